@@ -232,6 +232,10 @@ int upload_model(tmd_ctx *ctx)
   // table as float4 [n][k]
   std::vector<float> tabf(m.tab.size());
   for (size_t i = 0; i < tabf.size(); i++) tabf[i] = (float) m.tab[i];
+  // the end cells contribute nothing (ration.hpp:29): zero rows give H = dH/dr = 0
+  const size_t trow = (size_t) m.k * 4;
+  for (int n : {0, m.tab_n - 2, m.tab_n - 1})
+    if (n >= 0) std::fill_n(tabf.begin() + (size_t) n * trow, trow, 0.0f);
   hipError_t e = ctx->tab.ensure(tabf.size() * 4);
   if (e != hipSuccess) return hip_fail(ctx, e, "table alloc");
   e = hipMemcpy(ctx->tab.p, tabf.data(), tabf.size() * 4, hipMemcpyHostToDevice);

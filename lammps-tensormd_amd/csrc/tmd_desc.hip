@@ -1,23 +1,35 @@
-// Fused descriptor and force/virial kernels (gfx950, wave64).
+// Fused descriptor and force/virial kernels (gfx950, wave64), max_moment 0-3.
 //
-// One wavefront owns one atom.
-//  1. Sweep the atom's neighbor list (cutoff rc+skin) in chunks of 64: each
-//     lane forms one FP64 displacement, keeps 1e-10 < r^2 < rc^2
-//     (gpu/cuda/kernel.cu:1163) and finds the element slot b
-//     (tensormd.cpp:165-176).  Kept entries are compacted into LDS sorted
-//     by slot (ballot prefix counts), so later passes run on full lanes.
-//  2. For each chunk of 32 kept neighbors (two lanes per neighbor; 4 or 8
-//     for a short last chunk): geometry u = d/r (FP32 from FP64),
-//     monomials M_d(u), the Kerley-interpolated radial values H_k(r)
-//     (gpu/cuda/ration.cu:13-71) with lanes over (neighbor, filter), then
-//     P[b][k][d] += H_k M_d accumulated in registers: each lane owns a
-//     KT x DT block of (k, d) for every slot.
-//  3. Descriptor: G[b][k][m] = sum_d T[m][d] P^2 (m >= 1), G[b][k][0] = P0
-//     (= sign(P0) sqrt(P0^2), kernel.cu:1028-1061).
-//     Force: S = P * (2 sum_m T[m][d] g'_m), g'_0 = g_0/(2 G_0) guarded at
-//     1e-8 (kernel.cu:730-817); per neighbor U_k = S M, V_d = S H,
-//     F = scale (sum_k U_k H'_k) u + scale V . dM/dd (kernel.cu:559-646,
-//     :869-965); f_i += F, f_j -= F, virial -d (x) F (kernel.cu:1714-1758).
+// One wavefront owns one atom.  The moments are carried in 16 real spherical
+// harmonics Y_d(u) of degree 0..3 instead of the 20 monomials of the
+// reference: on unit vectors the two span the same space, and with the
+// normalisation of harmonics() the reference's tensor contractions are
+//   G_0 = P_0                         G_1 = sum_{l=1} P_d^2
+//   G_2 = P_0^2 / 3 + sum_{l=2} P_d^2     G_3 = 3/5 G_1 + sum_{l=3} P_d^2
+// (cos^2 and cos^3 in Legendre polynomials and the addition theorem; a
+// T-symmetric model drops the P_0^2 / 3 and 3/5 G_1 terms), where
+// P[b][k][d] = sum over the neighbors c of slot b of H_k(r_c) Y_d(u_c).
+//  1. Descriptor: sweep the atom's list (cutoff rc+skin) in chunks of 64,
+//     keep 1e-10 < r^2 < rc^2 (gpu/cuda/kernel.cu:1163), find the element
+//     slot b (tensormd.cpp:165-176) and compact the kept entries sorted by
+//     slot (ballot prefix counts).  The force kernel reuses that list.
+//  2. Staging: one lane per kept neighbor forms the FP64 geometry and writes
+//     a row of LDS: its harmonics, and the radial-table cell and offsets.
+//  3. Radial functions: 4 adjacent lanes per neighbor, 16 neighbors at a
+//     time; for each of a lane's filters the 4 lanes read 64 contiguous
+//     bytes of the table row (Kerley interpolation, gpu/cuda/ration.cu:13-71).
+//     H goes through LDS into the operand layouts of the matrix cores.
+//  4. P = Y^T H on v_mfma_f32_16x16x4_f32: 16 harmonics x 16 filters per
+//     tile, 4 neighbors per instruction.
+//     Force, slot by slot: S = dE/dP from P and dE/dG (kernel.cu:730-817),
+//     then per tile of 16 neighbors U = S Y and V = S^T H on the matrix
+//     cores, F = scale (sum_k U_k H'_k) u + scale V . dY/dd
+//     (kernel.cu:559-646, :869-965); f_i += F, f_j -= F, virial -d (x) F
+//     (kernel.cu:1714-1758), one lane per neighbor.
+//
+// MFMA operand layout (16x16x4): lane l holds A[l % 16][l / 16] and
+// B[l / 16][l % 16]; accumulator element i of lane l is
+// D[4 (l / 16) + i][l % 16].
 //
 // Nothing per neighbor is stored in HBM: the reference materialises R, M,
 // H, dH/dr, P, dE/dS, V, F1, F2 per padded slot (kernel.cu:1545-1582).
@@ -27,67 +39,258 @@ namespace tmd {
 
 namespace {
 
-constexpr int kMS = 24;  // LDS stride of a monomial row (16-byte aligned)
+typedef float f32x4v __attribute__((ext_vector_type(4)));
 
-constexpr int kChunkRows = 32;  // neighbors staged at a time
+constexpr int kNY = 16;  // harmonics of degree 0..3: degree l starts at l^2
+// LDS row of a staged neighbor: 16 harmonics, then q, dx - q and the table
+// cell.  A stride of 20 words puts the 16-byte accesses of 16 rows on
+// distinct banks.
+constexpr int kRow = 20;
 
+// Filters are taken in blocks of FBL (all of them up to K = 32, else 32).
 template <int K>
 struct Tiling {
-  // each lane owns KT filters x DT monomials of every slot
-  static constexpr int KT = K == 16 ? 1 : (K <= 32 ? 2 : (K == 64 ? 4 : 8));
-  static constexpr int DT = (K == 24) ? 4 : 5;
-  static constexpr int NDG = kND / DT;
-  static constexpr int LANES = (K / KT) * NDG;  // 60 or 64
-  // H and dH: [half][kChunk][HS] with the filters of a half in a row of odd
-  // stride HS = K/2 + 1: the 64 lanes of a neighbor pass (32 rows x 2 halves)
-  // hit 64 distinct banks
-  static constexpr int KH = K / 2;
-  static constexpr int HS = KH + 1;
-  static constexpr int HALF = kChunkRows * HS;  // floats per half
-  // S rows of one slot, padded so that slots b and b + 2 start on different banks
-  static constexpr int SSTR = K * kND + 4;
-  // LDS offset of filter k of row c
-  __host__ __device__ static constexpr int hidx(int c, int k)
-  {
-    return (k >= KH ? HALF + k - KH : k) + c * HS;
+  static constexpr int FBL = K <= 32 ? K : 32;
+  static constexpr int NFB = FBL / 4;          // filters of a block per lane
+  static constexpr int NB = K / FBL;           // blocks
+  static constexpr int CT = (FBL + 15) / 16;   // filter tiles per block
+  static constexpr int KT = NB * CT;           // filter tiles
+  // the second tile of K = 24 holds 8 filters, the others 16
+  static constexpr int nper(int t) { return (K == 24 && t == 1) ? 2 : 4; }  // filters per lane group
+  // H of 16 neighbors, [16][HS]: HS / 4 is odd, so the quads of 16 rows hit
+  // distinct banks
+  static constexpr int HS = FBL + 4;
+  static constexpr int SS = kRow;              // stride of an S row
+  // S is kept in registers per slot up to K = 32, and its LDS then overlays H
+  static constexpr bool kSRegs = K <= 32;
+  static constexpr int HBUF = 16 * HS + 4;     // floats (the last tile of K = 24 reads past row 15)
+  static constexpr int SBUF = K * SS;
+  static constexpr int BUF = kSRegs ? (HBUF > SBUF ? HBUF : SBUF) : HBUF + SBUF;
+  // staged neighbors of the force kernel: what leaves 16 waves per CU
+  // (10 KB each) up to K = 32, 13 at K = 64 and 9 at K = 128
+  static constexpr int WIN = K < 32 ? 96 : (K == 32 ? 88 : 64);
+  // tiles of a slot whose H and dH stay in registers between P and the
+  // chain rule (2 NFB registers each)
+  static constexpr int RT = K == 16 ? 5 : (K == 24 ? 2 : (K == 32 ? 2 : 0));
+};
+
+// Y_d(u) in d order: 1 | x y z | 5 of degree 2 | 7 of degree 3, scaled so
+// that the sums of squares above hold.
+__device__ inline void harmonics(float x, float y, float z, float *Y)
+{
+  constexpr float r2 = 1.4142135623730951f, r6 = 2.4494897427831781f;
+  const float zz = z * z, xy = x * y, xxyy = (x - y) * (x + y);
+  Y[0] = 1.0f;
+  Y[1] = x;
+  Y[2] = y;
+  Y[3] = z;
+  Y[4] = fmaf(1.2247448713915890f, zz, -0.40824829046386302f);  // (3 z^2 - 1) / sqrt 6
+  Y[5] = r2 * x * z;
+  Y[6] = r2 * y * z;
+  Y[7] = 0.70710678118654752f * xxyy;
+  Y[8] = r2 * xy;
+  Y[9] = z * fmaf(1.5811388300841898f, zz, -0.94868329805051381f);  // z (5 z^2 - 3) / sqrt 10
+  const float p = fmaf(1.9364916731037085f, zz, -0.38729833462074170f);  // sqrt(3/20) (5 z^2 - 1)
+  Y[10] = p * x;
+  Y[11] = p * y;
+  Y[12] = 0.5f * r6 * z * xxyy;
+  Y[13] = r6 * xy * z;
+  Y[14] = 0.5f * x * fmaf(x, x, -3.0f * y * y);
+  Y[15] = 0.5f * y * fmaf(3.0f * x, x, -y * y);
+}
+
+// g = sum_d V_d dY_d/du (the polynomials above as functions of a free u)
+__device__ inline void harmonics_grad(float x, float y, float z, const float *V, float &gx, float &gy, float &gz)
+{
+  constexpr float r2 = 1.4142135623730951f, r6 = 2.4494897427831781f, a10 = 3.8729833462074170f;
+  const float zz = z * z, xxyy = (x - y) * (x + y);
+  const float p = fmaf(1.9364916731037085f, zz, -0.38729833462074170f);
+  const float x2 = r2 * x, y2 = r2 * y, z2 = r2 * z, x6 = r6 * x, y6 = r6 * y, z6 = r6 * z;
+  const float d14 = 1.5f * xxyy, xy3 = 3.0f * x * y;
+  gx = V[1] + z2 * V[5] + x2 * V[7] + y2 * V[8] + p * V[10] + x6 * z * V[12] + y6 * z * V[13] + d14 * V[14] +
+      xy3 * V[15];
+  gy = V[2] + z2 * V[6] - y2 * V[7] + x2 * V[8] + p * V[11] - y6 * z * V[12] + x6 * z * V[13] - xy3 * V[14] +
+      d14 * V[15];
+  gz = V[3] + z6 * V[4] + x2 * V[5] + y2 * V[6] + fmaf(4.7434164902525694f, zz, -0.94868329805051381f) * V[9] +
+      a10 * z * (x * V[10] + y * V[11]) + 0.5f * r6 * xxyy * V[12] + x6 * y * V[13];
+}
+
+// a's lanes 0-31 + 32-63 in lanes 0-31, b's in lanes 32-63
+__device__ inline float swap32_add(float a, float b)
+{
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+// rows of 16 lanes: row 0 of the result = a's rows 0 + 1, row 1 = b's rows
+// 0 + 1, row 2 = a's rows 2 + 3, row 3 = b's rows 2 + 3
+__device__ inline float swap16_add(float a, float b)
+{
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+__device__ inline double make_d(unsigned lo, unsigned hi)
+{
+  return __longlong_as_double((long long) (((unsigned long long) hi << 32) | lo));
+}
+
+__device__ inline double swap32_add(double a, double b)
+{
+  const unsigned long long ua = (unsigned long long) __double_as_longlong(a), ub = (unsigned long long) __double_as_longlong(b);
+  const auto l = __builtin_amdgcn_permlane32_swap((unsigned) ua, (unsigned) ub, false, false);
+  const auto h = __builtin_amdgcn_permlane32_swap((unsigned) (ua >> 32), (unsigned) (ub >> 32), false, false);
+  return make_d(l[0], h[0]) + make_d(l[1], h[1]);
+}
+
+__device__ inline double swap16_add(double a, double b)
+{
+  const unsigned long long ua = (unsigned long long) __double_as_longlong(a), ub = (unsigned long long) __double_as_longlong(b);
+  const auto l = __builtin_amdgcn_permlane16_swap((unsigned) ua, (unsigned) ub, false, false);
+  const auto h = __builtin_amdgcn_permlane16_swap((unsigned) (ua >> 32), (unsigned) (ub >> 32), false, false);
+  return make_d(l[0], h[0]) + make_d(l[1], h[1]);
+}
+
+// Orders LDS accesses of the workgroup's only wave: its LDS instructions run
+// in order, so the compiler must keep the order and nothing has to be waited
+// for.
+__device__ inline void wave_sync()
+{
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+__device__ inline double row_sum_d(double v)
+{
+  v += dpp_d<kDppXor1>(v);
+  v += dpp_d<kDppXor2>(v);
+  v += dpp_d<kDppRor4>(v);
+  v += dpp_d<kDppRor8>(v);
+  return v;
+}
+
+// rows[c] of the n entries list[0..n)
+__device__ inline void stage(const ModelGeo &g, const Box &cell, const double4 &xi, const double4 *pos,
+                             const uint32_t *list, int n, float *rows)
+{
+  for (int c = threadIdx.x & 63; c < n; c += 64) {
+    NbrGeo ng;
+    nbr_geometry(g, cell, xi, pos, list[c], ng);
+    float Y[kNY];
+    harmonics(ng.ux, ng.uy, ng.uz, Y);
+    float4 *r = reinterpret_cast<float4 *>(rows + c * kRow);
+#pragma unroll
+    for (int q = 0; q < 4; q++) r[q] = make_float4(Y[4 * q], Y[4 * q + 1], Y[4 * q + 2], Y[4 * q + 3]);
+    // a table of one point has no cell: its only row is an end row
+    r[4] = make_float4(ng.q, ng.pq, __int_as_float(max(ng.n, 0)), 0.0f);
   }
-};
-
-// T[m][d] of a max_moment-3 descriptor (kDeg, kMult, plus the T-symmetric
-// extras T[2][0] = -1/3, T[3][1..3] = -3/5) for a lane-dependent d.
-__device__ inline float t_entry(int m, int d, int tsym)
-{
-  constexpr unsigned long long kMultBits = [] {
-    unsigned long long b = 0;
-    for (int i = 0; i < kND; i++) b |= (unsigned long long) kMult[i] << (3 * i);
-    return b;
-  }();
-  const int deg = d >= 10 ? 3 : (d >= 4 ? 2 : (d >= 1 ? 1 : 0));
-  float t = deg == m ? (float) ((kMultBits >> (3 * d)) & 7ull) : 0.0f;
-  if (tsym && m == 2 && d == 0) t = (float) (-1.0 / 3.0);
-  if (tsym && m == 3 && d >= 1 && d <= 3) t = (float) (-3.0 / 5.0);
-  return t;
+  wave_sync();
 }
 
-// True when monomials [d0, d0 + n) include one of degree m.
-__host__ __device__ constexpr bool group_has_degree(int d0, int n, int m)
+// Radial functions (and derivatives) of one block of filters for the tile of
+// neighbors rows[0..live), live >= 1: lane l holds the filters 4 i + l % 4
+// of neighbor l / 4.  The table's end cells are zero rows, and a lane past
+// the tile takes row 0: H = dH = 0 there without a mask.
+template <int K, bool DH>
+__device__ inline void radial_tile(const ModelGeo &g, const float4 *tab, const float *rows, int live,
+                                   int block, float *h, float *dh)
 {
-  for (int d = d0; d < d0 + n && d < kND; d++)
-    if (kDeg[d] == m) return true;
-  return false;
+  using T = Tiling<K>;
+  const int lane = threadIdx.x & 63, c = lane >> 2;
+  const float4 o = *reinterpret_cast<const float4 *>(rows + min(c, live - 1) * kRow + kNY);
+  const int n = c < live ? __float_as_int(o.z) : 0;
+  const float4 *row = tab + (size_t) n * K + block * T::FBL + (lane & 3);
+  float4 t[T::NFB];
+#pragma unroll
+  for (int i = 0; i < T::NFB; i++) t[i] = row[4 * i];
+#pragma unroll
+  for (int i = 0; i < T::NFB; i++) {
+    if constexpr (DH)
+      kerley(t[i], o.x, o.y, o.x - o.y, g.dxf, h[i], dh[i]);
+    else
+      h[i] = kerley_h(t[i], o.x, o.y);
+  }
 }
 
-constexpr int kChunk = kChunkRows;
-
-struct LDSMap {
-  uint32_t *kept;  // [cap] compacted, slot-sorted neighbor entries
-  float *M;        // [kChunk][kMS] monomials of the staged chunk
-  float *H;        // [2 halves][kChunk][HS] radial functions of the staged chunk
-};
-
-// descriptor LDS: kept list, monomials, radial functions
+// a block's values of the tile -> hb [16][HS]
 template <int K>
-__host__ __device__ inline size_t lds_layout(int cap, size_t *offs)
+__device__ inline void put_tile(const float *h, float *hb)
+{
+  using T = Tiling<K>;
+  const int lane = threadIdx.x & 63;
+  float *p = hb + (lane >> 2) * T::HS + (lane & 3);
+#pragma unroll
+  for (int i = 0; i < T::NFB; i++) p[4 * i] = h[i];
+}
+
+// the values of neighbor l % 16 in the chain-rule layout: lane group l / 16
+// holds nper(t) consecutive filters of tile t
+template <int K>
+__device__ inline void get_chain(const float *hb, float *h)
+{
+  using T = Tiling<K>;
+  const int lane = threadIdx.x & 63;
+  const float *p = hb + (lane & 15) * T::HS;
+#pragma unroll
+  for (int t = 0; t < T::CT; t++) {
+    if constexpr (K == 24) {
+      if (t == 1) {
+        const float2 v = *reinterpret_cast<const float2 *>(p + 16 + 2 * (lane >> 4));
+        h[4] = v.x;
+        h[5] = v.y;
+        continue;
+      }
+    }
+    const float4 v = *reinterpret_cast<const float4 *>(p + 16 * t + 4 * (lane >> 4));
+    h[4 * t] = v.x;
+    h[4 * t + 1] = v.y;
+    h[4 * t + 2] = v.z;
+    h[4 * t + 3] = v.w;
+  }
+}
+
+// P of a block's filters += the tile in rows[0..live) with H in hb:
+// P^T[d][k] of tile t in acc[t].  Rows past the tile hold H = 0.
+template <int K>
+__device__ inline void moments_tile(const float *rows, int live, const float *hb, f32x4v *acc)
+{
+  using T = Tiling<K>;
+  const int lane = threadIdx.x & 63;
+  float a[4], b[4][T::CT];
+#pragma unroll
+  for (int s = 0; s < 4; s++) {
+    const int c = 4 * s + (lane >> 4);
+    a[s] = rows[min(c, live - 1) * kRow + (lane & 15)];
+#pragma unroll
+    for (int t = 0; t < T::CT; t++) b[s][t] = hb[c * T::HS + 16 * t + (lane & 15)];
+  }
+#pragma unroll
+  for (int s = 0; s < 4; s++) {
+    if (4 * s >= live) break;
+#pragma unroll
+    for (int t = 0; t < T::CT; t++) acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[s], b[s][t], acc[t], 0, 0, 0);
+  }
+}
+
+// G[b][k][0..3] of one filter tile from its P^T: lane group m ends up with
+// component m of filter l % 16 (fixed-order sums over the groups).
+__device__ inline float g_components(const f32x4v &p, int tsym)
+{
+  const int grp = (threadIdx.x & 63) >> 4;
+  const float a = p[0] * p[0], b = p[1] * p[1] + p[2] * p[2] + p[3] * p[3];
+  const float c2 = tsym ? 0.0f : (1.0f / 3.0f), c3 = tsym ? 0.0f : 0.6f;
+  // degrees of a group's harmonics: 0 111 | 2222 | 2 333 | 3333
+  const float t0 = grp == 0 ? p[0] : 0.0f;
+  const float t1 = grp == 0 ? b : 0.0f;
+  const float t2 = grp == 0 ? c2 * a : (grp == 1 ? a + b : (grp == 2 ? a : 0.0f));
+  const float t3 = grp == 0 ? c3 * b : (grp == 1 ? 0.0f : (grp == 2 ? b : a + b));
+  return swap16_add(swap32_add(t0, t2), swap32_add(t1, t3));
+}
+
+// descriptor LDS: kept list, staged rows, H
+constexpr int kDescWin = 96;
+template <int K>
+__host__ __device__ inline size_t desc_lds(int cap, size_t *offs)
 {
   size_t o = 0;
   auto take = [&](size_t bytes) {
@@ -96,221 +299,81 @@ __host__ __device__ inline size_t lds_layout(int cap, size_t *offs)
     return r;
   };
   offs[0] = take((size_t) cap * 4);
-  offs[1] = take((size_t) kChunk * kMS * 4);
-  offs[2] = take((size_t) 2 * Tiling<K>::HALF * 4);
+  offs[1] = take((size_t) kDescWin * kRow * 4);
+  offs[2] = take((size_t) Tiling<K>::HBUF * 4);
   return o;
 }
 
-// force LDS: the staging area (monomials, radial functions), then P and S
-// of every slot [nelt][SSTR] at offs[0]: over the staging area when P is
-// built in one pass, after it when it takes several (the staging area is
-// still in use while the first passes' P is stored).  The kept list stays
-// in HBM.
-template <int K>
-__host__ __device__ inline size_t force_lds_layout(int nelt, bool multipass, size_t *offs)
-{
-  const size_t mreg = (size_t) kChunk * kMS * 4;
-  const size_t hreg = (size_t) 2 * Tiling<K>::HALF * 4;
-  const size_t preg = (size_t) nelt * Tiling<K>::SSTR * 4;
-  offs[1] = 0;
-  offs[2] = mreg;
-  if (multipass) {
-    offs[0] = (mreg + hreg + 15) & ~(size_t) 15;
-    return offs[0] + preg;
-  }
-  offs[0] = 0;
-  return mreg + hreg > preg ? mreg + hreg : preg;
-}
-
-template <int K>
-__device__ inline LDSMap carve(unsigned char *base, int cap)
-{
-  size_t offs[3];
-  lds_layout<K>(cap, offs);
-  LDSMap L;
-  L.kept = (uint32_t *) (base + offs[0]);
-  L.M = (float *) (base + offs[1]);
-  L.H = (float *) (base + offs[2]);
-  return L;
-}
-
-// Lanes per neighbor in the chain-rule pass: one lane per neighbor (a chunk
-// of 64) while more than 48 remain, then as lanes_per_nbr.  One wide chunk
-// runs the per-neighbor set-up and the force scatter once instead of twice.
-__device__ inline int chain_lanes(int rem) { return rem > 48 ? 1 : lanes_per_nbr(rem); }
-
-// table loads in flight per lane: divides K/2, K/4 and K/8
-template <int K>
-constexpr int kTabBatch = ((K / 8) % 4 == 0) ? 4 : K / 8;
-
-// Phase 2 staging of kept neighbors [base, base + 64/Lp) for the P
-// accumulation: Lp adjacent lanes per neighbor.  Each computes the
-// neighbor's geometry and interpolates K/Lp of the filters from the table
-// row of the neighbor's cell (immediate-offset loads, no per-element index
-// arithmetic).  Writes the monomials (M) and H to LDS.
-template <int K>
-__device__ inline void stage(const ModelGeo &g, const Box &cell, const double4 &xi,
-                             const double4 *pos, const float4 *tab, int base, int nk, int Lp,
-                             LDSMap &L)
-{
-  static_assert(kChunk == 32, "at most 32 neighbors staged at a time");
-  using T = Tiling<K>;
-  const int lane = threadIdx.x & 63;
-  const int c = lane / Lp, part = lane - c * Lp;
-  const int KL = K / Lp;
-  if (base + c < nk) {
-    NbrGeo ng;
-    nbr_geometry(g, cell, xi, pos, L.kept[base + c], ng);
-    if (part == 0) {
-      float M[kND];
-      monomials20(ng.ux, ng.uy, ng.uz, M);
-      float4 *Mr = reinterpret_cast<float4 *>(L.M + c * kMS);
-#pragma unroll
-      for (int q4 = 0; q4 < kND / 4; q4++)
-        Mr[q4] = make_float4(M[4 * q4], M[4 * q4 + 1], M[4 * q4 + 2], M[4 * q4 + 3]);
-    }
-    // the lane's filters lie in one half of the H layout (K/Lp divides K/2)
-    float *Hc = L.H + T::hidx(c, part * KL);
-    constexpr int B = kTabBatch<K>;
-    if (table_cell_live(g, ng.n)) {
-      const float4 *row = tab + (size_t) ng.n * K + part * KL;
-      // six rows per wait where they divide the lane's filters: the staging
-      // is latency-bound, and each wait covering more loads cuts the
-      // descriptor and the P rebuild by 7-8 % at K = 24 (twelve rows raise
-      // the descriptor to 143 VGPRs and lose)
-      constexpr int B6 = (K / 2) % 6 == 0 ? 6 : B;
-      if (KL % B6 == 0) {
-        for (int k0 = 0; k0 < KL; k0 += B6) {
-          float4 t[B6];
-#pragma unroll
-          for (int u = 0; u < B6; u++) t[u] = row[k0 + u];
-#pragma unroll
-          for (int u = 0; u < B6; u++) Hc[k0 + u] = kerley_h(t[u], ng.q, ng.pq);
-        }
-      } else {
-        for (int k0 = 0; k0 < KL; k0 += B) {
-          float4 t[B];
-#pragma unroll
-          for (int u = 0; u < B; u++) t[u] = row[k0 + u];
-#pragma unroll
-          for (int u = 0; u < B; u++) Hc[k0 + u] = kerley_h(t[u], ng.q, ng.pq);
-        }
-      }
-    } else {
-      for (int k = 0; k < KL; k++) Hc[k] = 0.0f;
-    }
-  }
-  __syncthreads();
-}
-
-// Phase 2 accumulation over the staged chunk into the lane's register block.
-// The pass covers nsl slots whose kept entries start at start[0..nsl]; slot
-// b of the pass accumulates into acc[b].
+// P of the nsl slots of one pass over the kept entries kept[start[0],
+// start[nsl]) (slot-sorted), then G.  Tiles of 16 neighbors run across slot
+// boundaries: each slot takes its own neighbors of a tile by zeroing the
+// harmonics of the others.
 template <int K, int NS>
-__device__ inline void accumulate(const LDSMap &L, const int *start, int nsl, int base,
-                                  float (*acc)[Tiling<K>::KT][Tiling<K>::DT])
+__device__ inline void descriptor_pass(const ModelGeo &g, const Box &cell, const double4 &xi, const double4 *pos,
+                                       const float4 *tab, const uint32_t *kept, const int *start, int nsl,
+                                       float *rows, float *hb, float *Grow, int b0, bool gbf16)
 {
   using T = Tiling<K>;
   const int lane = threadIdx.x & 63;
-  if (lane >= T::LANES) return;
-  const int kq = lane / T::NDG, dq = lane - (lane / T::NDG) * T::NDG;
-  const float *Hb = L.H + T::hidx(0, kq * T::KT);  // KT divides K/2: a lane's filters share a half
-  const float *Mb = L.M + dq * T::DT;
-#pragma unroll
-  for (int b = 0; b < NS; b++) {
-    if (b >= nsl) break;
-    int c0 = max(start[b] - base, 0), c1 = min(start[b + 1] - base, kChunk);
-#pragma unroll 4
-    for (int c = c0; c < c1; c++) {
-      float h[T::KT], m[T::DT];
-#pragma unroll
-      for (int a = 0; a < T::KT; a++) h[a] = Hb[c * T::HS + a];
-#pragma unroll
-      for (int q = 0; q < T::DT; q++) m[q] = Mb[c * kMS + q];
-#pragma unroll
-      for (int a = 0; a < T::KT; a++)
-#pragma unroll
-        for (int q = 0; q < T::DT; q++) acc[b][a][q] += h[a] * m[q];
-    }
-  }
-}
-
-// Phase 2: P of the nsl slots of one pass in the lane's register block, over
-// the kept entries L.kept[start[0], start[nsl]) (the list is slot-sorted, so
-// a pass stages only its own slots' neighbors).
-template <int K, int NS>
-__device__ inline void accumulate_P(const ModelGeo &g, const Box &cell, const double4 &xi,
-                                    const double4 *pos, const float4 *tab, LDSMap &L,
-                                    const int *start, int nsl,
-                                    float (*acc)[Tiling<K>::KT][Tiling<K>::DT])
-{
-  using T = Tiling<K>;
+  f32x4v acc[NS][T::KT];
 #pragma unroll
   for (int b = 0; b < NS; b++)
 #pragma unroll
-    for (int a = 0; a < T::KT; a++)
-#pragma unroll
-      for (int q = 0; q < T::DT; q++) acc[b][a][q] = 0.0f;
+    for (int t = 0; t < T::KT; t++) acc[b][t] = f32x4v{0, 0, 0, 0};
   const int end = start[nsl];
-  for (int base = start[0]; base < end;) {
-    const int Lp = lanes_per_nbr(end - base);
-    stage<K>(g, cell, xi, pos, tab, base, end, Lp, L);
-    accumulate<K, NS>(L, start, nsl, base, acc);
-    __syncthreads();
-    base += 64 / Lp;
+  for (int w0 = start[0]; w0 < end; w0 += kDescWin) {
+    const int nw = min(kDescWin, end - w0);
+    stage(g, cell, xi, pos, kept + w0, nw, rows);
+    for (int r0 = 0; r0 < nw; r0 += 16) {
+      const int live = min(16, nw - r0);
+      const float *rt = rows + r0 * kRow;
+#pragma unroll
+      for (int fb = 0; fb < T::NB; fb++) {
+        float h[T::NFB];
+        radial_tile<K, false>(g, tab, rt, live, fb, h, nullptr);
+        put_tile<K>(h, hb);
+        wave_sync();
+        float a[4], bo[4][T::CT];
+#pragma unroll
+        for (int s = 0; s < 4; s++) {
+          const int c = 4 * s + (lane >> 4);
+          a[s] = rt[min(c, live - 1) * kRow + (lane & 15)];
+#pragma unroll
+          for (int t = 0; t < T::CT; t++) bo[s][t] = hb[c * T::HS + 16 * t + (lane & 15)];
+        }
+#pragma unroll
+        for (int b = 0; b < NS; b++) {
+          if (b >= nsl) break;
+          const int lo = max(start[b] - w0 - r0, 0), hi = min(start[b + 1] - w0 - r0, live);
+          if (lo >= hi) continue;
+#pragma unroll
+          for (int s = 0; s < 4; s++) {
+            if (4 * s >= hi || 4 * s + 4 <= lo) continue;
+            const int c = 4 * s + (lane >> 4);
+            const float as = (c >= lo && c < hi) ? a[s] : 0.0f;
+#pragma unroll
+            for (int t = 0; t < T::CT; t++)
+              acc[b][fb * T::CT + t] =
+                  __builtin_amdgcn_mfma_f32_16x16x4f32(as, bo[s][t], acc[b][fb * T::CT + t], 0, 0, 0);
+          }
+        }
+        wave_sync();
+      }
+    }
   }
-}
-
-typedef float f32x4v __attribute__((ext_vector_type(4)));
-typedef __bf16 bf16x4v __attribute__((ext_vector_type(4)));
-
-// G[b0 + b][k][m] = sum_d T[m][d] P^2 (m >= 1) for the nsl slots of a pass:
-// partial sums over the lane's d block, then a sum over the NDG lanes that
-// share k; G[b][k][0] = P0 (= sign(P0) sqrt(P0^2)), held by the dq == 0 lane.
-// gbf16: the row is stored as BF16 (round to nearest even).
-template <int K, int NS>
-__device__ inline void write_G(const ModelGeo &g, float (*acc)[Tiling<K>::KT][Tiling<K>::DT],
-                               float *Grow, int b0, int nsl, bool gbf16)
-{
-  using T = Tiling<K>;
-  const int lane = threadIdx.x & 63;
-  const int kq = lane / T::NDG, dq = lane - (lane / T::NDG) * T::NDG;
-  const int gbase = kq * T::NDG;
-  float tc[kNM][T::DT];
-#pragma unroll
-  for (int m = 1; m < kNM; m++)
-#pragma unroll
-    for (int q = 0; q < T::DT; q++) tc[m][q] = t_entry(m, dq * T::DT + q, g.tsym);
 #pragma unroll
   for (int b = 0; b < NS; b++) {
     if (b >= nsl) break;
 #pragma unroll
-    for (int a = 0; a < T::KT; a++) {
-      float part[kNM] = {0, 0, 0, 0};
-#pragma unroll
-      for (int q = 0; q < T::DT; q++) {
-        float p2 = acc[b][a][q] * acc[b][a][q];
-#pragma unroll
-        for (int m = 1; m < kNM; m++) part[m] += tc[m][q] * p2;
-      }
-      // sum over the NDG lanes of the filter: only the d groups that hold a
-      // monomial of degree m add to G_m (the others' partial sums are exact
-      // zeros; the T-symmetric extras are in the d group 0, the lane itself)
-      float tot[kNM] = {0, part[1], part[2], part[3]};
-#pragma unroll
-      for (int t = 1; t < T::NDG; t++)
-#pragma unroll
-        for (int m = 1; m < kNM; m++)
-          if (group_has_degree(t * T::DT, T::DT, m)) tot[m] += __shfl(part[m], gbase + t);
-      if (lane < T::LANES && dq == 0) {
-        const int k = kq * T::KT + a;
-        const size_t o = ((size_t) (b0 + b) * K + k) * kNM;
-        if (gbf16) {
-          const f32x4v xv = {acc[b][a][0], tot[1], tot[2], tot[3]};
-          *reinterpret_cast<bf16x4v *>(reinterpret_cast<uint16_t *>(Grow) + o) = __builtin_convertvector(xv, bf16x4v);
-        } else {
-          *reinterpret_cast<float4 *>(Grow + o) = make_float4(acc[b][a][0], tot[1], tot[2], tot[3]);
-        }
+    for (int t = 0; t < T::KT; t++) {
+      const float v = g_components(acc[b][t], g.tsym);
+      const int k = 16 * t + (lane & 15);
+      if (k < K) {
+        const size_t o = ((size_t) (b0 + b) * K + k) * kNM + (lane >> 4);
+        if (gbf16)
+          reinterpret_cast<__bf16 *>(Grow)[o] = (__bf16) v;
+        else
+          Grow[o] = v;
       }
     }
   }
@@ -339,308 +402,347 @@ __global__ __launch_bounds__(64) void k_descriptor(ModelGeo g, Geom geo, const d
     for (int e = lane; e < nw; e += 64) Grow[e] = 0.0f;
     return;
   }
-  using T = Tiling<K>;
-  LDSMap L = carve<K>(smem, cap);
+  size_t offs[3];
+  desc_lds<K>(cap, offs);
+  uint32_t *kept = reinterpret_cast<uint32_t *>(smem + offs[0]);
+  float *rows = reinterpret_cast<float *>(smem + offs[1]);
+  float *hb = reinterpret_cast<float *>(smem + offs[2]);
   int start[kMaxElts + 1];
   const double4 xi = pos[i];
   const Box cell = load_box(geo, i);
   // phase 1: compaction
-  const int nk = compact(g, cell, xi, (int) xi.w, nbr + (size_t) i * cap, nn[i], pos, L.kept, start);
-  __syncthreads();
+  const int nk = compact(g, cell, xi, (int) xi.w, nbr + (size_t) i * cap, nn[i], pos, kept, start);
+  wave_sync();
   // the row's kept list with its slot starts, for the force kernel
-  auto write_kept = [&]() {
-    uint32_t *kr = kl + (size_t) row * kept_cache_words(cap);
-    if (lane == 0) {
-      kr[0] = (uint32_t) nk;
-      for (int b = 0; b <= g.nelt; b++) kr[1 + b] = (uint32_t) start[b];
-    }
-    for (int e = lane; e < nk; e += 64) kr[kKeptHdr + e] = L.kept[e];
-  };
+  uint32_t *kr = kl + (size_t) row * kept_cache_words(cap);
+  if (lane == 0) {
+    kr[0] = (uint32_t) nk;
+    for (int b = 0; b <= g.nelt; b++) kr[1 + b] = (uint32_t) start[b];
+  }
+  for (int e = lane; e < nk; e += 64) kr[kKeptHdr + e] = kept[e];
   if constexpr (!MP) {
-    float acc[NS][T::KT][T::DT];
-    accumulate_P<K, NS>(g, cell, xi, pos, tab, L, start, g.nelt, acc);
-    write_kept();
-    write_G<K, NS>(g, acc, Grow, 0, g.nelt, geo.g_bf16);
+    descriptor_pass<K, NS>(g, cell, xi, pos, tab, kept, start, g.nelt, rows, hb, Grow, 0, geo.g_bf16);
   } else {
     __shared__ int s_start[kMaxElts + 1];
     if (lane == 0)
       for (int b = 0; b <= g.nelt; b++) s_start[b] = start[b];
-    write_kept();
-    __syncthreads();
-    for (int b0 = 0; b0 < g.nelt; b0 += NS) {
-      const int nsl = min(NS, g.nelt - b0);
-      float acc[NS][T::KT][T::DT];
-      accumulate_P<K, NS>(g, cell, xi, pos, tab, L, s_start + b0, nsl, acc);
-      write_G<K, NS>(g, acc, Grow, b0, nsl, geo.g_bf16);
-    }
+    wave_sync();
+    for (int b0 = 0; b0 < g.nelt; b0 += NS)
+      descriptor_pass<K, NS>(g, cell, xi, pos, tab, kept, s_start + b0, min(NS, g.nelt - b0), rows, hb, Grow, b0,
+                             geo.g_bf16);
   }
 }
 
-// One chunk of the chain-rule pass: LP adjacent lanes per neighbor (neighbors
-// [base, base + 64/LP)), each over K/LP of the filters.  A lane recomputes
-// its neighbor's geometry and interpolates H and dH/dr of its filters in
-// registers, so the only LDS traffic is the broadcast read of S.  Adds the
-// neighbor forces to f_j (FP64 atomics) and to the atom's fi, wi.
-template <int K, int LP>
-__device__ inline void force_chunk(const ModelGeo &g, const Box &cell, const double4 &xi,
-                                   const double4 *pos, const float4 *tab, const float *PS,
-                                   const uint32_t *kept, const int *start, int base, int nk,
-                                   double scale, double *f, double *vatom, double *facc)
+// S = dE/dP of one slot from its P^T and dE/dG row (gslot[k][4]) -> sb
+// [k][SS]: S_0 = g_0 (dropped below |G_0| = 1e-8, kernel.cu:754-759)
+// + 2/3 g_2 P_0, S_d = 2 P_d (g_1 + 3/5 g_3 | g_2 | g_3) for degrees 1..3.
+template <int K>
+__device__ inline void slot_S(const f32x4v *p, const float4 *gv, int tsym, float *sb)
 {
   using T = Tiling<K>;
+  const int lane = threadIdx.x & 63, grp = lane >> 4;
+#pragma unroll
+  for (int t = 0; t < T::KT; t++) {
+    const float4 v = gv[t];
+    const float g2 = 2.0f * v.z, g3 = 2.0f * v.w;
+    const float g1 = tsym ? 2.0f * v.y : fmaf(0.6f, g3, 2.0f * v.y);
+    const float w0 = grp == 3 ? g3 : g2;                          // harmonic 4 grp (grp > 0)
+    const float w1 = grp == 0 ? g1 : (grp == 1 ? g2 : g3);        // the other three
+    const float g0 = fabsf(p[t][0]) < 1e-8f ? 0.0f : v.x;
+    const float s0 = tsym ? g0 : fmaf(p[t][0], g2 * (1.0f / 3.0f), g0);
+    const int k = 16 * t + (lane & 15);
+    if (k < K)
+      *reinterpret_cast<float4 *>(sb + k * T::SS + 4 * grp) =
+          make_float4(grp == 0 ? s0 : p[t][0] * w0, p[t][1] * w1, p[t][2] * w1, p[t][3] * w1);
+  }
+}
+
+// The S operands of one block for U (A[k][d], four MFMA steps of d = 4 g + s)
+// and V (A[d][k], one step per filter of a lane group).
+template <int K>
+struct SOps {
+  f32x4v u[Tiling<K>::CT];
+  float v[Tiling<K>::NFB];
+};
+
+template <int K>
+__device__ inline void load_S(const float *sb, int block, SOps<K> &o)
+{
+  using T = Tiling<K>;
+  const int lane = threadIdx.x & 63, r = lane & 15, grp = lane >> 4;
+  const float *s = sb + block * T::FBL * T::SS;
+#pragma unroll
+  for (int t = 0; t < T::CT; t++) {
+    // the U row r of the accumulator is the filter nper(t) (r / 4) + r % 4 of
+    // the tile (rows with r % 4 >= nper(t) repeat one and are not used)
+    const int np = T::nper(t);
+    const int f = 16 * t + (np == 4 ? r : 2 * (r >> 2) + (r & 1));
+    o.u[t] = *reinterpret_cast<const f32x4v *>(s + f * T::SS + 4 * grp);
+#pragma unroll
+    for (int i = 0; i < np; i++) o.v[4 * t + i] = s[(16 * t + np * grp + i) * T::SS + r];
+  }
+}
+
+// The chain rule of one block for a tile of neighbors (l % 16): f1 +=
+// sum_k U_k H'_k over the lane group's filters, v += V
+template <int K>
+__device__ inline void chain_block(const SOps<K> &o, const f32x4v &y, const float *h, const float *dh, float &f1,
+                                   f32x4v &v)
+{
+  using T = Tiling<K>;
+#pragma unroll
+  for (int t = 0; t < T::CT; t++) {
+    f32x4v u = {0, 0, 0, 0};
+#pragma unroll
+    for (int s = 0; s < 4; s++) u = __builtin_amdgcn_mfma_f32_16x16x4f32(o.u[t][s], y[s], u, 0, 0, 0);
+#pragma unroll
+    for (int i = 0; i < T::nper(t); i++)
+      v = __builtin_amdgcn_mfma_f32_16x16x4f32(o.v[4 * t + i], h[4 * t + i], v, 0, 0, 0);
+#pragma unroll
+    for (int i = 0; i < T::nper(t); i++) f1 = fmaf(u[i], dh[4 * t + i], f1);
+  }
+}
+
+// V and the lane group's f1 over the tile's harmonics and table offsets (the
+// tile needs them no more; neighbors past the tile belong to other slots)
+__device__ inline void put_V(float *rt, int live, float f1, const f32x4v &v)
+{
+  const int lane = threadIdx.x & 63, c = lane & 15, grp = lane >> 4;
+  if (c < live) {
+    *reinterpret_cast<f32x4v *>(rt + c * kRow + 4 * grp) = v;
+    rt[c * kRow + kNY + grp] = f1;
+  }
+}
+
+__device__ inline f32x4v get_Y(const float *rt, int live)
+{
   const int lane = threadIdx.x & 63;
-  const int c = lane / LP, sub = lane - c * LP;
-  constexpr int KL = K / LP;
-  {
-    const bool live = base + c < nk;
-    int b = 0;
-    while (b + 1 < g.nelt && base + c >= start[b + 1]) b++;
+  return *reinterpret_cast<const f32x4v *>(rt + min(lane & 15, live - 1) * kRow + 4 * (lane >> 4));
+}
+
+// The neighbor forces of list[0..n) from their V and f1 rows, one lane per
+// neighbor: f_j -= F (FP64 atomics); own force and virial summed over the
+// lanes in a fixed order into facc.
+__device__ inline void finish(const ModelGeo &g, const Box &cell, const double4 &xi, const double4 *pos,
+                              const uint32_t *list, int n, const float *rows, double scale, double *f,
+                              double *vatom, double *facc)
+{
+  const int lane = threadIdx.x & 63;
+  double cf[9];
+#pragma unroll
+  for (int q = 0; q < 9; q++) cf[q] = 0.0;
+  for (int c = lane; c < n; c += 64) {
     NbrGeo ng;
-    ng.ux = ng.uy = ng.uz = 0.0f;
-    ng.r = 1.0;
-    float V[kND];
+    nbr_geometry(g, cell, xi, pos, list[c], ng);
+    float V[kNY];
+    const float4 *r = reinterpret_cast<const float4 *>(rows + c * kRow);
 #pragma unroll
-    for (int q = 0; q < kND; q++) V[q] = 0.0f;
-    float f1 = 0.0f;
-    if (live) {
-      nbr_geometry(g, cell, xi, pos, kept[base + c], ng);
-      if (table_cell_live(g, ng.n)) {
-        float M[kND];
-        monomials20(ng.ux, ng.uy, ng.uz, M);
-        const float qp = ng.q - ng.pq;
-        const float4 *trow = tab + (size_t) ng.n * K + sub * KL;
-        const float *S = PS + (size_t) b * T::SSTR + sub * KL * kND;
-        // batches of B filters: load the table rows, interpolate H and dH/dr,
-        // then U_k = sum_d S_kd M_d (M_0 = 1), V_d += S_kd H_k (V_0 is not
-        // needed: dM_0/du = 0), f1 += U_k dH_k.  No software pipelining: four
-        // waves per SIMD hide the row latency, and a prefetch ring costs
-        // registers and copies (measured slower).  Six rows per batch where
-        // they divide the lane's filters (K = 24: 3 % faster than 3 or 8 rows;
-        // 12 rows spill), else the staging batch.
-        constexpr int B = KL % 6 == 0 ? 6 : kTabBatch<K>;
-#pragma unroll 1
-        for (int k0 = 0; k0 < KL; k0 += B) {
-          float4 t[B];
-#pragma unroll
-          for (int u = 0; u < B; u++) t[u] = trow[k0 + u];
-#pragma unroll
-          for (int u = 0; u < B; u++) {
-            float h, dh;
-            kerley(t[u], ng.q, ng.pq, qp, g.dxf, h, dh);
-            const float4 *Sk = reinterpret_cast<const float4 *>(S + (k0 + u) * kND);
-            float sv[kND];
-#pragma unroll
-            for (int q4 = 0; q4 < kND / 4; q4++) {
-              float4 v4 = Sk[q4];
-              sv[4 * q4] = v4.x;
-              sv[4 * q4 + 1] = v4.y;
-              sv[4 * q4 + 2] = v4.z;
-              sv[4 * q4 + 3] = v4.w;
-            }
-            float U = sv[0];
-#pragma unroll
-            for (int q = 1; q < kND; q++) U = fmaf(sv[q], M[q], U);
-#pragma unroll
-            for (int q = 1; q < kND; q++) V[q] = fmaf(sv[q], h, V[q]);
-            f1 = fmaf(U, dh, f1);
-          }
-        }
-      }
+    for (int q = 0; q < 4; q++) {
+      const float4 v = r[q];
+      V[4 * q] = v.x;
+      V[4 * q + 1] = v.y;
+      V[4 * q + 2] = v.z;
+      V[4 * q + 3] = v.w;
     }
-    // combine the Lp partial sums into the neighbor's first lane
-    if constexpr (LP >= 2) {
+    const float4 p = r[4];
+    const float f1 = (p.x + p.y) + (p.z + p.w);
+    const float x = ng.ux, y = ng.uy, z = ng.uz;
+    float gx, gy, gz;
+    harmonics_grad(x, y, z, V, gx, gy, gz);
+    const float gu = gx * x + gy * y + gz * z;
+    // 1-ulp hardware reciprocal (a division is a ten-instruction FP64 sequence)
+    const float rinv = __builtin_amdgcn_rcpf((float) ng.r);
+    // dE_i/dd = F1 + F2; du_b/dd_a = (delta_ab - u_a u_b)/r
+    const double F0 = (double) (f1 * x + (gx - gu * x) * rinv) * scale;
+    const double F1 = (double) (f1 * y + (gy - gu * y) * rinv) * scale;
+    const double F2 = (double) (f1 * z + (gz - gu * z) * rinv) * scale;
+    const int j = ng.j;
+    atomicAdd(&f[3 * (size_t) j + 0], -F0);
+    atomicAdd(&f[3 * (size_t) j + 1], -F1);
+    atomicAdd(&f[3 * (size_t) j + 2], -F2);
+    const double dx = ng.d[0], dy = ng.d[1], dz = ng.d[2];
+    const double v[6] = {-dx * F0, -dy * F1, -dz * F2, -dx * F1, -dx * F2, -dy * F2};
+    if (vatom) {
 #pragma unroll
-      for (int q = 1; q < kND; q++) V[q] += dpp_f<kDppXor1>(V[q]);
-      f1 += dpp_f<kDppXor1>(f1);
+      for (int q = 0; q < 6; q++) atomicAdd(&vatom[6 * (size_t) j + q], 0.5 * v[q]);
     }
-    if constexpr (LP >= 4) {
+    cf[0] += F0;
+    cf[1] += F1;
+    cf[2] += F2;
 #pragma unroll
-      for (int q = 1; q < kND; q++) V[q] += dpp_f<kDppXor2>(V[q]);
-      f1 += dpp_f<kDppXor2>(f1);
-    }
-    if constexpr (LP == 8) {
-#pragma unroll
-      for (int q = 1; q < kND; q++) V[q] += __shfl_xor(V[q], 4);
-      f1 += __shfl_xor(f1, 4);
-    }
-    double cf[9];
-#pragma unroll
-    for (int q = 0; q < 9; q++) cf[q] = 0.0;
-    if (live && sub == 0) {
-      const float x = ng.ux, y = ng.uy, z = ng.uz;
-      // g_beta = sum_d V_d dM_d/du_beta
-      float gx = V[1] + 2.f * x * V[4] + y * V[5] + z * V[6] + 3.f * x * x * V[10] +
-          2.f * x * y * V[11] + 2.f * x * z * V[12] + y * y * V[13] + y * z * V[14] + z * z * V[15];
-      float gy = V[2] + x * V[5] + 2.f * y * V[7] + z * V[8] + x * x * V[11] + 2.f * x * y * V[13] +
-          x * z * V[14] + 3.f * y * y * V[16] + 2.f * y * z * V[17] + z * z * V[18];
-      float gz = V[3] + x * V[6] + y * V[8] + 2.f * z * V[9] + x * x * V[12] + x * y * V[14] +
-          2.f * x * z * V[15] + y * y * V[17] + 2.f * y * z * V[18] + 3.f * z * z * V[19];
-      float gu = gx * x + gy * y + gz * z;
-      // 1-ulp hardware reciprocal (a division is a ten-instruction FP64 sequence)
-      float rinv = __builtin_amdgcn_rcpf((float) ng.r);
-      // dE_i/dd = F1 + F2; dM/dd_a = sum_b dM/du_b (delta_ab - u_a u_b)/r
-      double F0 = (double) (f1 * x + (gx - gu * x) * rinv) * scale;
-      double F1v = (double) (f1 * y + (gy - gu * y) * rinv) * scale;
-      double F2v = (double) (f1 * z + (gz - gu * z) * rinv) * scale;
-      const int j = ng.j;
-      atomicAdd(&f[3 * (size_t) j + 0], -F0);
-      atomicAdd(&f[3 * (size_t) j + 1], -F1v);
-      atomicAdd(&f[3 * (size_t) j + 2], -F2v);
-      const double dx = ng.d[0], dy = ng.d[1], dz = ng.d[2];
-      double v[6] = {-dx * F0, -dy * F1v, -dz * F2v, -dx * F1v, -dx * F2v, -dy * F2v};
-      if (vatom) {
-#pragma unroll
-        for (int q = 0; q < 6; q++) atomicAdd(&vatom[6 * (size_t) j + q], 0.5 * v[q]);
-      }
-      cf[0] = F0;
-      cf[1] = F1v;
-      cf[2] = F2v;
-#pragma unroll
-      for (int q = 0; q < 6; q++) cf[3 + q] = v[q];
-    }
-    // the chunk's own-force and virial sums, in a fixed lane order, into the
-    // atom's LDS accumulators (nothing FP64 is live through the filter loop);
-    // only each neighbor's first lane holds values
-#pragma unroll
-    for (int q = 0; q < 9; q++) cf[q] = wave_sum_d_lp<LP>(cf[q]);
-    if (lane == 0) {
-#pragma unroll
-      for (int q = 0; q < 9; q++) facc[q] += cf[q];
-    }
+    for (int q = 0; q < 6; q++) cf[3 + q] += v[q];
+  }
+  // nine sums over the lanes: pairs of quantities share the exchanges between
+  // the halves and between the rows, so that four of them remain per
+  // register for the sums within a row of 16 lanes
+  const double x0 = row_sum_d(swap16_add(swap32_add(cf[0], cf[1]), swap32_add(cf[2], cf[3])));
+  const double x1 = row_sum_d(swap16_add(swap32_add(cf[4], cf[5]), swap32_add(cf[6], cf[7])));
+  const double h8 = swap32_add(cf[8], cf[8]);
+  const double x2 = row_sum_d(swap16_add(h8, h8));
+  if ((lane & 15) == 0) {
+    const int q = ((lane >> 4) & 1) * 2 + (lane >> 5);  // rows hold quantities 0, 2, 1, 3
+    facc[q] += x0;
+    facc[4 + q] += x1;
+    if (lane == 0) facc[8] += x2;
   }
 }
 
-// 4 waves per SIMD (at most 128 VGPRs): the chain-rule pass hides its table
-// and LDS latency with more waves; the few spilled values live outside its loops
-// Waves per SIMD asked of the force kernel: 4 (at most 128 VGPRs, a few
-// values spilled outside the loops) where the P block of a lane is small;
-// the wider variants keep their registers and run fewer waves.
-template <int K, int NS>
-constexpr int kForceWaves = (K <= 24 && NS * Tiling<K>::KT * Tiling<K>::DT <= 40) ? 4 : 1;
+// Waves per SIMD asked of the force kernel: what its LDS leaves room for
+template <int K>
+constexpr int kForceWaves = K <= 32 ? 4 : (K == 64 ? 3 : 2);
 
-// P of the nsl slots of a pass -> LDS [b0 + b][k][d]
-template <int K, int NS>
-__device__ inline void store_P(float (*acc)[Tiling<K>::KT][Tiling<K>::DT], float *PS, int b0, int nsl)
-{
-  using T = Tiling<K>;
-  const int lane = threadIdx.x & 63;
-  if (lane < T::LANES) {
-    const int kq = lane / T::NDG, dq = lane - (lane / T::NDG) * T::NDG;
-#pragma unroll
-    for (int b = 0; b < NS; b++) {
-      if (b >= nsl) break;
-#pragma unroll
-      for (int a = 0; a < T::KT; a++)
-#pragma unroll
-        for (int q = 0; q < T::DT; q++)
-          PS[(size_t) (b0 + b) * T::SSTR + (kq * T::KT + a) * kND + dq * T::DT + q] = acc[b][a][q];
-    }
-  }
-}
-
-// NS, MP: as for k_descriptor
-template <int K, int NS, bool MP>
-__global__ __launch_bounds__(64, (kForceWaves<K, NS>)) void k_force(ModelGeo g, Geom geo, const double4 *pos, int cap,
+template <int K>
+__global__ __launch_bounds__(64, (kForceWaves<K>)) void k_force(ModelGeo g, Geom geo, const double4 *pos, int cap,
                                               const int *row2atom, int rbase, int nrows, const float4 *tab,
                                               const uint32_t *kl, const float *dEdG,
                                               const double *E, double scale, double *f,
                                               double *eatom, double *watom, double *vatom)
 {
   using T = Tiling<K>;
-  extern __shared__ __align__(16) unsigned char smem[];
+  __shared__ __align__(16) float rows[T::WIN * kRow];
+  __shared__ __align__(16) float buf[T::BUF];
+  __shared__ double facc[9];
   const int row = geo.order ? geo.order[rbase + (int) blockIdx.x] : rbase + (int) blockIdx.x;
   if (row >= nrows || (geo.dyn && row >= geo.dyn->rl.nrows)) return;
   const int lane = threadIdx.x & 63;
   const int i = row2atom[row];
   if (i < 0) return;  // padding row
-  size_t offs[3];
-  force_lds_layout<K>(g.nelt, MP, offs);
-  LDSMap L;
-  L.M = reinterpret_cast<float *>(smem + offs[1]);
-  L.H = reinterpret_cast<float *>(smem + offs[2]);
-  float *PS = reinterpret_cast<float *>(smem + offs[0]);
+  float *hb = buf, *sb = T::kSRegs ? buf : buf + T::HBUF;
   const double4 xi = pos[i];
   const Box cell = load_box(geo, i);
   // the descriptor kernel's kept list of this row (slot-sorted, within rc)
   const uint32_t *kr = kl + (size_t) row * kept_cache_words(cap);
   const int nk = (int) kr[0];
-  int start[kMaxElts + 1];
-  for (int b = 0; b <= g.nelt; b++) start[b] = (int) kr[1 + b];
   const uint32_t *kept = kr + kKeptHdr;
-  L.kept = const_cast<uint32_t *>(kept);
-  if constexpr (!MP) {
-    float acc[NS][T::KT][T::DT];
-    accumulate_P<K, NS>(g, cell, xi, pos, tab, L, start, g.nelt, acc);
-    // P -> LDS over the staging area (accumulate_P ends with a barrier)
-    store_P<K, NS>(acc, PS, 0, g.nelt);
-  } else {
-    __shared__ int s_start[kMaxElts + 1];
-    if (lane == 0)
-      for (int b = 0; b <= g.nelt; b++) s_start[b] = start[b];
-    __syncthreads();
-    for (int b0 = 0; b0 < g.nelt; b0 += NS) {
-      const int nsl = min(NS, g.nelt - b0);
-      float acc[NS][T::KT][T::DT];
-      accumulate_P<K, NS>(g, cell, xi, pos, tab, L, s_start + b0, nsl, acc);
-      store_P<K, NS>(acc, PS, b0, nsl);
-    }
-  }
-  __syncthreads();
-
-  // S[b][k][d] = P * sum_m 2 T[m][d] g'_m, in place: T[m][d] is the
-  // multiplicity of monomial d in its degree m, plus the T-symmetric extras
   const float *grow = dEdG + (size_t) row * g.nelt * K * kNM;
-  for (int e = lane; e < g.nelt * K; e += 64) {
-    float *P = PS + (size_t) (e / K) * T::SSTR + (e % K) * kND;
-    float4 gv = *reinterpret_cast<const float4 *>(grow + (size_t) e * kNM);
-    float G0 = P[0];
-    float g0 = (fabsf(G0) < 1e-8f) ? 0.0f : gv.x * __builtin_amdgcn_rcpf(G0) * 0.5f;
-    float w[kNM] = {2.0f * g0, 2.0f * gv.y, 2.0f * gv.z, 2.0f * gv.w};
-    float w0 = w[0], w1 = w[1];
-    if (g.tsym) {
-      w0 = fmaf(w[2], (float) (-1.0 / 3.0), w0);
-      w1 = fmaf(w[3], (float) (-3.0 / 5.0), w1);
-    }
-    P[0] *= w0;
-#pragma unroll
-    for (int d = 1; d < kND; d++) {
-      const float wd = kDeg[d] == 1 ? w1 : (kMult[d] == 1 ? w[kDeg[d]] : (float) kMult[d] * w[kDeg[d]]);
-      P[d] *= wd;
-    }
-  }
-  __syncthreads();
-
-  // Phase 3: the chain rule, chunk by chunk (1 lane per neighbor, or 2 / 4 / 8
-  // for a short last chunk)
-  // own force (3) and virial (6) of the atom, summed chunk by chunk
-  __shared__ double facc[9];
   if (lane < 9) facc[lane] = 0.0;
-  for (int base = 0; base < nk;) {
-    const int Lp = chain_lanes(nk - base);
-    if (Lp == 1)
-      force_chunk<K, 1>(g, cell, xi, pos, tab, PS, kept, start, base, nk, scale, f, vatom, facc);
-    else if (Lp == 2)
-      force_chunk<K, 2>(g, cell, xi, pos, tab, PS, kept, start, base, nk, scale, f, vatom, facc);
-    else if (Lp == 4)
-      force_chunk<K, 4>(g, cell, xi, pos, tab, PS, kept, start, base, nk, scale, f, vatom, facc);
-    else
-      force_chunk<K, 8>(g, cell, xi, pos, tab, PS, kept, start, base, nk, scale, f, vatom, facc);
-    base += 64 / Lp;
-  }
-  __syncthreads();
-  double fi[3], wi[6];
+  // Segments: the whole list where it fits the staged rows, else slot by
+  // slot; a slot that does not fit runs its P and its chain rule in windows.
+  const bool whole = nk <= T::WIN;
+  for (int b0 = 0; b0 < g.nelt;) {
+    const int b1 = whole ? g.nelt : b0 + 1;
+    const int lo = (int) kr[1 + b0], hi = (int) kr[1 + b1];
+    const bool one = hi - lo <= T::WIN;
+    if (one) stage(g, cell, xi, pos, kept + lo, hi - lo, rows);
+    for (int b = b0; b < b1; b++) {
+      const int s0 = (int) kr[1 + b], s1 = (int) kr[2 + b];
+      if (s0 >= s1) continue;
+      float4 gv[T::KT];
 #pragma unroll
-  for (int a = 0; a < 3; a++) fi[a] = facc[a];
+      for (int t = 0; t < T::KT; t++)
+        gv[t] = *reinterpret_cast<const float4 *>(grow + ((size_t) b * K + min(16 * t + (lane & 15), K - 1)) * kNM);
+      f32x4v acc[T::KT];
 #pragma unroll
-  for (int q = 0; q < 6; q++) wi[q] = facc[3 + q];
-
-  if (lane == 0) {
-    atomicAdd(&f[3 * (size_t) i + 0], fi[0]);
-    atomicAdd(&f[3 * (size_t) i + 1], fi[1]);
-    atomicAdd(&f[3 * (size_t) i + 2], fi[2]);
+      for (int t = 0; t < T::KT; t++) acc[t] = f32x4v{0, 0, 0, 0};
+      // P, then the chain rule, of a slot of at most RT tiles: H and dH are
+      // interpolated once and stay in registers in between
+      if constexpr (T::RT > 0) {
+        if (one && s1 - s0 <= 16 * T::RT) {
+          float h[T::RT][T::NFB], dh[T::RT][T::NFB];
+          float *rt = rows + (s0 - lo) * kRow;
+#pragma unroll
+          for (int q = 0; q < T::RT; q++) {
+            const int live = min(16, s1 - s0 - 16 * q);
+#pragma unroll
+            for (int k = 0; k < T::NFB; k++) h[q][k] = dh[q][k] = 0.0f;
+            if (live <= 0) continue;
+            float hq[T::NFB], dq[T::NFB];
+            radial_tile<K, true>(g, tab, rt + 16 * q * kRow, live, 0, hq, dq);
+            put_tile<K>(dq, hb);
+            wave_sync();
+            get_chain<K>(hb, dh[q]);
+            wave_sync();
+            put_tile<K>(hq, hb);
+            wave_sync();
+            get_chain<K>(hb, h[q]);
+            moments_tile<K>(rt + 16 * q * kRow, live, hb, acc);
+            wave_sync();
+          }
+          slot_S<K>(acc, gv, g.tsym, sb);
+          wave_sync();
+          SOps<K> so;
+          load_S<K>(sb, 0, so);
+          wave_sync();
+#pragma unroll
+          for (int q = 0; q < T::RT; q++) {
+            const int live = min(16, s1 - s0 - 16 * q);
+            if (live <= 0) break;
+            const f32x4v y = get_Y(rt + 16 * q * kRow, live);
+            float f1 = 0.0f;
+            f32x4v v = {0, 0, 0, 0};
+            chain_block<K>(so, y, h[q], dh[q], f1, v);
+            put_V(rt + 16 * q * kRow, live, f1, v);
+          }
+          continue;
+        }
+      }
+      // any other slot: H is interpolated again for the chain rule
+      for (int w0 = one ? lo : s0; w0 < s1; w0 += T::WIN) {
+        const int wn = min(T::WIN, (one ? hi : s1) - w0);
+        if (!one) stage(g, cell, xi, pos, kept + w0, wn, rows);
+        const int c0 = max(s0 - w0, 0), c1 = min(s1 - w0, wn);
+        for (int r0 = c0; r0 < c1; r0 += 16) {
+          const int live = min(16, c1 - r0);
+#pragma unroll
+          for (int fb = 0; fb < T::NB; fb++) {
+            float h[T::NFB];
+            radial_tile<K, false>(g, tab, rows + r0 * kRow, live, fb, h, nullptr);
+            put_tile<K>(h, hb);
+            wave_sync();
+            moments_tile<K>(rows + r0 * kRow, live, hb, acc + fb * T::CT);
+            wave_sync();
+          }
+        }
+      }
+      slot_S<K>(acc, gv, g.tsym, sb);
+      wave_sync();
+      SOps<K> so;
+      if constexpr (T::kSRegs) {
+        load_S<K>(sb, 0, so);
+        wave_sync();
+      }
+      for (int w0 = one ? lo : s0; w0 < s1; w0 += T::WIN) {
+        const int wn = min(T::WIN, (one ? hi : s1) - w0);
+        if (!one) stage(g, cell, xi, pos, kept + w0, wn, rows);
+        const int c0 = max(s0 - w0, 0), c1 = min(s1 - w0, wn);
+        for (int r0 = c0; r0 < c1; r0 += 16) {
+          const int live = min(16, c1 - r0);
+          float *rt = rows + r0 * kRow;
+          const f32x4v y = get_Y(rt, live);
+          float f1 = 0.0f;
+          f32x4v v = {0, 0, 0, 0};
+#pragma unroll 1
+          for (int fb = 0; fb < T::NB; fb++) {
+            float hq[T::NFB], dq[T::NFB], h[T::NFB], dh[T::NFB];
+            radial_tile<K, true>(g, tab, rt, live, fb, hq, dq);
+            put_tile<K>(dq, hb);
+            wave_sync();
+            get_chain<K>(hb, dh);
+            wave_sync();
+            put_tile<K>(hq, hb);
+            wave_sync();
+            get_chain<K>(hb, h);
+            wave_sync();
+            if constexpr (!T::kSRegs) load_S<K>(sb, fb, so);
+            chain_block<K>(so, y, h, dh, f1, v);
+          }
+          put_V(rt, live, f1, v);
+        }
+        if (!one) {
+          wave_sync();
+          finish(g, cell, xi, pos, kept + w0, wn, rows, scale, f, vatom, facc);
+          wave_sync();
+        }
+      }
+    }
+    wave_sync();
+    if (one) finish(g, cell, xi, pos, kept + lo, hi - lo, rows, scale, f, vatom, facc);
+    wave_sync();
+    b0 = b1;
   }
+  if (lane < 3) atomicAdd(&f[3 * (size_t) i + lane], facc[lane]);
   if (lane < 6) {
-    double v = wi[lane];
+    const double v = facc[3 + lane];
     watom[6 * (size_t) i + lane] = v;
     if (vatom) atomicAdd(&vatom[6 * (size_t) i + lane], 0.5 * v);
   }
@@ -653,7 +755,7 @@ hipError_t desc_impl(const ModelGeo &g, const Geom &geo, const double4 *pos, con
                      float *G, uint32_t *kl, hipStream_t s)
 {
   size_t offs[3];
-  size_t lds = lds_layout<K>(cap, offs);
+  size_t lds = desc_lds<K>(cap, offs);
   if (lds > 160 * 1024) return hipErrorInvalidConfiguration;
   if (hipError_t ae = hipFuncSetAttribute((const void *) k_descriptor<K, NS, MP>,
                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds);
@@ -664,40 +766,19 @@ hipError_t desc_impl(const ModelGeo &g, const Geom &geo, const double4 *pos, con
   return hipGetLastError();
 }
 
-template <int K, int NS, bool MP>
-hipError_t force_impl(const ModelGeo &g, const Geom &geo, const double4 *pos, int cap,
-                      const int *row2atom, int rbase, int nrows, const float4 *tab, const uint32_t *kl,
-                      const float *dEdG, const double *E, double scale, double *f, double *eatom,
-                      double *watom, double *vatom, hipStream_t s)
+// Slots per register pass of the descriptor: the smallest of 1, 2, 4, 8 that
+// holds nelt within a budget of 64 accumulators per lane; models with more
+// slots than the largest such count (k = 64: 4, k = 128: 2) take several
+// passes.
+template <int K>
+hipError_t dispatch_desc(const ModelGeo &g, const Geom &geo, const double4 *pos, const uint32_t *nbr,
+                         const int *nn, int cap, const int *row2atom, int rbase, int nrows, const float4 *tab,
+                         float *G, uint32_t *kl, hipStream_t s)
 {
-  size_t offs[3];
-  const size_t lds = force_lds_layout<K>(g.nelt, MP, offs);
-  if (lds > 160 * 1024) return hipErrorInvalidConfiguration;
-  if (hipError_t ae = hipFuncSetAttribute((const void *) k_force<K, NS, MP>,
-                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds);
-      ae != hipSuccess)
-    return ae;
-  k_force<K, NS, MP><<<nrows - rbase, 64, lds, s>>>(g, geo, pos, cap, row2atom, rbase, nrows, tab, kl, dEdG, E,
-                                                    scale, f, eatom, watom, vatom);
-  return hipGetLastError();
-}
-
-// Slots per register pass: the smallest of 1, 2, 4, 8 that holds nelt
-// within a budget of 128 accumulators per lane; models with more slots than
-// the largest such count (k = 64: 4, k = 128: 2) take several passes.
-template <int K, bool FORCE>
-hipError_t dispatch(const ModelGeo &g, const Geom &geo, const double4 *pos, const uint32_t *nbr,
-                    const int *nn, int cap, const int *row2atom, int rbase, int nrows, const float4 *tab,
-                    float *G, uint32_t *kl, const float *dEdG, const double *E, double scale,
-                    double *f, double *eatom, double *watom, double *vatom, hipStream_t s)
-{
-  constexpr int per = Tiling<K>::KT * Tiling<K>::DT;
-  constexpr int kMaxNS = 8 * per <= 128 ? 8 : (4 * per <= 128 ? 4 : (2 * per <= 128 ? 2 : 1));
-#define TMD_LAUNCH(NS, MP)                                                                          \
-  return FORCE ? force_impl<K, NS, MP>(g, geo, pos, cap, row2atom, rbase, nrows, tab, kl, dEdG, E,   \
-                                       scale, f, eatom, watom, vatom, s)                            \
-               : desc_impl<K, NS, MP>(g, geo, pos, nbr, nn, cap, row2atom, rbase, nrows, tab, G, kl, s);
-  static_assert(kMaxNS >= 2, "every filter count holds two slots per pass");
+  constexpr int per = Tiling<K>::KT * 4;
+  constexpr int kMaxNS = 8 * per <= 64 ? 8 : (4 * per <= 64 ? 4 : 2);
+#define TMD_LAUNCH(NS, MP) \
+  return desc_impl<K, NS, MP>(g, geo, pos, nbr, nn, cap, row2atom, rbase, nrows, tab, G, kl, s);
   if (g.nelt < 1 || g.nelt > kMaxElts) return hipErrorInvalidValue;
   if (g.nelt <= 1) TMD_LAUNCH(1, false)
   if (g.nelt <= 2) TMD_LAUNCH(2, false)
@@ -727,8 +808,7 @@ hipError_t launch_descriptor(const ModelGeo &g, const Geom &geo, const double4 *
     return launch_descriptor_hm(g, geo, pos, nbr, nn, cap, row2atom, nrows, tab, G, kl, stream, row_begin);
 #define TMD_K_CASE(K)                                                                                    \
   case K:                                                                                                \
-    return dispatch<K, false>(g, geo, pos, nbr, nn, cap, row2atom, row_begin, nrows, tab, G, kl, nullptr, \
-                              nullptr, 0, nullptr, nullptr, nullptr, nullptr, stream);
+    return dispatch_desc<K>(g, geo, pos, nbr, nn, cap, row2atom, row_begin, nrows, tab, G, kl, stream);
   switch (g.k) {
     TMD_K_CASE(16)
     TMD_K_CASE(24)
@@ -752,8 +832,9 @@ hipError_t launch_force(const ModelGeo &g, const Geom &geo, const double4 *pos, 
                            stream, row_begin);
 #define TMD_K_CASE(K)                                                                                       \
   case K:                                                                                                   \
-    return dispatch<K, true>(g, geo, pos, nullptr, nullptr, cap, row2atom, row_begin, nrows, tab, nullptr,  \
-                             const_cast<uint32_t *>(kl), dEdG, E, scale, f, eatom, watom, vatom, stream);
+    k_force<K><<<nrows - row_begin, 64, 0, stream>>>(g, geo, pos, cap, row2atom, row_begin, nrows, tab, kl, \
+                                                     dEdG, E, scale, f, eatom, watom, vatom);               \
+    return hipGetLastError();
   switch (g.k) {
     TMD_K_CASE(16)
     TMD_K_CASE(24)

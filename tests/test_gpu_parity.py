@@ -1009,3 +1009,59 @@ def test_fp8_mlp_error(tmp_path):
     e_l = _errs(got_l, ref_l, len(x))
     say("fp8 list-mode errors", e_l)
     assert e_l["dF"] <= 0.1 and e_l["dE"] <= 0.01
+
+
+def _cluster(rng, rc, counts):
+    """A center (type 1, atom 0) with counts[e] neighbors of type e + 1 at
+    0.35 rc .. 0.98 rc in random directions."""
+    t = np.concatenate([np.full(c, e + 1) for e, c in enumerate(counts)]).astype(np.int32)
+    u = rng.normal(size=(len(t), 3))
+    u /= np.linalg.norm(u, axis=1)[:, None]
+    x = u * rng.uniform(0.35, 0.98, size=(len(t), 1)) * rc
+    order = rng.permutation(len(t))
+    return np.concatenate([np.zeros((1, 3)), x[order]]), np.concatenate([[1], t[order]]).astype(np.int32)
+
+
+@pytest.mark.parametrize("k,nelt", [(16, 1), (16, 3), (24, 2), (24, 4), (32, 2), (64, 1), (64, 2),
+                                    (128, 1)])
+def test_force_tile_edges(tmp_path, k, nelt):
+    """Neighbor counts at the edges of the moment kernels' tiles: 4 neighbors
+    per matrix step, 16 per tile, the slots whose radial functions stay in
+    registers, and the staged windows (64, 88 and 96 neighbors), in one slot
+    and spread over the slots, empty slots among them.  One center per call;
+    forces, energies and the descriptor row against the FP64 oracle, bars as
+    for the reference's models (the FP32 floor of the same cluster)."""
+    path = W.write_model(str(tmp_path / "m.npz"), symbols=["Mo", "Nb", "Ta", "W"][:nelt],
+                         masses=[95.95, 92.906, 180.95, 183.84][:nelt], rmax=6.0, num_filters=k,
+                         layer_sizes=[64, 32, 1], actfn="tanh", seed=40 + k + nelt, radial_scale=0.1)
+    om = oracle.OracleModel(path, 0.001)
+    m = TensorMD(path, ["Mo", "Nb", "Ta", "W"][:nelt], "fp32", 0.001)
+    edges = [1, 3, 4, 5, 15, 16, 17, 31, 32, 33, 63, 64, 65, 79, 80, 81, 88, 89, 95, 96, 97, 112, 130]
+    rng = np.random.default_rng(7)
+    worst = 0.0
+    for n in edges:
+        for spread in range(2 if nelt > 1 else 1):
+            counts = [0] * nelt
+            if spread:
+                counts = list(np.bincount(rng.integers(0, nelt, n), minlength=nelt))
+            else:
+                counts[n % nelt] = n
+            x, t = _cluster(rng, om.rc, counts)
+            nl = np.zeros(len(x), dtype=np.int32)
+            nl[0] = n
+            args = ([0], nl, np.arange(1, n + 1))
+            ref = om.compute_list(len(x), x, t - 1, [0], nl, np.arange(1, n + 1), want_desc=True)
+            om.set_emulation(om.EMUL_DESC | om.EMUL_MLP | om.EMUL_FORCE)
+            emu = om.compute_list(len(x), x, t - 1, [0], nl, np.arange(1, n + 1))
+            om.set_emulation(0)
+            got = m.compute_list(len(x), x, t, *args)
+            G = m.descriptors_list(len(x), x, t, *args)[0]
+            e, fl = _errs(got, ref, 1), _errs(emu, ref, 1)
+            worst = max(worst, e["dF"])
+            assert e["dF"] <= max(F_TOL, 2.0 * fl["dF"]), (k, counts, e, fl)
+            assert e["dE"] <= max(1e-6, 2.0 * fl["dE"]), (k, counts, e, fl)
+            g0 = ref["G"][0]
+            assert abs(G - g0).max() <= 4e-6 * max(1.0, abs(g0).max()), (k, counts)
+            assert np.isfinite(got["vatom"]).all() and abs(got["vatom"] - ref["vatom"]).max() <= 6.0 * max(
+                F_TOL, 2.0 * fl["dF"])
+    say(k, nelt, "max |dF|", worst)
