@@ -226,12 +226,13 @@ int upload_model(tmd_ctx *ctx)
           }
   }
   g.rc2 = m.rc * m.rc;
-  g.dx = m.dx;
   g.xdx = m.xdx;
-  g.dxf = (float) m.dx;
-  // table as float4 [n][k]
+  g.rdx = 1.0 / m.dx;
+  g.rdxf = (float) g.rdx;
+  // table as float4 [n][k], in units of the grid step: (y, s dx, c1 dx^2, c2 dx^2)
   std::vector<float> tabf(m.tab.size());
-  for (size_t i = 0; i < tabf.size(); i++) tabf[i] = (float) m.tab[i];
+  const double unit[4] = {1.0, m.dx, m.dx * m.dx, m.dx * m.dx};
+  for (size_t i = 0; i < tabf.size(); i++) tabf[i] = (float) (m.tab[i] * unit[i % 4]);
   // the end cells contribute nothing (ration.hpp:29): zero rows give H = dH/dr = 0
   const size_t trow = (size_t) m.k * 4;
   for (int n : {0, m.tab_n - 2, m.tab_n - 1})

@@ -31,6 +31,13 @@
 // B[l / 16][l % 16]; accumulator element i of lane l is
 // D[4 (l / 16) + i][l % 16].
 //
+// What bounds the kernels (128,000 atoms, 4 elements, 24 filters, 63
+// neighbors): vector and matrix instructions, which do not overlap on a SIMD
+// here, fill about 95 % of the force kernel's time (0.38 + 0.19 of 0.61 ms;
+// 0.42 ms with neither matrix instructions nor atomics) and 86 % of the
+// descriptor's 0.32 ms.  With the monomials on the vector ALU they took 0.95
+// and 0.42 ms.
+//
 // Nothing per neighbor is stored in HBM: the reference materialises R, M,
 // H, dH/dr, P, dE/dS, V, F1, F2 per padded slot (kernel.cu:1545-1582).
 #include "tmd_desc_common.h"
@@ -42,7 +49,7 @@ namespace {
 typedef float f32x4v __attribute__((ext_vector_type(4)));
 
 constexpr int kNY = 16;  // harmonics of degree 0..3: degree l starts at l^2
-// LDS row of a staged neighbor: 16 harmonics, then q, dx - q and the table
+// LDS row of a staged neighbor: 16 harmonics, then q, 1 - q and the table
 // cell.  A stride of 20 words puts the 16-byte accesses of 16 rows on
 // distinct banks.
 constexpr int kRow = 20;
@@ -57,21 +64,22 @@ struct Tiling {
   static constexpr int KT = NB * CT;           // filter tiles
   // the second tile of K = 24 holds 8 filters, the others 16
   static constexpr int nper(int t) { return (K == 24 && t == 1) ? 2 : 4; }  // filters per lane group
-  // H of 16 neighbors, [16][HS]: HS / 4 is odd, so the quads of 16 rows hit
-  // distinct banks
-  static constexpr int HS = FBL + 4;
+  // H of 16 neighbors, [16][HS], and H with dH interleaved, [16][HD]: HS / 4
+  // and HD / 4 are odd, so the quads of 16 rows hit distinct banks
+  static constexpr int HS = FBL + 4, HD = 2 * FBL + 4;
   static constexpr int SS = kRow;              // stride of an S row
   // S is kept in registers per slot up to K = 32, and its LDS then overlays H
   static constexpr bool kSRegs = K <= 32;
-  static constexpr int HBUF = 16 * HS + 4;     // floats (the last tile of K = 24 reads past row 15)
+  // floats (the second tile of K = 24 reads 4 or 12 past row 15)
+  static constexpr int HBUF = 16 * HS + 4, DBUF = 16 * HD + (K == 24 ? 12 : 0);
   static constexpr int SBUF = K * SS;
-  static constexpr int BUF = kSRegs ? (HBUF > SBUF ? HBUF : SBUF) : HBUF + SBUF;
+  static constexpr int BUF = kSRegs ? (DBUF > SBUF ? DBUF : SBUF) : DBUF + SBUF;
   // staged neighbors of the force kernel: what leaves 16 waves per CU
-  // (10 KB each) up to K = 32, 13 at K = 64 and 9 at K = 128
-  static constexpr int WIN = K < 32 ? 96 : (K == 32 ? 88 : 64);
+  // (10 KB each) up to K = 32
+  static constexpr int WIN = K == 16 ? 96 : (K == 24 ? 84 : (K == 32 ? 72 : 64));
   // tiles of a slot whose H and dH stay in registers between P and the
   // chain rule (2 NFB registers each)
-  static constexpr int RT = K == 16 ? 5 : (K == 24 ? 2 : (K == 32 ? 2 : 0));
+  static constexpr int RT = K == 16 ? 5 : (K <= 32 ? 2 : 0);
 };
 
 // Y_d(u) in d order: 1 | x y z | 5 of degree 2 | 7 of degree 3, scaled so
@@ -169,89 +177,111 @@ __device__ inline double row_sum_d(double v)
   return v;
 }
 
+// The LDS row of neighbor e; d receives its displacement.
+__device__ inline void stage_row(const ModelGeo &g, const Box &cell, const double4 &xi, const double4 *pos,
+                                 uint32_t e, float *rowp, double d[3])
+{
+  NbrGeo ng;
+  nbr_geometry(g, cell, xi, pos, e, ng);
+  float Y[kNY];
+  harmonics(ng.ux, ng.uy, ng.uz, Y);
+  float4 *r = reinterpret_cast<float4 *>(rowp);
+#pragma unroll
+  for (int q = 0; q < 4; q++) r[q] = make_float4(Y[4 * q], Y[4 * q + 1], Y[4 * q + 2], Y[4 * q + 3]);
+  // a table of one point has no cell: its only row is an end row
+  r[4] = make_float4(ng.q, ng.pq, __int_as_float(max(ng.n, 0)), 0.0f);
+#pragma unroll
+  for (int q = 0; q < 3; q++) d[q] = ng.d[q];
+}
+
 // rows[c] of the n entries list[0..n)
 __device__ inline void stage(const ModelGeo &g, const Box &cell, const double4 &xi, const double4 *pos,
                              const uint32_t *list, int n, float *rows)
 {
   for (int c = threadIdx.x & 63; c < n; c += 64) {
-    NbrGeo ng;
-    nbr_geometry(g, cell, xi, pos, list[c], ng);
-    float Y[kNY];
-    harmonics(ng.ux, ng.uy, ng.uz, Y);
-    float4 *r = reinterpret_cast<float4 *>(rows + c * kRow);
-#pragma unroll
-    for (int q = 0; q < 4; q++) r[q] = make_float4(Y[4 * q], Y[4 * q + 1], Y[4 * q + 2], Y[4 * q + 3]);
-    // a table of one point has no cell: its only row is an end row
-    r[4] = make_float4(ng.q, ng.pq, __int_as_float(max(ng.n, 0)), 0.0f);
+    double d[3];
+    stage_row(g, cell, xi, pos, list[c], rows + c * kRow, d);
   }
   wave_sync();
 }
 
-// Radial functions (and derivatives) of one block of filters for the tile of
-// neighbors rows[0..live), live >= 1: lane l holds the filters 4 i + l % 4
-// of neighbor l / 4.  The table's end cells are zero rows, and a lane past
-// the tile takes row 0: H = dH = 0 there without a mask.
-template <int K, bool DH>
-__device__ inline void radial_tile(const ModelGeo &g, const float4 *tab, const float *rows, int live,
-                                   int block, float *h, float *dh)
+// The table rows of one block of filters for the tile of neighbors
+// rows[0..live), live >= 1: lane l takes the filters 4 i + l % 4 of neighbor
+// l / 4, so that 4 lanes read 64 contiguous bytes.  The table's end cells are
+// zero rows, and a lane past the tile takes row 0: H = dH = 0 there without
+// a mask.
+template <int K>
+struct TabTile {
+  float4 t[Tiling<K>::NFB];
+  float q, pq;
+};
+
+template <int K>
+__device__ inline void load_tile(const float4 *tab, const float *rows, int live, int block, TabTile<K> &o)
 {
   using T = Tiling<K>;
   const int lane = threadIdx.x & 63, c = lane >> 2;
-  const float4 o = *reinterpret_cast<const float4 *>(rows + min(c, live - 1) * kRow + kNY);
-  const int n = c < live ? __float_as_int(o.z) : 0;
+  const float4 v = *reinterpret_cast<const float4 *>(rows + min(c, live - 1) * kRow + kNY);
+  const int n = c < live ? __float_as_int(v.z) : 0;
+  o.q = v.x;
+  o.pq = v.y;
   const float4 *row = tab + (size_t) n * K + block * T::FBL + (lane & 3);
-  float4 t[T::NFB];
 #pragma unroll
-  for (int i = 0; i < T::NFB; i++) t[i] = row[4 * i];
-#pragma unroll
-  for (int i = 0; i < T::NFB; i++) {
-    if constexpr (DH)
-      kerley(t[i], o.x, o.y, o.x - o.y, g.dxf, h[i], dh[i]);
-    else
-      h[i] = kerley_h(t[i], o.x, o.y);
-  }
+  for (int i = 0; i < T::NFB; i++) o.t[i] = row[4 * i];
 }
 
-// a block's values of the tile -> hb [16][HS]
+// a block's H of the tile -> hb [16][HS]
 template <int K>
-__device__ inline void put_tile(const float *h, float *hb)
+__device__ inline void put_H(const TabTile<K> &o, float *hb)
 {
   using T = Tiling<K>;
   const int lane = threadIdx.x & 63;
   float *p = hb + (lane >> 2) * T::HS + (lane & 3);
 #pragma unroll
-  for (int i = 0; i < T::NFB; i++) p[4 * i] = h[i];
+  for (int i = 0; i < T::NFB; i++) p[4 * i] = kerley_h(o.t[i], o.q, o.pq);
 }
 
-// the values of neighbor l % 16 in the chain-rule layout: lane group l / 16
-// holds nper(t) consecutive filters of tile t
+// a block's H and dH = dx H' of the tile -> hb [16][HD]
 template <int K>
-__device__ inline void get_chain(const float *hb, float *h)
+__device__ inline void put_HD(const TabTile<K> &o, float *hb)
 {
   using T = Tiling<K>;
   const int lane = threadIdx.x & 63;
-  const float *p = hb + (lane & 15) * T::HS;
+  float *p = hb + (lane >> 2) * T::HD + 2 * (lane & 3);
 #pragma unroll
-  for (int t = 0; t < T::CT; t++) {
-    if constexpr (K == 24) {
-      if (t == 1) {
-        const float2 v = *reinterpret_cast<const float2 *>(p + 16 + 2 * (lane >> 4));
-        h[4] = v.x;
-        h[5] = v.y;
-        continue;
-      }
-    }
-    const float4 v = *reinterpret_cast<const float4 *>(p + 16 * t + 4 * (lane >> 4));
-    h[4 * t] = v.x;
-    h[4 * t + 1] = v.y;
-    h[4 * t + 2] = v.z;
-    h[4 * t + 3] = v.w;
+  for (int i = 0; i < T::NFB; i++) {
+    float2 v;
+    kerley(o.t[i], o.q, o.pq, o.q - o.pq, v.x, v.y);
+    *reinterpret_cast<float2 *>(p + 8 * i) = v;
   }
 }
 
-// P of a block's filters += the tile in rows[0..live) with H in hb:
-// P^T[d][k] of tile t in acc[t].  Rows past the tile hold H = 0.
+// H and dH of neighbor l % 16 in the chain-rule layout: lane group l / 16
+// holds nper(t) consecutive filters of tile t
 template <int K>
+__device__ inline void get_chain(const float *hb, float *h, float *dh)
+{
+  using T = Tiling<K>;
+  const int lane = threadIdx.x & 63, grp = lane >> 4;
+  const float *p = hb + (lane & 15) * T::HD;
+#pragma unroll
+  for (int t = 0; t < T::CT; t++) {
+    const int np = T::nper(t);
+#pragma unroll
+    for (int i = 0; i < np; i += 2) {
+      const float4 v = *reinterpret_cast<const float4 *>(p + 2 * (16 * t + np * grp + i));
+      h[4 * t + i] = v.x;
+      dh[4 * t + i] = v.y;
+      h[4 * t + i + 1] = v.z;
+      dh[4 * t + i + 1] = v.w;
+    }
+  }
+}
+
+// P of a block's filters += the tile in rows[0..live): P^T[d][k] of tile t
+// in acc[t].  Filter k of neighbor c is hb[c STR + k SK]; rows past the tile
+// hold H = 0.
+template <int K, int STR, int SK>
 __device__ inline void moments_tile(const float *rows, int live, const float *hb, f32x4v *acc)
 {
   using T = Tiling<K>;
@@ -262,7 +292,7 @@ __device__ inline void moments_tile(const float *rows, int live, const float *hb
     const int c = 4 * s + (lane >> 4);
     a[s] = rows[min(c, live - 1) * kRow + (lane & 15)];
 #pragma unroll
-    for (int t = 0; t < T::CT; t++) b[s][t] = hb[c * T::HS + 16 * t + (lane & 15)];
+    for (int t = 0; t < T::CT; t++) b[s][t] = hb[c * STR + SK * (16 * t + (lane & 15))];
   }
 #pragma unroll
   for (int s = 0; s < 4; s++) {
@@ -282,13 +312,13 @@ __device__ inline float g_components(const f32x4v &p, int tsym)
   // degrees of a group's harmonics: 0 111 | 2222 | 2 333 | 3333
   const float t0 = grp == 0 ? p[0] : 0.0f;
   const float t1 = grp == 0 ? b : 0.0f;
-  const float t2 = grp == 0 ? c2 * a : (grp == 1 ? a + b : (grp == 2 ? a : 0.0f));
-  const float t3 = grp == 0 ? c3 * b : (grp == 1 ? 0.0f : (grp == 2 ? b : a + b));
+  const float t2 = (grp == 0 ? c2 : (grp == 3 ? 0.0f : 1.0f)) * a + (grp == 1 ? 1.0f : 0.0f) * b;
+  const float t3 = (grp == 3 ? 1.0f : 0.0f) * a + (grp == 0 ? c3 : (grp == 1 ? 0.0f : 1.0f)) * b;
   return swap16_add(swap32_add(t0, t2), swap32_add(t1, t3));
 }
 
 // descriptor LDS: kept list, staged rows, H
-constexpr int kDescWin = 96;
+constexpr int kDescWin = 64;
 template <int K>
 __host__ __device__ inline size_t desc_lds(int cap, size_t *offs)
 {
@@ -329,9 +359,9 @@ __device__ inline void descriptor_pass(const ModelGeo &g, const Box &cell, const
       const float *rt = rows + r0 * kRow;
 #pragma unroll
       for (int fb = 0; fb < T::NB; fb++) {
-        float h[T::NFB];
-        radial_tile<K, false>(g, tab, rt, live, fb, h, nullptr);
-        put_tile<K>(h, hb);
+        TabTile<K> tt;
+        load_tile<K>(tab, rt, live, fb, tt);
+        put_H<K>(tt, hb);
         wave_sync();
         float a[4], bo[4][T::CT];
 #pragma unroll
@@ -484,7 +514,7 @@ __device__ inline void load_S(const float *sb, int block, SOps<K> &o)
 }
 
 // The chain rule of one block for a tile of neighbors (l % 16): f1 +=
-// sum_k U_k H'_k over the lane group's filters, v += V
+// sum_k U_k dH_k over the lane group's filters, v += V
 template <int K>
 __device__ inline void chain_block(const SOps<K> &o, const f32x4v &y, const float *h, const float *dh, float &f1,
                                    f32x4v &v)
@@ -520,61 +550,87 @@ __device__ inline f32x4v get_Y(const float *rt, int live)
   return *reinterpret_cast<const f32x4v *>(rt + min(lane & 15, live - 1) * kRow + 4 * (lane >> 4));
 }
 
-// The neighbor forces of list[0..n) from their V and f1 rows, one lane per
-// neighbor: f_j -= F (FP64 atomics); own force and virial summed over the
-// lanes in a fixed order into facc.
-__device__ inline void finish(const ModelGeo &g, const Box &cell, const double4 &xi, const double4 *pos,
-                              const uint32_t *list, int n, const float *rows, double scale, double *f,
-                              double *vatom, double *facc)
+// The force F of one neighbor (displacement d, atom j) from its V and f1 row;
+// the row then holds F, j and, with vatom, -d (x) F for scatter(), and cf has own force
+// and virial added.
+struct ForceRow {
+  double F[3];
+  double v[6];
+  int j;
+};
+static_assert(sizeof(ForceRow) <= kRow * sizeof(float) && kRow % 2 == 0, "a force row overlays a staged row");
+
+__device__ inline void neighbor_force(const ModelGeo &g, const double d[3], int j, float *rowp, double scale,
+                                      bool vatom, double *cf)
+{
+  const double r2 = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
+  const double ri = rsqrt_fp64(r2);
+  const float x = (float) (d[0] * ri), y = (float) (d[1] * ri), z = (float) (d[2] * ri);
+  float V[kNY];
+  const float4 *r = reinterpret_cast<const float4 *>(rowp);
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    const float4 v = r[q];
+    V[4 * q] = v.x;
+    V[4 * q + 1] = v.y;
+    V[4 * q + 2] = v.z;
+    V[4 * q + 3] = v.w;
+  }
+  const float4 p = r[4];
+  const float f1 = ((p.x + p.y) + (p.z + p.w)) * g.rdxf;
+  float gx, gy, gz;
+  harmonics_grad(x, y, z, V, gx, gy, gz);
+  const float gu = gx * x + gy * y + gz * z;
+  const float rinv = (float) ri;
+  // dE_i/dd = F1 + F2; du_b/dd_a = (delta_ab - u_a u_b)/r
+  const double F0 = (double) (f1 * x + (gx - gu * x) * rinv) * scale;
+  const double F1 = (double) (f1 * y + (gy - gu * y) * rinv) * scale;
+  const double F2 = (double) (f1 * z + (gz - gu * z) * rinv) * scale;
+  const double v[6] = {-d[0] * F0, -d[1] * F1, -d[2] * F2, -d[0] * F1, -d[0] * F2, -d[1] * F2};
+  ForceRow *o = reinterpret_cast<ForceRow *>(rowp);
+  o->F[0] = F0;
+  o->F[1] = F1;
+  o->F[2] = F2;
+  if (vatom) {
+#pragma unroll
+    for (int q = 0; q < 6; q++) o->v[q] = v[q];
+  }
+  o->j = j;
+  cf[0] += F0;
+  cf[1] += F1;
+  cf[2] += F2;
+#pragma unroll
+  for (int q = 0; q < 6; q++) cf[3 + q] += v[q];
+}
+
+// f_j -= F (and the neighbor half of the per-atom virials) of the n neighbors
+// in rows, FP64 atomics with adjacent lanes on adjacent components: they are
+// executed at the memory side, one request per line of 64 bytes, and a
+// neighbor's three components in three instructions were three requests
+// (13.5 M requests and at least 640 us for the 24 M atomics of 128,000 atoms).
+__device__ inline void scatter(const float *rows, int n, double *f, double *vatom)
 {
   const int lane = threadIdx.x & 63;
-  double cf[9];
-#pragma unroll
-  for (int q = 0; q < 9; q++) cf[q] = 0.0;
-  for (int c = lane; c < n; c += 64) {
-    NbrGeo ng;
-    nbr_geometry(g, cell, xi, pos, list[c], ng);
-    float V[kNY];
-    const float4 *r = reinterpret_cast<const float4 *>(rows + c * kRow);
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-      const float4 v = r[q];
-      V[4 * q] = v.x;
-      V[4 * q + 1] = v.y;
-      V[4 * q + 2] = v.z;
-      V[4 * q + 3] = v.w;
-    }
-    const float4 p = r[4];
-    const float f1 = (p.x + p.y) + (p.z + p.w);
-    const float x = ng.ux, y = ng.uy, z = ng.uz;
-    float gx, gy, gz;
-    harmonics_grad(x, y, z, V, gx, gy, gz);
-    const float gu = gx * x + gy * y + gz * z;
-    // 1-ulp hardware reciprocal (a division is a ten-instruction FP64 sequence)
-    const float rinv = __builtin_amdgcn_rcpf((float) ng.r);
-    // dE_i/dd = F1 + F2; du_b/dd_a = (delta_ab - u_a u_b)/r
-    const double F0 = (double) (f1 * x + (gx - gu * x) * rinv) * scale;
-    const double F1 = (double) (f1 * y + (gy - gu * y) * rinv) * scale;
-    const double F2 = (double) (f1 * z + (gz - gu * z) * rinv) * scale;
-    const int j = ng.j;
-    atomicAdd(&f[3 * (size_t) j + 0], -F0);
-    atomicAdd(&f[3 * (size_t) j + 1], -F1);
-    atomicAdd(&f[3 * (size_t) j + 2], -F2);
-    const double dx = ng.d[0], dy = ng.d[1], dz = ng.d[2];
-    const double v[6] = {-dx * F0, -dy * F1, -dz * F2, -dx * F1, -dx * F2, -dy * F2};
-    if (vatom) {
-#pragma unroll
-      for (int q = 0; q < 6; q++) atomicAdd(&vatom[6 * (size_t) j + q], 0.5 * v[q]);
-    }
-    cf[0] += F0;
-    cf[1] += F1;
-    cf[2] += F2;
-#pragma unroll
-    for (int q = 0; q < 6; q++) cf[3 + q] += v[q];
+  for (int t = lane; t < 3 * n; t += 64) {
+    const int c = t / 3, q = t - 3 * c;
+    const ForceRow *o = reinterpret_cast<const ForceRow *>(rows + c * kRow);
+    atomicAdd(&f[3 * (size_t) o->j + q], -o->F[q]);
   }
-  // nine sums over the lanes: pairs of quantities share the exchanges between
-  // the halves and between the rows, so that four of them remain per
-  // register for the sums within a row of 16 lanes
+  if (vatom)
+    for (int t = lane; t < 6 * n; t += 64) {
+      const int c = t / 6, q = t - 6 * c;
+      const ForceRow *o = reinterpret_cast<const ForceRow *>(rows + c * kRow);
+      atomicAdd(&vatom[6 * (size_t) o->j + q], 0.5 * o->v[q]);
+    }
+}
+
+// facc += the lanes' own force and virial, in a fixed order.  Pairs of
+// quantities share the exchanges between the halves and between the rows, so
+// that four of them remain per register for the sums within a row of 16
+// lanes.
+__device__ inline void add_sums(const double *cf, double *facc)
+{
+  const int lane = threadIdx.x & 63;
   const double x0 = row_sum_d(swap16_add(swap32_add(cf[0], cf[1]), swap32_add(cf[2], cf[3])));
   const double x1 = row_sum_d(swap16_add(swap32_add(cf[4], cf[5]), swap32_add(cf[6], cf[7])));
   const double h8 = swap32_add(cf[8], cf[8]);
@@ -584,6 +640,64 @@ __device__ inline void finish(const ModelGeo &g, const Box &cell, const double4 
     facc[q] += x0;
     facc[4 + q] += x1;
     if (lane == 0) facc[8] += x2;
+  }
+}
+
+// dE/dG of one slot: filter l % 16 of every tile
+template <int K>
+__device__ inline void load_dEdG(const float *gslot, float4 *gv)
+{
+#pragma unroll
+  for (int t = 0; t < Tiling<K>::KT; t++)
+    gv[t] = *reinterpret_cast<const float4 *>(gslot + min(16 * t + (int) (threadIdx.x & 15), K - 1) * kNM);
+}
+
+// P += the staged neighbors rows[0..n) of one slot
+template <int K>
+__device__ inline void slot_moments(const float4 *tab, const float *rows, int n, float *hb, f32x4v *acc)
+{
+  using T = Tiling<K>;
+  for (int r0 = 0; r0 < n; r0 += 16) {
+    const int live = min(16, n - r0);
+#pragma unroll
+    for (int fb = 0; fb < T::NB; fb++) {
+      TabTile<K> tt;
+      load_tile<K>(tab, rows + r0 * kRow, live, fb, tt);
+      put_H<K>(tt, hb);
+      wave_sync();
+      moments_tile<K, T::HS, 1>(rows + r0 * kRow, live, hb, acc + fb * T::CT);
+      wave_sync();
+    }
+  }
+}
+
+// V and f1 of the staged neighbors rows[0..n) of one slot, over their rows.
+// so: the slot's S operands where they fit registers, else read from sb.
+template <int K>
+__device__ inline void slot_chain(const float4 *tab, float *rows, int n, const float *sb,
+                                  SOps<K> &so, float *hb)
+{
+  using T = Tiling<K>;
+  for (int r0 = 0; r0 < n; r0 += 16) {
+    const int live = min(16, n - r0);
+    float *rt = rows + r0 * kRow;
+    const f32x4v y = get_Y(rt, live);
+    float f1 = 0.0f;
+    f32x4v v = {0, 0, 0, 0};
+#pragma unroll 1
+    for (int fb = 0; fb < T::NB; fb++) {
+      TabTile<K> tt;
+      load_tile<K>(tab, rt, live, fb, tt);
+      if constexpr (!T::kSRegs) load_S<K>(sb, fb, so);
+      put_HD<K>(tt, hb);
+      wave_sync();
+      float h[T::NFB], dh[T::NFB];
+      get_chain<K>(hb, h, dh);
+      wave_sync();
+      chain_block<K>(so, y, h, dh, f1, v);
+    }
+    put_V(rt, live, f1, v);
+    wave_sync();
   }
 }
 
@@ -607,92 +721,135 @@ __global__ __launch_bounds__(64, (kForceWaves<K>)) void k_force(ModelGeo g, Geom
   const int lane = threadIdx.x & 63;
   const int i = row2atom[row];
   if (i < 0) return;  // padding row
-  float *hb = buf, *sb = T::kSRegs ? buf : buf + T::HBUF;
+  float *hb = buf, *sb = T::kSRegs ? buf : buf + T::DBUF;
   const double4 xi = pos[i];
   const Box cell = load_box(geo, i);
-  // the descriptor kernel's kept list of this row (slot-sorted, within rc)
+  // the descriptor kernel's kept list of this row (slot-sorted, within rc):
+  // the header in one register per lane, and the first two chunks' entries
+  // read beside it (indices clamped into the row)
   const uint32_t *kr = kl + (size_t) row * kept_cache_words(cap);
-  const int nk = (int) kr[0];
   const uint32_t *kept = kr + kKeptHdr;
+  const uint32_t hdr = kr[lane & 15];
+  const uint32_t e0 = kept[min(lane, cap - 1)], e1 = kept[min(64 + lane, cap - 1)];
+  const int nk = (int) __builtin_amdgcn_readlane((int) hdr, 0);
+  auto start = [&](int b) { return (int) __builtin_amdgcn_readlane((int) hdr, 1 + b); };
   const float *grow = dEdG + (size_t) row * g.nelt * K * kNM;
   if (lane < 9) facc[lane] = 0.0;
-  // Segments: the whole list where it fits the staged rows, else slot by
-  // slot; a slot that does not fit runs its P and its chain rule in windows.
-  const bool whole = nk <= T::WIN;
-  for (int b0 = 0; b0 < g.nelt;) {
-    const int b1 = whole ? g.nelt : b0 + 1;
-    const int lo = (int) kr[1 + b0], hi = (int) kr[1 + b1];
-    const bool one = hi - lo <= T::WIN;
-    if (one) stage(g, cell, xi, pos, kept + lo, hi - lo, rows);
-    for (int b = b0; b < b1; b++) {
-      const int s0 = (int) kr[1 + b], s1 = (int) kr[2 + b];
-      if (s0 >= s1) continue;
+  if (nk <= T::WIN) {
+    // the whole list is staged at once; two lanes' worth of neighbors at most
+    static_assert(T::WIN <= 128, "the list fits two chunks");
+    double d0[3] = {0.0, 0.0, 0.0};
+    if (lane < nk) stage_row(g, cell, xi, pos, e0, rows + lane * kRow, d0);
+    if (64 + lane < nk) {
+      double d1[3];
+      stage_row(g, cell, xi, pos, e1, rows + (64 + lane) * kRow, d1);
+    }
+    wave_sync();
+    auto next_slot = [&](int b) {
+      while (b < g.nelt && start(b) >= start(b + 1)) b++;
+      return b;
+    };
+    int b = next_slot(0);
+    // the table rows of the next tile of filters are requested before the
+    // present one goes through the matrix cores: the wave would otherwise
+    // wait for them tile after tile
+    TabTile<K> tt;
+    auto request = [&](int bb) {
+      if (T::RT > 0 && bb < g.nelt) load_tile<K>(tab, rows + start(bb) * kRow, min(16, start(bb + 1) - start(bb)), 0, tt);
+    };
+    request(b);
+    while (b < g.nelt) {
+      const int s0 = start(b), n = start(b + 1) - s0;
+      const int bn = next_slot(b + 1);
+      float *rt = rows + s0 * kRow;
       float4 gv[T::KT];
-#pragma unroll
-      for (int t = 0; t < T::KT; t++)
-        gv[t] = *reinterpret_cast<const float4 *>(grow + ((size_t) b * K + min(16 * t + (lane & 15), K - 1)) * kNM);
+      load_dEdG<K>(grow + (size_t) b * K * kNM, gv);
       f32x4v acc[T::KT];
 #pragma unroll
       for (int t = 0; t < T::KT; t++) acc[t] = f32x4v{0, 0, 0, 0};
-      // P, then the chain rule, of a slot of at most RT tiles: H and dH are
-      // interpolated once and stay in registers in between
+      SOps<K> so;
+      bool done = false;
       if constexpr (T::RT > 0) {
-        if (one && s1 - s0 <= 16 * T::RT) {
+        // a slot of at most RT tiles: H and dH are interpolated once and stay
+        // in registers between P and the chain rule
+        if (n <= 16 * T::RT) {
           float h[T::RT][T::NFB], dh[T::RT][T::NFB];
-          float *rt = rows + (s0 - lo) * kRow;
 #pragma unroll
           for (int q = 0; q < T::RT; q++) {
-            const int live = min(16, s1 - s0 - 16 * q);
+            const int live = min(16, n - 16 * q);
+            if (live > 0) {
+              put_HD<K>(tt, hb);
+              wave_sync();
+              if (n > 16 * (q + 1))
+                load_tile<K>(tab, rt + 16 * (q + 1) * kRow, min(16, n - 16 * (q + 1)), 0, tt);
+              else
+                request(bn);
+              get_chain<K>(hb, h[q], dh[q]);
+              moments_tile<K, T::HD, 2>(rt + 16 * q * kRow, live, hb, acc);
+              wave_sync();
+            } else {
 #pragma unroll
-            for (int k = 0; k < T::NFB; k++) h[q][k] = dh[q][k] = 0.0f;
-            if (live <= 0) continue;
-            float hq[T::NFB], dq[T::NFB];
-            radial_tile<K, true>(g, tab, rt + 16 * q * kRow, live, 0, hq, dq);
-            put_tile<K>(dq, hb);
-            wave_sync();
-            get_chain<K>(hb, dh[q]);
-            wave_sync();
-            put_tile<K>(hq, hb);
-            wave_sync();
-            get_chain<K>(hb, h[q]);
-            moments_tile<K>(rt + 16 * q * kRow, live, hb, acc);
-            wave_sync();
+              for (int k = 0; k < T::NFB; k++) h[q][k] = dh[q][k] = 0.0f;
+            }
           }
           slot_S<K>(acc, gv, g.tsym, sb);
           wave_sync();
-          SOps<K> so;
           load_S<K>(sb, 0, so);
           wave_sync();
 #pragma unroll
           for (int q = 0; q < T::RT; q++) {
-            const int live = min(16, s1 - s0 - 16 * q);
-            if (live <= 0) break;
-            const f32x4v y = get_Y(rt + 16 * q * kRow, live);
-            float f1 = 0.0f;
-            f32x4v v = {0, 0, 0, 0};
-            chain_block<K>(so, y, h[q], dh[q], f1, v);
-            put_V(rt + 16 * q * kRow, live, f1, v);
+            const int live = min(16, n - 16 * q);
+            if (live > 0) {
+              const f32x4v y = get_Y(rt + 16 * q * kRow, live);
+              float f1 = 0.0f;
+              f32x4v v = {0, 0, 0, 0};
+              chain_block<K>(so, y, h[q], dh[q], f1, v);
+              put_V(rt + 16 * q * kRow, live, f1, v);
+            }
           }
-          continue;
+          done = true;
         }
       }
-      // any other slot: H is interpolated again for the chain rule
-      for (int w0 = one ? lo : s0; w0 < s1; w0 += T::WIN) {
-        const int wn = min(T::WIN, (one ? hi : s1) - w0);
-        if (!one) stage(g, cell, xi, pos, kept + w0, wn, rows);
-        const int c0 = max(s0 - w0, 0), c1 = min(s1 - w0, wn);
-        for (int r0 = c0; r0 < c1; r0 += 16) {
-          const int live = min(16, c1 - r0);
-#pragma unroll
-          for (int fb = 0; fb < T::NB; fb++) {
-            float h[T::NFB];
-            radial_tile<K, false>(g, tab, rows + r0 * kRow, live, fb, h, nullptr);
-            put_tile<K>(h, hb);
-            wave_sync();
-            moments_tile<K>(rows + r0 * kRow, live, hb, acc + fb * T::CT);
-            wave_sync();
-          }
+      if (!done) {
+        slot_moments<K>(tab, rt, n, hb, acc);
+        slot_S<K>(acc, gv, g.tsym, sb);
+        wave_sync();
+        if constexpr (T::kSRegs) {
+          load_S<K>(sb, 0, so);
+          wave_sync();
         }
+        slot_chain<K>(tab, rt, n, sb, so, hb);
+        request(bn);
+      }
+      b = bn;
+    }
+    wave_sync();
+    double cf[9];
+#pragma unroll
+    for (int q = 0; q < 9; q++) cf[q] = 0.0;
+    if (lane < nk) neighbor_force(g, d0, (int) (e0 & kNbrJMask), rows + lane * kRow, scale, vatom, cf);
+    if (64 + lane < nk) {
+      double d1[3];
+      displacement(xi, pos[e1 & kNbrJMask], e1 >> kNbrJBits, cell, d1);
+      neighbor_force(g, d1, (int) (e1 & kNbrJMask), rows + (64 + lane) * kRow, scale, vatom, cf);
+    }
+    wave_sync();
+    scatter(rows, nk, f, vatom);
+    add_sums(cf, facc);
+  } else {
+    // a longer list: slot by slot, P and then the chain rule in windows
+    for (int b = 0; b < g.nelt; b++) {
+      const int s0 = start(b), s1 = start(b + 1);
+      if (s0 >= s1) continue;
+      float4 gv[T::KT];
+      load_dEdG<K>(grow + (size_t) b * K * kNM, gv);
+      f32x4v acc[T::KT];
+#pragma unroll
+      for (int t = 0; t < T::KT; t++) acc[t] = f32x4v{0, 0, 0, 0};
+      for (int w0 = s0; w0 < s1; w0 += T::WIN) {
+        const int wn = min(T::WIN, s1 - w0);
+        stage(g, cell, xi, pos, kept + w0, wn, rows);
+        slot_moments<K>(tab, rows, wn, hb, acc);
       }
       slot_S<K>(acc, gv, g.tsym, sb);
       wave_sync();
@@ -701,45 +858,27 @@ __global__ __launch_bounds__(64, (kForceWaves<K>)) void k_force(ModelGeo g, Geom
         load_S<K>(sb, 0, so);
         wave_sync();
       }
-      for (int w0 = one ? lo : s0; w0 < s1; w0 += T::WIN) {
-        const int wn = min(T::WIN, (one ? hi : s1) - w0);
-        if (!one) stage(g, cell, xi, pos, kept + w0, wn, rows);
-        const int c0 = max(s0 - w0, 0), c1 = min(s1 - w0, wn);
-        for (int r0 = c0; r0 < c1; r0 += 16) {
-          const int live = min(16, c1 - r0);
-          float *rt = rows + r0 * kRow;
-          const f32x4v y = get_Y(rt, live);
-          float f1 = 0.0f;
-          f32x4v v = {0, 0, 0, 0};
-#pragma unroll 1
-          for (int fb = 0; fb < T::NB; fb++) {
-            float hq[T::NFB], dq[T::NFB], h[T::NFB], dh[T::NFB];
-            radial_tile<K, true>(g, tab, rt, live, fb, hq, dq);
-            put_tile<K>(dq, hb);
-            wave_sync();
-            get_chain<K>(hb, dh);
-            wave_sync();
-            put_tile<K>(hq, hb);
-            wave_sync();
-            get_chain<K>(hb, h);
-            wave_sync();
-            if constexpr (!T::kSRegs) load_S<K>(sb, fb, so);
-            chain_block<K>(so, y, h, dh, f1, v);
-          }
-          put_V(rt, live, f1, v);
+      for (int w0 = s0; w0 < s1; w0 += T::WIN) {
+        const int wn = min(T::WIN, s1 - w0);
+        if (s1 - s0 > T::WIN) stage(g, cell, xi, pos, kept + w0, wn, rows);
+        slot_chain<K>(tab, rows, wn, sb, so, hb);
+        double cf[9];
+#pragma unroll
+        for (int q = 0; q < 9; q++) cf[q] = 0.0;
+        for (int c = lane; c < wn; c += 64) {
+          const uint32_t e = kept[w0 + c];
+          double d[3];
+          displacement(xi, pos[e & kNbrJMask], e >> kNbrJBits, cell, d);
+          neighbor_force(g, d, (int) (e & kNbrJMask), rows + c * kRow, scale, vatom, cf);
         }
-        if (!one) {
-          wave_sync();
-          finish(g, cell, xi, pos, kept + w0, wn, rows, scale, f, vatom, facc);
-          wave_sync();
-        }
+        wave_sync();
+        scatter(rows, wn, f, vatom);
+        add_sums(cf, facc);
+        wave_sync();
       }
     }
-    wave_sync();
-    if (one) finish(g, cell, xi, pos, kept + lo, hi - lo, rows, scale, f, vatom, facc);
-    wave_sync();
-    b0 = b1;
   }
+  wave_sync();
   if (lane < 3) atomicAdd(&f[3 * (size_t) i + lane], facc[lane]);
   if (lane < 6) {
     const double v = facc[3 + lane];

@@ -27,13 +27,19 @@ __device__ inline void displacement(const double4 &xi, const double4 &xj, uint32
                                     const Box &c, double d[3])
 {
 #pragma clang fp contract(off)
+  d[0] = xj.x - xi.x;
+  d[1] = xj.y - xi.y;
+  d[2] = xj.z - xi.z;
+  // no image shift in the whole wave (list mode, and most atoms of a large
+  // cell): nothing to decode or add
+  if (__builtin_amdgcn_ballot_w64(code != kShiftCenter) == 0ull) return;
   int s0 = (int) (code / 49u) - 3, s1 = (int) ((code / 7u) % 7u) - 3, s2 = (int) (code % 7u) - 3;
   double sh0 = ((double) s0 * c.h[0] + (double) s1 * c.h[3]) + (double) s2 * c.h[6];
   double sh1 = ((double) s0 * c.h[1] + (double) s1 * c.h[4]) + (double) s2 * c.h[7];
   double sh2 = ((double) s0 * c.h[2] + (double) s1 * c.h[5]) + (double) s2 * c.h[8];
-  d[0] = (xj.x - xi.x) + sh0;
-  d[1] = (xj.y - xi.y) + sh1;
-  d[2] = (xj.z - xi.z) + sh2;
+  d[0] += sh0;
+  d[1] += sh1;
+  d[2] += sh2;
 }
 
 __device__ inline double dist2(const double d[3])
@@ -67,34 +73,35 @@ __device__ inline void monomials20(float x, float y, float z, float *M)
   M[19] = z * zz;
 }
 
-// Kerley rational interpolation of one filter (gpu/cuda/ration.cu:59-68),
-// table entry t = (y, s, c1, c2), q = r - n dx, p = dx - q, qp = q - p:
+// Kerley rational interpolation of one filter (gpu/cuda/ration.cu:59-68) in
+// units of the grid step: table entry t = (y, s dx, c1 dx^2, c2 dx^2),
+// q = r / dx - n, p = 1 - q, qp = q - p:
 //   w = |c2 p| / (|c2 p| + |c1 q|)  (0 when both vanish)
 //   c = c2 + w (c1 - c2),  h = y + q (s - p c),
-//   dh/dr = s + (q - p) c + dx w (1 - w) (c1 - c2)
-// (the last term is the reference's dx (c - c2)(1 - w)).  The max() stands
-// for its "denominator > 0" test: a zero denominator has a zero numerator.
-// The caller zeroes the two end cells.
-__device__ inline float kerley_w(float4 t, float q, float p)
+//   dx dh/dr = s + (q - p) c + w (1 - w) (c1 - c2)
+// (the last term is the reference's dx (c - c2)(1 - w)).  Evaluated through
+// 1 - w = |c1 q| / den: the smallest normal number added to |c1 q| makes the
+// denominator positive and 1 - w = 1 when both vanish, and is lost in
+// rounding otherwise.
+__device__ inline float kerley_w1(float4 t, float q, float p)
 {
-  float a = fabsf(t.w) * fabsf(p);
-  float den = fmaf(fabsf(t.z), fabsf(q), a);
-  return a * __builtin_amdgcn_rcpf(fmaxf(den, 1.17549435e-38f));  // 1-ulp reciprocal
+  const float b = fmaf(fabsf(t.z), fabsf(q), 1.17549435e-38f);
+  return b * __builtin_amdgcn_rcpf(fmaf(fabsf(t.w), fabsf(p), b));  // 1-ulp reciprocal
 }
 
 __device__ inline float kerley_h(float4 t, float q, float p)
 {
-  float c = fmaf(kerley_w(t, q, p), t.z - t.w, t.w);
+  const float c = fmaf(kerley_w1(t, q, p), t.w - t.z, t.z);
   return fmaf(q, fmaf(-p, c, t.y), t.x);
 }
 
-__device__ inline void kerley(float4 t, float q, float p, float qp, float dx, float &h, float &dh)
+__device__ inline void kerley(float4 t, float q, float p, float qp, float &h, float &dxdh)
 {
-  float w = kerley_w(t, q, p);
-  float dc = t.z - t.w;
-  float c = fmaf(w, dc, t.w);
+  const float w = kerley_w1(t, q, p);
+  const float dc = t.w - t.z;
+  const float c = fmaf(w, dc, t.z);
   h = fmaf(q, fmaf(-p, c, t.y), t.x);
-  dh = fmaf(dx * dc, fmaf(-w, w, w), fmaf(qp, c, t.y));
+  dxdh = fmaf(dc, fmaf(w, w, -w), fmaf(qp, c, t.y));
 }
 
 // Cross-lane moves within a row of 16 lanes (DPP: no LDS traffic).
@@ -259,7 +266,8 @@ __device__ inline double rsqrt_fp64(double r2)
 }
 
 // Geometry of one kept neighbor: FP64 displacement, unit vector and r, and
-// the radial-table cell n with the offsets q, dx - q (ration.cu:29-32).
+// the radial-table cell n with the offsets q = r / dx - n, 1 - q
+// (ration.cu:29-32).
 struct NbrGeo {
   double d[3];
   double r;
@@ -280,9 +288,9 @@ __device__ inline void nbr_geometry(const ModelGeo &g, const Box &cell, const do
   o.uy = (float) (o.d[1] * rinv);
   o.uz = (float) (o.d[2] * rinv);
   o.n = min(g.tab_n - 2, (int) (o.r * g.xdx));
-  double qd = o.r - (double) o.n * g.dx;
+  const double qd = o.r * g.rdx - (double) o.n;
   o.q = (float) qd;
-  o.pq = (float) (g.dx - qd);
+  o.pq = (float) (1.0 - qd);
 }
 
 // the end cells of the table are zero (ration.hpp:29)

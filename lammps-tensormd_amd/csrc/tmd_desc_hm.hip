@@ -289,7 +289,7 @@ __global__ __launch_bounds__(64) void k_force_hm(ModelGeo g, Geom geo, const dou
           const float4 *trow = tab + (size_t) ng.n * K;
           for (int k = 0; k < K; k++) {
             float h, dh;
-            kerley(trow[k], ng.q, ng.pq, qp, g.dxf, h, dh);
+            kerley(trow[k], ng.q, ng.pq, qp, h, dh);
             const float *Sk = Pl + k * ND;
             float U = 0.0f;
 #pragma unroll
@@ -300,6 +300,7 @@ __global__ __launch_bounds__(64) void k_force_hm(ModelGeo g, Geom geo, const dou
             }
             f1 = fmaf(U, dh, f1);
           }
+          f1 *= g.rdxf;  // dh is dx dH/dr
           // g_beta = sum_d V_d dM_d/du_beta
           float px[MM + 1], py[MM + 1], pz[MM + 1];
           px[0] = py[0] = pz[0] = 1.0f;

@@ -47,8 +47,10 @@ struct ModelGeo {
   int mm;    // max_moment as evaluated: 3 (0-2 are padded to 3), 4 or 5
   uint32_t slots[kMaxElts];
   double rc2;
-  double dx, xdx;
-  float dxf;
+  // grid step dx of the radial table: xdx finds the cell (the model's 1 / dx,
+  // rounded to FP32 in a precision-32 model), rdx = 1 / dx scales offsets
+  double xdx, rdx;
+  float rdxf;
 };
 
 // Row layout of the MLP: rows are atoms grouped by element; each element
