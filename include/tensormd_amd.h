@@ -215,9 +215,9 @@ int tmd_md_run(tmd_system *sys, int nsteps, double dt, double *epot, double *eki
 int tmd_md_step_async(tmd_system *sys, double dt);
 /* Run nsteps MD steps with HIP events recorded on the library stream
  * between phases; ms[0..6] = mean ms per step spent in: neighbor
- * maintenance, descriptor kernel, MLP kernel, force kernel, FP64
- * reductions (with the force-buffer clears), integration, and the whole
- * step. */
+ * rebuilds, descriptor kernel, MLP kernel, force kernel, FP64
+ * reductions (with the second half kick), the first half kick, drift,
+ * displacement check and force-buffer clear, and the whole step. */
 int tmd_md_profile(tmd_system *sys, int nsteps, double dt, double *ms);
 /* Sampled kernel timing inside tmd_md_run.  No counterpart in the reference
  * (benchmark instrumentation: kernel durations measured over a timed run).

@@ -478,11 +478,7 @@ int run_chain(tmd_ctx *ctx, Workspace &w, const Chain &c, hipStream_t s, PhaseEv
     if (e != hipSuccess) return hip_fail(ctx, e, "mlp launch");
   }
   if (pe && (e = hipEventRecord(pe->ev[2], s)) != hipSuccess) return hip_fail(ctx, e, "timing event");
-  if (c.dyn)
-    e = launch_zero_atoms(c.f, 3, (int) (c.fbytes / (3 * sizeof(double))), c.dyn, s);
-  else
-    e = launch_zero(c.f, c.fbytes, s);
-  if (e != hipSuccess) return hip_fail(ctx, e, "zero f");
+  if (!c.f_cleared && (e = launch_zero(c.f, c.fbytes, s)) != hipSuccess) return hip_fail(ctx, e, "zero f");
   if (c.vatom && (e = launch_zero(c.vatom, c.vbytes, s)) != hipSuccess)
     return hip_fail(ctx, e, "zero vatom");
   if (c.zero_ew && (e = launch_zero(eatom, (size_t) c.natoms * 7 * sizeof(double), s)) != hipSuccess)
@@ -493,10 +489,28 @@ int run_chain(tmd_ctx *ctx, Workspace &w, const Chain &c, hipStream_t s, PhaseEv
                    watom, c.vatom, s);
   if (e != hipSuccess) return hip_fail(ctx, e, "force launch");
   if (pe && (e = hipEventRecord(pe->ev[4], s)) != hipSuccess) return hip_fail(ctx, e, "timing event");
-  if (c.struct_off)
-    e = launch_reduce_struct(eatom, watom, c.struct_off, c.nstruct, c.struct_out, s, c.dyn);
-  else
-    e = launch_reduce_ev(eatom, watom, c.natoms, (double *) w.red.p, s);
+  unsigned long long *ctl = c.nb ? c.nb->ctl : nullptr;
+  const double trig2 = c.nb ? c.nb->trig2 : 0.0;
+  if (c.struct_off) {
+    e = launch_reduce_struct(eatom, watom, c.struct_off, c.nstruct, c.struct_out, ctl, trig2, s, c.dyn);
+  } else {
+    StepTail t{};
+    t.eatom = eatom;
+    t.watom = watom;
+    t.n = c.natoms;
+    t.out = (double *) w.red.p;
+    t.ctl = ctl;
+    t.trig2 = trig2;
+    t.pos = c.pos;
+    t.v = c.v;
+    t.f = c.f;
+    t.dtfm = c.dtfm;
+    t.mass = c.mass;
+    t.hist = c.hist;
+    t.counter = c.hist_counter;
+    t.hist_cap = c.hist_cap;
+    e = launch_step_tail(t, s);
+  }
   if (e != hipSuccess) return hip_fail(ctx, e, "reduce launch");
   if (pe && (e = hipEventRecord(pe->ev[5], s)) != hipSuccess) return hip_fail(ctx, e, "timing event");
   return TMD_OK;

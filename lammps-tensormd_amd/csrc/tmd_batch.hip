@@ -109,6 +109,10 @@ __global__ void k_batch_unpack(const unsigned char *stage, BatchCaps caps, Batch
     }
     a.pos[q] = p;
   }
+  // cleared for this batch's list build and force sums
+  for (int q = tid; q < 3 * n; q += stride) a.f[q] = 0.0;
+  for (int q = tid; q < d.nbins; q += stride) a.bin_count[q] = 0;
+  if (tid == 0) *a.bin_total = 0;
   if (bad) atomicOr(&a.dyn->pad, 1);
 }
 

@@ -152,6 +152,60 @@ __device__ inline double wave_sum_d_lp(double v)
   return v;
 }
 
+// a's lanes 0-31 + 32-63 in lanes 0-31, b's in lanes 32-63
+__device__ inline float swap32_add(float a, float b)
+{
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+// rows of 16 lanes: row 0 of the result = a's rows 0 + 1, row 1 = b's rows
+// 0 + 1, row 2 = a's rows 2 + 3, row 3 = b's rows 2 + 3
+__device__ inline float swap16_add(float a, float b)
+{
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+__device__ inline double make_d(unsigned lo, unsigned hi)
+{
+  return __longlong_as_double((long long) (((unsigned long long) hi << 32) | lo));
+}
+
+__device__ inline double swap32_add(double a, double b)
+{
+  const unsigned long long ua = (unsigned long long) __double_as_longlong(a), ub = (unsigned long long) __double_as_longlong(b);
+  const auto l = __builtin_amdgcn_permlane32_swap((unsigned) ua, (unsigned) ub, false, false);
+  const auto h = __builtin_amdgcn_permlane32_swap((unsigned) (ua >> 32), (unsigned) (ub >> 32), false, false);
+  return make_d(l[0], h[0]) + make_d(l[1], h[1]);
+}
+
+__device__ inline double swap16_add(double a, double b)
+{
+  const unsigned long long ua = (unsigned long long) __double_as_longlong(a), ub = (unsigned long long) __double_as_longlong(b);
+  const auto l = __builtin_amdgcn_permlane16_swap((unsigned) ua, (unsigned) ub, false, false);
+  const auto h = __builtin_amdgcn_permlane16_swap((unsigned) (ua >> 32), (unsigned) (ub >> 32), false, false);
+  return make_d(l[0], h[0]) + make_d(l[1], h[1]);
+}
+
+// Orders LDS accesses of the workgroup's only wave: its LDS instructions run
+// in order, so the compiler must keep the order and nothing has to be waited
+// for.
+__device__ inline void wave_sync()
+{
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+__device__ inline double row_sum_d(double v)
+{
+  v += dpp_d<kDppXor1>(v);
+  v += dpp_d<kDppXor2>(v);
+  v += dpp_d<kDppRor4>(v);
+  v += dpp_d<kDppRor8>(v);
+  return v;
+}
+
 __device__ inline unsigned lane_rank(unsigned long long m)
 {
   return __builtin_amdgcn_mbcnt_hi((unsigned) (m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned) m, 0u));

@@ -121,19 +121,27 @@ struct NbrBuild {
   const CellInfo *cells;   // [ncells] (device)
   const int *atom_struct;  // [n] cell of each atom, or null (one cell)
   const BatchDims *dyn;    // device extents (n, nbins) when non-null
-  int *bin_count;     // [nbins + 1]
-  int *bin_start;     // [nbins + 1]
-  int *bin_cursor;    // [nbins]
+  int *bin_count;     // [nbins]
+  int *bin_start;     // [nbins]
+  int *bin_total;     // [1] atoms placed so far
   int *bin_atoms;     // [n]
   int *atom_bin;      // [n] flat bin
+  int *atom_rank;     // [n] arrival rank in the bin
   int *atom_bc;       // [n][3] bin coordinates
+  double4 *sorted;    // [n] positions in bin order, w = atom index
   double *x_build;    // [n][4]
   unsigned long long *ctl;  // [0] max d^2 bits, [1] force flag, [2] overflow, [3] build count
 };
 
-hipError_t nbr_step(const NbrBuild &nb, double4 *pos, uint32_t *nbr, int *nn, hipStream_t stream);
-// force the next nbr_step to rebuild (device-side flag; graph-safe)
-hipError_t nbr_force_rebuild(const NbrBuild &nb, hipStream_t stream);
+// One neighbor-list update: a check (nbr_check, or launch_vv_first, which
+// moves the atoms first), the rebuild kernels, which return at once when none
+// is due, and at the end of the evaluation the reset of the control word
+// (StepTail / launch_reduce_struct).
+hipError_t nbr_check(const NbrBuild &nb, const double4 *pos, hipStream_t stream);
+hipError_t nbr_rebuild(const NbrBuild &nb, double4 *pos, uint32_t *nbr, int *nn, hipStream_t stream);
+// first half kick and drift, the displacement check, and f = 0
+hipError_t launch_vv_first(const NbrBuild &nb, int n, double4 *pos, double *v, double *f, const double *dtfm,
+                           double dt, hipStream_t stream);
 
 // ---- descriptor / force -------------------------------------------------------
 // Geometry of an evaluation: cells[atom_struct[i]] (atom_struct null: cells[0]).
@@ -253,9 +261,10 @@ struct BatchArrays {
   int *row2atom;      // [rows]
   double4 *pos;       // [atoms]
   const double *struct_out;  // [structs][7]
-  const double *f;           // [atoms][3]
+  double *f;                 // [atoms][3]
   const double *eatom;       // [atoms]
   unsigned long long *ctl;   // neighbor control word
+  int *bin_count, *bin_total;
 };
 // Dense host staging of a batch: BatchDims | struct_off[ns+1] | cells[ns] |
 // atom_struct[n] | row2atom[nrows] | pos[n].  Byte offsets from the start:
@@ -276,7 +285,8 @@ __host__ __device__ inline void batch_stage_offsets(int ns, int n, int nrows, si
 // atoms, structures, error flag) | struct_out[ns][7] | f[n][3] | eatom[n].
 inline size_t batch_out_bytes(int ns, int n) { return 8 * (8 + 7 * (size_t) ns + 4 * (size_t) n); }
 // Copy a staged batch (host memory, read by the kernels) into the slot's
-// device arrays, clamping every count and index to the capacities.
+// device arrays, clamping every count and index to the capacities; forces and
+// bin counts of the batch are cleared.
 hipError_t launch_batch_unpack(const void *stage, const BatchCaps &caps, const BatchArrays &a,
                                hipStream_t stream);
 // Write a finished batch's results to host memory `out` and clear the
@@ -288,33 +298,36 @@ hipError_t launch_batch_pack(void *out, const BatchCaps &caps, const BatchArrays
 hipError_t launch_zero(void *p, size_t bytes, hipStream_t stream);
 // plain device-to-device copy (bandwidth calibration)
 hipError_t launch_copy(const void *src, void *dst, size_t bytes, hipStream_t stream);
-// out[0] = sum_i eatom[i]; out[1..6] = sum_i watom[i][*], i < n (fixed order)
-hipError_t launch_reduce_ev(const double *eatom, const double *watom, int n, double *out,
-                            hipStream_t stream);
+// What follows the force kernel of one evaluation: out[0] = sum_i eatom[i]
+// and out[1..6] = sum_i watom[i][*] (fixed order; out holds 8 + 8 kSumParts
+// doubles), the neighbor list's control word reset (ctl non-null), and, with
+// v non-null, the second half kick of velocity Verlet and the kinetic energy
+// sum(m v^2)/2 * mvv2e; with hist non-null the step's energies recorded at
+// hist[2 n], n = (*counter)++ (safe to replay in a graph).
+struct StepTail {
+  const double *eatom, *watom;
+  int n;
+  double *out;
+  unsigned long long *ctl;
+  double trig2;
+  const double4 *pos;
+  double *v;
+  const double *f, *dtfm, *mass;
+  double *hist;
+  unsigned long long *counter;
+  int hist_cap;
+};
+constexpr int kSumParts = 240;
+hipError_t launch_step_tail(const StepTail &t, hipStream_t stream);
 // per structure s: out[7 s + 0] = sum eatom, out[7 s + 1..6] = sum watom over
-// atoms [off[s], off[s+1])
+// atoms [off[s], off[s+1]); resets ctl
 // (with dyn: nstruct is the capacity, dyn->nstruct the live count)
 hipError_t launch_reduce_struct(const double *eatom, const double *watom, const int *off,
-                                int nstruct, double *out, hipStream_t stream,
-                                const BatchDims *dyn = nullptr);
-// p[0 .. per_atom * dyn->natoms) = 0 (grid sized for cap_atoms)
-hipError_t launch_zero_atoms(double *p, int per_atom, int cap_atoms, const BatchDims *dyn,
-                             hipStream_t stream);
-hipError_t launch_vv_first(int n, double4 *pos, double *v, const double *f,
-                           const double *dtfm_by_elem, double dt, hipStream_t stream);
-hipError_t launch_vv_second(int n, const double4 *pos, double *v, const double *f,
-                            const double *dtfm_by_elem, hipStream_t stream);
-// kinetic energy sum(m v^2)/2 * mvv2e into out[0] (out zeroed inside)
-hipError_t launch_ekin(int n, const double4 *pos, const double *v, const double *mass_by_elem,
-                       double *out, hipStream_t stream);
-// per-step energy history through a device counter (safe to replay in a graph)
+                                int nstruct, double *out, unsigned long long *ctl, double trig2,
+                                hipStream_t stream, const BatchDims *dyn = nullptr);
 // *acc += sum of the kept-neighbor counts of the real rows (row2atom >= 0)
 // in the kept-list cache kl (words per row)
 hipError_t launch_sum_kept(const uint32_t *kl, size_t words, const int *row2atom, int nrows,
                            unsigned long long *acc, hipStream_t s);
-hipError_t launch_record_step(const double *epot, const double *ekin, double *hist,
-                              unsigned long long *counter, int cap, hipStream_t stream);
-// copy e (per-step scalars) into history slots
-hipError_t launch_copy_scalar(const double *src, double *dst, hipStream_t stream);
 
 }  // namespace tmd

@@ -118,7 +118,8 @@ struct tmd_ctx {
 namespace tmd {
 // Optional events recorded between the phases of one evaluation:
 // [0] start, [1] after descriptor, [2] after MLP, [3] after the force-buffer
-// clears (just before the force kernel), [4] after force, [5] after reductions
+// clears (just before the force kernel), [4] after force, [5] after the sums
+// (with the second half kick in an MD step)
 struct PhaseEvents {
   hipEvent_t ev[6];
 };
@@ -143,8 +144,9 @@ struct Chain {
   const int *nn = nullptr;
   int cap = 0;
   double scale = 1.0;
-  double *f = nullptr;       // zeroed, then accumulated
+  double *f = nullptr;       // zeroed unless f_cleared, then accumulated
   size_t fbytes = 0;
+  bool f_cleared = false;    // an earlier kernel of this evaluation cleared f
   double *vatom = nullptr;   // optional; zeroed, then accumulated
   size_t vbytes = 0;
   int natoms = 0;            // eatom/watom entries (in w.ew)
@@ -152,6 +154,15 @@ struct Chain {
   const int *struct_off = nullptr;  // per-structure sums into struct_out[7 s ..]
   int nstruct = 0;
   double *struct_out = nullptr;     // (null struct_off: one sum into w.red[0..6])
+  // the list whose control word the evaluation resets (null in list mode)
+  const NbrBuild *nb = nullptr;
+  // the second half of a velocity-Verlet step rides on the sums: velocities,
+  // per-element constants, and optionally the energy history (StepTail)
+  double *v = nullptr;
+  const double *dtfm = nullptr, *mass = nullptr;
+  double *hist = nullptr;
+  unsigned long long *hist_counter = nullptr;
+  int hist_cap = 0;
   int rtile = 0;
   const BatchDims *dyn = nullptr;   // device extents of a batch (capture-once graphs)
   // BF16 descriptor rows where the MLP launch takes them (mlp_bf16_rows):

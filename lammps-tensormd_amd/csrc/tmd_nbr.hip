@@ -18,6 +18,8 @@
 // different structures never see each other.
 #include "tmd_device.h"
 
+#include <algorithm>
+
 namespace tmd {
 
 namespace {
@@ -55,18 +57,33 @@ __device__ inline bool rebuild_due(const unsigned long long *ctl, double trig2)
   return ctl[1] != 0ull || m > trig2;
 }
 
-// max |x - x_build|^2 over atoms -> ctl[0] (as ordered bits of a positive double)
-__global__ void k_nb_check(NbrBuild nb, const double4 *pos, const double *xb, unsigned long long *ctl)
+// Inclusive sum over the lanes (DPP: shifts within rows of 16, then the row
+// totals 15 -> 16.., 31 -> 32.. broadcast to the rows behind).
+__device__ inline int wave_scan(int v)
 {
-  const int n = live_atoms(nb);
-  if ((int) (blockIdx.x * blockDim.x) >= n) return;
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  double d2 = 0.0;
-  if (i < n) {
-    double4 p = pos[i];
-    double dx = p.x - xb[4 * i], dy = p.y - xb[4 * i + 1], dz = p.z - xb[4 * i + 2];
-    d2 = dx * dx + dy * dy + dz * dz;
-  }
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, false);  // row_shr:1
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, false);  // row_shr:2
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, false);  // row_shr:4
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, false);  // row_shr:8
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false);  // row_bcast:15 into rows 1 and 3
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false);  // row_bcast:31 into rows 2 and 3
+  return v;
+}
+
+// Clears the bin counts for a build that may follow in this step: part `id`
+// of `stride` threads.  Runs in the kernel before the build's first one.
+__device__ inline void clear_bins(const NbrBuild &nb, int id, int stride)
+{
+  const int nbins = live_bins(nb, nb.nbins);
+  for (int b = id; b < nbins; b += stride) nb.bin_count[b] = 0;
+  if (id == 0) *nb.bin_total = 0;
+}
+
+// ctl[0] = the largest d2 of the workgroups whose largest exceeds the trigger
+// (as ordered bits of a positive double): no one else's matters, and one
+// atomic per workgroup on one word cost 5 us at 128,000 atoms.
+__device__ inline void report_move(double d2, double trig2, unsigned long long *ctl)
+{
   for (int o = 32; o > 0; o >>= 1) d2 = fmax(d2, __shfl_xor(d2, o));
   __shared__ double wmax[16];
   if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = d2;
@@ -74,16 +91,55 @@ __global__ void k_nb_check(NbrBuild nb, const double4 *pos, const double *xb, un
   if (threadIdx.x == 0) {
     double m = 0.0;
     for (int w = 0; w < (int) (blockDim.x >> 6); w++) m = fmax(m, wmax[w]);
-    if (m > 0.0) atomicMax(&ctl[0], (unsigned long long) __double_as_longlong(m));
+    if (m > trig2) atomicMax(&ctl[0], (unsigned long long) __double_as_longlong(m));
   }
 }
 
-// wrap into the cell, remember build positions, bin the atoms
-__global__ void k_nb_bin(NbrBuild nb, double4 *pos)
+__device__ inline double moved2(const NbrBuild &nb, int i, const double4 &p)
 {
-  if (!rebuild_due(nb.ctl, nb.trig2)) return;
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= live_atoms(nb)) return;
+  const double dx = p.x - nb.x_build[4 * (size_t) i], dy = p.y - nb.x_build[4 * (size_t) i + 1],
+               dz = p.z - nb.x_build[4 * (size_t) i + 2];
+  return dx * dx + dy * dy + dz * dz;
+}
+
+// max |x - x_build|^2 over atoms, and the bin counts cleared
+__global__ void k_nb_check(NbrBuild nb, const double4 *pos)
+{
+  const int n = live_atoms(nb);
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  clear_bins(nb, i, gridDim.x * blockDim.x);
+  report_move(i < n ? moved2(nb, i, pos[i]) : 0.0, nb.trig2, nb.ctl);
+}
+
+// First half of a velocity-Verlet step (src/fix_nve.cpp:64-98) with the
+// displacement check of the new positions; the forces, read here, are
+// cleared for the force kernel.
+__global__ void k_vv_first(NbrBuild nb, int n, double4 *pos, double *v, double *f, const double *dtfm, double dt)
+{
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  clear_bins(nb, i, gridDim.x * blockDim.x);
+  double d2 = 0.0;
+  if (i < n) {
+    double4 p = pos[i];
+    const double c = dtfm[(int) p.w];
+    const size_t q = 3 * (size_t) i;
+    const double vx = v[q] + c * f[q], vy = v[q + 1] + c * f[q + 1], vz = v[q + 2] + c * f[q + 2];
+    v[q] = vx;
+    v[q + 1] = vy;
+    v[q + 2] = vz;
+    f[q] = f[q + 1] = f[q + 2] = 0.0;
+    p.x += dt * vx;
+    p.y += dt * vy;
+    p.z += dt * vz;
+    pos[i] = p;
+    d2 = moved2(nb, i, p);
+  }
+  report_move(d2, nb.trig2, nb.ctl);
+}
+
+// wrap atom i into its cell, remember its build position; returns its bin
+__device__ inline int bin_atom(const NbrBuild &nb, double4 *pos, int i)
+{
   const CellInfo &c = cell_of(nb, i);
   double4 p = pos[i];
   double f[3];
@@ -98,186 +154,267 @@ __global__ void k_nb_bin(NbrBuild nb, double4 *pos)
     pos[i] = p;
     for (int a = 0; a < 3; a++) f[a] -= s[a];
   }
-  nb.x_build[4 * i + 0] = p.x;
-  nb.x_build[4 * i + 1] = p.y;
-  nb.x_build[4 * i + 2] = p.z;
+  nb.x_build[4 * (size_t) i + 0] = p.x;
+  nb.x_build[4 * (size_t) i + 1] = p.y;
+  nb.x_build[4 * (size_t) i + 2] = p.z;
   int b[3];
   for (int a = 0; a < 3; a++) {
     int q = (int) floor(f[a] * c.nb[a]);
     b[a] = min(max(q, 0), c.nb[a] - 1);
-    nb.atom_bc[3 * i + a] = b[a];
+    nb.atom_bc[3 * (size_t) i + a] = b[a];
   }
-  int flat = c.bin_base + (b[0] * c.nb[1] + b[1]) * c.nb[2] + b[2];
-  nb.atom_bin[i] = flat;
-  atomicAdd(&nb.bin_count[flat], 1);
+  return c.bin_base + (b[0] * c.nb[1] + b[1]) * c.nb[2] + b[2];
 }
 
-// exclusive scan of bin counts (single workgroup of 1024 threads)
-__global__ void k_nb_scan(NbrBuild nb, int nbins)
+// An atom and its position at its place in the bin-sorted order: w holds
+// the index (exact in FP64).
+__device__ inline double4 sorted_entry(const double4 &p, int i) { return make_double4(p.x, p.y, p.z, (double) i); }
+
+// ---- bins of a large system: one kernel per phase ----
+// Each atom's bin, and an arrival rank within it (any order).
+__global__ void k_nb_bin(NbrBuild nb, double4 *pos)
 {
   if (!rebuild_due(nb.ctl, nb.trig2)) return;
-  nbins = live_bins(nb, nbins);
-  __shared__ int part[1024];
-  int t = threadIdx.x;
-  int per = (nbins + 1023) / 1024;
-  int lo = t * per, hi = min(lo + per, nbins);
-  int s = 0;
-  for (int b = lo; b < hi; b++) s += nb.bin_count[b];
-  part[t] = s;
-  __syncthreads();
-  for (int o = 1; o < 1024; o <<= 1) {
-    int v = (t >= o) ? part[t - o] : 0;
-    __syncthreads();
-    part[t] += v;
-    __syncthreads();
-  }
-  int run = (t == 0) ? 0 : part[t - 1];
-  for (int b = lo; b < hi; b++) {
-    nb.bin_start[b] = run;
-    nb.bin_cursor[b] = run;
-    run += nb.bin_count[b];
-  }
-  if (t == 1023) nb.bin_start[nbins] = part[1023];
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= live_atoms(nb)) return;
+  const int flat = bin_atom(nb, pos, i);
+  nb.atom_bin[i] = flat;
+  nb.atom_rank[i] = atomicAdd(&nb.bin_count[flat], 1);
+}
+
+// Room for every bin's atoms: consecutive within 64 bins, the groups of 64
+// in any order (one counter update per group; the list kernel reads bins
+// through their starts, so their order does not reach the list).
+__global__ void k_nb_alloc(NbrBuild nb, int nbins)
+{
+  if (!rebuild_due(nb.ctl, nb.trig2)) return;
+  const int b = blockIdx.x * blockDim.x + threadIdx.x, lane = threadIdx.x & 63;
+  const bool in = b < live_bins(nb, nbins);
+  const int cnt = in ? nb.bin_count[b] : 0;
+  const int incl = wave_scan(cnt);
+  int base = 0;
+  if (lane == 63) base = atomicAdd(nb.bin_total, incl);
+  base = __shfl(base, 63);
+  if (in) nb.bin_start[b] = base + incl - cnt;
 }
 
 __global__ void k_nb_fill(NbrBuild nb)
 {
   if (!rebuild_due(nb.ctl, nb.trig2)) return;
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= live_atoms(nb)) return;
-  int slot = atomicAdd(&nb.bin_cursor[nb.atom_bin[i]], 1);
-  nb.bin_atoms[slot] = i;
+  nb.bin_atoms[nb.bin_start[nb.atom_bin[i]] + nb.atom_rank[i]] = i;
 }
 
-// make the order inside each bin deterministic (ascending atom index)
-__global__ void k_nb_sortbins(NbrBuild nb, int nbins)
+// Ascending atom index inside each bin (a deterministic order): an atom's
+// place is the number of smaller indices among its bin's atoms.
+__global__ void k_nb_sort(NbrBuild nb, const double4 *pos)
 {
   if (!rebuild_due(nb.ctl, nb.trig2)) return;
-  int b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= live_bins(nb, nbins)) return;
-  int lo = nb.bin_start[b], hi = nb.bin_start[b + 1];
-  for (int p = lo + 1; p < hi; p++) {
-    int v = nb.bin_atoms[p];
-    int q = p - 1;
-    while (q >= lo && nb.bin_atoms[q] > v) {
-      nb.bin_atoms[q + 1] = nb.bin_atoms[q];
-      q--;
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= live_atoms(nb)) return;
+  const int b = nb.atom_bin[i], lo = nb.bin_start[b], cnt = nb.bin_count[b];
+  int r = 0;
+  for (int q = 0; q < cnt; q++) r += nb.bin_atoms[lo + q] < i ? 1 : 0;
+  nb.sorted[lo + r] = sorted_entry(pos[i], i);
+}
+
+// ---- bins of a small system: the same phases in one workgroup ----
+constexpr int kSmall = 4096;  // atoms and bins at most
+
+__global__ __launch_bounds__(1024) void k_nb_small(NbrBuild nb, double4 *pos, int nbins)
+{
+  if (!rebuild_due(nb.ctl, nb.trig2)) return;
+  __shared__ int count[kSmall], start[kSmall], atoms[kSmall], wsum[16];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int n = min(live_atoms(nb), kSmall);
+  nbins = min(live_bins(nb, nbins), kSmall);
+  for (int b = t; b < kSmall; b += 1024) count[b] = 0;
+  __syncthreads();
+  int bin[kSmall / 1024], rank[kSmall / 1024];
+#pragma unroll
+  for (int u = 0; u < kSmall / 1024; u++) {
+    const int i = u * 1024 + t;
+    bin[u] = rank[u] = 0;
+    if (i < n) {
+      bin[u] = min(bin_atom(nb, pos, i), kSmall - 1);
+      rank[u] = atomicAdd(&count[bin[u]], 1);
     }
-    nb.bin_atoms[q + 1] = v;
+  }
+  __syncthreads();
+  // exclusive scan, 4 consecutive bins per thread
+  int c[4], sum = 0;
+#pragma unroll
+  for (int u = 0; u < 4; u++) {
+    c[u] = count[4 * t + u];
+    sum += c[u];
+  }
+  const int incl = wave_scan(sum);
+  if (lane == 63) wsum[wave] = incl;
+  __syncthreads();
+  int run = incl - sum;
+  for (int w = 0; w < wave; w++) run += wsum[w];
+#pragma unroll
+  for (int u = 0; u < 4; u++) {
+    const int b = 4 * t + u;
+    start[b] = run;
+    if (b < nbins) {
+      nb.bin_start[b] = run;
+      nb.bin_count[b] = c[u];
+    }
+    run += c[u];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < kSmall / 1024; u++) {
+    const int i = u * 1024 + t;
+    if (i < n) atoms[start[bin[u]] + rank[u]] = i;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < kSmall / 1024; u++) {
+    const int i = u * 1024 + t;
+    if (i >= n) continue;
+    const int lo = start[bin[u]], cnt = count[bin[u]];
+    int r = 0;
+    for (int q = 0; q < cnt; q++) r += atoms[lo + q] < i ? 1 : 0;
+    nb.sorted[lo + r] = sorted_entry(pos[i], i);
   }
 }
 
-// One wavefront per atom, one lane per stencil bin (rounds of 64 bins in
-// the stencil order o0, o1, o2): each lane counts the kept candidates of its
-// bin, a prefix sum over the lanes gives each bin its output offset, and the
-// lanes write their entries there.  The list order is the serial walk's
-// (stencil order, then ascending atom index within a bin), with ~2 rounds of
-// a few candidates per lane instead of one thread walking ~400 candidates.
+// floor(a / b) for |a|, b < 2^20, ib = 1 / b: a + 1/2 is at least 1 / (2 b)
+// away from a multiple of b, relative to which the rounding of the product is
+// small.
+__device__ inline int small_div(int a, float ib) { return (int) floorf(((float) a + 0.5f) * ib); }
+
+// One wavefront per atom.  Its stencil bins (in the order o0, o1, o2) are
+// read one per lane; the lanes write their bins' places in the sorted order
+// to LDS behind one another (a prefix sum of the counts), and the wave then
+// takes 64 of these candidates at a time: one contiguous 32-byte load per
+// lane, and a ballot places the kept ones.  The list order is the serial
+// walk's: stencil order, then ascending atom index within a bin.
+// Workgroups of the list kernel at most: they stride over the atoms, so that
+// the steps without a rebuild do not launch one wave per atom to return.
+constexpr int kListBlocks = 4096;
+constexpr int kCand = 768;  // candidates held in LDS per wave; longer stencils take several rounds
+
 __global__ __launch_bounds__(256) void k_nb_list(NbrBuild nb, const double4 *pos, uint32_t *nbr, int *nn)
 {
   if (!rebuild_due(nb.ctl, nb.trig2)) return;
+  __shared__ uint32_t s_cand[4][kCand];
   const int lane = threadIdx.x & 63;
-  const int i = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
-  if (i >= live_atoms(nb)) return;
-  const CellInfo &c = cell_of(nb, i);
-  const double4 xi = pos[i];
-  const int bc0 = nb.atom_bc[3 * i], bc1 = nb.atom_bc[3 * i + 1], bc2 = nb.atom_bc[3 * i + 2];
-  const int n0 = c.nb[0], n1 = c.nb[1], n2 = c.nb[2];
-  const int w1 = 2 * c.reach[1] + 1, w2 = 2 * c.reach[2] + 1;
-  const int nst = (2 * c.reach[0] + 1) * w1 * w2;
-  uint32_t *out = nbr + (size_t) i * nb.cap;
-  int base = 0;  // entries of the earlier rounds (wave-uniform)
-  for (int r0 = 0; r0 < nst; r0 += 64) {
-    const int sidx = r0 + lane;
-    int lo = 0, hi = 0, s0 = 0, s1 = 0, s2 = 0;
-    if (sidx < nst) {
-      const int o0 = sidx / (w1 * w2) - c.reach[0];
-      const int o1 = (sidx / w2) % w1 - c.reach[1];
-      const int o2 = sidx % w2 - c.reach[2];
-      const int q0 = bc0 + o0, q1 = bc1 + o1, q2 = bc2 + o2;
-      s0 = (q0 >= 0) ? q0 / n0 : -((-q0 + n0 - 1) / n0);
-      s1 = (q1 >= 0) ? q1 / n1 : -((-q1 + n1 - 1) / n1);
-      s2 = (q2 >= 0) ? q2 / n2 : -((-q2 + n2 - 1) / n2);
-      const int t0 = q0 - s0 * n0, t1 = q1 - s1 * n1, t2 = q2 - s2 * n2;
-      const int b = c.bin_base + (t0 * n1 + t1) * n2 + t2;
-      lo = nb.bin_start[b];
-      hi = nb.bin_start[b + 1];
-    }
-    const bool self_image = s0 == 0 && s1 == 0 && s2 == 0;
-    auto kept = [&](int j) {
-      if (j == i && self_image) return false;
-      double d[3];
-      displacement(xi, pos[j], s0, s1, s2, c, d);
-      return dist2(d) <= nb.cut2;
-    };
-    int cnt = 0;
-    for (int p = lo; p < hi; p++) cnt += kept(nb.bin_atoms[p]) ? 1 : 0;
-    // exclusive prefix sum of the lane counts
-    int incl = cnt;
+  uint32_t *cand = s_cand[threadIdx.x >> 6];
+  const int n = live_atoms(nb);
+  for (int i = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6)); i < n; i += 4 * gridDim.x) {
+    const CellInfo &c = cell_of(nb, i);
+    const double4 xi = pos[i];
+    const int bc0 = nb.atom_bc[3 * (size_t) i], bc1 = nb.atom_bc[3 * (size_t) i + 1],
+              bc2 = nb.atom_bc[3 * (size_t) i + 2];
+    const int n0 = c.nb[0], n1 = c.nb[1], n2 = c.nb[2];
+    const int w2 = 2 * c.reach[2] + 1, w12 = (2 * c.reach[1] + 1) * w2;
+    const int nst = (2 * c.reach[0] + 1) * w12;
+    const float iw2 = 1.0f / (float) w2, iw12 = 1.0f / (float) w12;
+    const float in0 = 1.0f / (float) n0, in1 = 1.0f / (float) n1, in2 = 1.0f / (float) n2;
+    uint32_t *out = nbr + (size_t) i * nb.cap;
+    int base = 0;    // entries written so far (wave-uniform)
+    int ncand = 0;   // candidates held in LDS (wave-uniform)
+    auto flush = [&]() {
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      // four loads per lane in flight: the wave waits for memory, not for arithmetic
+      for (int t0 = 0; t0 < ncand; t0 += 256) {
+        uint32_t e[4];
+        double4 xj[4];
 #pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int v = __shfl_up(incl, o);
-      if (lane >= o) incl += v;
-    }
-    int k = base + incl - cnt;
-    const uint32_t code = (uint32_t) ((s0 + 3) * 49 + (s1 + 3) * 7 + (s2 + 3)) << kNbrJBits;
-    for (int p = lo; p < hi; p++) {
-      const int j = nb.bin_atoms[p];
-      if (kept(j)) {
-        if (k < nb.cap) out[k] = (uint32_t) j | code;
-        k++;
+        for (int u = 0; u < 4; u++) e[u] = cand[min(t0 + 64 * u + lane, ncand - 1)];
+#pragma unroll
+        for (int u = 0; u < 4; u++) xj[u] = nb.sorted[e[u] & kNbrJMask];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+          if (t0 + 64 * u >= ncand) break;
+          const uint32_t code = e[u] >> kNbrJBits;
+          double d[3] = {xj[u].x - xi.x, xj[u].y - xi.y, xj[u].z - xi.z};
+          // most waves of a large cell hold no image: nothing to decode or add
+          if (__builtin_amdgcn_ballot_w64(code != kShiftCenter) != 0ull) {
+            const int s0 = (int) (code / 49u) - 3, s1 = (int) ((code / 7u) % 7u) - 3, s2 = (int) (code % 7u) - 3;
+            displacement(xi, xj[u], s0, s1, s2, c, d);
+          }
+          const int j = (int) xj[u].w;
+          const bool keep = t0 + 64 * u + lane < ncand && dist2(d) <= nb.cut2 && !(j == i && code == kShiftCenter);
+          const unsigned long long m = __ballot(keep);
+          const int k = base + (int) __builtin_amdgcn_mbcnt_hi((unsigned) (m >> 32),
+                                                               __builtin_amdgcn_mbcnt_lo((unsigned) m, 0u));
+          if (keep && k < nb.cap) out[k] = (uint32_t) j | (code << kNbrJBits);
+          base += __popcll(m);
+        }
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      ncand = 0;
+    };
+    for (int r0 = 0; r0 < nst; r0 += 64) {
+      const int sidx = r0 + lane;
+      int lo = 0, cnt = 0;
+      uint32_t code = 0;
+      if (sidx < nst) {
+        const int i0 = small_div(sidx, iw12), rem = sidx - i0 * w12, i1 = small_div(rem, iw2);
+        const int q0 = bc0 + i0 - c.reach[0], q1 = bc1 + i1 - c.reach[1], q2 = bc2 + rem - i1 * w2 - c.reach[2];
+        const int s0 = small_div(q0, in0), s1 = small_div(q1, in1), s2 = small_div(q2, in2);
+        const int t0 = q0 - s0 * n0, t1 = q1 - s1 * n1, t2 = q2 - s2 * n2;
+        const int b = c.bin_base + (t0 * n1 + t1) * n2 + t2;
+        lo = nb.bin_start[b];
+        cnt = nb.bin_count[b];
+        code = (uint32_t) ((s0 + 3) * 49 + (s1 + 3) * 7 + (s2 + 3)) << kNbrJBits;
+      }
+      // this round's candidates in order, as many at a time as fit
+      const int incl = wave_scan(cnt);
+      const int excl = incl - cnt, total = __builtin_amdgcn_readlane(incl, 63);
+      if (ncand + total > kCand) flush();
+      for (int w0 = 0; w0 < total; w0 += kCand) {  // one pass unless the round alone overfills LDS
+        const int wend = min(total, w0 + kCand);
+        const int q0 = max(0, w0 - excl), q1 = min(cnt, wend - excl);
+        for (int q = q0; q < q1; q++) cand[ncand + excl + q - w0] = (uint32_t) (lo + q) | code;
+        ncand += wend - w0;
+        if (wend < total) flush();
       }
     }
-    base += __shfl(incl, 63);
+    flush();
+    if (lane == 0) {
+      nn[i] = min(base, nb.cap);
+      if (base > nb.cap) atomicMax(&nb.ctl[2], (unsigned long long) base);
+    }
   }
-  if (lane == 0) {
-    nn[i] = min(base, nb.cap);
-    if (base > nb.cap) atomicMax(&nb.ctl[2], (unsigned long long) base);
-  }
-}
-
-__global__ void k_nb_done(NbrBuild nb, int nbins)
-{
-  // runs as one workgroup: clear counts for the next build, reset the control word
-  bool due = rebuild_due(nb.ctl, nb.trig2);
-  nbins = live_bins(nb, nbins);
-  __syncthreads();
-  if (due) {
-    for (int b = threadIdx.x; b <= nbins; b += blockDim.x) nb.bin_count[b] = 0;
-    if (threadIdx.x == 0) nb.ctl[3] += 1ull;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    nb.ctl[0] = 0ull;
-    nb.ctl[1] = 0ull;
-  }
-}
-
-__global__ void k_nb_force(unsigned long long *ctl)
-{
-  if (threadIdx.x == 0) ctl[1] = 1ull;
 }
 
 }  // namespace
 
-hipError_t nbr_force_rebuild(const NbrBuild &nb, hipStream_t stream)
+hipError_t nbr_check(const NbrBuild &nb, const double4 *pos, hipStream_t stream)
 {
-  k_nb_force<<<1, 64, 0, stream>>>(nb.ctl);
+  if (nb.n <= 0) return hipSuccess;
+  k_nb_check<<<(nb.n + 1023) / 1024, 1024, 0, stream>>>(nb, pos);
   return hipGetLastError();
 }
 
-hipError_t nbr_step(const NbrBuild &nb, double4 *pos, uint32_t *nbr, int *nn, hipStream_t stream)
+hipError_t launch_vv_first(const NbrBuild &nb, int n, double4 *pos, double *v, double *f, const double *dtfm,
+                           double dt, hipStream_t stream)
+{
+  k_vv_first<<<(n + 255) / 256, 256, 0, stream>>>(nb, n, pos, v, f, dtfm, dt);
+  return hipGetLastError();
+}
+
+hipError_t nbr_rebuild(const NbrBuild &nb, double4 *pos, uint32_t *nbr, int *nn, hipStream_t stream)
 {
   if (nb.n <= 0) return hipSuccess;
-  const int nbins = nb.nbins;
-  int blocks = (nb.n + 255) / 256;
-  k_nb_check<<<(nb.n + 1023) / 1024, 1024, 0, stream>>>(nb, pos, nb.x_build, nb.ctl);
-  k_nb_bin<<<blocks, 256, 0, stream>>>(nb, pos);
-  k_nb_scan<<<1, 1024, 0, stream>>>(nb, nbins);
-  k_nb_fill<<<blocks, 256, 0, stream>>>(nb);
-  k_nb_sortbins<<<(nbins + 255) / 256, 256, 0, stream>>>(nb, nbins);
-  k_nb_list<<<(nb.n + 3) / 4, 256, 0, stream>>>(nb, pos, nbr, nn);
-  k_nb_done<<<1, 1024, 0, stream>>>(nb, nbins);
+  const int blocks = (nb.n + 255) / 256;
+  if (nb.n <= kSmall && nb.nbins <= kSmall) {
+    k_nb_small<<<1, 1024, 0, stream>>>(nb, pos, nb.nbins);
+  } else {
+    k_nb_bin<<<blocks, 256, 0, stream>>>(nb, pos);
+    k_nb_alloc<<<(nb.nbins + 255) / 256, 256, 0, stream>>>(nb, nb.nbins);
+    k_nb_fill<<<blocks, 256, 0, stream>>>(nb);
+    k_nb_sort<<<blocks, 256, 0, stream>>>(nb, pos);
+  }
+  k_nb_list<<<std::min((nb.n + 3) / 4, kListBlocks), 256, 0, stream>>>(nb, pos, nbr, nn);
   return hipGetLastError();
 }
 

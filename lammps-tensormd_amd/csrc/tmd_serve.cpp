@@ -81,7 +81,7 @@ struct Slot {
   hipStream_t stream = nullptr;
   hipEvent_t ev_start = nullptr, ev_done = nullptr;
   Workspace w;  // pos, nbr, nn, f, ew, G, dEdG, E, row2atom, cells
-  DeviceBuffer dyn, soff, astruct, sout, bins, atominfo, xbuild, ctl;
+  DeviceBuffer dyn, soff, astruct, sout, bins, atominfo, xbuild, sorted, ctl;
   unsigned char *stage = nullptr;  // pinned host (device-visible)
   double *out = nullptr;           // pinned host (device-visible)
   unsigned char *stage_dev = nullptr;
@@ -131,11 +131,11 @@ size_t bytes_per_atom(const tmd_ctx *ctx, int listcap)
   const size_t gw = (size_t) ctx->model.gwidth();
   return 8 * gw + 8 /*E*/ + 4 /*row2atom*/ + 4 * (size_t) listcap + 4 /*nn*/ + 32 /*pos*/ +
       4 * kept_cache_words(listcap) /*kept lists*/ +
-      24 /*f*/ + 56 /*eatom, watom*/ + 4 /*atom_struct*/ + 12 /*bins*/ + 20 /*atom bins*/ +
-      32 /*x_build*/ + 48 /*staging, output*/;
+      24 /*f*/ + 56 /*eatom, watom*/ + 4 /*atom_struct*/ + 8 /*bins*/ + 24 /*atom bins*/ +
+      64 /*x_build, sorted positions*/ + 48 /*staging, output*/;
 }
 
-BatchArrays arrays_of(Slot &sl)
+BatchArrays arrays_of(Slot &sl, const BatchCaps &full)
 {
   BatchArrays a;
   a.dyn = (BatchDims *) sl.dyn.p;
@@ -145,9 +145,11 @@ BatchArrays arrays_of(Slot &sl)
   a.row2atom = (int *) sl.w.row2atom.p;
   a.pos = (double4 *) sl.w.pos.p;
   a.struct_out = (const double *) sl.sout.p;
-  a.f = (const double *) sl.w.f.p;
+  a.f = (double *) sl.w.f.p;
   a.eatom = (const double *) sl.w.ew.p;
   a.ctl = (unsigned long long *) sl.ctl.p;
+  a.bin_count = (int *) sl.bins.p;
+  a.bin_total = (int *) sl.bins.p + 2 * (size_t) full.bins;
   return a;
 }
 
@@ -193,8 +195,9 @@ int create_slot(Server *S, Slot &sl, int listcap)
   if ((rc = chk(sl.soff.ensure(4 * (size_t) (c.structs + 1)), "serve: offsets"))) return rc;
   if ((rc = chk(sl.astruct.ensure(4 * (size_t) c.atoms), "serve: atom structure"))) return rc;
   if ((rc = chk(sl.sout.ensure(56 * (size_t) c.structs), "serve: sums"))) return rc;
-  if ((rc = chk(sl.bins.ensure(sizeof(int) * (3 * (size_t) (c.bins + 1) + 1)), "serve: bins"))) return rc;
-  if ((rc = chk(sl.atominfo.ensure(sizeof(int) * 5 * (size_t) c.atoms), "serve: atom bins"))) return rc;
+  if ((rc = chk(sl.bins.ensure(sizeof(int) * (2 * (size_t) c.bins + 1)), "serve: bins"))) return rc;
+  if ((rc = chk(sl.atominfo.ensure(sizeof(int) * 6 * (size_t) c.atoms), "serve: atom bins"))) return rc;
+  if ((rc = chk(sl.sorted.ensure(sizeof(double4) * c.atoms), "serve: sorted positions"))) return rc;
   if ((rc = chk(sl.xbuild.ensure(sizeof(double) * 4 * (size_t) c.atoms), "serve: x_build"))) return rc;
   if ((rc = chk(sl.ctl.ensure(sizeof(unsigned long long) * 8), "serve: ctl"))) return rc;
   if ((rc = alloc_list(S, sl, listcap))) return rc;
@@ -249,7 +252,7 @@ int enqueue_batch(Server *S, Slot &sl, const Bucket &b, int rtile)
 {
   tmd_ctx *ctx = S->ctx;
   hipStream_t st = sl.stream;
-  BatchArrays a = arrays_of(sl);
+  BatchArrays a = arrays_of(sl, S->full);
   hipError_t e = launch_batch_unpack(sl.stage_dev, b.caps, a, st);
   if (e != hipSuccess) return hip_fail(ctx, e, "serve: unpack");
   NbrBuild nb{};
@@ -261,17 +264,19 @@ int enqueue_batch(Server *S, Slot &sl, const Bucket &b, int rtile)
   nb.cells = a.cells;
   nb.atom_struct = a.atom_struct;
   nb.dyn = a.dyn;
-  int *bins = (int *) sl.bins.p;
-  nb.bin_count = bins;
-  nb.bin_start = bins + (S->full.bins + 1);
-  nb.bin_cursor = bins + 2 * (S->full.bins + 1);
+  nb.bin_count = a.bin_count;
+  nb.bin_start = a.bin_count + S->full.bins;
+  nb.bin_total = a.bin_total;
   int *ai = (int *) sl.atominfo.p;
+  const size_t na = (size_t) S->full.atoms;
   nb.bin_atoms = ai;
-  nb.atom_bin = ai + S->full.atoms;
-  nb.atom_bc = ai + 2 * (size_t) S->full.atoms;
+  nb.atom_bin = ai + na;
+  nb.atom_rank = ai + 2 * na;
+  nb.atom_bc = ai + 3 * na;
+  nb.sorted = (double4 *) sl.sorted.p;
   nb.x_build = (double *) sl.xbuild.p;
   nb.ctl = a.ctl;
-  e = nbr_step(nb, a.pos, (uint32_t *) sl.w.nbr.p, (int *) sl.w.nn.p, st);
+  e = nbr_rebuild(nb, a.pos, (uint32_t *) sl.w.nbr.p, (int *) sl.w.nn.p, st);
   if (e != hipSuccess) return hip_fail(ctx, e, "serve: neighbor build");
   sl.w.rl.nrows = b.caps.rows;  // grid extent; live layout is on the device
   Chain c;
@@ -284,6 +289,8 @@ int enqueue_batch(Server *S, Slot &sl, const Bucket &b, int rtile)
   c.cap = sl.listcap;
   c.f = (double *) sl.w.f.p;
   c.fbytes = 24 * (size_t) b.caps.atoms;
+  c.f_cleared = true;  // by the unpack kernel
+  c.nb = &nb;
   c.natoms = S->full.atoms;  // eatom/watom layout of the slot
   c.struct_off = a.struct_off;
   c.nstruct = b.caps.structs;

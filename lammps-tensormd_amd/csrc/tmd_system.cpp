@@ -25,7 +25,7 @@ struct tmd_system {
   int nbins = 0;
   Workspace w;
   std::vector<int> row2atom;
-  DeviceBuffer vel, dtfm, mass, bins, atominfo, xbuild, ctl, hist;
+  DeviceBuffer vel, dtfm, mass, bins, atominfo, xbuild, sorted, ctl, hist;
   DeviceBuffer snap;  // x, v, f at the start of the current run segment
   DeviceBuffer order;  // rows in atom order (the descriptor and force kernels' launch order)
   bool have_forces = false;
@@ -159,21 +159,45 @@ Chain sys_chain(tmd_system *s)
   c.f = (double *) s->w.f.p;
   c.fbytes = sizeof(double) * 3 * (size_t) s->n;
   c.natoms = s->n;
+  c.nb = &s->nb;
   c.g_bf16 = true;
   return c;
 }
 
-int sys_forces(tmd_system *s, PhaseEvents *pe = nullptr)
+// One force evaluation at the current positions.  step: it ends an MD step,
+// whose launch_vv_first has checked the displacements and cleared f (its
+// velocities and history are in the chain).
+int sys_forces(tmd_system *s, const Chain &c, bool step, PhaseEvents *pe = nullptr)
 {
   hipStream_t st = s->ctx->stream;
-  hipError_t e = nbr_step(s->nb, (double4 *) s->w.pos.p, (uint32_t *) s->w.nbr.p, (int *) s->w.nn.p, st);
+  hipError_t e = step ? hipSuccess : nbr_check(s->nb, (const double4 *) s->w.pos.p, st);
+  if (e == hipSuccess)
+    e = nbr_rebuild(s->nb, (double4 *) s->w.pos.p, (uint32_t *) s->w.nbr.p, (int *) s->w.nn.p, st);
   if (e != hipSuccess) return hip_fail(s->ctx, e, "neighbor build");
-  int rc = run_chain(s->ctx, s->w, sys_chain(s), st, pe);
+  int rc = run_chain(s->ctx, s->w, c, st, pe);
   if (rc != TMD_OK || !pe) return rc;
   // the kept-neighbor counts of this evaluation, for the sampled work per launch
   e = launch_sum_kept((const uint32_t *) s->w.kl.p, kept_cache_words(s->nb.cap),
                       (const int *) s->w.row2atom.p, s->w.rl.nrows, (unsigned long long *) s->tkept.p, st);
   return e == hipSuccess ? TMD_OK : hip_fail(s->ctx, e, "kept count");
+}
+
+// The chain of an MD step: the second half kick and, with hist, the energy
+// history ride on its sums.
+constexpr int kHist = 4096;
+Chain step_chain(tmd_system *s, bool want_hist)
+{
+  Chain c = sys_chain(s);
+  c.f_cleared = true;
+  c.v = (double *) s->vel.p;
+  c.dtfm = (const double *) s->dtfm.p;
+  c.mass = (const double *) s->mass.p;
+  if (want_hist) {
+    c.hist = (double *) s->hist.p;
+    c.hist_counter = (unsigned long long *) (c.hist + 2 * kHist);
+    c.hist_cap = kHist;
+  }
+  return c;
 }
 
 // the control words read after the queued work: an overflow grows the list
@@ -325,20 +349,23 @@ int tmd_system_create(tmd_ctx *ctx, int natoms, const double *x, const int *type
   if ((rc = chk(s->vel.ensure(sizeof(double) * 3 * (size_t) natoms), "v alloc"))) return rc;
   if ((rc = chk(s->dtfm.ensure(sizeof(double) * kMaxElts), "dtfm alloc"))) return rc;
   if ((rc = chk(s->mass.ensure(sizeof(double) * kMaxElts), "mass alloc"))) return rc;
-  if ((rc = chk(s->bins.ensure(sizeof(int) * (3 * (size_t) (s->nbins + 1) + 1)), "bins alloc"))) return rc;
-  if ((rc = chk(s->atominfo.ensure(sizeof(int) * 5 * (size_t) natoms), "atom bins alloc"))) return rc;
+  if ((rc = chk(s->bins.ensure(sizeof(int) * (2 * (size_t) s->nbins + 1)), "bins alloc"))) return rc;
+  if ((rc = chk(s->atominfo.ensure(sizeof(int) * 6 * (size_t) natoms), "atom bins alloc"))) return rc;
+  if ((rc = chk(s->sorted.ensure(sizeof(double4) * (size_t) natoms), "sorted positions alloc"))) return rc;
   if ((rc = chk(s->xbuild.ensure(sizeof(double) * 4 * (size_t) natoms), "xbuild alloc"))) return rc;
   if ((rc = chk(s->ctl.ensure(sizeof(unsigned long long) * 8), "ctl alloc"))) return rc;
-  if ((rc = chk(s->hist.ensure(sizeof(double) * (2 * 4096 + 4096 + 64)), "hist alloc"))) return rc;
+  if ((rc = chk(s->hist.ensure(sizeof(double) * (2 * kHist + 1)), "hist alloc"))) return rc;
   if ((rc = alloc_list(s.get(), cap))) return rc;
   int *bins = (int *) s->bins.p;
   s->nb.bin_count = bins;
-  s->nb.bin_start = bins + (s->nbins + 1);
-  s->nb.bin_cursor = bins + 2 * (s->nbins + 1);
+  s->nb.bin_start = bins + s->nbins;
+  s->nb.bin_total = bins + 2 * (size_t) s->nbins;
   int *ai = (int *) s->atominfo.p;
   s->nb.bin_atoms = ai;
   s->nb.atom_bin = ai + natoms;
-  s->nb.atom_bc = ai + 2 * (size_t) natoms;
+  s->nb.atom_rank = ai + 2 * (size_t) natoms;
+  s->nb.atom_bc = ai + 3 * (size_t) natoms;
+  s->nb.sorted = (double4 *) s->sorted.p;
   s->nb.x_build = (double *) s->xbuild.p;
   s->nb.ctl = (unsigned long long *) s->ctl.p;
   s->nb.cells = (const CellInfo *) s->w.cells.p;
@@ -416,7 +443,7 @@ int tmd_system_compute(tmd_system *s)
     return hip_fail(s->ctx, de, "hipSetDevice");
   if (int rc = resolve_pending(s); rc != TMD_OK) return rc;
   for (int attempt = 0; attempt < 4; attempt++) {
-    int rc = sys_forces(s);
+    int rc = sys_forces(s, sys_chain(s), false);
     if (rc != TMD_OK) return rc;
     bool over = false;
     rc = check_overflow(s, &over);
@@ -512,28 +539,12 @@ int md_run_impl(tmd_system *s, int nsteps, double dt, double *epot, double *ekin
   }
   double *hist = (double *) s->hist.p;
   const bool want_hist = epot || ekin;
-  // layout of the history buffer: [0, 2*kHist) pairs, then scratch
-  const int kHist = 4096;
-  double *ekin_out = hist + 2 * kHist;
-  unsigned long long *counter = (unsigned long long *) (hist + 2 * kHist + 4096);
+  unsigned long long *counter = (unsigned long long *) (hist + 2 * kHist);
   auto enqueue_step = [&](PhaseEvents *pe) -> int {
-    hipError_t er;
-    if ((er = launch_vv_first(s->n, (double4 *) s->w.pos.p, (double *) s->vel.p, (const double *) s->w.f.p,
-                              (const double *) s->dtfm.p, dt, st)) != hipSuccess)
-      return hip_fail(s->ctx, er, "vv first");
-    int rc = sys_forces(s, pe);
-    if (rc != TMD_OK) return rc;
-    if ((er = launch_vv_second(s->n, (const double4 *) s->w.pos.p, (double *) s->vel.p,
-                               (const double *) s->w.f.p, (const double *) s->dtfm.p, st)) != hipSuccess)
-      return hip_fail(s->ctx, er, "vv second");
-    if (want_hist) {
-      if ((er = launch_ekin(s->n, (const double4 *) s->w.pos.p, (const double *) s->vel.p,
-                            (const double *) s->mass.p, ekin_out, st)) != hipSuccess)
-        return hip_fail(s->ctx, er, "ekin");
-      if ((er = launch_record_step((const double *) s->w.red.p, ekin_out, hist, counter, kHist, st)) != hipSuccess)
-        return hip_fail(s->ctx, er, "history");
-    }
-    return TMD_OK;
+    hipError_t er = launch_vv_first(s->nb, s->n, (double4 *) s->w.pos.p, (double *) s->vel.p, (double *) s->w.f.p,
+                                    (const double *) s->dtfm.p, dt, st);
+    if (er != hipSuccess) return hip_fail(s->ctx, er, "vv first");
+    return sys_forces(s, step_chain(s, want_hist), true, pe);
   };
   if (s->use_graph && (!s->step_graph || s->graph_hist != want_hist)) {
     if (s->step_graph) {
@@ -744,25 +755,23 @@ int tmd_md_profile(tmd_system *s, int nsteps, double dt, double *ms)
     for (int k = 0; k < 6; k++) pe.ev[k] = E[3 + k];
     e = hipEventRecord(E[0], st);
     if (e == hipSuccess)
-      e = launch_vv_first(s->n, (double4 *) s->w.pos.p, (double *) s->vel.p, (const double *) s->w.f.p,
+      e = launch_vv_first(s->nb, s->n, (double4 *) s->w.pos.p, (double *) s->vel.p, (double *) s->w.f.p,
                           (const double *) s->dtfm.p, dt, st);
     if (e == hipSuccess) e = hipEventRecord(E[1], st);
     if (e == hipSuccess)
-      e = nbr_step(s->nb, (double4 *) s->w.pos.p, (uint32_t *) s->w.nbr.p, (int *) s->w.nn.p, st);
+      e = nbr_rebuild(s->nb, (double4 *) s->w.pos.p, (uint32_t *) s->w.nbr.p, (int *) s->w.nn.p, st);
     if (e == hipSuccess) e = hipEventRecord(E[2], st);
     if (e == hipSuccess) {
-      rc = run_chain(s->ctx, s->w, sys_chain(s), st, &pe);
+      rc = run_chain(s->ctx, s->w, step_chain(s, false), st, &pe);
       if (rc != TMD_OK) return rc;
     }
-    if (e == hipSuccess)
-      e = launch_vv_second(s->n, (const double4 *) s->w.pos.p, (double *) s->vel.p,
-                           (const double *) s->w.f.p, (const double *) s->dtfm.p, st);
     if (e == hipSuccess) e = hipEventRecord(E[9], st);
   }
   if (e == hipSuccess) e = hipStreamSynchronize(st);
   if (e != hipSuccess) return hip_fail(s->ctx, e, "profile");
-  // phases: neighbor(1-2), descriptor(3-4), mlp(4-5), force kernel(6-7),
-  // reductions + force-buffer clears(7-8, 5-6), integrate(0-1, 8-9)
+  // phases: neighbor rebuild(1-2), descriptor(3-4), mlp(4-5), force kernel(6-7),
+  // sums with the second half kick(7-8, 5-6), first half kick, drift and
+  // displacement check(0-1, 8-9)
   double acc[7] = {0, 0, 0, 0, 0, 0, 0};
   auto el = [&](hipEvent_t a, hipEvent_t b) {
     float t = 0.f;

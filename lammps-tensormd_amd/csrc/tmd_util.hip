@@ -1,15 +1,14 @@
 // Small device kernels: buffer clearing (a kernel, so it is safe inside
-// captured graphs), fixed-order FP64 reductions of energy/virial and kinetic
-// energy, and the two velocity-Verlet half steps (src/fix_nve.cpp:64-130).
-#include "tmd_device.h"
+// captured graphs), and what follows the force kernel: fixed-order FP64
+// reductions of energy/virial and kinetic energy with the second half of the
+// velocity-Verlet step (src/fix_nve.cpp:102-130).
+#include "tmd_desc_common.h"
 
 #include <algorithm>
 
 namespace tmd {
 
 namespace {
-
-constexpr int kRedParts = 240;
 
 __global__ void k_zero(uint4 *p, size_t n16, unsigned char *tail, size_t ntail)
 {
@@ -19,8 +18,6 @@ __global__ void k_zero(uint4 *p, size_t n16, unsigned char *tail, size_t ntail)
   if (i < ntail) tail[i] = 0;
 }
 
-// Each block writes one partial; the final kernel adds partials in order,
-// so the result does not depend on scheduling.
 // sums of eatom[i], watom[i][0..5] over atoms [lo, hi) by one 256-thread
 // workgroup, in a fixed order; thread 0..6 of the result hold the 7 sums
 __device__ inline void block_sum7(const double *eatom, const double *watom, int lo, int hi,
@@ -42,115 +39,104 @@ __device__ inline void block_sum7(const double *eatom, const double *watom, int 
   if (t < 7) res[t] = sh[t][0];
 }
 
-__global__ void k_reduce_ev_part(const double *eatom, const double *watom, int n, double *part)
+// The control word of the neighbor list after an evaluation: a build counted
+// if one was due, flags cleared for the next step.
+__device__ inline void reset_ctl(unsigned long long *ctl, double trig2)
 {
-  __shared__ double sh[7][256];
-  block_sum7(eatom, watom, 0, n, blockIdx.x * 256, gridDim.x * 256, sh,
-             part + (size_t) blockIdx.x * 7);
-}
-
-// one wave per quantity; fixed shuffle tree (deterministic)
-__global__ void k_reduce_ev_final(const double *part, int nparts, double *out)
-{
-  const int q = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  if (q >= 7) return;
-  double s = 0.0;
-  for (int p = lane; p < nparts; p += 64) s += part[(size_t) p * 7 + q];
-  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
-  if (lane == 0) out[q] = s;
+  if (ctl[1] != 0ull || __longlong_as_double((long long) ctl[0]) > trig2) ctl[3] += 1ull;
+  ctl[0] = 0ull;
+  ctl[1] = 0ull;
 }
 
 // one workgroup per structure
 __global__ void k_reduce_struct(const double *eatom, const double *watom, const int *off,
-                                int nstruct, double *out, const BatchDims *dyn)
+                                int nstruct, double *out, unsigned long long *ctl, double trig2, const BatchDims *dyn)
 {
   __shared__ double sh[7][256];
   const int st = blockIdx.x;
+  if (st == 0 && threadIdx.x == 0) reset_ctl(ctl, trig2);
   if (st >= nstruct || (dyn && st >= dyn->nstruct)) return;
   block_sum7(eatom, watom, off[st], off[st + 1], 0, 256, sh, out + (size_t) st * 7);
 }
 
-__global__ void k_vv_first(int n, double4 *pos, double *v, const double *f, const double *dtfm,
-                           double dt)
+// tot[0..7] = energy, virial, sum m v^2 (held by the workgroup) -> results
+__device__ inline void finish_step(const StepTail &a, const double *tot)
 {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  double4 p = pos[i];
-  double c = dtfm[(int) p.w];
-  double vx = v[3 * i] + c * f[3 * i];
-  double vy = v[3 * i + 1] + c * f[3 * i + 1];
-  double vz = v[3 * i + 2] + c * f[3 * i + 2];
-  v[3 * i] = vx;
-  v[3 * i + 1] = vy;
-  v[3 * i + 2] = vz;
-  p.x += dt * vx;
-  p.y += dt * vy;
-  p.z += dt * vz;
-  pos[i] = p;
-}
-
-__global__ void k_vv_second(int n, const double4 *pos, double *v, const double *f, const double *dtfm)
-{
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  double c = dtfm[(int) pos[i].w];
-  v[3 * i] += c * f[3 * i];
-  v[3 * i + 1] += c * f[3 * i + 1];
-  v[3 * i + 2] += c * f[3 * i + 2];
-}
-
-__global__ void k_ekin_part(int n, const double4 *pos, const double *v, const double *mass,
-                            double *part)
-{
-  __shared__ double sh[256];
-  int t = threadIdx.x;
-  double s = 0.0;
-  for (int i = blockIdx.x * 256 + t; i < n; i += gridDim.x * 256) {
-    double m = mass[(int) pos[i].w];
-    s += m * (v[3 * i] * v[3 * i] + v[3 * i + 1] * v[3 * i + 1] + v[3 * i + 2] * v[3 * i + 2]);
-  }
-  sh[t] = s;
-  __syncthreads();
-  for (int o = 128; o > 0; o >>= 1) {
-    if (t < o) sh[t] += sh[t + o];
-    __syncthreads();
-  }
-  if (t == 0) part[blockIdx.x] = sh[0];
-}
-
-__global__ void k_ekin_final(const double *part, int nparts, double *out)
-{
-  const int lane = threadIdx.x & 63;
-  double s = 0.0;
-  for (int p = lane; p < nparts; p += 64) s += part[p];
-  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
-  if (threadIdx.x == 0) out[0] = 0.5 * 1.0364269e-4 * s;  // mvv2e, metal units
-}
-
-__global__ void k_zero_atoms(double *p, int per_atom, const BatchDims *dyn)
-{
-  size_t n = (size_t) per_atom * dyn->natoms;
-  size_t i = (size_t) blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = 0.0;
-}
-
-__global__ void k_copy_scalar(const double *src, double *dst)
-{
-  if (threadIdx.x == 0) dst[0] = src[0];
-}
-
-// hist[2*n] = epot, hist[2*n+1] = ekin, n = counter++ (graph-replay safe)
-__global__ void k_record_step(const double *epot, const double *ekin, double *hist,
-                              unsigned long long *counter, int cap)
-{
-  if (threadIdx.x == 0) {
-    unsigned long long n = counter[0];
-    if (n < (unsigned long long) cap) {
-      hist[2 * n] = epot[0];
-      hist[2 * n + 1] = ekin ? ekin[0] : 0.0;
+  const int t = threadIdx.x;
+  if (t < 7) a.out[t] = tot[t];
+  if (t != 0) return;
+  if (a.ctl) reset_ctl(a.ctl, a.trig2);
+  if (a.hist) {
+    const unsigned long long n = a.counter[0];
+    if (n < (unsigned long long) a.hist_cap) {
+      a.hist[2 * n] = tot[0];
+      a.hist[2 * n + 1] = 0.5 * 1.0364269e-4 * tot[7];  // mvv2e, metal units
     }
-    counter[0] = n + 1;
+    a.counter[0] = n + 1;
   }
+}
+
+// Sums over the atoms, and the second half of a velocity-Verlet step
+// (src/fix_nve.cpp:102-130) in the same pass.  Each workgroup writes its
+// partial sums, added in a fixed order by k_step_final; the only workgroup
+// of a small system finishes by itself.
+__global__ __launch_bounds__(1024) void k_step_sums(StepTail a)
+{
+  __shared__ double sh[16][8];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, nw = blockDim.x >> 6;
+  double s[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll 2
+  for (int i = blockIdx.x * blockDim.x + t; i < a.n; i += gridDim.x * blockDim.x) {
+    s[0] += a.eatom[i];
+#pragma unroll
+    for (int q = 0; q < 6; q++) s[1 + q] += a.watom[6 * (size_t) i + q];
+    if (a.v) {
+      const int e = (int) a.pos[i].w;
+      const double c = a.dtfm[e];
+      double v2 = 0.0;
+#pragma unroll
+      for (int q = 0; q < 3; q++) {
+        const size_t p = 3 * (size_t) i + q;
+        const double v = a.v[p] + c * a.f[p];
+        a.v[p] = v;
+        v2 += v * v;
+      }
+      s[7] += a.mass[e] * v2;
+    }
+  }
+  // pairs of quantities share the exchanges between halves and rows
+  const double x0 = row_sum_d(swap16_add(swap32_add(s[0], s[1]), swap32_add(s[2], s[3])));
+  const double x1 = row_sum_d(swap16_add(swap32_add(s[4], s[5]), swap32_add(s[6], s[7])));
+  if ((lane & 15) == 0) {
+    const int q = ((lane >> 4) & 1) * 2 + (lane >> 5);  // rows hold quantities 0, 2, 1, 3
+    sh[wave][q] = x0;
+    sh[wave][4 + q] = x1;
+  }
+  __syncthreads();
+  double r = 0.0;
+  if (t < 8)
+    for (int w = 0; w < nw; w++) r += sh[w][t];
+  if (gridDim.x > 1) {
+    if (t < 8) a.out[8 + 8 * (size_t) blockIdx.x + t] = r;
+    return;
+  }
+  __syncthreads();
+  if (t < 8) sh[0][t] = r;
+  __syncthreads();
+  finish_step(a, sh[0]);
+}
+
+// one wave per quantity; fixed shuffle tree (deterministic)
+__global__ __launch_bounds__(512) void k_step_final(StepTail a, int nparts)
+{
+  __shared__ double tot[8];
+  const int q = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  double s = 0.0;
+  for (int p = lane; p < nparts; p += 64) s += a.out[8 + 8 * (size_t) p + q];
+  s = wave_sum_d(s);
+  if (lane == 0) tot[q] = s;
+  __syncthreads();
+  finish_step(a, tot);
 }
 
 __global__ void k_copy(const uint4 *__restrict__ src, uint4 *__restrict__ dst, size_t n16)
@@ -178,52 +164,26 @@ hipError_t launch_zero(void *p, size_t bytes, hipStream_t s)
   return hipGetLastError();
 }
 
-hipError_t launch_reduce_ev(const double *eatom, const double *watom, int n, double *out,
-                            hipStream_t s)
+hipError_t launch_step_tail(const StepTail &t, hipStream_t s)
 {
-  double *part = out + 8;  // out holds 8 + kRedParts*7 doubles
-  k_reduce_ev_part<<<kRedParts, 256, 0, s>>>(eatom, watom, n, part);
-  k_reduce_ev_final<<<1, 448, 0, s>>>(part, kRedParts, out);
+  // one workgroup up to 2,048 atoms: two atoms per thread cost less than a
+  // second launch
+  if (t.n <= 2048) {
+    k_step_sums<<<1, 1024, 0, s>>>(t);
+  } else {
+    const int parts = std::min(kSumParts, (t.n + 255) / 256);
+    k_step_sums<<<parts, 256, 0, s>>>(t);
+    k_step_final<<<1, 512, 0, s>>>(t, parts);
+  }
   return hipGetLastError();
 }
 
 hipError_t launch_reduce_struct(const double *eatom, const double *watom, const int *off,
-                                int nstruct, double *out, hipStream_t s, const BatchDims *dyn)
+                                int nstruct, double *out, unsigned long long *ctl, double trig2,
+                                hipStream_t s, const BatchDims *dyn)
 {
   if (nstruct <= 0) return hipSuccess;
-  k_reduce_struct<<<nstruct, 256, 0, s>>>(eatom, watom, off, nstruct, out, dyn);
-  return hipGetLastError();
-}
-
-hipError_t launch_zero_atoms(double *p, int per_atom, int cap_atoms, const BatchDims *dyn,
-                             hipStream_t s)
-{
-  size_t n = (size_t) per_atom * cap_atoms;
-  if (n == 0) return hipSuccess;
-  k_zero_atoms<<<(unsigned) ((n + 255) / 256), 256, 0, s>>>(p, per_atom, dyn);
-  return hipGetLastError();
-}
-
-hipError_t launch_vv_first(int n, double4 *pos, double *v, const double *f, const double *dtfm,
-                           double dt, hipStream_t s)
-{
-  k_vv_first<<<(n + 255) / 256, 256, 0, s>>>(n, pos, v, f, dtfm, dt);
-  return hipGetLastError();
-}
-
-hipError_t launch_vv_second(int n, const double4 *pos, double *v, const double *f,
-                            const double *dtfm, hipStream_t s)
-{
-  k_vv_second<<<(n + 255) / 256, 256, 0, s>>>(n, pos, v, f, dtfm);
-  return hipGetLastError();
-}
-
-hipError_t launch_ekin(int n, const double4 *pos, const double *v, const double *mass, double *out,
-                       hipStream_t s)
-{
-  double *part = out + 8;
-  k_ekin_part<<<kRedParts, 256, 0, s>>>(n, pos, v, mass, part);
-  k_ekin_final<<<1, 64, 0, s>>>(part, kRedParts, out);
+  k_reduce_struct<<<nstruct, 256, 0, s>>>(eatom, watom, off, nstruct, out, ctl, trig2, dyn);
   return hipGetLastError();
 }
 
@@ -245,19 +205,6 @@ hipError_t launch_sum_kept(const uint32_t *kl, size_t words, const int *row2atom
 {
   if (nrows <= 0) return hipSuccess;
   k_sum_kept<<<(nrows + 255) / 256, 256, 0, s>>>(kl, words, row2atom, nrows, acc);
-  return hipGetLastError();
-}
-
-hipError_t launch_record_step(const double *epot, const double *ekin, double *hist,
-                              unsigned long long *counter, int cap, hipStream_t s)
-{
-  k_record_step<<<1, 64, 0, s>>>(epot, ekin, hist, counter, cap);
-  return hipGetLastError();
-}
-
-hipError_t launch_copy_scalar(const double *src, double *dst, hipStream_t s)
-{
-  k_copy_scalar<<<1, 64, 0, s>>>(src, dst);
   return hipGetLastError();
 }
 

@@ -1065,3 +1065,47 @@ def test_force_tile_edges(tmp_path, k, nelt):
             assert np.isfinite(got["vatom"]).all() and abs(got["vatom"] - ref["vatom"]).max() <= 6.0 * max(
                 F_TOL, 2.0 * fl["dF"])
     say(k, nelt, "max |dF|", worst)
+
+
+@pytest.mark.parametrize("cells,a", [((16, 16, 8), 3.2), ((16, 16, 9), 3.2), ((3, 3, 3), 3.2),
+                                     ((9, 9, 9), 1.5)])
+def test_neighbor_build_paths(synth_models, cells, a):
+    """The list builds at the edges of their ranges: bins in one workgroup (at
+    most 4,096 atoms and bins) and in separate kernels, stencils that span
+    several periodic images, and a crystal so dense that one round of stencil
+    bins has more candidates than the list kernel holds.  The set of (i, j,
+    image) entries equals the oracle's, and each atom's entries have no
+    duplicates."""
+    x, t, cell = W.crystal("bcc", a, cells, nelt=4, sigma=0.03, seed=61)
+    m = TensorMD(synth_models["c2"], ["Mo", "Nb", "Ta", "W"], "fp32", 0.001)
+    s = m.system(x, t, cell, skin=1.0)
+    s.compute()
+    off, j, sh = s.neighbors()
+    xw = s.get()["x"]
+    ro, rj, rs = oracle.neighbors(xw, cell, m.cutoff + 1.0, cap_per_atom=1800 if a < 2 else 200)
+    assert np.array_equal(off, ro)
+    i = np.repeat(np.arange(len(x)), np.diff(off))
+    key = lambda jj, ss: ((i * len(x) + jj) * 343 + (ss[:, 0] + 3) * 49 + (ss[:, 1] + 3) * 7 + ss[:, 2] + 3)
+    got = np.sort(key(j.astype(np.int64), sh.astype(np.int64)))
+    ref = np.sort(key(rj.astype(np.int64), rs.astype(np.int64)))
+    assert np.array_equal(got, ref) and (np.diff(got) > 0).all()
+
+
+@pytest.mark.parametrize("cells", [(8, 16, 8), (5, 5, 41), (9, 16, 8)])
+def test_step_sums(synth_models, cells):
+    """Sums of an MD step in one workgroup (2,048 atoms at most) and in
+    several: total energy and virial against the per-atom values, the recorded
+    kinetic energies against the velocities."""
+    x, t, cell = W.crystal("bcc", 3.2, cells, nelt=4, sigma=0.05, seed=62)
+    mass = np.array([95.95, 92.906, 180.95, 183.84])[t - 1]
+    v = W.maxwell_boltzmann(mass, 300.0, seed=63)
+    s = TensorMD(synth_models["c2"], ["Mo", "Nb", "Ta", "W"], "fp32", 0.001).system(x, t, cell, skin=1.0)
+    s.set_velocities(v)
+    ep, ek = s.md_run(3, 0.001)
+    r = s.get()
+    # FP64 sums of n terms: n eps sum |term| bounds the difference
+    eps = np.finfo(float).eps * len(x)
+    assert abs(ep[-1] - r["eatom"].sum()) <= eps * abs(r["eatom"]).sum() and r["energy"] == ep[-1]
+    assert abs(ek[-1] - W.kinetic_energy(mass, r["v"])) <= eps * ek[-1]
+    assert abs(ek[0] - W.kinetic_energy(mass, v)) < 0.05 * ek[0]
+    assert np.all(np.diff(ek) != 0.0) and np.all(np.diff(ep) != 0.0)
