@@ -460,7 +460,7 @@ int run_chain(tmd_ctx *ctx, Workspace &w, const Chain &c, hipStream_t s, PhaseEv
   uint32_t *kl = (uint32_t *) w.kl.p;
   if (pe && (e = hipEventRecord(pe->ev[0], s)) != hipSuccess) return hip_fail(ctx, e, "timing event");
   Geom geo = c.geo;
-  geo.g_bf16 = c.g_bf16 && !ctx->model.tdnp && ctx->geo.mm <= 3 && mlp_bf16_rows(ctx->mlp, mode, c.rtile);
+  geo.g_bf16 = c.g_bf16 && !ctx->model.tdnp && ctx->geo.mm <= 3 && mlp_bf16_rows(ctx->mlp, mode);
   w.g_bf16 = geo.g_bf16;
   e = launch_descriptor(ctx->geo, geo, c.pos, c.nbr, c.nn, c.cap, row2atom, w.rl.nrows,
                         (const float4 *) ctx->tab.p, (float *) w.G.p, kl, s);

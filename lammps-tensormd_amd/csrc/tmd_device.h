@@ -108,6 +108,8 @@ struct MlpParams {
   int offGH, ldGH;
   int offRS;   // FP8: per-row scale and inverse scale [2][R] (floats, byte offset)
   int offQ, ldq;  // FP8: the next GEMM's B operand rows, quantized [R][ldq] (bytes)
+  int stage_g, g_over;  // descriptor rows staged in LDS; over the activations
+  int offX, ldx;        // the staged rows [R][ldx]
   int storeD;  // D_l kept in LDS (otherwise recomputed from H_l: tanh)
 };
 
@@ -209,8 +211,8 @@ hipError_t launch_mlp(int mode, const RowLayout &rl, const MlpParams &mp, const 
                       const BatchDims *dyn = nullptr, int row_begin = 0, int row_end = -1,
                       bool g_bf16 = false);
 // the MLP launch takes BF16 descriptor rows: BF16 mode, tanh, a compile-time
-// layer shape, 32-row tiles
-bool mlp_bf16_rows(const MlpParams &mp, int mode, int rtile);
+// layer shape
+bool mlp_bf16_rows(const MlpParams &mp, int mode);
 size_t mlp_lds_bytes(const MlpParams &mp, int mode, int R, MlpParams *out);
 // the fast (aligned) MLP kernel applies: required by the FP8 mode
 bool mlp_fast_ok(const MlpParams &mp, int mode);

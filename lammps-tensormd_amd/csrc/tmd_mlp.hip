@@ -4,7 +4,7 @@
 // one cuBLAS GEMM + one bias/activation kernel per layer, activations in
 // HBM) and the CPU dense path (src/ML-TENSORMD/nnp.cpp:246-366).
 //
-// A workgroup (4 waves) owns R rows of one element (rows are element-sorted
+// A workgroup owns R rows of one element (rows are element-sorted
 // and each element group starts at a multiple of 64, so R | 64 keeps a tile
 // inside one element).  Every hidden activation H_l and derivative
 // D_l = act'(z_l) of the tile stays in LDS; the waves split each layer's
@@ -475,6 +475,13 @@ __device__ inline typename Frag<MODE>::A ld_x(const T *X, int ld, int r0, int k,
   }
 }
 
+// Waves of a workgroup.  Eight share a tile's rows: each reads half the
+// weights that four would, a small system's few tiles have twice the loads in
+// flight, and the FP32 modes, whose LDS admits two workgroups per CU, run
+// four waves per SIMD instead of two (FP32 network of 2,000 atoms 65 -> 40 us,
+// of 128,000 atoms 785 -> 694 us against four waves; 16 waves are slower).
+constexpr int NW = 8;
+
 // 8 consecutive values of row r at column c: the FP32 descriptor rows in
 // HBM (XG) or a BF16 LDS tile
 template <bool XG>
@@ -502,7 +509,8 @@ __device__ inline bool quantize_g_rows(const float *G, int gw, int grow0, int wi
                                        int ldq)
 {
   constexpr int kMaxChunks = 8;
-  const int tpr = 256 / R;
+  const int tpr = min(64, (int) blockDim.x / R);
+  if ((int) threadIdx.x >= tpr * R) return width <= kMaxChunks * tpr * 8;
   if (width > kMaxChunks * tpr * 8) return false;
   const int r = threadIdx.x / tpr, part = threadIdx.x - r * tpr;
   float v[kMaxChunks][8];
@@ -542,7 +550,8 @@ __device__ inline bool quantize_g_rows(const float *G, int gw, int grow0, int wi
 __device__ inline void quantize_rows_max(const uint16_t *X, int ld, int w, int R, const unsigned *rin,
                                          unsigned *rnext, float *rs, uint8_t *Q, int ldq)
 {
-  const int tpr = 256 / R;
+  const int tpr = min(64, (int) blockDim.x / R);
+  if ((int) threadIdx.x >= tpr * R) return;
   const int r = threadIdx.x / tpr, part = threadIdx.x - r * tpr;
   const float m = __uint_as_float(rin[r]);
   const float sc = m > 0.0f ? m * (1.0f / 440.0f) : 1.0f, ri = 1.0f / sc;
@@ -589,7 +598,8 @@ template <bool XG>
 __device__ inline void quantize_rows(const uint16_t *X, int ld, const float *G, int gw, int grow0, int w, int R,
                                      const float *rinv, uint8_t *Q, int ldq)
 {
-  const int tpr = 256 / R;
+  const int tpr = min(64, (int) blockDim.x / R);
+  if ((int) threadIdx.x >= tpr * R) return;
   const int r = threadIdx.x / tpr, part = threadIdx.x - r * tpr;
   const float ri = rinv[r];
 #pragma unroll 4
@@ -615,19 +625,11 @@ struct GRaw<0> {
   f32x4 v;
 };
 
-// GB: the descriptor rows are stored as BF16 (the BF16 mode's operand
-// values, rounded once by the descriptor kernel), read 16 bytes per lane
-template <int MODE, bool GB = false>
+template <int MODE>
 __device__ inline GRaw<MODE> ld_graw(const float *G, int gw, int grow, int k)
 {
   const int lane = threadIdx.x & 63;
   GRaw<MODE> g;
-  if constexpr (GB) {
-    static_assert(MODE == 1, "BF16 descriptor rows feed the BF16 mode only");
-    const uint16_t *pb = reinterpret_cast<const uint16_t *>(G) + (size_t) (grow + (lane & 15)) * gw + k;
-    g.lo = *reinterpret_cast<const float4 *>(pb + (lane >> 4) * 8);
-    return g;
-  }
   const float *p = G + (size_t) (grow + (lane & 15)) * gw + k;
   if constexpr (MODE == 0) {
     g.v = *reinterpret_cast<const f32x4 *>(p + (lane >> 4) * 4);
@@ -639,12 +641,10 @@ __device__ inline GRaw<MODE> ld_graw(const float *G, int gw, int grow, int k)
   return g;
 }
 
-template <int MODE, bool GB = false>
+template <int MODE>
 __device__ inline typename Frag<MODE>::A cvt_graw(const GRaw<MODE> &g, float ri)
 {
-  if constexpr (GB) {
-    return __builtin_bit_cast(bf16x8, g.lo);
-  } else if constexpr (MODE == 0) {
+  if constexpr (MODE == 0) {
     return g.v;
   } else if constexpr (MODE == 1) {
     f32x8 xv = {g.lo.x, g.lo.y, g.lo.z, g.lo.w, g.hi.x, g.hi.y, g.hi.z, g.hi.w};
@@ -682,14 +682,15 @@ __device__ inline f32x4 mma(typename Frag<MODE>::A a, typename Frag<MODE>::A b, 
 // FP8: per-row scale of the next GEMM's B operand (the rows of X, or of the
 // descriptor rows G): rs[r] = max_c |x[r][c]| / 440 (1 for a zero row),
 // rs[R + r] = 1 / rs[r]; every value then fits e4m3 (|x| <= 448).
-// Threads per row (256 / R consecutive threads) each take 8 consecutive
+// The threads of a row (consecutive lanes) each take 8 consecutive
 // values at a time; the loops are unrolled so that several loads are in
 // flight (the descriptor rows come from HBM).
 template <bool XG>
 __device__ inline void row_scales(const uint16_t *X, int ld, const float *G, int gw, int grow0,
                                   int width, int R, float *rs)
 {
-  const int tpr = 256 / R;  // threads per row: 16, 8 or 4 consecutive lanes
+  const int tpr = min(64, (int) blockDim.x / R);  // threads per row: consecutive lanes of one wave
+  if ((int) threadIdx.x >= tpr * R) return;
   const int r = threadIdx.x / tpr, part = threadIdx.x - r * tpr;
   float m = 0.0f;
 #pragma unroll 4
@@ -736,7 +737,56 @@ __device__ inline void st4(uint16_t *p, const float v[4])
   *reinterpret_cast<uint2 *>(p) = x;
 }
 
-// acc[j][r] = 16 output columns (tile t0 + 4 j) x 16 rows (r * 16 ..) of
+// Layer 0: the tile's descriptor rows, read once with every load in flight,
+// -> X [R][ld] in the activations' type (the BF16 mode rounds FP32 rows here,
+// once for all waves; GB rows are BF16 already).  Reading them step by step
+// as MFMA operands put one trip to HBM into every step of the inner loop.
+template <int MODE, int R, bool GB, int GW, typename T>
+__device__ inline void stage_g(const float *G, int gw_, int grow0, T *X, int ld)
+{
+  static_assert(MODE != 2, "FP8 rows are quantized instead");
+  const int gw = GW ? GW : gw_;
+  const int cpr = gw / 8, total = R * cpr;  // 8 values at a time
+  constexpr int kIt = GW ? (R * (GW / 8) + 64 * NW - 1) / (64 * NW) : 2;
+  auto at = [&](int q, int &r, int &c) {
+    r = q / cpr;
+    c = (q - r * cpr) * 8;
+  };
+  for (int q0 = threadIdx.x; q0 < total; q0 += kIt * 64 * NW) {
+    float4 v[kIt][2];
+#pragma unroll
+    for (int i = 0; i < kIt; i++) {
+      int r, c;
+      at(min(q0 + i * 64 * NW, total - 1), r, c);
+      if constexpr (GB) {
+        v[i][0] = *reinterpret_cast<const float4 *>(reinterpret_cast<const uint16_t *>(G) + (size_t) (grow0 + r) * gw + c);
+      } else {
+        const float4 *p = reinterpret_cast<const float4 *>(G + (size_t) (grow0 + r) * gw + c);
+        v[i][0] = p[0];
+        v[i][1] = p[1];
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < kIt; i++) {
+      const int q = q0 + i * 64 * NW;
+      if (q >= total) break;
+      int r, c;
+      at(q, r, c);
+      T *x = X + r * ld + c;
+      if constexpr (GB) {
+        *reinterpret_cast<float4 *>(x) = v[i][0];
+      } else if constexpr (MODE == 1) {
+        const f32x8 xv = {v[i][0].x, v[i][0].y, v[i][0].z, v[i][0].w, v[i][1].x, v[i][1].y, v[i][1].z, v[i][1].w};
+        *reinterpret_cast<bf16x8 *>(x) = __builtin_convertvector(xv, bf16x8);
+      } else {
+        reinterpret_cast<float4 *>(x)[0] = v[i][0];
+        reinterpret_cast<float4 *>(x)[1] = v[i][1];
+      }
+    }
+  }
+}
+
+// acc[j][r] = 16 output columns (tile t0 + NW j) x 16 rows (r * 16 ..) of
 // W X^T, summed over the inner dimension K, for the wave's NTW tiles.
 //
 // Global operands (the weights, and the descriptor rows of layer 0) go
@@ -746,7 +796,7 @@ __device__ inline void st4(uint16_t *p, const float v[4])
 // same number of loads (past the last step they repeat it), which lets the
 // compiler wait for exactly the step being consumed.  Activations in LDS
 // are read at the step that uses them.
-template <int MODE, int R, bool XG, int NTW, typename T, bool GB = false>
+template <int MODE, int R, bool XG, int NTW, typename T>
 __device__ inline void gemm_t(const void *W, int t0, const T *X, int ldx, const float *G, int gw,
                               int grow0, int K, const float *rinv, f32x4 (&acc)[4][R / 16])
 {
@@ -767,10 +817,10 @@ __device__ inline void gemm_t(const void *W, int t0, const T *X, int ldx, const 
   auto issue = [&](F(&as)[NTW], GRaw<MODE>(&gs)[RT], int s) {
     const int sc = min(s, nst - 1), k = sc * KS;
 #pragma unroll
-    for (int j = 0; j < NTW; j++) as[j] = ld_a<MODE>(W, t0 + 4 * j, sc, nst);
+    for (int j = 0; j < NTW; j++) as[j] = ld_a<MODE>(W, t0 + NW * j, sc, nst);
     if constexpr (XG) {
 #pragma unroll
-      for (int r = 0; r < RT; r++) gs[r] = ld_graw<MODE, GB>(G, gw, grow0 + r * 16, k);
+      for (int r = 0; r < RT; r++) gs[r] = ld_graw<MODE>(G, gw, grow0 + r * 16, k);
     }
   };
 #pragma unroll
@@ -786,7 +836,7 @@ __device__ inline void gemm_t(const void *W, int t0, const T *X, int ldx, const 
 #pragma unroll
         for (int r = 0; r < RT; r++) {
           if constexpr (XG)
-            b[r] = cvt_graw<MODE, GB>(g[i][r], ri[r]);
+            b[r] = cvt_graw<MODE>(g[i][r], ri[r]);
           else
             b[r] = ld_x<MODE>(X, ldx, r * 16, s * KS, ri[r]);
         }
@@ -800,28 +850,27 @@ __device__ inline void gemm_t(const void *W, int t0, const T *X, int ldx, const 
 }
 
 // gemm_t for a runtime tile count ntw in 1..4 (wave-uniform)
-template <int MODE, int R, bool XG, typename T, bool GB = false>
+template <int MODE, int R, bool XG, typename T>
 __device__ inline void gemm_n(const void *W, int t0, int ntw, const T *X, int ldx, const float *G,
                               int gw, int grow0, int K, const float *rinv, f32x4 (&acc)[4][R / 16])
 {
   if (ntw >= 4)
-    gemm_t<MODE, R, XG, 4, T, GB>(W, t0, X, ldx, G, gw, grow0, K, rinv, acc);
+    gemm_t<MODE, R, XG, 4, T>(W, t0, X, ldx, G, gw, grow0, K, rinv, acc);
   else if (ntw == 3)
-    gemm_t<MODE, R, XG, 3, T, GB>(W, t0, X, ldx, G, gw, grow0, K, rinv, acc);
+    gemm_t<MODE, R, XG, 3, T>(W, t0, X, ldx, G, gw, grow0, K, rinv, acc);
   else if (ntw == 2)
-    gemm_t<MODE, R, XG, 2, T, GB>(W, t0, X, ldx, G, gw, grow0, K, rinv, acc);
+    gemm_t<MODE, R, XG, 2, T>(W, t0, X, ldx, G, gw, grow0, K, rinv, acc);
   else
-    gemm_t<MODE, R, XG, 1, T, GB>(W, t0, X, ldx, G, gw, grow0, K, rinv, acc);
+    gemm_t<MODE, R, XG, 1, T>(W, t0, X, ldx, G, gw, grow0, K, rinv, acc);
 }
 
 }  // namespace
 
-// Waves per SIMD asked of the fast kernel (more tiles in flight hide the L2
-// latency of the weight operands): 4 for BF16 and 16-row tiles, 3 for FP32
-// and FP8 32-row tiles, 2 for 64-row tiles (their accumulators and rings
-// need up to 256 VGPRs).
-template <int MODE, int R>
-constexpr int kMlpWaves = R == 64 ? 2 : ((MODE == 1 || R == 16) ? 4 : 3);
+// Waves per SIMD asked of the fast kernel; a workgroup has two.  Four where
+// the registers allow it (the compile-time shapes, and the FP32 and BF16
+// modes up to 32 rows), else two.
+template <int MODE, int R, int SH>
+constexpr int kMlpWaves = SH ? 4 : ((R <= 32 && MODE <= 1) ? 4 : 2);
 
 // bytes per weight of the fast kernel's A operands
 template <int MODE>
@@ -847,7 +896,7 @@ struct MlpShape<2> {  // 384-256-256-128-1
 
 // GB: Gd holds BF16 descriptor rows (MODE 1 only)
 template <int MODE, int ACT, int R, int SH = 0, bool GB = false>
-__global__ __launch_bounds__(256, (kMlpWaves<MODE, R>)) void k_mlp_fast(RowLayout rl_cap, MlpParams mp, const float *Gd,
+__global__ __launch_bounds__(64 * NW, (kMlpWaves<MODE, R, SH>)) void k_mlp_fast(RowLayout rl_cap, MlpParams mp, const float *Gd,
                                                   double *E, float *dEdG, const BatchDims *dyn, int rbase)
 {
   const RowLayout rl = dyn ? dyn->rl : rl_cap;
@@ -876,6 +925,16 @@ __global__ __launch_bounds__(256, (kMlpWaves<MODE, R>)) void k_mlp_fast(RowLayou
     if (threadIdx.x < 2 * R) rmax[threadIdx.x] = 0u;
   }
 
+  // layer 0's input in LDS; with g_over it lies over the activations, which a
+  // barrier then keeps from being written before every wave has read it
+  T *X0 = sm + mp.offX;
+  if constexpr (MODE != 2) {
+    if (SH || mp.stage_g) {
+      stage_g<MODE, R, GB, SH ? MlpShape<SH>::w(0) : 0>(Gd, gw, row0, X0, mp.ldx);
+      __syncthreads();
+    }
+  }
+
   // ---------------- forward ----------------
 #pragma unroll kLayerUnroll
   for (int l = 0; l < L - 1; l++) {
@@ -886,8 +945,8 @@ __global__ __launch_bounds__(256, (kMlpWaves<MODE, R>)) void k_mlp_fast(RowLayou
     T *H = sm + mp.offH[l];
     T *D = sm + mp.offD[l];
     const int ldo = mp.ld[l + 1];
-    const T *Hin = l > 0 ? sm + mp.offH[l - 1] : nullptr;
-    const int ldi = mp.ld[l];
+    const T *Hin = l > 0 ? sm + mp.offH[l - 1] : X0;
+    const int ldi = l > 0 ? mp.ld[l] : mp.ldx;
     const int NT = N / 16;
     unsigned *rnext = rmax + ((l + 1) & 1) * R;  // FP8: maxima of this layer's output
     if constexpr (MODE == 2) {
@@ -903,24 +962,31 @@ __global__ __launch_bounds__(256, (kMlpWaves<MODE, R>)) void k_mlp_fast(RowLayou
       __syncthreads();
     }
     const float *wsc = MODE == 2 ? mp.swf[l] + (size_t) e * N : nullptr;
-    for (int tb = 0; tb < NT; tb += 16) {
+    const bool over = MODE != 2 && l == 0 && (SH || mp.g_over);  // one pass covers the layer
+    for (int tb = 0; tb < NT; tb += 4 * NW) {
       const int t0 = tb + wave;
-      const int ntw = t0 < NT ? min(4, (NT - t0 + 3) / 4) : 0;
-      if (ntw == 0) continue;
+      const int ntw = t0 < NT ? min(4, (NT - t0 + NW - 1) / NW) : 0;
+      if (ntw == 0 && !over) continue;
       f32x4 acc[4][RT];
       float mx[RT];  // FP8: the lane's largest |h| per row tile
 #pragma unroll
       for (int r = 0; r < RT; r++) mx[r] = 0.0f;
-      if constexpr (MODE == 2)
-        gemm_n<MODE, R, false, uint8_t>(W, t0, ntw, Q, mp.ldq, nullptr, gw, row0, K, rs + R, acc);
-      else if (l == 0)
-        gemm_n<MODE, R, true, T, GB>(W, t0, ntw, nullptr, 0, Gd, gw, row0, K, rs + R, acc);
-      else
-        gemm_n<MODE, R, false, T>(W, t0, ntw, Hin, ldi, nullptr, gw, row0, K, rs + R, acc);
+      if (ntw > 0) {
+        if constexpr (MODE == 2)
+          gemm_n<MODE, R, false, uint8_t>(W, t0, ntw, Q, mp.ldq, nullptr, gw, row0, K, rs + R, acc);
+        else if (!SH && l == 0 && !mp.stage_g)
+          gemm_n<MODE, R, true, T>(W, t0, ntw, nullptr, 0, Gd, gw, row0, K, rs + R, acc);
+        else
+          gemm_n<MODE, R, false, T>(W, t0, ntw, Hin, ldi, nullptr, gw, row0, K, rs + R, acc);
+      }
+      if (over) {
+        __syncthreads();
+        if (ntw == 0) continue;
+      }
 #pragma unroll
       for (int j = 0; j < 4; j++) {
         if (j >= ntw) continue;
-        const int c0 = (t0 + 4 * j) * 16 + cq;
+        const int c0 = (t0 + NW * j) * 16 + cq;
         float bv[4] = {0.f, 0.f, 0.f, 0.f};
         if (bias) ld4(bias + c0, bv);
         float ws[4] = {1.f, 1.f, 1.f, 1.f};
@@ -958,7 +1024,7 @@ __global__ __launch_bounds__(256, (kMlpWaves<MODE, R>)) void k_mlp_fast(RowLayou
     const int ld = mp.ld[L - 1];
     const float *w = mp.wout + (size_t) e * mp.wstride[L - 1];
     const float bo = mp.bout ? mp.bout[(size_t) e * mp.bstride[L - 1]] : 0.0f;
-    for (int r = wave; r < R; r += 4) {
+    for (int r = wave; r < R; r += NW) {
       double s = 0.0;
       for (int k = lane; k < K; k += 64) s += (double) (to_f<T>(H[r * ld + k]) * w[k]);
       for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
@@ -973,7 +1039,7 @@ __global__ __launch_bounds__(256, (kMlpWaves<MODE, R>)) void k_mlp_fast(RowLayou
     T *D = sm + mp.offD[L - 2];
     T *gH = sm + mp.offGH;
     const int ld = mp.ld[L - 1];
-    for (int q = threadIdx.x; q < R * N; q += 256) {
+    for (int q = threadIdx.x; q < R * N; q += 64 * NW) {
       int r = q / N, c = q - r * N;
       float v = to_f<T>(D[r * ld + c]);
       D[r * ld + c] = from_f<T>(w[c] * (mp.storeD ? v : 1.0f - v * v));
@@ -1009,9 +1075,9 @@ __global__ __launch_bounds__(256, (kMlpWaves<MODE, R>)) void k_mlp_fast(RowLayou
       __syncthreads();
     }
     const float *wsc = MODE == 2 ? mp.swb[l] + (size_t) e * K : nullptr;
-    for (int tb = 0; tb < NT; tb += 16) {
+    for (int tb = 0; tb < NT; tb += 4 * NW) {
       const int t0 = tb + wave;
-      const int ntw = t0 < NT ? min(4, (NT - t0 + 3) / 4) : 0;
+      const int ntw = t0 < NT ? min(4, (NT - t0 + NW - 1) / NW) : 0;
       if (ntw == 0) continue;
       f32x4 acc[4][RT];
       float mx[RT];  // FP8: the lane's largest |G| per row tile
@@ -1024,7 +1090,7 @@ __global__ __launch_bounds__(256, (kMlpWaves<MODE, R>)) void k_mlp_fast(RowLayou
 #pragma unroll
       for (int j = 0; j < 4; j++) {
         if (j >= ntw) continue;
-        const int c0 = (t0 + 4 * j) * 16 + cq;
+        const int c0 = (t0 + NW * j) * 16 + cq;
         float ws[4] = {1.f, 1.f, 1.f, 1.f};
         if (MODE == 2) ld4(wsc + c0, ws);
 #pragma unroll
@@ -1077,37 +1143,37 @@ int mlp_shape(const MlpParams &mp)
   return 0;
 }
 
+// Tiles at which a mode's compile-time shapes are built: those that
+// tile_rows() takes.
+template <int MODE, int R>
+constexpr bool kShapeTile = R <= 32 || MODE == 1;
+
 // k_mlp_fast with the model's compile-time shape where one exists (tanh
-// models at each mode's default tile), else the generic widths.  Measured
-// (128k- and 1M-atom systems): BF16 MLP -8% and -7%, split BF16 -5%, FP8
-// -36% (78 instead of 128 VGPRs), FP32 -2.5% on the first shape; FP32 on
-// the second shape spills (168 VGPRs) and runs 8% slower, so it keeps the
-// generic kernel.
+// models), else the generic widths.  The constant tile counts, inner steps
+// and ring shapes save registers (BF16 80 instead of 118 VGPRs at 32 rows)
+// and scalar instructions: BF16 network -8 %, FP8 -36 % when measured alone.
 template <int MODE, int A, int R>
 hipError_t launch_fast(dim3 grid, size_t lds, hipStream_t s, const RowLayout &rl, const MlpParams &mp,
-                       const float *G, double *E, float *dEdG, const BatchDims *dyn, int rb, bool gb = false)
+                       const float *G, double *E, float *dEdG, const BatchDims *dyn, int rb, bool gb)
 {
   auto go = [&](auto kern) -> hipError_t {
     if (hipError_t ae = hipFuncSetAttribute((const void *) kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds);
         ae != hipSuccess)
       return ae;
-    kern<<<grid, 256, lds, s>>>(rl, mp, G, E, dEdG, dyn, rb);
+    kern<<<grid, 64 * NW, lds, s>>>(rl, mp, G, E, dEdG, dyn, rb);
     return hipGetLastError();
   };
-  if constexpr (MODE == 1 && A == 2 && R == 32) {
-    if (gb) {
-      const int sh = mlp_shape(mp);
-      if (sh == 1) return go(k_mlp_fast<MODE, A, R, 1, true>);
-      if (sh == 2) return go(k_mlp_fast<MODE, A, R, 2, true>);
-      return hipErrorInvalidValue;
+  if constexpr (A == 2 && kShapeTile<MODE, R>) {
+    const int sh = mlp_shape(mp);
+    if constexpr (MODE == 1) {
+      if (gb && sh == 1) return go(k_mlp_fast<MODE, A, R, 1, true>);
+      if (gb && sh == 2) return go(k_mlp_fast<MODE, A, R, 2, true>);
     }
+    if (gb) return hipErrorInvalidValue;
+    if (sh == 1) return go(k_mlp_fast<MODE, A, R, 1>);
+    if (sh == 2) return go(k_mlp_fast<MODE, A, R, 2>);
   }
   if (gb) return hipErrorInvalidValue;
-  if constexpr (A == 2 && R == (MODE == 2 ? 16 : 32)) {
-    const int sh = mlp_shape(mp);
-    if (sh == 1) return go(k_mlp_fast<MODE, A, R, 1>);
-    if (sh == 2 && MODE != 0) return go(k_mlp_fast<MODE, A, R, 2>);
-  }
   return go(k_mlp_fast<MODE, A, R, 0>);
 }
 
@@ -1236,6 +1302,23 @@ size_t mlp_lds_bytes(const MlpParams &mp, int mode, int R, MlpParams *out)
   m.ldGH = f32lds ? maxw + 4 : maxw + 8;
   m.offGH = (int) off;
   if (anyres) off += (size_t) R * m.ldGH;
+  // the fast kernel's staged descriptor rows: over the activations where the
+  // first layer's outputs fit one pass of the waves, else behind them, or
+  // not staged where that is too much
+  m.stage_g = m.g_over = 0;
+  m.offX = 0;
+  m.ldx = f32lds ? mp.sizes[0] + 4 : mp.sizes[0] + 8;
+  if (mode != 2 && mlp_fast_ok(mp, mode)) {
+    const size_t xn = (size_t) R * m.ldx;
+    if (mp.sizes[1] / 16 <= 4 * NW && xn * esz <= 128 * 1024) {
+      m.stage_g = m.g_over = 1;
+      off = std::max(off, xn);
+    } else if ((off + xn) * esz <= 80 * 1024) {
+      m.stage_g = 1;
+      m.offX = (int) off;
+      off += xn;
+    }
+  }
   size_t bytes = (off * esz + 15) & ~(size_t) 15;
   m.offRS = (int) bytes;
   m.offQ = 0;
@@ -1253,28 +1336,42 @@ size_t mlp_lds_bytes(const MlpParams &mp, int mode, int R, MlpParams *out)
   return bytes;
 }
 
-bool mlp_bf16_rows(const MlpParams &mp, int mode, int rtile)
+bool mlp_bf16_rows(const MlpParams &mp, int mode)
 {
-  if (mode != 1 || !mlp_fast_ok(mp, 1) || mp.act != 2 || mlp_shape(mp) == 0) return false;
-  if (rtile != 0 && rtile != 32) return false;
-  return mlp_lds_bytes(mp, 1, 32, nullptr) <= 160 * 1024;  // the 32-row tile is the one taken
+  return mode == 1 && mlp_fast_ok(mp, 1) && mp.act == 2 && mlp_shape(mp) != 0;
 }
+
+namespace {
+// Rows per tile.  16 while 32-row tiles would not give every CU one (a tile
+// is a serial chain of layers, and its length goes with its rows); 64 in the
+// BF16 mode once they give every CU two (half the weight reads, and their
+// accumulators still fit four waves per SIMD); else 32.  us, network alone,
+// 384-256-128-64-1:   16 rows  32 rows  64 rows
+//   BF16     2,000      18.0     22.2     29.9
+//           16,000      40.3     29.8     33.2
+//          128,000       240      177      145
+//   FP32     2,000      40.1     58.8      101
+//           16,000       107     94.4      103
+//          128,000       775      694      750
+int tile_rows(int mode, int nrows)
+{
+  constexpr int kCUs = 256;
+  if (nrows <= 32 * kCUs) return 16;
+  return mode == 1 && nrows >= 64 * 2 * kCUs ? 64 : 32;
+}
+}  // namespace
 
 hipError_t launch_mlp(int mode, const RowLayout &rl, const MlpParams &mp, const float *G, double *E,
                       float *dEdG, hipStream_t s, int rtile, const BatchDims *dyn, int row_begin,
                       int row_end, bool g_bf16)
 {
-  if (g_bf16 && !mlp_bf16_rows(mp, mode, rtile)) return hipErrorInvalidValue;
+  if (g_bf16 && !mlp_bf16_rows(mp, mode)) return hipErrorInvalidValue;
   if (row_end < 0 || row_end > rl.nrows) row_end = rl.nrows;
   if (row_begin < 0 || row_begin > row_end) return hipErrorInvalidValue;
   if (row_end == row_begin) return hipSuccess;
   const size_t limit = 160 * 1024;
-  // 32-row tiles by default: several workgroups per CU hide the LDS/L2
-  // latency better than one 64-row tile, at twice the (L2-resident) weight
-  // traffic.  FP8: 16-row tiles (its 32-byte K=128 operands need 152 VGPRs
-  // at 32 rows, 3 waves per SIMD; 128 and 4 waves at 16 rows, 2.5% faster
-  // on the 1M-atom C4 system).  rtile (16/32/64) overrides the first choice.
-  int Rs[3] = {mode == 2 ? 16 : 32, 16, 16};
+  // rtile (16/32/64) overrides the rule
+  int Rs[3] = {mlp_fast_ok(mp, mode) ? tile_rows(mode, row_end - row_begin) : 32, 16, 16};
   if (rtile == 16 || rtile == 32 || rtile == 64) Rs[0] = rtile;
   for (int q = 0; q < 3; q++) {
     int R = Rs[q];
