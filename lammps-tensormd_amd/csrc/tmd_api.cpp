@@ -500,6 +500,7 @@ int run_chain(tmd_ctx *ctx, Workspace &w, const Chain &c, hipStream_t s, PhaseEv
     t.n = c.natoms;
     t.out = (double *) w.red.p;
     t.ctl = ctl;
+    t.ctl_host = c.ctl_host;
     t.trig2 = trig2;
     t.pos = c.pos;
     t.v = c.v;

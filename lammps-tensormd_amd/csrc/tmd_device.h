@@ -311,6 +311,7 @@ struct StepTail {
   int n;
   double *out;
   unsigned long long *ctl;
+  unsigned long long *ctl_host;  // with ctl: receives its 4 words (host memory)
   double trig2;
   const double4 *pos;
   double *v;
@@ -321,6 +322,24 @@ struct StepTail {
 };
 constexpr int kSumParts = 240;
 hipError_t launch_step_tail(const StepTail &t, hipStream_t stream);
+// Host transfers of a system's state, through page-locked memory that the
+// kernels read and write themselves.
+// x [n][3] -> pos (elements kept) of atoms [first, first + n)
+hipError_t launch_set_positions(int first, int n, const double *x, double4 *pos, unsigned long long *ctl,
+                                hipStream_t stream);
+// atoms [first, first + n) -> out: x [n][3], v [n][3], f [n][3], eatom [n],
+// those asked for, one behind the other
+struct StateOut {
+  const double4 *pos;
+  const double *v, *f, *eatom;
+  double *out;
+};
+hipError_t launch_pack_state(int first, int n, const StateOut &s, hipStream_t stream);
+// dst[0..n) = src[0..n), n <= 64
+hipError_t launch_copy_small(const double *src, double *dst, int n, hipStream_t stream);
+// pos, v and f to (save) or from snap [n](pos | v | f); counter = 0
+hipError_t launch_snapshot(int n, bool save, double4 *pos, double *v, double *f, void *snap,
+                           unsigned long long *counter, hipStream_t stream);
 // per structure s: out[7 s + 0] = sum eatom, out[7 s + 1..6] = sum watom over
 // atoms [off[s], off[s+1]); resets ctl
 // (with dyn: nstruct is the capacity, dyn->nstruct the live count)

@@ -157,8 +157,10 @@ struct Chain {
   // the list whose control word the evaluation resets (null in list mode)
   const NbrBuild *nb = nullptr;
   // the second half of a velocity-Verlet step rides on the sums: velocities,
-  // per-element constants, and optionally the energy history (StepTail)
+  // per-element constants, and optionally the energy history (StepTail);
+  // ctl_host receives the control word (host memory)
   double *v = nullptr;
+  unsigned long long *ctl_host = nullptr;
   const double *dtfm = nullptr, *mass = nullptr;
   double *hist = nullptr;
   unsigned long long *hist_counter = nullptr;
@@ -200,6 +202,13 @@ struct ListResources {
   unsigned char *host = nullptr;
   size_t host_bytes = 0;
 };
+// The copies, on the process's host worker threads where they are large.
+struct HostCopy {
+  void *dst;
+  const void *src;
+  size_t bytes;
+};
+void copy_threads(const HostCopy *c, int n);
 // serial >= 0 (tmd_compute_list_serial): the list is reused from the
 // previous call with the same serial and shape; serial < 0: always packed.
 int list_compute(tmd_ctx *ctx, const ListArgs &a, const ListResources &r, long long serial);

@@ -25,7 +25,7 @@ struct tmd_system {
   int nbins = 0;
   Workspace w;
   std::vector<int> row2atom;
-  DeviceBuffer vel, dtfm, mass, bins, atominfo, xbuild, sorted, ctl, hist;
+  DeviceBuffer vel, dtfm, mass, bins, atominfo, xbuild, sorted, ctl, xin;
   DeviceBuffer snap;  // x, v, f at the start of the current run segment
   DeviceBuffer order;  // rows in atom order (the descriptor and force kernels' launch order)
   bool have_forces = false;
@@ -44,13 +44,20 @@ struct tmd_system {
   double tsum[3] = {0, 0, 0};    // descriptor, MLP, force kernel ms summed over the samples
   double tkept_sum = 0;          // kept neighbors summed over the samples (all atoms)
   long long tsamples = 0;
-  // a step of tmd_md_step_async whose list-capacity check is still open:
-  // the control words are copied into pinned memory behind it, and the
-  // event marks the copy; the next call on the system resolves it
+  // a step of tmd_md_step_async whose list-capacity check is still open: its
+  // control word is in host_state once the event has passed; the next call on
+  // the system resolves it
   bool pending = false;
   double pending_dt = 0;
   hipEvent_t pend_ev = nullptr;
-  PinnedBuffer pend_ctl;
+  // page-locked memory that kernels read or write: the control word and the
+  // energy history of the last steps, positions and velocities on their way
+  // in (until their events), results on their way out
+  PinnedBuffer host_state, in_x, in_v, out;
+  unsigned long long *ctl_host() const { return (unsigned long long *) host_state.p; }
+  double *hist_host() const { return (double *) host_state.p + 8; }
+  unsigned long long *step_counter() const { return (unsigned long long *) ctl.p + 4; }
+  hipEvent_t ev_x = nullptr, ev_v = nullptr;
 };
 
 namespace tmd {
@@ -160,6 +167,7 @@ Chain sys_chain(tmd_system *s)
   c.fbytes = sizeof(double) * 3 * (size_t) s->n;
   c.natoms = s->n;
   c.nb = &s->nb;
+  c.ctl_host = s->ctl_host();
   c.g_bf16 = true;
   return c;
 }
@@ -184,7 +192,7 @@ int sys_forces(tmd_system *s, const Chain &c, bool step, PhaseEvents *pe = nullp
 
 // The chain of an MD step: the second half kick and, with hist, the energy
 // history ride on its sums.
-constexpr int kHist = 4096;
+constexpr int kSeg = 200;  // steps of a run segment
 Chain step_chain(tmd_system *s, bool want_hist)
 {
   Chain c = sys_chain(s);
@@ -193,17 +201,18 @@ Chain step_chain(tmd_system *s, bool want_hist)
   c.dtfm = (const double *) s->dtfm.p;
   c.mass = (const double *) s->mass.p;
   if (want_hist) {
-    c.hist = (double *) s->hist.p;
-    c.hist_counter = (unsigned long long *) (c.hist + 2 * kHist);
-    c.hist_cap = kHist;
+    c.hist = s->hist_host();
+    c.hist_counter = s->step_counter();
+    c.hist_cap = kSeg;
   }
   return c;
 }
 
-// the control words read after the queued work: an overflow grows the list
-// and asks for a rebuild
-int apply_overflow(tmd_system *s, const unsigned long long *ctl, bool *overflow)
+// the control word that the queued work, now done, has left in host memory:
+// an overflow grows the list and asks for a rebuild
+int apply_overflow(tmd_system *s, bool *overflow)
 {
+  const unsigned long long *ctl = s->ctl_host();
   s->nbuilds_seen = (int) ctl[3];
   *overflow = ctl[2] != 0;
   if (*overflow) {
@@ -226,14 +235,32 @@ int apply_overflow(tmd_system *s, const unsigned long long *ctl, bool *overflow)
 // overflow check after the queued work (waits for it)
 int check_overflow(tmd_system *s, bool *overflow)
 {
-  unsigned long long ctl[4];
-  hipError_t e = hipMemcpyAsync(ctl, s->ctl.p, sizeof(ctl), hipMemcpyDeviceToHost, s->ctx->stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(s->ctx->stream);
-  if (e != hipSuccess) return hip_fail(s->ctx, e, "device step");
-  return apply_overflow(s, ctl, overflow);
+  if (hipError_t e = hipStreamSynchronize(s->ctx->stream); e != hipSuccess)
+    return hip_fail(s->ctx, e, "device step");
+  return apply_overflow(s, overflow);
 }
 
 int md_run_impl(tmd_system *s, int nsteps, double dt, double *epot, double *ekin, bool defer);
+
+hipError_t snapshot(tmd_system *s, bool save)
+{
+  return launch_snapshot(s->n, save, (double4 *) s->w.pos.p, (double *) s->vel.p, (double *) s->w.f.p, s->snap.p,
+                         s->step_counter(), s->ctx->stream);
+}
+
+// Waits until the last transfer from a staging buffer has left it.
+hipError_t staging_free(hipEvent_t &ev)
+{
+  if (!ev) return hipEventCreateWithFlags(&ev, hipEventDisableTiming);  // never used so far
+  return hipEventSynchronize(ev);
+}
+
+// Atoms staged at a time on the way in or out (page-locked memory stays
+// below 64 MB).
+constexpr int kIoAtoms = 800000;
+// Up to this many atoms the kernel reads the staged positions itself; more
+// are copied to the device first, at the full rate of the copy engine.
+constexpr int kDirectIn = 4096;
 
 // Closes the open step of tmd_md_step_async: waits for it and, if its list
 // overflowed, restores the snapshot taken before it and runs it again with
@@ -243,18 +270,10 @@ int resolve_pending(tmd_system *s)
   if (!s->pending) return TMD_OK;
   s->pending = false;
   if (hipError_t e = hipEventSynchronize(s->pend_ev); e != hipSuccess) return hip_fail(s->ctx, e, "device step");
-  unsigned long long ctl[4];
-  std::memcpy(ctl, s->pend_ctl.p, sizeof(ctl));
   bool over = false;
-  int rc = apply_overflow(s, ctl, &over);
+  int rc = apply_overflow(s, &over);
   if (rc != TMD_OK || !over) return rc;
-  const size_t xb = sizeof(double4) * (size_t) s->n, vb = 24 * (size_t) s->n;
-  unsigned char *snap = (unsigned char *) s->snap.p;
-  hipStream_t st = s->ctx->stream;
-  hipError_t e = hipMemcpyAsync(s->w.pos.p, snap, xb, hipMemcpyDeviceToDevice, st);
-  if (e == hipSuccess) e = hipMemcpyAsync(s->vel.p, snap + xb, vb, hipMemcpyDeviceToDevice, st);
-  if (e == hipSuccess) e = hipMemcpyAsync(s->w.f.p, snap + xb + vb, vb, hipMemcpyDeviceToDevice, st);
-  if (e != hipSuccess) return hip_fail(s->ctx, e, "snapshot restore");
+  if (hipError_t e = snapshot(s, false); e != hipSuccess) return hip_fail(s->ctx, e, "snapshot restore");
   return md_run_impl(s, 1, s->pending_dt, nullptr, nullptr, false);
 }
 
@@ -354,7 +373,8 @@ int tmd_system_create(tmd_ctx *ctx, int natoms, const double *x, const int *type
   if ((rc = chk(s->sorted.ensure(sizeof(double4) * (size_t) natoms), "sorted positions alloc"))) return rc;
   if ((rc = chk(s->xbuild.ensure(sizeof(double) * 4 * (size_t) natoms), "xbuild alloc"))) return rc;
   if ((rc = chk(s->ctl.ensure(sizeof(unsigned long long) * 8), "ctl alloc"))) return rc;
-  if ((rc = chk(s->hist.ensure(sizeof(double) * (2 * kHist + 1)), "hist alloc"))) return rc;
+  if ((rc = chk(s->host_state.ensure((8 + 2 * kSeg) * sizeof(double)), "host state alloc"))) return rc;
+  std::memset(s->host_state.p, 0, 8 * sizeof(double));
   if ((rc = alloc_list(s.get(), cap))) return rc;
   int *bins = (int *) s->bins.p;
   s->nb.bin_count = bins;
@@ -394,7 +414,8 @@ void tmd_system_destroy(tmd_system *s)
   hipSetDevice(s->ctx->device);
   hipStreamSynchronize(s->ctx->stream);
   if (s->step_graph) hipGraphExecDestroy(s->step_graph);
-  if (s->pend_ev) hipEventDestroy(s->pend_ev);
+  for (hipEvent_t ev : {s->pend_ev, s->ev_x, s->ev_v})
+    if (ev) hipEventDestroy(ev);
   for (auto &pe : s->tev)
     for (auto &ev : pe.ev) hipEventDestroy(ev);
   delete s;
@@ -406,20 +427,23 @@ int tmd_system_set_positions(tmd_system *s, const double *x)
   if (hipError_t de = hipSetDevice(s->ctx->device); de != hipSuccess)
     return hip_fail(s->ctx, de, "hipSetDevice");
   if (int rc = resolve_pending(s); rc != TMD_OK) return rc;
-  std::vector<double4> pos(s->n);
   hipStream_t st = s->ctx->stream;
-  hipError_t e = hipMemcpyAsync(pos.data(), s->w.pos.p, sizeof(double4) * s->n, hipMemcpyDeviceToHost, st);
-  if (e == hipSuccess) e = hipStreamSynchronize(st);
-  if (e != hipSuccess) return hip_fail(s->ctx, e, "set positions");
-  for (int i = 0; i < s->n; i++) {
-    pos[i].x = x[3 * i];
-    pos[i].y = x[3 * i + 1];
-    pos[i].z = x[3 * i + 2];
+  hipError_t e = hipSuccess;
+  for (int first = 0; first < s->n && e == hipSuccess; first += kIoAtoms) {
+    const int n = std::min(kIoAtoms, s->n - first);
+    const size_t bytes = 3 * sizeof(double) * (size_t) n;
+    if ((e = staging_free(s->ev_x)) != hipSuccess || (e = s->in_x.ensure(bytes)) != hipSuccess) break;
+    const HostCopy cp{s->in_x.p, x + 3 * (size_t) first, bytes};
+    copy_threads(&cp, 1);
+    const double *src = (const double *) s->in_x.p;
+    if (n > kDirectIn) {
+      if ((e = s->xin.ensure(bytes)) != hipSuccess) break;
+      if ((e = hipMemcpyAsync(s->xin.p, s->in_x.p, bytes, hipMemcpyHostToDevice, st)) != hipSuccess) break;
+      src = (const double *) s->xin.p;
+    }
+    e = launch_set_positions(first, n, src, (double4 *) s->w.pos.p, (unsigned long long *) s->ctl.p, st);
+    if (e == hipSuccess) e = hipEventRecord(s->ev_x, st);
   }
-  unsigned long long force_build = 1ull;
-  e = hipMemcpyAsync(s->w.pos.p, pos.data(), sizeof(double4) * s->n, hipMemcpyHostToDevice, st);
-  if (e == hipSuccess) e = hipMemcpyAsync((unsigned long long *) s->ctl.p + 1, &force_build, 8, hipMemcpyHostToDevice, st);
-  if (e == hipSuccess) e = hipStreamSynchronize(st);
   if (e != hipSuccess) return hip_fail(s->ctx, e, "set positions");
   s->have_forces = false;
   return TMD_OK;
@@ -431,7 +455,17 @@ int tmd_system_set_velocities(tmd_system *s, const double *v)
   if (hipError_t de = hipSetDevice(s->ctx->device); de != hipSuccess)
     return hip_fail(s->ctx, de, "hipSetDevice");
   if (int rc = resolve_pending(s); rc != TMD_OK) return rc;
-  hipError_t e = hipMemcpy(s->vel.p, v, sizeof(double) * 3 * (size_t) s->n, hipMemcpyHostToDevice);
+  hipError_t e = hipSuccess;
+  for (int first = 0; first < s->n && e == hipSuccess; first += kIoAtoms) {
+    const int n = std::min(kIoAtoms, s->n - first);
+    const size_t bytes = 3 * sizeof(double) * (size_t) n;
+    if ((e = staging_free(s->ev_v)) != hipSuccess || (e = s->in_v.ensure(bytes)) != hipSuccess) break;
+    const HostCopy cp{s->in_v.p, v + 3 * (size_t) first, bytes};
+    copy_threads(&cp, 1);
+    e = hipMemcpyAsync((double *) s->vel.p + 3 * (size_t) first, s->in_v.p, bytes, hipMemcpyHostToDevice,
+                       s->ctx->stream);
+    if (e == hipSuccess) e = hipEventRecord(s->ev_v, s->ctx->stream);
+  }
   if (e != hipSuccess) return hip_fail(s->ctx, e, "set velocities");
   return TMD_OK;
 }
@@ -464,26 +498,41 @@ int tmd_system_get(tmd_system *s, double *x, double *v, double *f, double *eatom
     return hip_fail(s->ctx, de, "hipSetDevice");
   if (int rc = resolve_pending(s); rc != TMD_OK) return rc;
   hipStream_t st = s->ctx->stream;
-  std::vector<double4> pos;
-  double red[7];
   hipError_t e = hipSuccess;
-  if (x) {
-    pos.resize(s->n);
-    e = hipMemcpyAsync(pos.data(), s->w.pos.p, sizeof(double4) * s->n, hipMemcpyDeviceToHost, st);
+  const int per = (x ? 3 : 0) + (v ? 3 : 0) + (f ? 3 : 0) + (eatom ? 1 : 0);
+  double red[8];
+  const int chunk = std::min(s->n, kIoAtoms);
+  // the sums ride in front of the first chunk
+  if ((e = s->out.ensure(sizeof(double) * (8 + (size_t) per * chunk))) != hipSuccess)
+    return hip_fail(s->ctx, e, "tmd_system_get");
+  double *sums = (double *) s->out.p, *data = sums + 8;
+  StateOut o{};
+  if (x) o.pos = (const double4 *) s->w.pos.p;
+  if (v) o.v = (const double *) s->vel.p;
+  if (f) o.f = (const double *) s->w.f.p;
+  if (eatom) o.eatom = (const double *) s->w.ew.p;
+  o.out = data;
+  if (energy || virial) e = launch_copy_small((const double *) s->w.red.p, sums, 7, st);
+  for (int first = 0; first == 0 || first < s->n; first += chunk) {
+    const int n = std::min(chunk, s->n - first);
+    if (e == hipSuccess) e = launch_pack_state(first, n, o, st);
+    if (e == hipSuccess) e = hipStreamSynchronize(st);
+    if (e != hipSuccess) return hip_fail(s->ctx, e, "tmd_system_get");
+    const double *src = data;
+    HostCopy cp[4];
+    int nc = 0;
+    auto take = [&](double *dst, int w) {
+      if (!dst) return;
+      cp[nc++] = {dst + (size_t) w * first, src, sizeof(double) * (size_t) w * n};
+      src += (size_t) w * n;
+    };
+    take(x, 3);
+    take(v, 3);
+    take(f, 3);
+    take(eatom, 1);
+    copy_threads(cp, nc);
   }
-  if (e == hipSuccess && v) e = hipMemcpyAsync(v, s->vel.p, sizeof(double) * 3 * (size_t) s->n, hipMemcpyDeviceToHost, st);
-  if (e == hipSuccess && f) e = hipMemcpyAsync(f, s->w.f.p, sizeof(double) * 3 * (size_t) s->n, hipMemcpyDeviceToHost, st);
-  if (e == hipSuccess && (energy || virial)) e = hipMemcpyAsync(red, s->w.red.p, sizeof(red), hipMemcpyDeviceToHost, st);
-  if (e == hipSuccess && eatom)
-    e = hipMemcpyAsync(eatom, s->w.ew.p, sizeof(double) * (size_t) s->n, hipMemcpyDeviceToHost, st);
-  if (e == hipSuccess) e = hipStreamSynchronize(st);
-  if (e != hipSuccess) return hip_fail(s->ctx, e, "tmd_system_get");
-  if (x)
-    for (int i = 0; i < s->n; i++) {
-      x[3 * i] = pos[i].x;
-      x[3 * i + 1] = pos[i].y;
-      x[3 * i + 2] = pos[i].z;
-    }
+  std::memcpy(red, sums, sizeof(red));
   if (energy) *energy = red[0];
   if (virial)
     for (int q = 0; q < 6; q++) virial[q] = red[1 + q];
@@ -537,9 +586,7 @@ int md_run_impl(tmd_system *s, int nsteps, double dt, double *epot, double *ekin
     int rc = tmd_system_compute(s);
     if (rc != TMD_OK) return rc;
   }
-  double *hist = (double *) s->hist.p;
   const bool want_hist = epot || ekin;
-  unsigned long long *counter = (unsigned long long *) (hist + 2 * kHist);
   auto enqueue_step = [&](PhaseEvents *pe) -> int {
     hipError_t er = launch_vv_first(s->nb, s->n, (double4 *) s->w.pos.p, (double *) s->vel.p, (double *) s->w.f.p,
                                     (const double *) s->dtfm.p, dt, st);
@@ -570,7 +617,6 @@ int md_run_impl(tmd_system *s, int nsteps, double dt, double *epot, double *ekin
   // neighbor-list overflow inside a segment (a truncated list) grows the
   // list and reruns the segment from the snapshot, so no step ever uses a
   // truncated list.
-  const int kSeg = 200;
   const int every = s->time_every;
   if (every > 0) {
     const size_t need = (size_t) (kSeg + every - 1) / every;
@@ -585,35 +631,19 @@ int md_run_impl(tmd_system *s, int nsteps, double dt, double *epot, double *ekin
   }
   const size_t xb = sizeof(double4) * (size_t) s->n, vb = 24 * (size_t) s->n;
   if ((e = s->snap.ensure(xb + 2 * vb)) != hipSuccess) return hip_fail(s->ctx, e, "snapshot alloc");
-  unsigned char *snap = (unsigned char *) s->snap.p;
-  auto copy3 = [&](bool save) -> hipError_t {
-    hipError_t er;
-    void *a[3] = {s->w.pos.p, s->vel.p, s->w.f.p};
-    void *b[3] = {snap, snap + xb, snap + xb + vb};
-    size_t n[3] = {xb, vb, vb};
-    for (int q = 0; q < 3; q++)
-      if ((er = hipMemcpyAsync(save ? b[q] : a[q], save ? a[q] : b[q], n[q], hipMemcpyDeviceToDevice, st)) !=
-          hipSuccess)
-        return er;
-    return hipSuccess;
-  };
   for (int done = 0; done < nsteps;) {
     int nrun = std::min(kSeg, nsteps - done);
-    if ((e = copy3(true)) != hipSuccess) return hip_fail(s->ctx, e, "snapshot");
+    if ((e = snapshot(s, true)) != hipSuccess) return hip_fail(s->ctx, e, "snapshot");
     bool over = true;
     if (defer) {
-      // one step behind its snapshot; the control words follow it into
-      // pinned memory, read by resolve_pending
+      // one step behind its snapshot; its control word, left in host memory,
+      // is read by resolve_pending
       if (!s->pend_ev && (e = hipEventCreateWithFlags(&s->pend_ev, hipEventDisableTiming)) != hipSuccess)
         return hip_fail(s->ctx, e, "step event");
-      if ((e = s->pend_ctl.ensure(4 * sizeof(unsigned long long))) != hipSuccess)
-        return hip_fail(s->ctx, e, "step control staging");
       if (s->use_graph)
         e = hipGraphLaunch(s->step_graph, st);
       else if (int rc = enqueue_step(nullptr); rc != TMD_OK)
         return rc;
-      if (e == hipSuccess)
-        e = hipMemcpyAsync(s->pend_ctl.p, s->ctl.p, 4 * sizeof(unsigned long long), hipMemcpyDeviceToHost, st);
       if (e == hipSuccess) e = hipEventRecord(s->pend_ev, st);
       if (e != hipSuccess) return hip_fail(s->ctx, e, "step launch");
       s->pending = true;
@@ -621,11 +651,6 @@ int md_run_impl(tmd_system *s, int nsteps, double dt, double *epot, double *ekin
       return TMD_OK;
     }
     for (int attempt = 0; attempt < 4 && over; attempt++) {
-      if (want_hist) {
-        // stream-ordered clear (this loop is never captured into a graph)
-        if ((e = hipMemsetAsync(counter, 0, sizeof(unsigned long long), st)) != hipSuccess)
-          return hip_fail(s->ctx, e, "history reset");
-      }
       if (every > 0) {
         if ((e = hipMemsetAsync(s->tkept.p, 0, sizeof(unsigned long long), st)) != hipSuccess)
           return hip_fail(s->ctx, e, "timing reset");
@@ -665,7 +690,7 @@ int md_run_impl(tmd_system *s, int nsteps, double dt, double *epot, double *ekin
         s->tsamples += nsamp;
       }
       if (over) {
-        if ((e = copy3(false)) != hipSuccess) return hip_fail(s->ctx, e, "snapshot restore");
+        if ((e = snapshot(s, false)) != hipSuccess) return hip_fail(s->ctx, e, "snapshot restore");
         if (s->use_graph && !s->step_graph) {  // the list grew: capture again
           hipGraph_t graph;
           if ((e = hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal)) != hipSuccess)
@@ -685,9 +710,7 @@ int md_run_impl(tmd_system *s, int nsteps, double dt, double *epot, double *ekin
     }
     if (over) return sys_fail(s, TMD_ERR_CAPACITY, "neighbor list overflow persists after growing the list");
     if (want_hist) {
-      std::vector<double> h(2 * (size_t) nrun);
-      if ((e = hipMemcpy(h.data(), hist, sizeof(double) * 2 * nrun, hipMemcpyDeviceToHost)) != hipSuccess)
-        return hip_fail(s->ctx, e, "history copy");
+      const double *h = s->hist_host();  // the stream is idle
       for (int q = 0; q < nrun; q++) {
         if (epot) epot[done + q] = h[2 * q];
         if (ekin) ekin[done + q] = h[2 * q + 1];

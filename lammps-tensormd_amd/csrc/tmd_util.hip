@@ -65,7 +65,11 @@ __device__ inline void finish_step(const StepTail &a, const double *tot)
   const int t = threadIdx.x;
   if (t < 7) a.out[t] = tot[t];
   if (t != 0) return;
-  if (a.ctl) reset_ctl(a.ctl, a.trig2);
+  if (a.ctl) {
+    reset_ctl(a.ctl, a.trig2);
+    if (a.ctl_host)
+      for (int q = 0; q < 4; q++) a.ctl_host[q] = a.ctl[q];
+  }
   if (a.hist) {
     const unsigned long long n = a.counter[0];
     if (n < (unsigned long long) a.hist_cap) {
@@ -139,6 +143,84 @@ __global__ __launch_bounds__(512) void k_step_final(StepTail a, int nparts)
   finish_step(a, tot);
 }
 
+__global__ void k_set_positions(int first, int n, const double *x, double4 *pos, unsigned long long *ctl)
+{
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i == 0) ctl[1] = 1ull;  // rebuild the list
+  if (i >= n) return;
+  double4 p = pos[first + i];
+  p.x = x[3 * (size_t) i];
+  p.y = x[3 * (size_t) i + 1];
+  p.z = x[3 * (size_t) i + 2];
+  pos[first + i] = p;
+}
+
+__global__ void k_copy_small(const double *src, double *dst, int n)
+{
+  if ((int) threadIdx.x < n) dst[threadIdx.x] = src[threadIdx.x];
+}
+
+// One thread per value, so that a wave writes 512 contiguous bytes.
+__global__ void k_pack_state(int first, int n, StateOut s)
+{
+  const size_t n3 = 3 * (size_t) n, total = (s.pos ? n3 : 0) + (s.v ? n3 : 0) + (s.f ? n3 : 0) + (s.eatom ? n : 0);
+  const size_t f3 = 3 * (size_t) first, stride = (size_t) gridDim.x * blockDim.x;
+  for (size_t t = (size_t) blockIdx.x * blockDim.x + threadIdx.x; t < total; t += stride) {
+    size_t q = t;
+    double val = 0.0;
+    bool done = false;
+    if (s.pos) {
+      if (q < n3) {
+        val = reinterpret_cast<const double *>(s.pos + first + q / 3)[q % 3];
+        done = true;
+      } else {
+        q -= n3;
+      }
+    }
+    if (!done && s.v) {
+      if (q < n3) {
+        val = s.v[f3 + q];
+        done = true;
+      } else {
+        q -= n3;
+      }
+    }
+    if (!done && s.f) {
+      if (q < n3) {
+        val = s.f[f3 + q];
+        done = true;
+      } else {
+        q -= n3;
+      }
+    }
+    if (!done) val = s.eatom[first + q];
+    s.out[t] = val;
+  }
+}
+
+__global__ void k_snapshot(int n, bool save, double4 *pos, double *v, double *f, double4 *sp, double *sv, double *sf,
+                           unsigned long long *counter)
+{
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i == 0) counter[0] = 0ull;
+  if (i >= n) return;
+  if (save)
+    sp[i] = pos[i];
+  else
+    pos[i] = sp[i];
+#pragma unroll
+  for (int q = 0; q < 3; q++) {
+    const size_t k = (size_t) q * n + i;  // any order: both sides are [n][3]
+    if (save) {
+      sv[k] = v[k];
+      sf[k] = f[k];
+    } else {
+      v[k] = sv[k];
+      f[k] = sf[k];
+    }
+  }
+}
+
 __global__ void k_copy(const uint4 *__restrict__ src, uint4 *__restrict__ dst, size_t n16)
 {
   size_t i = (size_t) blockIdx.x * blockDim.x + threadIdx.x;
@@ -152,6 +234,37 @@ hipError_t launch_copy(const void *src, void *dst, size_t bytes, hipStream_t s)
 {
   size_t n16 = bytes / 16;
   k_copy<<<8192, 256, 0, s>>>((const uint4 *) src, (uint4 *) dst, n16);
+  return hipGetLastError();
+}
+
+hipError_t launch_set_positions(int first, int n, const double *x, double4 *pos, unsigned long long *ctl,
+                                hipStream_t s)
+{
+  if (n <= 0) return hipSuccess;
+  k_set_positions<<<(n + 255) / 256, 256, 0, s>>>(first, n, x, pos, ctl);
+  return hipGetLastError();
+}
+
+hipError_t launch_pack_state(int first, int n, const StateOut &o, hipStream_t s)
+{
+  const size_t total = (size_t) n * ((o.pos ? 3 : 0) + (o.v ? 3 : 0) + (o.f ? 3 : 0) + (o.eatom ? 1 : 0));
+  if (total == 0) return hipSuccess;
+  k_pack_state<<<(int) std::min<size_t>(2048, (total + 255) / 256), 256, 0, s>>>(first, n, o);
+  return hipGetLastError();
+}
+
+hipError_t launch_copy_small(const double *src, double *dst, int n, hipStream_t s)
+{
+  k_copy_small<<<1, 64, 0, s>>>(src, dst, n);
+  return hipGetLastError();
+}
+
+hipError_t launch_snapshot(int n, bool save, double4 *pos, double *v, double *f, void *snap,
+                           unsigned long long *counter, hipStream_t s)
+{
+  double4 *sp = static_cast<double4 *>(snap);
+  double *sv = reinterpret_cast<double *>(sp + n), *sf = sv + 3 * (size_t) n;
+  k_snapshot<<<(n + 255) / 256, 256, 0, s>>>(n, save, pos, v, f, sp, sv, sf, counter);
   return hipGetLastError();
 }
 
