@@ -200,7 +200,7 @@ hipError_t launch_force_hm(const ModelGeo &g, const Geom &geo, const double4 *po
 // scales, activations and gradients with per-row scales; FP32 accumulation),
 // 3 split bf16 (hi + lo operands, three BF16 products each).
 // E[row] (FP64 output sum) and dEdG[row][width] (fp32).  rtile: rows per
-// workgroup (16, 32 or 64; 0 = default).
+// workgroup (16, 32 or 64, with the fast FP32 kernel also 4 or 8; 0 = default).
 // With dyn, rl gives the capacity (grid) and dyn->rl the live layout.
 // Rows [row_begin, row_end) only (row_end < 0: to rl.nrows); both bounds
 // are multiples of 64 (element blocks start on such rows).

@@ -113,6 +113,16 @@ __device__ inline float from_f<float>(float v) { return v; }
 template <>
 __device__ inline uint16_t from_f<uint16_t>(float v) { return f2bf(v); }
 
+// The tile of block b of the first n: blocks go to the eight XCDs in turn, and
+// each XCD takes a contiguous run of tiles, so that its L2 holds the weights
+// of one or two elements instead of all of them.
+__device__ inline int xcd_tile(int b, int n)
+{
+  constexpr int kXcds = 8;
+  const int x = b % kXcds, i = b / kXcds;
+  return x * (n / kXcds) + min(x, n % kXcds) + i;
+}
+
 __device__ inline int tile_elem(const RowLayout &rl, int row0)
 {
   int e = 0;
@@ -455,14 +465,24 @@ __device__ inline typename Frag<MODE>::A ld_a(const void *A, int t, int s, int n
     return reinterpret_cast<const i32x8 *>(A)[idx];
 }
 
-// B operand (activations of rows r0..r0+15) from a row-major LDS tile;
+// Rows of one row tile of the fast kernel: 16, and 4 in tiles of fewer than
+// 16 rows (FP32), whose products are v_mfma_f32_4x4x1_16b_f32.  Its 16 blocks
+// are the four quads of a tile's 16 columns times the four lane groups, each
+// group with inner values of its own as in the 16x16x4 form, so that both
+// read the same weight fragments; the four groups' sums are added at the end
+// (group_sum).
+template <int R>
+constexpr int kRB = R < 16 ? 4 : 16;
+
+// B operand (activations of rows r0..r0+RB-1) from a row-major LDS tile;
 // FP8: scaled by the row's inverse scale ri
-template <int MODE, typename T>
+template <int MODE, int RB, typename T>
 __device__ inline typename Frag<MODE>::A ld_x(const T *X, int ld, int r0, int k, float ri)
 {
   const int lane = threadIdx.x & 63;
+  static_assert(RB == 16 || MODE == 0, "4-row tiles are FP32");
   if constexpr (MODE == 0) {
-    return *reinterpret_cast<const f32x4 *>(X + (r0 + (lane & 15)) * ld + k + (lane >> 4) * 4);
+    return *reinterpret_cast<const f32x4 *>(X + (r0 + (lane & (RB - 1))) * ld + k + (lane >> 4) * 4);
   } else if constexpr (MODE == 1) {
     return *reinterpret_cast<const bf16x8 *>(X + (r0 + (lane & 15)) * ld + k + (lane >> 4) * 8);
   } else if constexpr (MODE == 3) {
@@ -658,10 +678,15 @@ __device__ inline typename Frag<MODE>::A cvt_graw(const GRaw<MODE> &g, float ri)
   }
 }
 
-template <int MODE>
+template <int MODE, int RB>
 __device__ inline f32x4 mma(typename Frag<MODE>::A a, typename Frag<MODE>::A b, f32x4 c)
 {
-  if constexpr (MODE == 0) {
+  if constexpr (MODE == 0 && RB == 4) {
+    c = __builtin_amdgcn_mfma_f32_4x4x1f32(a[0], b[0], c, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f32_4x4x1f32(a[1], b[1], c, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f32_4x4x1f32(a[2], b[2], c, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_4x4x1f32(a[3], b[3], c, 0, 0, 0);
+  } else if constexpr (MODE == 0) {
     c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[0], b[0], c, 0, 0, 0);
     c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[1], b[1], c, 0, 0, 0);
     c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[2], b[2], c, 0, 0, 0);
@@ -706,6 +731,19 @@ __device__ inline void row_scales(const uint16_t *X, int ld, const float *G, int
     rs[r] = sc;
     rs[R + r] = 1.0f / sc;
   }
+}
+
+// Lane group m: component m of the accumulators, summed over the four groups
+// (each exchange between the halves or the rows of lanes serves two sums).
+__device__ inline float group_sum(const f32x4 &c)
+{
+  auto halves = [](float a, float b) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  };
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(halves(c[0], c[2])),
+                                                  __float_as_uint(halves(c[1], c[3])), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
 // 4 consecutive values of a row-major LDS tile (8- or 16-byte aligned)
@@ -792,16 +830,17 @@ __device__ inline void stage_g(const float *G, int gw_, int grow0, T *X, int ld)
 // Global operands (the weights, and the descriptor rows of layer 0) go
 // through a register ring D steps deep, D = (fragments budget) / NTW (2 for
 // layer 0, whose ring also holds its raw rows), so a load has D - 1 steps of
-// MFMA work to arrive in.  Every step issues the
+// MFMA work to arrive in; twice the budget in tiles of fewer than 16 rows,
+// whose steps are short.  Every step issues the
 // same number of loads (past the last step they repeat it), which lets the
 // compiler wait for exactly the step being consumed.  Activations in LDS
 // are read at the step that uses them.
 template <int MODE, int R, bool XG, int NTW, typename T>
 __device__ inline void gemm_t(const void *W, int t0, const T *X, int ldx, const float *G, int gw,
-                              int grow0, int K, const float *rinv, f32x4 (&acc)[4][R / 16])
+                              int grow0, int K, const float *rinv, f32x4 (&acc)[4][R / kRB<R>])
 {
-  constexpr int KS = kFastKS<MODE>, RT = R / 16;
-  constexpr int DW = 8 / NTW;
+  constexpr int KS = kFastKS<MODE>, RB = kRB<R>, RT = R / RB;
+  constexpr int DW = (RB == 4 ? 16 : 8) / NTW;
   constexpr int D = XG ? 2 : (DW >= 2 ? DW : 2);  // layer 0 also rings its raw rows
   using F = typename Frag<MODE>::A;
 #pragma unroll
@@ -838,12 +877,12 @@ __device__ inline void gemm_t(const void *W, int t0, const T *X, int ldx, const 
           if constexpr (XG)
             b[r] = cvt_graw<MODE>(g[i][r], ri[r]);
           else
-            b[r] = ld_x<MODE>(X, ldx, r * 16, s * KS, ri[r]);
+            b[r] = ld_x<MODE, RB>(X, ldx, r * RB, s * KS, ri[r]);
         }
 #pragma unroll
         for (int j = 0; j < NTW; j++)
 #pragma unroll
-          for (int r = 0; r < RT; r++) acc[j][r] = mma<MODE>(a[i][j], b[r], acc[j][r]);
+          for (int r = 0; r < RT; r++) acc[j][r] = mma<MODE, RB>(a[i][j], b[r], acc[j][r]);
       }
     }
   }
@@ -852,7 +891,7 @@ __device__ inline void gemm_t(const void *W, int t0, const T *X, int ldx, const 
 // gemm_t for a runtime tile count ntw in 1..4 (wave-uniform)
 template <int MODE, int R, bool XG, typename T>
 __device__ inline void gemm_n(const void *W, int t0, int ntw, const T *X, int ldx, const float *G,
-                              int gw, int grow0, int K, const float *rinv, f32x4 (&acc)[4][R / 16])
+                              int gw, int grow0, int K, const float *rinv, f32x4 (&acc)[4][R / kRB<R>])
 {
   if (ntw >= 4)
     gemm_t<MODE, R, XG, 4, T>(W, t0, X, ldx, G, gw, grow0, K, rinv, acc);
@@ -868,9 +907,10 @@ __device__ inline void gemm_n(const void *W, int t0, int ntw, const T *X, int ld
 
 // Waves per SIMD asked of the fast kernel; a workgroup has two.  Four where
 // the registers allow it (the compile-time shapes, and the FP32 and BF16
-// modes up to 32 rows), else two.
+// modes up to 32 rows), else two; two in tiles of fewer than 16 rows, which
+// are taken where a CU has one tile.
 template <int MODE, int R, int SH>
-constexpr int kMlpWaves = SH ? 4 : ((R <= 32 && MODE <= 1) ? 4 : 2);
+constexpr int kMlpWaves = R < 16 ? 2 : SH ? 4 : ((R <= 32 && MODE <= 1) ? 4 : 2);
 
 // bytes per weight of the fast kernel's A operands
 template <int MODE>
@@ -897,15 +937,16 @@ struct MlpShape<2> {  // 384-256-256-128-1
 // GB: Gd holds BF16 descriptor rows (MODE 1 only)
 template <int MODE, int ACT, int R, int SH = 0, bool GB = false>
 __global__ __launch_bounds__(64 * NW, (kMlpWaves<MODE, R, SH>)) void k_mlp_fast(RowLayout rl_cap, MlpParams mp, const float *Gd,
-                                                  double *E, float *dEdG, const BatchDims *dyn, int rbase)
+                                                  double *E, float *dEdG, const BatchDims *dyn, int rbase, int rend)
 {
   const RowLayout rl = dyn ? dyn->rl : rl_cap;
   using T = typename Traits<MODE>::T;
-  constexpr int RT = R / 16;
+  constexpr int RB = kRB<R>, RT = R / RB;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   T *sm = reinterpret_cast<T *>(smem_raw);
-  const int row0 = rbase + (int) blockIdx.x * R;
-  if (row0 >= rl.nrows) return;
+  const int tiles = (min(rl.nrows, rend) - rbase) / R;
+  if ((int) blockIdx.x >= tiles) return;
+  const int row0 = rbase + xcd_tile(blockIdx.x, tiles) * R;
   const int e = tile_elem(rl, row0);
   // wave index made wave-uniform for the compiler: tile bounds and guards
   // derived from it are scalar branches
@@ -916,6 +957,7 @@ __global__ __launch_bounds__(64 * NW, (kMlpWaves<MODE, R, SH>)) void k_mlp_fast(
   const int L = SH ? MlpShape<SH>::nl : mp.nl;
   const int cq = 4 * (lane >> 4);  // first of the lane's 4 output columns in a tile
   const int rq = lane & 15;        // the lane's row in a row tile
+  const int c4 = (lane & 12) + (lane >> 4);  // 4-row tiles: the lane's output column in a tile
   float *rs = reinterpret_cast<float *>(smem_raw + mp.offRS);  // FP8 row scales [2][R]
   uint8_t *Q = smem_raw + mp.offQ;                              // FP8 B operand rows [R][ldq]
   // FP8 row maxima [2][R]: GEMM g (forward layer l: g = l; backward layer
@@ -986,6 +1028,20 @@ __global__ __launch_bounds__(64 * NW, (kMlpWaves<MODE, R, SH>)) void k_mlp_fast(
 #pragma unroll
       for (int j = 0; j < 4; j++) {
         if (j >= ntw) continue;
+        if constexpr (RB == 4) {  // one output per lane and row tile
+          const int c = (t0 + NW * j) * 16 + c4;
+          const float bv = bias ? bias[c] : 0.0f;
+#pragma unroll
+          for (int r = 0; r < RT; r++) {
+            const int row = r * RB + (lane & 3);
+            float dz;
+            float h = act_f<ACT>(group_sum(acc[j][r]) + bv, dz);
+            if (mp.res[l]) h += Hin[row * ldi + c];
+            H[row * ldo + c] = h;
+            if (mp.storeD) D[row * ldo + c] = dz;
+          }
+          continue;
+        }
         const int c0 = (t0 + NW * j) * 16 + cq;
         float bv[4] = {0.f, 0.f, 0.f, 0.f};
         if (bias) ld4(bias + c0, bv);
@@ -1090,6 +1146,24 @@ __global__ __launch_bounds__(64 * NW, (kMlpWaves<MODE, R, SH>)) void k_mlp_fast(
 #pragma unroll
       for (int j = 0; j < 4; j++) {
         if (j >= ntw) continue;
+        if constexpr (RB == 4) {
+          const int c = (t0 + NW * j) * 16 + c4;
+#pragma unroll
+          for (int r = 0; r < RT; r++) {
+            const int row = r * RB + (lane & 3);
+            float v = group_sum(acc[j][r]);
+            if (mp.res[l]) v += gH[row * mp.ldGH + c];
+            if (l == 0) {
+              dEdG[(size_t) (row0 + row) * gw + c] = v;
+            } else {
+              T *D = sm + mp.offD[l - 1] + row * mp.ld[l] + c;
+              const float d = *D;
+              *D = v * (mp.storeD ? d : 1.0f - d * d);
+              if (mp.res[l - 1]) gH[row * mp.ldGH + c] = v;
+            }
+          }
+          continue;
+        }
         const int c0 = (t0 + NW * j) * 16 + cq;
         float ws[4] = {1.f, 1.f, 1.f, 1.f};
         if (MODE == 2) ld4(wsc + c0, ws);
@@ -1160,7 +1234,7 @@ hipError_t launch_fast(dim3 grid, size_t lds, hipStream_t s, const RowLayout &rl
     if (hipError_t ae = hipFuncSetAttribute((const void *) kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds);
         ae != hipSuccess)
       return ae;
-    kern<<<grid, 64 * NW, lds, s>>>(rl, mp, G, E, dEdG, dyn, rb);
+    kern<<<grid, 64 * NW, lds, s>>>(rl, mp, G, E, dEdG, dyn, rb, rb + (int) grid.x * R);
     return hipGetLastError();
   };
   if constexpr (A == 2 && kShapeTile<MODE, R>) {
@@ -1184,7 +1258,7 @@ hipError_t launch_r(const RowLayout &rl, const MlpParams &mp, const float *G, do
   if (rb % R || re % R) return hipErrorInvalidValue;
   dim3 grid((re - rb) / R);
   const bool fast = mlp_fast_ok(mp, MODE);
-  if constexpr (MODE == 2 || MODE == 3) {  // FP8 and split BF16 exist on the fast path only
+  if constexpr (MODE == 2 || MODE == 3 || R < 16) {  // these exist on the fast path only
     if (!fast) return hipErrorInvalidConfiguration;
 #define TMD_MLP8_CASE(A)                                                                         \
   case A:                                                                                        \
@@ -1282,7 +1356,7 @@ size_t mlp_lds_bytes(const MlpParams &mp, int mode, int R, MlpParams *out)
   bool anyres = false;
   for (int l = 0; l <= mp.nl - 1; l++) {
     int w = mp.sizes[l];
-    m.ld[l] = f32lds ? w + 4 : w + 8;
+    m.ld[l] = R < 16 ? w + 16 : (f32lds ? w + 4 : w + 8);
   }
   for (int l = 0; l < mp.nl - 1; l++)
     if (mp.res[l]) anyres = true;
@@ -1299,7 +1373,7 @@ size_t mlp_lds_bytes(const MlpParams &mp, int mode, int R, MlpParams *out)
       off += (size_t) R * m.ld[l + 1];
     }
   }
-  m.ldGH = f32lds ? maxw + 4 : maxw + 8;
+  m.ldGH = R < 16 ? maxw + 16 : (f32lds ? maxw + 4 : maxw + 8);
   m.offGH = (int) off;
   if (anyres) off += (size_t) R * m.ldGH;
   // the fast kernel's staged descriptor rows: over the activations where the
@@ -1307,7 +1381,7 @@ size_t mlp_lds_bytes(const MlpParams &mp, int mode, int R, MlpParams *out)
   // not staged where that is too much
   m.stage_g = m.g_over = 0;
   m.offX = 0;
-  m.ldx = f32lds ? mp.sizes[0] + 4 : mp.sizes[0] + 8;
+  m.ldx = m.ld[0];
   if (mode != 2 && mlp_fast_ok(mp, mode)) {
     const size_t xn = (size_t) R * m.ldx;
     if (mp.sizes[1] / 16 <= 4 * NW && xn * esz <= 128 * 1024) {
@@ -1345,17 +1419,31 @@ namespace {
 // Rows per tile.  16 while 32-row tiles would not give every CU one (a tile
 // is a serial chain of layers, and its length goes with its rows); 64 in the
 // BF16 mode once they give every CU two (half the weight reads, and their
-// accumulators still fit four waves per SIMD); else 32.  us, network alone,
-// 384-256-128-64-1:   16 rows  32 rows  64 rows
-//   BF16     2,000      18.0     22.2     29.9
-//           16,000      40.3     29.8     33.2
-//          128,000       240      177      145
-//   FP32     2,000      40.1     58.8      101
-//           16,000       107     94.4      103
-//          128,000       775      694      750
-int tile_rows(int mode, int nrows)
+// accumulators still fit four waves per SIMD); else 32.  FP32 tiles of 4 and
+// 8 rows while those give no CU a second one: a lone 16-row tile is bound by
+// its CU's matrix cores, 0.11 us per 1,000 weights, so they pay where that is
+// most of its time (16 K weights: 15.9 us at 16 rows, 16.4 and 17.3 at 4 and
+// 8; 82 K: 32.7, 29.5 and 32.4).  us, network alone, 384-256-128-64-1
+// (139 K weights):     4 rows   8 rows  16 rows  32 rows  64 rows
+//   FP32       128      18.3     23.5     32.5     52.0
+//            1,024      22.1     24.3     32.6     52.4
+//            2,000      30.9     29.0     35.0     53.8
+//            3,456      53.6     38.4     38.5     55.6
+//            8,192      95.6     68.7     56.7     58.8
+//           16,000       184      127      105     93.5      103
+//   BF16     2,000                        15.8     18.3     25.1
+//            8,192                        25.0     25.5     32.1
+//           16,000                        40.0     29.8     34.2
+//           35,152                        73.2     66.5     65.1
+//          128,000                         245      191      150
+int tile_rows(const MlpParams &mp, int mode, int nrows)
 {
   constexpr int kCUs = 256;
+  if (mode == 0 && nrows <= 8 * kCUs) {
+    long w = 0;
+    for (int l = 0; l < mp.nl - 1; l++) w += (long) mp.sizes[l] * mp.sizes[l + 1];
+    if (w >= 64 * 1024) return nrows <= 4 * kCUs ? 4 : 8;
+  }
   if (nrows <= 32 * kCUs) return 16;
   return mode == 1 && nrows >= 64 * 2 * kCUs ? 64 : 32;
 }
@@ -1370,9 +1458,10 @@ hipError_t launch_mlp(int mode, const RowLayout &rl, const MlpParams &mp, const 
   if (row_begin < 0 || row_begin > row_end) return hipErrorInvalidValue;
   if (row_end == row_begin) return hipSuccess;
   const size_t limit = 160 * 1024;
-  // rtile (16/32/64) overrides the rule
-  int Rs[3] = {mlp_fast_ok(mp, mode) ? tile_rows(mode, row_end - row_begin) : 32, 16, 16};
-  if (rtile == 16 || rtile == 32 || rtile == 64) Rs[0] = rtile;
+  // rtile (16/32/64, FP32 fast kernel also 4/8) overrides the rule
+  const bool fast = mlp_fast_ok(mp, mode);
+  int Rs[3] = {fast ? tile_rows(mp, mode, row_end - row_begin) : 32, 16, 16};
+  if (rtile == 16 || rtile == 32 || rtile == 64 || (mode == 0 && fast && (rtile == 4 || rtile == 8))) Rs[0] = rtile;
   for (int q = 0; q < 3; q++) {
     int R = Rs[q];
     MlpParams m;
@@ -1381,6 +1470,8 @@ hipError_t launch_mlp(int mode, const RowLayout &rl, const MlpParams &mp, const 
     if (mode == 0) {
       if (R == 64) return launch_r<0, 64>(rl, m, G, E, dEdG, lds, s, dyn, row_begin, row_end);
       if (R == 32) return launch_r<0, 32>(rl, m, G, E, dEdG, lds, s, dyn, row_begin, row_end);
+      if (R == 4) return launch_r<0, 4>(rl, m, G, E, dEdG, lds, s, dyn, row_begin, row_end);
+      if (R == 8) return launch_r<0, 8>(rl, m, G, E, dEdG, lds, s, dyn, row_begin, row_end);
       return launch_r<0, 16>(rl, m, G, E, dEdG, lds, s, dyn, row_begin, row_end);
     }
     if (mode == 3) {

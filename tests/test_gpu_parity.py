@@ -1109,3 +1109,75 @@ def test_step_sums(synth_models, cells):
     assert abs(ek[-1] - W.kinetic_energy(mass, r["v"])) <= eps * ek[-1]
     assert abs(ek[0] - W.kinetic_energy(mass, v)) < 0.05 * ek[0]
     assert np.all(np.diff(ek) != 0.0) and np.all(np.diff(ep) != 0.0)
+
+
+def _network_spread(z, G, nl, act, resnet, u_op):
+    """E, dE/dG of one element's network in FP64 on the descriptor rows G, and
+    the spread that rounding gives an FP32 evaluation whose operands are
+    rounded with relative error u_op each: independent errors add in quadrature,
+    a sum of n products has sqrt(n) u times the norm of its terms, and an
+    activation or its derivative a few u."""
+    u = 2.0 ** -24
+    Ws = [z["weights_0_%d" % l].astype(np.float32).astype(float) for l in range(nl)]
+    bs = [z["biases_0_%d" % l].astype(np.float32).astype(float) for l in range(nl)]
+    w = Ws[-1].reshape(-1)
+
+    def product(x, ex, W_, b=0.0):  # spread of x W + b
+        return np.sqrt((W_.shape[0] * u * u + 2 * u_op * u_op) * (x * x @ (W_ * W_) + b * b) + ex * ex @ (W_ * W_))
+
+    H, eH, D = G.astype(float), 0.0 * G, []
+    for W_, b in zip(Ws[:-1], bs[:-1]):
+        a, e = H @ W_ + b, product(H, eH, W_, b)
+        if act == "tanh":
+            h = np.tanh(a)
+            d = 1 - h * h
+            eh = np.hypot(np.hypot(d * e, 8 * u), u_op * h)
+            ed = np.hypot(2 * h * eh, 2 * u)
+        else:
+            r = np.sqrt(a * a + 4)
+            h = 0.5 * (a + r)
+            d = h / r
+            eh, ed = np.hypot(d * e, 8 * u * np.maximum(h, 1)), np.hypot(2 / r ** 3 * e, 8 * u)
+        res = resnet and W_.shape[0] == W_.shape[1]
+        D.append((d, ed, res))
+        H, eH = (h + H, np.hypot(np.hypot(eh, eH), u * (h + H))) if res else (h, eh)
+    E = H @ w + float(bs[-1].reshape(-1)[0])
+    sE = np.sqrt(((2 * u * H * w) ** 2 + (eH * w) ** 2).sum(1) + (2 * u * E) ** 2)
+    g, eg = np.broadcast_to(w, H.shape), 0.0 * H
+    for (d, ed, res), W_ in zip(D[::-1], Ws[-2::-1]):
+        gd = g * d
+        gi, ei = gd @ W_.T, product(gd, np.hypot(np.hypot(eg * d, g * ed), 2 * u * gd), W_.T)
+        g, eg = (gi + g, np.hypot(np.hypot(ei, eg), u * (gi + g))) if res else (gi, ei)
+    return E, sE, g, eg
+
+
+@pytest.mark.parametrize("prec,k,layers,act,resnet,cells", [
+    ("fp32", 24, [256, 128, 128, 1], "tanh", False, [(3, 3, 3), (8, 8, 8), (8, 8, 9), (8, 16, 8), (8, 16, 9),
+                                                     (16, 16, 16), (8, 16, 33)]),
+    ("fp32", 64, [128, 128, 128, 128, 1], "squareplus", True, [(5, 5, 5), (8, 16, 8), (9, 16, 8)]),
+    ("fp32", 16, [64, 64, 1], "tanh", False, [(3, 3, 3), (8, 8, 8)]),
+    ("fp32", 32, [576, 64, 1], "tanh", False, [(5, 5, 5), (8, 8, 9), (8, 16, 9), (8, 16, 33)]),
+    ("bf16", 24, [256, 128, 128, 1], "tanh", False, [(16, 16, 16), (8, 16, 33), (16, 32, 31), (16, 32, 32)]),
+])
+def test_network_tiles(tmp_path, prec, k, layers, act, resnet, cells):
+    """The network alone at the row counts where its tiles change (4, 8, 16, 32
+    and 64 rows), with few and many weights, with skips, and with a first layer
+    too wide for its descriptor rows to be staged over the activations: energies
+    and dE/dG on the exported descriptor rows against FP64, within eight times
+    the spread of the arithmetic's rounding."""
+    path = W.write_model(str(tmp_path / "m.npz"), symbols=["W"], masses=[183.84], rmax=5.0, num_filters=k,
+                         layer_sizes=layers, actfn=act, use_resnet_dt=resnet, seed=70 + k, radial_scale=0.2)
+    z = dict(np.load(path))
+    m = TensorMD(path, ["W"], prec, 0.001)
+    for c in cells:
+        x, t, cell = W.crystal("bcc", 3.2, c, nelt=1, sigma=0.08, seed=71)
+        say("case: network", prec, layers, act, len(x), "atoms")
+        s = m.system(x, t, cell, skin=0.6)
+        r = s.compute()
+        G, dG = s.descriptors(m.info()["width"])
+        s.close()
+        E, sE, g, sg = _network_spread(z, G, len(layers), act, resnet, 2.0 ** -9 if prec == "bf16" else 0.0)
+        e0, e1 = abs(r["eatom"] - E) / sE, abs(dG - g) / sg
+        say("largest error / spread: E", e0.max(), "dE/dG", e1.max(), "rms dE/dG error",
+            float(np.sqrt(((dG - g) ** 2).mean())), "rms dE/dG", float(np.sqrt((g ** 2).mean())))
+        assert e0.max() <= 8.0 and e1.max() <= 8.0, (len(x), e0.max(), e1.max())
