@@ -24,7 +24,7 @@
 // Operand layouts (16x16 tiles): A lane l holds row l%16, k-group l/16;
 // B lane l holds column l%16, k-group l/16; C lane l holds rows
 // 4*(l/16)+i, column l%16.
-#include "tmd_device.h"
+#include "tmd_desc_common.h"
 
 namespace tmd {
 
@@ -39,16 +39,35 @@ typedef float f32x8 __attribute__((ext_vector_type(8)));
 typedef int i32x8 __attribute__((ext_vector_type(8)));
 __device__ inline float bf2f(uint16_t v) { return __uint_as_float(((uint32_t) v) << 16); }
 
+// tanh without branches, so that a lane's values overlap: below 1 the odd
+// polynomial x + x u p(u), u = x^2 (p fitted to the relative error on [0, 1],
+// 5e-9), above it 1 - 2 / (exp(2 |x|) + 1).  Largest error 1.3 ulp and rms
+// 1.63e-8 over normal and uniform [-6, 6] arguments; the library's, two
+// divergent branches, has 1.4 ulp and 1.70e-8 there.
+__device__ inline float tanh_f32(float x)
+{
+  const float e = __builtin_amdgcn_exp2f(fabsf(x) * 2.8853900817779268f);  // 2 / ln 2
+  const float r = fmaf(-2.0f, __builtin_amdgcn_rcpf(e + 1.0f), 1.0f);
+  const float u = x * x;
+  float p = -3.58451881e-4f;
+  p = fmaf(p, u, 2.30136419e-3f);
+  p = fmaf(p, u, -7.94610591e-3f);
+  p = fmaf(p, u, 2.14866572e-2f);
+  p = fmaf(p, u, -5.38798026e-2f);
+  p = fmaf(p, u, 1.33323446e-1f);
+  p = fmaf(p, u, -3.33332954e-1f);
+  return fabsf(x) >= 1.0f ? copysignf(r, x) : fmaf(x * u, p, x);
+}
+
 // activation value and derivative (nnp.cu:9-49, activation.hpp:158-261).
 // FAST (BF16 and FP8 modes, whose operands are rounded to 8 significant bits
-// or fewer): tanh from one exp and one 1-ulp hardware reciprocal,
-// tanh z = 1 - 2 / (exp(2z) + 1) (a correctly rounded reciprocal is a
-// ten-instruction division sequence).
+// or fewer): exp, reciprocal and square root are the hardware's (1 ulp), as
+// in tanh z = 1 - 2 / (exp(2z) + 1).
 template <int ACT, bool FAST = false>
 __device__ inline float act_f(float z, float &dz)
 {
-  if (ACT == 2 && FAST) {
-    float h = 1.0f - 2.0f * __builtin_amdgcn_rcpf(__expf(2.0f * z) + 1.0f);
+  if (ACT == 2) {
+    float h = FAST ? 1.0f - 2.0f * __builtin_amdgcn_rcpf(__expf(2.0f * z) + 1.0f) : tanh_f32(z);
     dz = 1.0f - h * h;
     return h;
   }
@@ -57,16 +76,26 @@ __device__ inline float act_f(float z, float &dz)
     float h = (z < 13.942385f) ? log1pf(ez) : z;
     dz = 1.0f / (1.0f + 1.0f / ez);
     return h;
-  } else if (ACT == 2) {
-    float h = tanhf(z);
-    dz = 1.0f - h * h;
-    return h;
   } else if (ACT == 3) {
-    // squareplus (z + sqrt(z^2 + 4)) / 2; for z < 0 the same value as
-    // 2 / (sqrt(z^2 + 4) - z), which does not cancel in FP32
-    float s = sqrtf(z * z + 4.0f);
-    float h = z >= 0.0f ? 0.5f * (z + s) : 2.0f / (s - z);
-    dz = h / s;
+    // squareplus h = (z + s) / 2, s = sqrt(z^2 + 4); for z < 0 the same value
+    // as 2 / (s - z), which does not cancel in FP32.  h' = h / s.
+    if (FAST) {
+      const float s = __builtin_amdgcn_sqrtf(fmaf(z, z, 4.0f)), w = s + fabsf(z);
+      const float h = z < 0.0f ? 2.0f * __builtin_amdgcn_rcpf(w) : 0.5f * w;
+      dz = h * __builtin_amdgcn_rcpf(s);
+      return h;
+    }
+    // root, reciprocals and quotient each corrected once by their residual:
+    // the errors of the correctly rounded operations (rms 7.37e-8 and 2.65e-8
+    // of h and h' over the arguments above) without their range scaling and
+    // branches.  z is bounded below to keep the residuals finite.
+    const float zc = fmaxf(z, -1e18f), a = fmaf(zc, zc, 4.0f), r0 = __builtin_amdgcn_rsqf(a), s0 = a * r0;
+    const float s = fmaf(fmaf(-s0, s0, a), 0.5f * r0, s0), r = fmaf(fmaf(-s, r0, 1.0f), r0, r0), w = s - zc;
+    float q = __builtin_amdgcn_rcpf(w);
+    q = fmaf(fmaf(-w, q, 1.0f), q, q);
+    const float h = z < 0.0f ? 2.0f * q : 0.5f * (z + s);
+    dz = h * r;
+    dz = fmaf(fmaf(-dz, s, h), r, dz);
     return h;
   }
   dz = z >= 0.0f ? 1.0f : 0.0f;
@@ -733,17 +762,10 @@ __device__ inline void row_scales(const uint16_t *X, int ld, const float *G, int
   }
 }
 
-// Lane group m: component m of the accumulators, summed over the four groups
-// (each exchange between the halves or the rows of lanes serves two sums).
+// Lane group m: component m of the accumulators, summed over the four groups.
 __device__ inline float group_sum(const f32x4 &c)
 {
-  auto halves = [](float a, float b) {
-    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
-    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-  };
-  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(halves(c[0], c[2])),
-                                                  __float_as_uint(halves(c[1], c[3])), false, false);
-  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  return swap16_add(swap32_add(c[0], c[2]), swap32_add(c[1], c[3]));
 }
 
 // 4 consecutive values of a row-major LDS tile (8- or 16-byte aligned)
@@ -1073,33 +1095,39 @@ __global__ __launch_bounds__(64 * NW, (kMlpWaves<MODE, R, SH>)) void k_mlp_fast(
     __syncthreads();
   }
 
-  // ---------------- output layer: E = H w + b (FP64 sum) ----------------
-  {
-    const int K = width(L - 1);
-    const T *H = sm + mp.offH[L - 2];
-    const int ld = mp.ld[L - 1];
-    const float *w = mp.wout + (size_t) e * mp.wstride[L - 1];
-    const float bo = mp.bout ? mp.bout[(size_t) e * mp.bstride[L - 1]] : 0.0f;
-    for (int r = wave; r < R; r += NW) {
-      double s = 0.0;
-      for (int k = lane; k < K; k += 64) s += (double) (to_f<T>(H[r * ld + k]) * w[k]);
-      for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
-      if (lane == 0) E[row0 + r] = s + (double) bo;
-    }
-  }
-  __syncthreads();
-  // seed: G_{L-2} = w_out * D_{L-2} (in the D slot); dE/dH = w_out for a resnet layer
+  // ---------------- output layer ----------------
+  // E = H w + b (FP64 sum) and the seed G_{L-2} = w_out * D_{L-2} (in the D
+  // slot; dE/dH = w_out for a resnet layer) in one pass: a wave takes whole
+  // rows, so that it may overwrite what it has read, four at a time, whose
+  // sums share the exchanges between halves and rows of lanes.
   {
     const int N = width(L - 1);
-    const float *w = mp.wout + (size_t) e * mp.wstride[L - 1];
+    T *H = sm + mp.offH[L - 2];
     T *D = sm + mp.offD[L - 2];
     T *gH = sm + mp.offGH;
     const int ld = mp.ld[L - 1];
-    for (int q = threadIdx.x; q < R * N; q += 64 * NW) {
-      int r = q / N, c = q - r * N;
-      float v = to_f<T>(D[r * ld + c]);
-      D[r * ld + c] = from_f<T>(w[c] * (mp.storeD ? v : 1.0f - v * v));
-      if (mp.res[L - 2]) gH[r * mp.ldGH + c] = from_f<T>(w[c]);
+    const float *w = mp.wout + (size_t) e * mp.wstride[L - 1];
+    const float bo = mp.bout ? mp.bout[(size_t) e * mp.bstride[L - 1]] : 0.0f;
+    constexpr int kRows = R >= 4 * NW ? 4 : (R >= 2 * NW ? 2 : 1);
+    for (int r0 = wave; r0 < R; r0 += kRows * NW) {
+      double s[4] = {0.0, 0.0, 0.0, 0.0};
+      for (int k = lane; k < N; k += 64) {
+        const float wk = w[k];
+#pragma unroll
+        for (int q = 0; q < kRows; q++) {
+          const int r = r0 + q * NW;
+          const float hv = to_f<T>(H[r * ld + k]);
+          const float dv = mp.storeD ? to_f<T>(D[r * ld + k]) : 1.0f - hv * hv;
+          s[q] += (double) (hv * wk);
+          D[r * ld + k] = from_f<T>(wk * dv);
+          if (mp.res[L - 2]) gH[r * mp.ldGH + k] = from_f<T>(wk);
+        }
+      }
+      const double x = kRows == 1 ? swap32_add(s[0], s[0]) : swap32_add(s[0], s[1]);
+      const double v = row_sum_d(swap16_add(x, kRows == 4 ? swap32_add(s[2], s[3]) : x));
+      // rows of 16 lanes hold the sums 0, 2, 1, 3
+      const int q = ((lane >> 4) & 1) * 2 + (lane >> 5);
+      if ((lane & 15) == 0 && q < kRows) E[row0 + r0 + q * NW] = v + (double) bo;
     }
   }
   __syncthreads();
