@@ -217,7 +217,8 @@ int tmd_md_step_async(tmd_system *sys, double dt);
  * between phases; ms[0..6] = mean ms per step spent in: neighbor
  * rebuilds, descriptor kernel, MLP kernel, force kernel, FP64
  * reductions (with the second half kick), the first half kick, drift,
- * displacement check and force-buffer clear, and the whole step. */
+ * displacement check and force-buffer clear (up to 2,048 atoms also the
+ * bins of a rebuild), and the whole step. */
 int tmd_md_profile(tmd_system *sys, int nsteps, double dt, double *ms);
 /* Sampled kernel timing inside tmd_md_run.  No counterpart in the reference
  * (benchmark instrumentation: kernel durations measured over a timed run).

@@ -140,8 +140,11 @@ struct NbrBuild {
 // is due, and at the end of the evaluation the reset of the control word
 // (StepTail / launch_reduce_struct).
 hipError_t nbr_check(const NbrBuild &nb, const double4 *pos, hipStream_t stream);
-hipError_t nbr_rebuild(const NbrBuild &nb, double4 *pos, uint32_t *nbr, int *nn, hipStream_t stream);
-// first half kick and drift, the displacement check, and f = 0
+// after_vv: launch_vv_first came before it on the same system
+hipError_t nbr_rebuild(const NbrBuild &nb, double4 *pos, uint32_t *nbr, int *nn, hipStream_t stream,
+                       bool after_vv = false);
+// first half kick and drift, the displacement check, and f = 0; for a small
+// system also the bins of a rebuild that is due
 hipError_t launch_vv_first(const NbrBuild &nb, int n, double4 *pos, double *v, double *f, const double *dtfm,
                            double dt, hipStream_t stream);
 

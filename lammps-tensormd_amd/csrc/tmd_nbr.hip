@@ -111,30 +111,32 @@ __global__ void k_nb_check(NbrBuild nb, const double4 *pos)
   report_move(i < n ? moved2(nb, i, pos[i]) : 0.0, nb.trig2, nb.ctl);
 }
 
-// First half of a velocity-Verlet step (src/fix_nve.cpp:64-98) with the
-// displacement check of the new positions; the forces, read here, are
-// cleared for the force kernel.
+// First half of a velocity-Verlet step of one atom (src/fix_nve.cpp:64-98),
+// its force cleared for the force kernel; returns its displacement^2 since the build.
+__device__ inline double vv_atom(const NbrBuild &nb, int i, double4 *pos, double *v, double *f, const double *dtfm,
+                                 double dt)
+{
+  double4 p = pos[i];
+  const double c = dtfm[(int) p.w];
+  const size_t q = 3 * (size_t) i;
+  const double vx = v[q] + c * f[q], vy = v[q + 1] + c * f[q + 1], vz = v[q + 2] + c * f[q + 2];
+  v[q] = vx;
+  v[q + 1] = vy;
+  v[q + 2] = vz;
+  f[q] = f[q + 1] = f[q + 2] = 0.0;
+  p.x += dt * vx;
+  p.y += dt * vy;
+  p.z += dt * vz;
+  pos[i] = p;
+  return moved2(nb, i, p);
+}
+
+// That half step with the displacement check of the new positions.
 __global__ void k_vv_first(NbrBuild nb, int n, double4 *pos, double *v, double *f, const double *dtfm, double dt)
 {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   clear_bins(nb, i, gridDim.x * blockDim.x);
-  double d2 = 0.0;
-  if (i < n) {
-    double4 p = pos[i];
-    const double c = dtfm[(int) p.w];
-    const size_t q = 3 * (size_t) i;
-    const double vx = v[q] + c * f[q], vy = v[q + 1] + c * f[q + 1], vz = v[q + 2] + c * f[q + 2];
-    v[q] = vx;
-    v[q + 1] = vy;
-    v[q + 2] = vz;
-    f[q] = f[q + 1] = f[q + 2] = 0.0;
-    p.x += dt * vx;
-    p.y += dt * vy;
-    p.z += dt * vz;
-    pos[i] = p;
-    d2 = moved2(nb, i, p);
-  }
-  report_move(d2, nb.trig2, nb.ctl);
+  report_move(i < n ? vv_atom(nb, i, pos, v, f, dtfm, dt) : 0.0, nb.trig2, nb.ctl);
 }
 
 // wrap atom i into its cell, remember its build position; returns its bin
@@ -221,11 +223,32 @@ __global__ void k_nb_sort(NbrBuild nb, const double4 *pos)
 
 // ---- bins of a small system: the same phases in one workgroup ----
 constexpr int kSmall = 4096;  // atoms and bins at most
+// Atoms up to which the workgroup also takes the first half of an MD step:
+// two atoms per thread cost less than a launch of their own.
+constexpr int kSmallStep = 2048;
 
-__global__ __launch_bounds__(1024) void k_nb_small(NbrBuild nb, double4 *pos, int nbins)
+bool small_build(const NbrBuild &nb) { return nb.n <= kSmall && nb.nbins <= kSmall; }
+bool small_step(const NbrBuild &nb) { return small_build(nb) && nb.n <= kSmallStep && !nb.dyn; }
+
+template <bool VV>
+__global__ __launch_bounds__(1024) void k_nb_small(NbrBuild nb, double4 *pos, int nbins, double *v, double *f,
+                                                   const double *dtfm, double dt)
 {
-  if (!rebuild_due(nb.ctl, nb.trig2)) return;
   __shared__ int count[kSmall], start[kSmall], atoms[kSmall], wsum[16];
+  if constexpr (VV) {
+    const bool flagged = rebuild_due(nb.ctl, nb.trig2);
+    double d2 = 0.0;
+#pragma unroll
+    for (int u = 0; u < kSmallStep / 1024; u++) {
+      const int i = u * 1024 + (int) threadIdx.x;
+      if (i < nb.n) d2 = fmax(d2, vv_atom(nb, i, pos, v, f, dtfm, dt));
+    }
+    const bool moved = __syncthreads_or(d2 > nb.trig2);
+    if (moved) report_move(d2, nb.trig2, nb.ctl);  // the list kernel reads it
+    if (!flagged && !moved) return;
+  } else if (!rebuild_due(nb.ctl, nb.trig2)) {
+    return;
+  }
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const int n = min(live_atoms(nb), kSmall);
   nbins = min(live_bins(nb, nbins), kSmall);
@@ -398,16 +421,21 @@ hipError_t nbr_check(const NbrBuild &nb, const double4 *pos, hipStream_t stream)
 hipError_t launch_vv_first(const NbrBuild &nb, int n, double4 *pos, double *v, double *f, const double *dtfm,
                            double dt, hipStream_t stream)
 {
-  k_vv_first<<<(n + 255) / 256, 256, 0, stream>>>(nb, n, pos, v, f, dtfm, dt);
+  if (n == nb.n && small_step(nb))
+    k_nb_small<true><<<1, 1024, 0, stream>>>(nb, pos, nb.nbins, v, f, dtfm, dt);
+  else
+    k_vv_first<<<(n + 255) / 256, 256, 0, stream>>>(nb, n, pos, v, f, dtfm, dt);
   return hipGetLastError();
 }
 
-hipError_t nbr_rebuild(const NbrBuild &nb, double4 *pos, uint32_t *nbr, int *nn, hipStream_t stream)
+hipError_t nbr_rebuild(const NbrBuild &nb, double4 *pos, uint32_t *nbr, int *nn, hipStream_t stream, bool after_vv)
 {
   if (nb.n <= 0) return hipSuccess;
   const int blocks = (nb.n + 255) / 256;
-  if (nb.n <= kSmall && nb.nbins <= kSmall) {
-    k_nb_small<<<1, 1024, 0, stream>>>(nb, pos, nb.nbins);
+  if (after_vv && small_step(nb)) {
+    // binned by launch_vv_first
+  } else if (small_build(nb)) {
+    k_nb_small<false><<<1, 1024, 0, stream>>>(nb, pos, nb.nbins, nullptr, nullptr, nullptr, 0.0);
   } else {
     k_nb_bin<<<blocks, 256, 0, stream>>>(nb, pos);
     k_nb_alloc<<<(nb.nbins + 255) / 256, 256, 0, stream>>>(nb, nb.nbins);

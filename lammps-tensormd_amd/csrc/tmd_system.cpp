@@ -180,7 +180,7 @@ int sys_forces(tmd_system *s, const Chain &c, bool step, PhaseEvents *pe = nullp
   hipStream_t st = s->ctx->stream;
   hipError_t e = step ? hipSuccess : nbr_check(s->nb, (const double4 *) s->w.pos.p, st);
   if (e == hipSuccess)
-    e = nbr_rebuild(s->nb, (double4 *) s->w.pos.p, (uint32_t *) s->w.nbr.p, (int *) s->w.nn.p, st);
+    e = nbr_rebuild(s->nb, (double4 *) s->w.pos.p, (uint32_t *) s->w.nbr.p, (int *) s->w.nn.p, st, step);
   if (e != hipSuccess) return hip_fail(s->ctx, e, "neighbor build");
   int rc = run_chain(s->ctx, s->w, c, st, pe);
   if (rc != TMD_OK || !pe) return rc;
@@ -782,7 +782,7 @@ int tmd_md_profile(tmd_system *s, int nsteps, double dt, double *ms)
                           (const double *) s->dtfm.p, dt, st);
     if (e == hipSuccess) e = hipEventRecord(E[1], st);
     if (e == hipSuccess)
-      e = nbr_rebuild(s->nb, (double4 *) s->w.pos.p, (uint32_t *) s->w.nbr.p, (int *) s->w.nn.p, st);
+      e = nbr_rebuild(s->nb, (double4 *) s->w.pos.p, (uint32_t *) s->w.nbr.p, (int *) s->w.nn.p, st, true);
     if (e == hipSuccess) e = hipEventRecord(E[2], st);
     if (e == hipSuccess) {
       rc = run_chain(s->ctx, s->w, step_chain(s, false), st, &pe);

@@ -41,9 +41,21 @@ __device__ inline void block_sum7(const double *eatom, const double *watom, int 
 
 // The control word of the neighbor list after an evaluation: a build counted
 // if one was due, flags cleared for the next step.
-__device__ inline void reset_ctl(unsigned long long *ctl, double trig2)
+struct Ctl {
+  unsigned long long w[4];
+};
+
+__device__ inline Ctl load_ctl(const unsigned long long *ctl)
 {
-  if (ctl[1] != 0ull || __longlong_as_double((long long) ctl[0]) > trig2) ctl[3] += 1ull;
+  Ctl c;
+  for (int q = 0; q < 4; q++) c.w[q] = ctl[q];
+  return c;
+}
+
+__device__ inline void reset_ctl(unsigned long long *ctl, Ctl &c, double trig2)
+{
+  if (c.w[1] != 0ull || __longlong_as_double((long long) c.w[0]) > trig2) ctl[3] = ++c.w[3];
+  c.w[0] = c.w[1] = 0ull;
   ctl[0] = 0ull;
   ctl[1] = 0ull;
 }
@@ -54,24 +66,41 @@ __global__ void k_reduce_struct(const double *eatom, const double *watom, const 
 {
   __shared__ double sh[7][256];
   const int st = blockIdx.x;
-  if (st == 0 && threadIdx.x == 0) reset_ctl(ctl, trig2);
+  if (st == 0 && threadIdx.x == 0) {
+    Ctl c = load_ctl(ctl);
+    reset_ctl(ctl, c, trig2);
+  }
   if (st >= nstruct || (dyn && st >= dyn->nstruct)) return;
   block_sum7(eatom, watom, off[st], off[st + 1], 0, 256, sh, out + (size_t) st * 7);
 }
 
+// What the end of a step needs of memory, requested before the sums.
+struct StepEnd {
+  Ctl ctl;
+  unsigned long long n;
+};
+
+__device__ inline StepEnd load_end(const StepTail &a)
+{
+  StepEnd e{};
+  if (a.ctl) e.ctl = load_ctl(a.ctl);
+  if (a.hist) e.n = a.counter[0];
+  return e;
+}
+
 // tot[0..7] = energy, virial, sum m v^2 (held by the workgroup) -> results
-__device__ inline void finish_step(const StepTail &a, const double *tot)
+__device__ inline void finish_step(const StepTail &a, StepEnd &end, const double *tot)
 {
   const int t = threadIdx.x;
   if (t < 7) a.out[t] = tot[t];
   if (t != 0) return;
   if (a.ctl) {
-    reset_ctl(a.ctl, a.trig2);
+    reset_ctl(a.ctl, end.ctl, a.trig2);
     if (a.ctl_host)
-      for (int q = 0; q < 4; q++) a.ctl_host[q] = a.ctl[q];
+      for (int q = 0; q < 4; q++) a.ctl_host[q] = end.ctl.w[q];
   }
   if (a.hist) {
-    const unsigned long long n = a.counter[0];
+    const unsigned long long n = end.n;
     if (n < (unsigned long long) a.hist_cap) {
       a.hist[2 * n] = tot[0];
       a.hist[2 * n + 1] = 0.5 * 1.0364269e-4 * tot[7];  // mvv2e, metal units
@@ -88,6 +117,8 @@ __global__ __launch_bounds__(1024) void k_step_sums(StepTail a)
 {
   __shared__ double sh[16][8];
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6, nw = blockDim.x >> 6;
+  StepEnd end{};
+  if (gridDim.x == 1 && t == 0) end = load_end(a);
   double s[8] = {0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll 2
   for (int i = blockIdx.x * blockDim.x + t; i < a.n; i += gridDim.x * blockDim.x) {
@@ -127,7 +158,7 @@ __global__ __launch_bounds__(1024) void k_step_sums(StepTail a)
   __syncthreads();
   if (t < 8) sh[0][t] = r;
   __syncthreads();
-  finish_step(a, sh[0]);
+  finish_step(a, end, sh[0]);
 }
 
 // one wave per quantity; fixed shuffle tree (deterministic)
@@ -135,12 +166,14 @@ __global__ __launch_bounds__(512) void k_step_final(StepTail a, int nparts)
 {
   __shared__ double tot[8];
   const int q = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  StepEnd end{};
+  if (threadIdx.x == 0) end = load_end(a);
   double s = 0.0;
   for (int p = lane; p < nparts; p += 64) s += a.out[8 + 8 * (size_t) p + q];
   s = wave_sum_d(s);
   if (lane == 0) tot[q] = s;
   __syncthreads();
-  finish_step(a, tot);
+  finish_step(a, end, tot);
 }
 
 __global__ void k_set_positions(int first, int n, const double *x, double4 *pos, unsigned long long *ctl)

@@ -1181,3 +1181,23 @@ def test_network_tiles(tmp_path, prec, k, layers, act, resnet, cells):
         say("largest error / spread: E", e0.max(), "dE/dG", e1.max(), "rms dE/dG error",
             float(np.sqrt(((dG - g) ** 2).mean())), "rms dE/dG", float(np.sqrt((g ** 2).mean())))
         assert e0.max() <= 8.0 and e1.max() <= 8.0, (len(x), e0.max(), e1.max())
+
+
+@pytest.mark.parametrize("cells", [(4, 4, 4), (8, 8, 8), (8, 8, 9), (8, 8, 16), (8, 8, 17)])
+def test_md_rebuilds_small(synth_models, cells):
+    """MD steps whose first half bins the atoms itself (2,048 atoms at most)
+    and those that leave it to kernels of their own: after several rebuilds
+    the forces equal those of a new system at the same positions."""
+    x, t, cell = W.crystal("bcc", 3.2, cells, nelt=4, sigma=0.05, seed=81)
+    mass = np.array([95.95, 92.906, 180.95, 183.84])[t - 1]
+    m = TensorMD(synth_models["c2"], ["Mo", "Nb", "Ta", "W"], "fp32", 0.001)
+    s = m.system(x, t, cell, skin=0.3)
+    s.set_velocities(W.maxwell_boltzmann(mass, 3000.0, seed=82))
+    s.md_run(40, 0.002)
+    r = s.get()
+    ref = m.system(r["x"], t, cell, skin=1.0).compute()
+    say("case:", len(x), "atoms,", s.nbuilds, "builds, max |dF|", abs(r["f"] - ref["f"]).max())
+    assert s.nbuilds >= 3
+    # both are FP32 evaluations of the same positions
+    assert abs(r["f"] - ref["f"]).max() <= 2 * F_TOL * max(1.0, abs(ref["f"]).max())
+    assert abs(r["energy"] - ref["energy"]) / len(x) <= 2e-6
