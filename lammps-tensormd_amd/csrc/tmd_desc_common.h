@@ -213,13 +213,19 @@ __device__ inline unsigned lane_rank(unsigned long long m)
 
 // Phase 1: compact the kept entries (slot-sorted).  start[b] .. start[b+1].
 __device__ inline int kept_slot(const ModelGeo &g, const Box &cell, const double4 &xi, int ei,
-                                uint32_t e, const double4 &xj)
+                                uint32_t e, const double4 &xj, double d[3])
 {
-  double d[3];
   displacement(xi, xj, e >> kNbrJBits, cell, d);
   double r2 = dist2(d);
   return (r2 < g.rc2 && r2 > 1e-10) ? (int) ((g.slots[ei] >> (4 * (int) xj.w)) & 15u)
                                     : -1;  // kernel.cu:1163
+}
+
+__device__ inline int kept_slot(const ModelGeo &g, const Box &cell, const double4 &xi, int ei,
+                                uint32_t e, const double4 &xj)
+{
+  double d[3];
+  return kept_slot(g, cell, xi, ei, e, xj, d);
 }
 
 // Lists of at most 64 NCH entries: every entry's slot stays in registers.
@@ -330,11 +336,9 @@ struct NbrGeo {
   int n, j;
 };
 
-__device__ inline void nbr_geometry(const ModelGeo &g, const Box &cell, const double4 &xi,
-                                    const double4 *pos, uint32_t e, NbrGeo &o)
+// from the displacement o.d
+__device__ inline void nbr_geometry(const ModelGeo &g, NbrGeo &o)
 {
-  o.j = (int) (e & kNbrJMask);
-  displacement(xi, pos[o.j], e >> kNbrJBits, cell, o.d);
   double r2 = o.d[0] * o.d[0] + o.d[1] * o.d[1] + o.d[2] * o.d[2];
   double rinv = rsqrt_fp64(r2);
   o.r = r2 * rinv;
@@ -345,6 +349,14 @@ __device__ inline void nbr_geometry(const ModelGeo &g, const Box &cell, const do
   const double qd = o.r * g.rdx - (double) o.n;
   o.q = (float) qd;
   o.pq = (float) (1.0 - qd);
+}
+
+__device__ inline void nbr_geometry(const ModelGeo &g, const Box &cell, const double4 &xi,
+                                    const double4 *pos, uint32_t e, NbrGeo &o)
+{
+  o.j = (int) (e & kNbrJMask);
+  displacement(xi, pos[o.j], e >> kNbrJBits, cell, o.d);
+  nbr_geometry(g, o);
 }
 
 // the end cells of the table are zero (ration.hpp:29)

@@ -198,6 +198,19 @@ hipError_t launch_force_hm(const ModelGeo &g, const Geom &geo, const double4 *po
                            double *eatom, double *watom, double *vatom, hipStream_t stream,
                            int row_begin = 0);
 
+// Several waves per atom, for small systems (tmd_desc_wide.hip): the waves that
+// the two kernels take for so many rows (1: the kernels of one wave), and
+// the launches, which launch_descriptor/launch_force call.
+int desc_waves(const ModelGeo &g, int rows, int cap);
+int force_waves(const ModelGeo &g, int rows);
+hipError_t launch_descriptor_wide(const ModelGeo &g, const Geom &geo, const double4 *pos, const uint32_t *nbr,
+                                  const int *nn, int cap, const int *row2atom, int nrows, const float4 *tab, float *G,
+                                  uint32_t *kl, hipStream_t stream, int row_begin);
+hipError_t launch_force_wide(const ModelGeo &g, const Geom &geo, const double4 *pos, int cap, const int *row2atom,
+                             int nrows, const float4 *tab, const uint32_t *kl, const float *dEdG, const double *E,
+                             double scale, double *f, double *eatom, double *watom, double *vatom, hipStream_t stream,
+                             int row_begin);
+
 // ---- MLP ----------------------------------------------------------------------
 // mode: 0 fp32, 1 bf16, 2 fp8 (e4m3 operands: weights with per-output-channel
 // scales, activations and gradients with per-row scales; FP32 accumulation),

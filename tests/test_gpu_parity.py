@@ -1201,3 +1201,53 @@ def test_md_rebuilds_small(synth_models, cells):
     # both are FP32 evaluations of the same positions
     assert abs(r["f"] - ref["f"]).max() <= 2 * F_TOL * max(1.0, abs(ref["f"]).max())
     assert abs(r["energy"] - ref["energy"]) / len(x) <= 2e-6
+
+
+@pytest.mark.parametrize("k,nelt", [(16, 1), (24, 4), (32, 2)])
+def test_waves_per_atom(tmp_path, k, nelt):
+    """The moment kernels with four, two and one wave per atom (by the number
+    of rows): clusters of the tile edges' sizes as the centers of one call,
+    repeated until the next kernels are taken.  Descriptor rows and forces of
+    every copy against the FP64 oracle, bars as in test_force_tile_edges."""
+    path = W.write_model(str(tmp_path / "m.npz"), symbols=["Mo", "Nb", "Ta", "W"][:nelt],
+                         masses=[95.95, 92.906, 180.95, 183.84][:nelt], rmax=6.0, num_filters=k,
+                         layer_sizes=[64, 32, 1], actfn="tanh", seed=90 + k + nelt, radial_scale=0.1)
+    om = oracle.OracleModel(path, 0.001)
+    m = TensorMD(path, ["Mo", "Nb", "Ta", "W"][:nelt], "fp32", 0.001)
+    rng = np.random.default_rng(9)
+    cl = []
+    for n in [1, 4, 5, 16, 17, 32, 33, 48, 49, 64, 65, 72, 73, 84, 85, 96, 97, 112]:
+        for spread in range(2):
+            counts = np.bincount(rng.integers(0, nelt, n), minlength=nelt) if spread else [n] + [0] * (nelt - 1)
+            cl.append(_cluster(rng, om.rc, list(counts)))
+    nl = [len(t) - 1 for _, t in cl]
+    first = np.concatenate([[0], np.cumsum([len(t) for _, t in cl])[:-1]])
+    x1 = np.concatenate([x for x, _ in cl])
+    t1 = np.concatenate([t for _, t in cl])
+
+    def call(copies):  # the centers' lists of `copies` repetitions
+        size = len(t1)
+        il, num, flat = [], np.zeros(copies * size, dtype=np.int32), []
+        for c in range(copies):
+            for f0, n in zip(first, nl):
+                il.append(c * size + f0)
+                num[c * size + f0] = n
+                flat.append(c * size + f0 + np.arange(1, n + 1))
+        return np.tile(x1, (copies, 1)), np.tile(t1, copies), il, num, np.concatenate(flat)
+
+    x, t, il, num, flat = call(1)
+    ref = om.compute_list(len(x), x, t - 1, il, num, flat, want_desc=True)
+    om.set_emulation(om.EMUL_DESC | om.EMUL_MLP | om.EMUL_FORCE)
+    emu = om.compute_list(len(x), x, t - 1, il, num, flat)
+    om.set_emulation(0)
+    bar = max(F_TOL, 2.0 * float(abs(emu["f"] - ref["f"]).max()))
+    g0 = ref["G"]
+    for copies in (1, 18, 30, 60):
+        x, t, il, num, flat = call(copies)
+        say("case:", len(il), "rows,", k, nelt)
+        got = m.compute_list(len(x), x, t, il, num, flat)
+        G = m.descriptors_list(len(x), x, t, il, num, flat)[np.array(il)].reshape(copies, len(nl), -1)
+        assert abs(got["f"].reshape(copies, -1, 3) - ref["f"]).max() <= bar
+        assert abs(got["vatom"].reshape(copies, -1, 6) - ref["vatom"]).max() <= 6.0 * bar
+        assert abs(got["energy"] / copies - ref["energy"]) <= 1e-6 * len(nl)
+        assert abs(G - g0).max() <= 4e-6 * max(1.0, abs(g0).max())
