@@ -231,8 +231,9 @@ __device__ inline float g_components(const f32x4v &p, int tsym)
   return swap16_add(swap32_add(t0, t2), swap32_add(t1, t3));
 }
 
-// descriptor LDS: kept list, staged rows, H
-constexpr int kDescWin = 64;
+// descriptor LDS: kept list and staged rows, or the rows of all kept
+// neighbors; H
+constexpr int kDescWin = 64, kDescAll = 88;
 template <int K>
 __host__ __device__ inline size_t desc_lds(int cap, size_t *offs)
 {
@@ -244,6 +245,7 @@ __host__ __device__ inline size_t desc_lds(int cap, size_t *offs)
   };
   offs[0] = take((size_t) cap * 4);
   offs[1] = take((size_t) kDescWin * kRow * 4);
+  o = o > kDescAll * kRow * 4 ? o : kDescAll * kRow * 4;
   offs[2] = take((size_t) Tiling<K>::HBUF * 4);
   return o;
 }
@@ -252,16 +254,15 @@ __host__ __device__ inline size_t desc_lds(int cap, size_t *offs)
 // sorted) += the tile of `live` neighbors from entry `first` on, staged in
 // rt.  Tiles run across slot boundaries: each slot takes its own neighbors
 // of a tile by zeroing the harmonics of the others.
-template <int K, int NS>
-__device__ inline void descriptor_tile(const float4 *tab, const float *rt, int first, int live, int fb,
+template <int K, int NS, typename Next>
+__device__ inline void descriptor_tile(TabTile<K> &tt, const Next &next, const float *rt, int first, int live, int fb,
                                        const int *start, int nsl, float *hb, f32x4v (&acc)[NS][Tiling<K>::KT])
 {
   using T = Tiling<K>;
   const int lane = threadIdx.x & 63;
-  TabTile<K> tt;
-  load_tile<K>(tab, rt, live, fb, tt);
   put_H<K>(tt, hb);
   wave_sync();
+  next();
   float a[4], bo[4][T::CT];
 #pragma unroll
   for (int s = 0; s < 4; s++) {
@@ -309,7 +310,7 @@ __device__ inline void store_g(const f32x4v &p, int b, int t, int tsym, float *G
 template <int K, int NS>
 __device__ inline void descriptor_pass(const ModelGeo &g, const Box &cell, const double4 &xi, const double4 *pos,
                                        const float4 *tab, const uint32_t *kept, const int *start, int nsl,
-                                       float *rows, float *hb, float *Grow, int b0, bool gbf16)
+                                       float *rows, float *hb, float *Grow, int b0, bool gbf16, bool staged = false)
 {
   using T = Tiling<K>;
   const int lane = threadIdx.x & 63;
@@ -319,15 +320,22 @@ __device__ inline void descriptor_pass(const ModelGeo &g, const Box &cell, const
 #pragma unroll
     for (int t = 0; t < T::KT; t++) acc[b][t] = f32x4v{0, 0, 0, 0};
   const int end = start[nsl];
-  for (int w0 = start[0]; w0 < end; w0 += kDescWin) {
-    const int nw = min(kDescWin, end - w0);
-    stage(g, cell, xi, pos, kept + w0, nw, rows);
+  const int win = staged ? end : kDescWin;
+  for (int w0 = start[0]; w0 < end; w0 += win) {
+    const int nw = min(win, end - w0);
+    if (!staged) stage(g, cell, xi, pos, kept + w0, nw, rows);
+    TabTile<K> tt;
+    load_tile<K>(tab, rows, min(16, nw), 0, tt);
     for (int r0 = 0; r0 < nw; r0 += 16) {
       const int live = min(16, nw - r0);
       const float *rt = rows + r0 * kRow;
 #pragma unroll
       for (int fb = 0; fb < T::NB; fb++) {
-        descriptor_tile<K, NS>(tab, rt, w0 + r0, live, fb, start, nsl, hb, acc);
+        auto next = [&]() {
+          const int r = fb + 1 < T::NB ? r0 : r0 + 16;
+          if (r < nw) load_tile<K>(tab, rows + r * kRow, min(16, nw - r), (fb + 1) % T::NB, tt);
+        };
+        descriptor_tile<K, NS>(tt, next, rt, w0 + r0, live, fb, start, nsl, hb, acc);
         wave_sync();
       }
     }
@@ -356,14 +364,69 @@ __device__ inline void descriptor_row(const ModelGeo &g, const Geom &geo, int ro
   uint32_t *kept = reinterpret_cast<uint32_t *>(smem + offs[0]);
   float *rows = reinterpret_cast<float *>(smem + offs[1]);
   float *hb = reinterpret_cast<float *>(smem + offs[2]);
+  float *all = reinterpret_cast<float *>(smem);  // kDescAll rows, over the kept list and the window
   int start[kMaxElts + 1];
   const double4 xi = pos[i];
   const Box cell = load_box(geo, i);
+  uint32_t *kr = kl + (size_t) row * kept_cache_words(cap);
+  if constexpr (!MP) {
+    // a list of at most two entries per lane: their geometry stays in
+    // registers, and the kept ones are staged from there instead of being
+    // gathered and displaced a second time (128,000 atoms, with the table rows
+    // of the next tile requested ahead: 334 -> 302 us)
+    const int nraw = nn[i];
+    if (nraw <= 128) {
+      const uint32_t *list = nbr + (size_t) i * cap;
+      const int last = max(nraw - 1, 0);
+      uint32_t ent[2];
+      double4 xj[2];
+      NbrGeo ng[2];
+      int slot[2], rank[2] = {0, 0};
+#pragma unroll
+      for (int c = 0; c < 2; c++) {
+        const uint32_t e = list[min(64 * c + lane, last)];
+        ent[c] = 64 * c + lane < nraw ? e : 0u;
+      }
+#pragma unroll
+      for (int c = 0; c < 2; c++) xj[c] = pos[ent[c] & kNbrJMask];
+#pragma unroll
+      for (int c = 0; c < 2; c++) {
+        const int sl = kept_slot(g, cell, xi, (int) xi.w, ent[c], xj[c], ng[c].d);
+        slot[c] = 64 * c + lane < nraw ? sl : -1;
+      }
+      int nk = 0;
+      for (int b = 0; b < g.nelt; b++) {
+        start[b] = nk;
+#pragma unroll
+        for (int c = 0; c < 2; c++) {
+          const unsigned long long m = __ballot(slot[c] == b);
+          if (slot[c] == b) rank[c] = nk + (int) lane_rank(m);
+          nk += __popcll(m);
+        }
+      }
+      start[g.nelt] = nk;
+      if (nk <= kDescAll) {
+#pragma unroll
+        for (int c = 0; c < 2; c++)
+          if (slot[c] >= 0) {
+            kr[kKeptHdr + rank[c]] = ent[c];
+            nbr_geometry(g, ng[c]);
+            put_row(ng[c], all + rank[c] * kRow);
+          }
+        if (lane == 0) {
+          kr[0] = (uint32_t) nk;
+          for (int b = 0; b <= g.nelt; b++) kr[1 + b] = (uint32_t) start[b];
+        }
+        wave_sync();
+        descriptor_pass<K, NS>(g, cell, xi, pos, tab, nullptr, start, g.nelt, all, hb, Grow, 0, geo.g_bf16, true);
+        return;
+      }
+    }
+  }
   // phase 1: compaction
   const int nk = compact(g, cell, xi, (int) xi.w, nbr + (size_t) i * cap, nn[i], pos, kept, start);
   wave_sync();
   // the row's kept list with its slot starts, for the force kernel
-  uint32_t *kr = kl + (size_t) row * kept_cache_words(cap);
   if (lane == 0) {
     kr[0] = (uint32_t) nk;
     for (int b = 0; b <= g.nelt; b++) kr[1 + b] = (uint32_t) start[b];

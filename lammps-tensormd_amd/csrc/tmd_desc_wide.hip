@@ -96,7 +96,9 @@ __global__ __launch_bounds__(64 * W) void k_descriptor_wide(ModelGeo g, Geom geo
 #pragma unroll
         for (int t = 0; t < T::KT; t++) acc[b][t] = f32x4v{0, 0, 0, 0};
       for (int r0 = 16 * wave; r0 < nk; r0 += 16 * W) {
-        descriptor_tile<K, NS>(tab, sh.rows + r0 * kRow, r0, min(16, nk - r0), 0, start, g.nelt, sh.hb[wave], acc);
+        TabTile<K> tt;
+        load_tile<K>(tab, sh.rows + r0 * kRow, min(16, nk - r0), 0, tt);
+        descriptor_tile<K, NS>(tt, [] {}, sh.rows + r0 * kRow, r0, min(16, nk - r0), 0, start, g.nelt, sh.hb[wave], acc);
         wave_sync();
       }
 #pragma unroll
