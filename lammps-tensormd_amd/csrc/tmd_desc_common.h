@@ -48,31 +48,6 @@ __device__ inline double dist2(const double d[3])
   return d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
 }
 
-__device__ inline void monomials20(float x, float y, float z, float *M)
-{
-  float xx = x * x, xy = x * y, xz = x * z, yy = y * y, yz = y * z, zz = z * z;
-  M[0] = 1.0f;
-  M[1] = x;
-  M[2] = y;
-  M[3] = z;
-  M[4] = xx;
-  M[5] = xy;
-  M[6] = xz;
-  M[7] = yy;
-  M[8] = yz;
-  M[9] = zz;
-  M[10] = x * xx;
-  M[11] = x * xy;
-  M[12] = x * xz;
-  M[13] = x * yy;
-  M[14] = x * yz;
-  M[15] = x * zz;
-  M[16] = y * yy;
-  M[17] = y * yz;
-  M[18] = y * zz;
-  M[19] = z * zz;
-}
-
 // Kerley rational interpolation of one filter (gpu/cuda/ration.cu:59-68) in
 // units of the grid step: table entry t = (y, s dx, c1 dx^2, c2 dx^2),
 // q = r / dx - n, p = 1 - q, qp = q - p:
@@ -110,12 +85,6 @@ __device__ inline void kerley(float4 t, float q, float p, float qp, float &h, fl
 constexpr int kDppXor1 = 0xB1, kDppXor2 = 0x4E, kDppRor4 = 0x124, kDppRor8 = 0x128;
 
 template <int CTRL>
-__device__ inline float dpp_f(float v)
-{
-  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xF, 0xF, false));
-}
-
-template <int CTRL>
 __device__ inline double dpp_d(double v)
 {
   long long b = __double_as_longlong(v);
@@ -131,21 +100,6 @@ __device__ inline double wave_sum_d(double v)
   v += dpp_d<kDppXor1>(v);
   v += dpp_d<kDppXor2>(v);
   v += dpp_d<kDppRor4>(v);
-  v += dpp_d<kDppRor8>(v);
-  v += __shfl_xor(v, 16);
-  v += __shfl_xor(v, 32);
-  return v;
-}
-
-// The same sum when only lanes that are multiples of LP (1, 2, 4 or 8) hold
-// non-zero values; the total is exact in lane 0 (the first steps, which
-// would only add zeros there, are skipped).
-template <int LP>
-__device__ inline double wave_sum_d_lp(double v)
-{
-  if constexpr (LP < 2) v += dpp_d<kDppXor1>(v);
-  if constexpr (LP < 4) v += dpp_d<kDppXor2>(v);
-  if constexpr (LP < 8) v += dpp_d<kDppRor4>(v);
   v += dpp_d<kDppRor8>(v);
   v += __shfl_xor(v, 16);
   v += __shfl_xor(v, 32);
@@ -361,11 +315,6 @@ __device__ inline void nbr_geometry(const ModelGeo &g, const Box &cell, const do
 
 // the end cells of the table are zero (ration.hpp:29)
 __device__ inline bool table_cell_live(const ModelGeo &g, int n) { return n > 0 && n < g.tab_n - 2; }
-
-// Lanes per neighbor for a chunk when `rem` kept neighbors remain: 2 (a
-// chunk of 32 neighbors), 4 (16) or 8 (8).  A short last chunk spreads each
-// neighbor's filters over more lanes instead of leaving lanes idle.
-__device__ inline int lanes_per_nbr(int rem) { return rem > 16 ? 2 : (rem > 8 ? 4 : 8); }
 
 }  // namespace
 
