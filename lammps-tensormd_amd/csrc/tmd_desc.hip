@@ -34,8 +34,8 @@
 // What bounds the kernels (128,000 atoms, 4 elements, 24 filters, 63
 // neighbors): vector and matrix instructions, which do not overlap on a SIMD
 // here, fill about 95 % of the force kernel's time (0.38 + 0.19 of 0.61 ms;
-// 0.42 ms with neither matrix instructions nor atomics) and 86 % of the
-// descriptor's 0.32 ms.  With the monomials on the vector ALU they took 0.95
+// 0.42 ms with neither matrix instructions nor atomics) and 90 % of the
+// descriptor's 0.30 ms.  With the monomials on the vector ALU they took 0.95
 // and 0.42 ms.
 //
 // Nothing per neighbor is stored in HBM: the reference materialises R, M,
@@ -265,7 +265,7 @@ hipError_t launch_descriptor(const ModelGeo &g, const Geom &geo, const double4 *
   if (geo.order && row_begin != 0) return hipErrorInvalidValue;  // an order covers whole launches
   if (g.mm > 3)
     return launch_descriptor_hm(g, geo, pos, nbr, nn, cap, row2atom, nrows, tab, G, kl, stream, row_begin);
-  if (desc_waves(g, nrows - row_begin, cap) > 1)
+  if (!geo.dyn && desc_waves(g, nrows - row_begin, cap) > 1)
     return launch_descriptor_wide(g, geo, pos, nbr, nn, cap, row2atom, nrows, tab, G, kl, stream, row_begin);
 #define TMD_K_CASE(K)                                                                                    \
   case K:                                                                                                \
@@ -291,7 +291,7 @@ hipError_t launch_force(const ModelGeo &g, const Geom &geo, const double4 *pos, 
   if (g.mm > 3)
     return launch_force_hm(g, geo, pos, cap, row2atom, nrows, tab, kl, dEdG, E, scale, f, eatom, watom, vatom,
                            stream, row_begin);
-  if (force_waves(g, nrows - row_begin) > 1)
+  if (!geo.dyn && force_waves(g, nrows - row_begin) > 1)
     return launch_force_wide(g, geo, pos, cap, row2atom, nrows, tab, kl, dEdG, E, scale, f, eatom, watom, vatom,
                              stream, row_begin);
 #define TMD_K_CASE(K)                                                                                       \

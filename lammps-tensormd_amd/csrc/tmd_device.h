@@ -200,7 +200,9 @@ hipError_t launch_force_hm(const ModelGeo &g, const Geom &geo, const double4 *po
 
 // Several waves per atom, for small systems (tmd_desc_wide.hip): the waves that
 // the two kernels take for so many rows (1: the kernels of one wave), and
-// the launches, which launch_descriptor/launch_force call.
+// the launches, which launch_descriptor/launch_force call.  Not for batches
+// (Geom::dyn): their sums' order, and so a structure's last bits, must not
+// depend on the batch's capacity.
 int desc_waves(const ModelGeo &g, int rows, int cap);
 int force_waves(const ModelGeo &g, int rows);
 hipError_t launch_descriptor_wide(const ModelGeo &g, const Geom &geo, const double4 *pos, const uint32_t *nbr,
@@ -216,7 +218,10 @@ hipError_t launch_force_wide(const ModelGeo &g, const Geom &geo, const double4 *
 // scales, activations and gradients with per-row scales; FP32 accumulation),
 // 3 split bf16 (hi + lo operands, three BF16 products each).
 // E[row] (FP64 output sum) and dEdG[row][width] (fp32).  rtile: rows per
-// workgroup (16, 32 or 64, with the fast FP32 kernel also 4 or 8; 0 = default).
+// workgroup (16, 32 or 64; 0 = default).  The fast FP32 kernel takes 4 or 8 by
+// default for few rows, which sums in another order than the larger tiles
+// (those agree bit for bit): not with dyn, so that a structure's result does
+// not depend on its batch's capacity.
 // With dyn, rl gives the capacity (grid) and dyn->rl the live layout.
 // Rows [row_begin, row_end) only (row_end < 0: to rl.nrows); both bounds
 // are multiples of 64 (element blocks start on such rows).

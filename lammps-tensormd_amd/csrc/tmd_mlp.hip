@@ -8,13 +8,14 @@
 // and each element group starts at a multiple of 64, so R | 64 keeps a tile
 // inside one element).  Every hidden activation H_l and derivative
 // D_l = act'(z_l) of the tile stays in LDS; the waves split each layer's
-// output columns 16 at a time, reading A from LDS (layer 0: the FP32
-// descriptor rows from HBM) and streaming the element's weights from L2
-// straight into MFMA B operands.  The backward pass reuses the D_l slots for
+// output columns 16 at a time, reading activations from LDS (layer 0: the
+// staged descriptor rows) and streaming the element's weights from L2
+// straight into MFMA operands.  The backward pass reuses the D_l slots for
 // G_l = dE/dH_l * D_l and writes dE/dG (FP32) to HBM.  HBM traffic per atom
 // is the descriptor read plus the gradient write.
 //
-// FP32 mode: v_mfma_f32_16x16x4_f32; BF16 mode: v_mfma_f32_16x16x32_bf16
+// FP32 mode: v_mfma_f32_16x16x4_f32 (4x4x1 in tiles of fewer than 16 rows);
+// BF16 mode: v_mfma_f32_16x16x32_bf16
 // (operands rounded to BF16, FP32 accumulation; H/D kept as BF16 in LDS).
 // Split-BF16 mode (fast kernel only): every operand x is carried as
 // hi = bf16(x) and lo = bf16(x - hi), and each product as the three BF16
@@ -1464,10 +1465,10 @@ namespace {
 //           16,000                        40.0     29.8     34.2
 //           35,152                        73.2     66.5     65.1
 //          128,000                         245      191      150
-int tile_rows(const MlpParams &mp, int mode, int nrows)
+int tile_rows(const MlpParams &mp, int mode, int nrows, bool batch)
 {
   constexpr int kCUs = 256;
-  if (mode == 0 && nrows <= 8 * kCUs) {
+  if (mode == 0 && nrows <= 8 * kCUs && !batch) {
     long w = 0;
     for (int l = 0; l < mp.nl - 1; l++) w += (long) mp.sizes[l] * mp.sizes[l + 1];
     if (w >= 64 * 1024) return nrows <= 4 * kCUs ? 4 : 8;
@@ -1486,10 +1487,9 @@ hipError_t launch_mlp(int mode, const RowLayout &rl, const MlpParams &mp, const 
   if (row_begin < 0 || row_begin > row_end) return hipErrorInvalidValue;
   if (row_end == row_begin) return hipSuccess;
   const size_t limit = 160 * 1024;
-  // rtile (16/32/64, FP32 fast kernel also 4/8) overrides the rule
-  const bool fast = mlp_fast_ok(mp, mode);
-  int Rs[3] = {fast ? tile_rows(mp, mode, row_end - row_begin) : 32, 16, 16};
-  if (rtile == 16 || rtile == 32 || rtile == 64 || (mode == 0 && fast && (rtile == 4 || rtile == 8))) Rs[0] = rtile;
+  // rtile (16/32/64) overrides the rule
+  int Rs[3] = {mlp_fast_ok(mp, mode) ? tile_rows(mp, mode, row_end - row_begin, dyn != nullptr) : 32, 16, 16};
+  if (rtile == 16 || rtile == 32 || rtile == 64) Rs[0] = rtile;
   for (int q = 0; q < 3; q++) {
     int R = Rs[q];
     MlpParams m;

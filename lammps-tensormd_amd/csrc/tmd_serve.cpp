@@ -318,8 +318,7 @@ int tune_bucket(Server *S, Slot &sl, Bucket &b)
   for (int e = 0; e <= kMaxElts; e++) rl.row_off[e] = std::min(e, nelt) * per;
   rl.row_off[nelt] = b.caps.rows;
   for (int e = nelt + 1; e <= kMaxElts; e++) rl.row_off[e] = b.caps.rows;
-  const int cand[5] = {16, 32, 64, 4, 8};
-  const int ncand = mode == 0 && mlp_fast_ok(ctx->mlp, mode) ? 5 : 3;
+  const int cand[3] = {16, 32, 64};
   float best = 1e30f;
   int pick = 0;
   hipEvent_t e0, e1;
@@ -328,7 +327,7 @@ int tune_bucket(Server *S, Slot &sl, Bucket &b)
     hipEventDestroy(e0);
     return serve_fail(ctx, TMD_ERR_DEVICE, "serve: event");
   }
-  for (int q = 0; q < ncand; q++) {
+  for (int q = 0; q < 3; q++) {
     MlpParams m;
     if (mlp_lds_bytes(ctx->mlp, mode, cand[q], &m) > 160 * 1024) continue;
     hipError_t e = launch_mlp(mode, rl, ctx->mlp, (const float *) sl.w.G.p, (double *) sl.w.E.p,
