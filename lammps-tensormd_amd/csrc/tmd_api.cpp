@@ -491,9 +491,7 @@ int run_chain(tmd_ctx *ctx, Workspace &w, const Chain &c, hipStream_t s, PhaseEv
   if (pe && (e = hipEventRecord(pe->ev[4], s)) != hipSuccess) return hip_fail(ctx, e, "timing event");
   unsigned long long *ctl = c.nb ? c.nb->ctl : nullptr;
   const double trig2 = c.nb ? c.nb->trig2 : 0.0;
-  if (c.struct_off) {
-    e = launch_reduce_struct(eatom, watom, c.struct_off, c.nstruct, c.struct_out, ctl, trig2, s, c.dyn);
-  } else {
+  if (!c.no_sums) {
     StepTail t{};
     t.eatom = eatom;
     t.watom = watom;

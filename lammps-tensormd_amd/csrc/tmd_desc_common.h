@@ -316,6 +316,27 @@ __device__ inline void nbr_geometry(const ModelGeo &g, const Box &cell, const do
 // the end cells of the table are zero (ration.hpp:29)
 __device__ inline bool table_cell_live(const ModelGeo &g, int n) { return n > 0 && n < g.tab_n - 2; }
 
+// The control word of the neighbor list after an evaluation: a build counted
+// if one was due, flags cleared for the next step.
+struct Ctl {
+  unsigned long long w[4];
+};
+
+__device__ inline Ctl load_ctl(const unsigned long long *ctl)
+{
+  Ctl c;
+  for (int q = 0; q < 4; q++) c.w[q] = ctl[q];
+  return c;
+}
+
+__device__ inline void reset_ctl(unsigned long long *ctl, Ctl &c, double trig2)
+{
+  if (c.w[1] != 0ull || __longlong_as_double((long long) c.w[0]) > trig2) ctl[3] = ++c.w[3];
+  c.w[0] = c.w[1] = 0ull;
+  ctl[0] = 0ull;
+  ctl[1] = 0ull;
+}
+
 }  // namespace
 
 }  // namespace tmd

@@ -132,13 +132,13 @@ struct NbrBuild {
   int *atom_bc;       // [n][3] bin coordinates
   double4 *sorted;    // [n] positions in bin order, w = atom index
   double *x_build;    // [n][4]
-  unsigned long long *ctl;  // [0] max d^2 bits, [1] force flag, [2] overflow, [3] build count
+  unsigned long long *ctl;  // [0] max d^2 bits, [1] force flag, [2] overflow, [3] build count, [5] batch error
 };
 
 // One neighbor-list update: a check (nbr_check, or launch_vv_first, which
 // moves the atoms first), the rebuild kernels, which return at once when none
 // is due, and at the end of the evaluation the reset of the control word
-// (StepTail / launch_reduce_struct).
+// (StepTail / launch_batch_finish).
 hipError_t nbr_check(const NbrBuild &nb, const double4 *pos, hipStream_t stream);
 // after_vv: launch_vv_first came before it on the same system
 hipError_t nbr_rebuild(const NbrBuild &nb, double4 *pos, uint32_t *nbr, int *nn, hipStream_t stream,
@@ -283,9 +283,9 @@ struct BatchArrays {
   int *atom_struct;   // [atoms]
   int *row2atom;      // [rows]
   double4 *pos;       // [atoms]
-  const double *struct_out;  // [structs][7]
   double *f;                 // [atoms][3]
   const double *eatom;       // [atoms]
+  const double *watom;       // [atoms][6]
   unsigned long long *ctl;   // neighbor control word
   int *bin_count, *bin_total;
 };
@@ -305,17 +305,18 @@ __host__ __device__ inline void batch_stage_offsets(int ns, int n, int nrows, si
   off[6] = off[5];
 }
 // Dense host output of a batch: 8 header doubles (list overflow count,
-// atoms, structures, error flag) | struct_out[ns][7] | f[n][3] | eatom[n].
+// atoms, structures, error flag) | energy and virial[ns][7] | f[n][3] |
+// eatom[n].
 inline size_t batch_out_bytes(int ns, int n) { return 8 * (8 + 7 * (size_t) ns + 4 * (size_t) n); }
 // Copy a staged batch (host memory, read by the kernels) into the slot's
 // device arrays, clamping every count and index to the capacities; forces and
 // bin counts of the batch are cleared.
 hipError_t launch_batch_unpack(const void *stage, const BatchCaps &caps, const BatchArrays &a,
                                hipStream_t stream);
-// Write a finished batch's results to host memory `out` and clear the
-// list-overflow word.
-hipError_t launch_batch_pack(void *out, const BatchCaps &caps, const BatchArrays &a,
-                             hipStream_t stream);
+// Sum a finished batch's structures (fixed order), write its results to host
+// memory `out` and reset the control word.
+hipError_t launch_batch_finish(void *out, const BatchCaps &caps, const BatchArrays &a,
+                               hipStream_t stream);
 
 // ---- reductions / integration ---------------------------------------------------
 hipError_t launch_zero(void *p, size_t bytes, hipStream_t stream);
@@ -361,12 +362,6 @@ hipError_t launch_copy_small(const double *src, double *dst, int n, hipStream_t 
 // pos, v and f to (save) or from snap [n](pos | v | f); counter = 0
 hipError_t launch_snapshot(int n, bool save, double4 *pos, double *v, double *f, void *snap,
                            unsigned long long *counter, hipStream_t stream);
-// per structure s: out[7 s + 0] = sum eatom, out[7 s + 1..6] = sum watom over
-// atoms [off[s], off[s+1]); resets ctl
-// (with dyn: nstruct is the capacity, dyn->nstruct the live count)
-hipError_t launch_reduce_struct(const double *eatom, const double *watom, const int *off,
-                                int nstruct, double *out, unsigned long long *ctl, double trig2,
-                                hipStream_t stream, const BatchDims *dyn = nullptr);
 // *acc += sum of the kept-neighbor counts of the real rows (row2atom >= 0)
 // in the kept-list cache kl (words per row)
 hipError_t launch_sum_kept(const uint32_t *kl, size_t words, const int *row2atom, int nrows,

@@ -151,9 +151,7 @@ struct Chain {
   size_t vbytes = 0;
   int natoms = 0;            // eatom/watom entries (in w.ew)
   bool zero_ew = false;      // some atoms own no row: clear eatom/watom first
-  const int *struct_off = nullptr;  // per-structure sums into struct_out[7 s ..]
-  int nstruct = 0;
-  double *struct_out = nullptr;     // (null struct_off: one sum into w.red[0..6])
+  bool no_sums = false;      // leaves the sums and the control word to the caller
   // the list whose control word the evaluation resets (null in list mode)
   const NbrBuild *nb = nullptr;
   // the second half of a velocity-Verlet step rides on the sums: velocities,

@@ -81,7 +81,7 @@ struct Slot {
   hipStream_t stream = nullptr;
   hipEvent_t ev_start = nullptr, ev_done = nullptr;
   Workspace w;  // pos, nbr, nn, f, ew, G, dEdG, E, row2atom, cells
-  DeviceBuffer dyn, soff, astruct, sout, bins, atominfo, xbuild, sorted, ctl;
+  DeviceBuffer dyn, soff, astruct, bins, atominfo, xbuild, sorted, ctl;
   unsigned char *stage = nullptr;  // pinned host (device-visible)
   double *out = nullptr;           // pinned host (device-visible)
   unsigned char *stage_dev = nullptr;
@@ -144,9 +144,9 @@ BatchArrays arrays_of(Slot &sl, const BatchCaps &full)
   a.atom_struct = (int *) sl.astruct.p;
   a.row2atom = (int *) sl.w.row2atom.p;
   a.pos = (double4 *) sl.w.pos.p;
-  a.struct_out = (const double *) sl.sout.p;
   a.f = (double *) sl.w.f.p;
   a.eatom = (const double *) sl.w.ew.p;
+  a.watom = a.eatom + full.atoms;
   a.ctl = (unsigned long long *) sl.ctl.p;
   a.bin_count = (int *) sl.bins.p;
   a.bin_total = (int *) sl.bins.p + 2 * (size_t) full.bins;
@@ -194,7 +194,6 @@ int create_slot(Server *S, Slot &sl, int listcap)
   if ((rc = chk(sl.dyn.ensure(sizeof(BatchDims)), "serve: header"))) return rc;
   if ((rc = chk(sl.soff.ensure(4 * (size_t) (c.structs + 1)), "serve: offsets"))) return rc;
   if ((rc = chk(sl.astruct.ensure(4 * (size_t) c.atoms), "serve: atom structure"))) return rc;
-  if ((rc = chk(sl.sout.ensure(56 * (size_t) c.structs), "serve: sums"))) return rc;
   if ((rc = chk(sl.bins.ensure(sizeof(int) * (2 * (size_t) c.bins + 1)), "serve: bins"))) return rc;
   if ((rc = chk(sl.atominfo.ensure(sizeof(int) * 6 * (size_t) c.atoms), "serve: atom bins"))) return rc;
   if ((rc = chk(sl.sorted.ensure(sizeof(double4) * c.atoms), "serve: sorted positions"))) return rc;
@@ -292,16 +291,14 @@ int enqueue_batch(Server *S, Slot &sl, const Bucket &b, int rtile)
   c.f_cleared = true;  // by the unpack kernel
   c.nb = &nb;
   c.natoms = S->full.atoms;  // eatom/watom layout of the slot
-  c.struct_off = a.struct_off;
-  c.nstruct = b.caps.structs;
-  c.struct_out = (double *) sl.sout.p;
+  c.no_sums = true;  // with the results' copy
   c.rtile = rtile;
   c.dyn = a.dyn;
   c.g_bf16 = true;
   int rc = run_chain(ctx, sl.w, c, st);
   if (rc != TMD_OK) return rc;
-  e = launch_batch_pack(sl.out_dev, b.caps, a, st);
-  if (e != hipSuccess) return hip_fail(ctx, e, "serve: pack");
+  e = launch_batch_finish(sl.out_dev, b.caps, a, st);
+  if (e != hipSuccess) return hip_fail(ctx, e, "serve: results");
   return TMD_OK;
 }
 

@@ -18,62 +18,6 @@ __global__ void k_zero(uint4 *p, size_t n16, unsigned char *tail, size_t ntail)
   if (i < ntail) tail[i] = 0;
 }
 
-// sums of eatom[i], watom[i][0..5] over atoms [lo, hi) by one 256-thread
-// workgroup, in a fixed order; thread 0..6 of the result hold the 7 sums
-__device__ inline void block_sum7(const double *eatom, const double *watom, int lo, int hi,
-                                  int stride_lo, int stride, double (*sh)[256], double *res)
-{
-  int t = threadIdx.x;
-  double v[7] = {0, 0, 0, 0, 0, 0, 0};
-  for (int i = lo + stride_lo + t; i < hi; i += stride) {
-    v[0] += eatom[i];
-    for (int q = 0; q < 6; q++) v[1 + q] += watom[(size_t) i * 6 + q];
-  }
-  for (int q = 0; q < 7; q++) sh[q][t] = v[q];
-  __syncthreads();
-  for (int o = 128; o > 0; o >>= 1) {
-    if (t < o)
-      for (int q = 0; q < 7; q++) sh[q][t] += sh[q][t + o];
-    __syncthreads();
-  }
-  if (t < 7) res[t] = sh[t][0];
-}
-
-// The control word of the neighbor list after an evaluation: a build counted
-// if one was due, flags cleared for the next step.
-struct Ctl {
-  unsigned long long w[4];
-};
-
-__device__ inline Ctl load_ctl(const unsigned long long *ctl)
-{
-  Ctl c;
-  for (int q = 0; q < 4; q++) c.w[q] = ctl[q];
-  return c;
-}
-
-__device__ inline void reset_ctl(unsigned long long *ctl, Ctl &c, double trig2)
-{
-  if (c.w[1] != 0ull || __longlong_as_double((long long) c.w[0]) > trig2) ctl[3] = ++c.w[3];
-  c.w[0] = c.w[1] = 0ull;
-  ctl[0] = 0ull;
-  ctl[1] = 0ull;
-}
-
-// one workgroup per structure
-__global__ void k_reduce_struct(const double *eatom, const double *watom, const int *off,
-                                int nstruct, double *out, unsigned long long *ctl, double trig2, const BatchDims *dyn)
-{
-  __shared__ double sh[7][256];
-  const int st = blockIdx.x;
-  if (st == 0 && threadIdx.x == 0) {
-    Ctl c = load_ctl(ctl);
-    reset_ctl(ctl, c, trig2);
-  }
-  if (st >= nstruct || (dyn && st >= dyn->nstruct)) return;
-  block_sum7(eatom, watom, off[st], off[st + 1], 0, 256, sh, out + (size_t) st * 7);
-}
-
 // What the end of a step needs of memory, requested before the sums.
 struct StepEnd {
   Ctl ctl;
@@ -321,15 +265,6 @@ hipError_t launch_step_tail(const StepTail &t, hipStream_t s)
     k_step_sums<<<parts, 256, 0, s>>>(t);
     k_step_final<<<1, 512, 0, s>>>(t, parts);
   }
-  return hipGetLastError();
-}
-
-hipError_t launch_reduce_struct(const double *eatom, const double *watom, const int *off,
-                                int nstruct, double *out, unsigned long long *ctl, double trig2,
-                                hipStream_t s, const BatchDims *dyn)
-{
-  if (nstruct <= 0) return hipSuccess;
-  k_reduce_struct<<<nstruct, 256, 0, s>>>(eatom, watom, off, nstruct, out, ctl, trig2, dyn);
   return hipGetLastError();
 }
 
