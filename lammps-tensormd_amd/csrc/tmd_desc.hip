@@ -265,7 +265,7 @@ hipError_t launch_descriptor(const ModelGeo &g, const Geom &geo, const double4 *
   if (geo.order && row_begin != 0) return hipErrorInvalidValue;  // an order covers whole launches
   if (g.mm > 3)
     return launch_descriptor_hm(g, geo, pos, nbr, nn, cap, row2atom, nrows, tab, G, kl, stream, row_begin);
-  if (!geo.dyn && desc_waves(g, nrows - row_begin, cap) > 1)
+  if (!geo.dyn && desc_wide_ok(g, nrows - row_begin))
     return launch_descriptor_wide(g, geo, pos, nbr, nn, cap, row2atom, nrows, tab, G, kl, stream, row_begin);
 #define TMD_K_CASE(K)                                                                                    \
   case K:                                                                                                \

@@ -21,17 +21,18 @@ namespace {
 // order.  Lists or kept counts beyond the workgroup's room are left to its
 // first wave.  (Figures at force_waves.)
 constexpr int kWideRows = 96;  // staged neighbors of the descriptor
+constexpr int kDescWaves = 4;
 
-template <int K, int NS, int W>
+template <int K, int NS>
 struct DescWide {
   float rows[kWideRows * kRow];
-  float hb[W][Tiling<K>::HBUF];
-  f32x4v part[W][NS * Tiling<K>::KT][64];
-  int cnt[kMaxElts][W];
+  float hb[kDescWaves][Tiling<K>::HBUF];
+  f32x4v part[kDescWaves][NS * Tiling<K>::KT][64];
+  int cnt[kMaxElts][kDescWaves];
 };
 
-template <int K, int NS, int W>
-__global__ __launch_bounds__(64 * W) void k_descriptor_wide(ModelGeo g, Geom geo, const double4 *pos,
+template <int K, int NS>
+__global__ __launch_bounds__(64 * kDescWaves) void k_descriptor_wide(ModelGeo g, Geom geo, const double4 *pos,
                                                                 const uint32_t *nbr, const int *nn, int cap,
                                                                 const int *row2atom, int rbase, int nrows,
                                                                 const float4 *tab, float *G, uint32_t *kl)
@@ -43,10 +44,10 @@ __global__ __launch_bounds__(64 * W) void k_descriptor_wide(ModelGeo g, Geom geo
   float *Grow;
   const int i = descriptor_begin(g, geo, K, row, row2atom, G, Grow);
   if (i < 0) return;
-  DescWide<K, NS, W> &sh = *reinterpret_cast<DescWide<K, NS, W> *>(smem);
+  DescWide<K, NS> &sh = *reinterpret_cast<DescWide<K, NS> *>(smem);
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int nraw = nn[i];
-  if (nraw <= 64 * W) {
+  if (nraw <= 64 * kDescWaves) {
     const uint32_t *list = nbr + (size_t) i * cap;
     const uint32_t le = list[min(tid, max(nraw - 1, 0))];
     const uint32_t e = tid < nraw ? le : 0u;
@@ -68,7 +69,7 @@ __global__ __launch_bounds__(64 * W) void k_descriptor_wide(ModelGeo g, Geom geo
       start[b] = nk;
       if (b < g.nelt) {
 #pragma unroll
-        for (int w = 0; w < W; w++) {
+        for (int w = 0; w < kDescWaves; w++) {
           if (slot == b && w < wave) rank += sh.cnt[b][w];
           nk += sh.cnt[b][w];
         }
@@ -95,7 +96,7 @@ __global__ __launch_bounds__(64 * W) void k_descriptor_wide(ModelGeo g, Geom geo
       for (int b = 0; b < NS; b++)
 #pragma unroll
         for (int t = 0; t < T::KT; t++) acc[b][t] = f32x4v{0, 0, 0, 0};
-      for (int r0 = 16 * wave; r0 < nk; r0 += 16 * W) {
+      for (int r0 = 16 * wave; r0 < nk; r0 += 16 * kDescWaves) {
         TabTile<K> tt;
         load_tile<K>(tab, sh.rows + r0 * kRow, min(16, nk - r0), 0, tt);
         descriptor_tile<K, NS>(tt, [] {}, sh.rows + r0 * kRow, r0, min(16, nk - r0), 0, start, g.nelt, sh.hb[wave], acc);
@@ -106,10 +107,10 @@ __global__ __launch_bounds__(64 * W) void k_descriptor_wide(ModelGeo g, Geom geo
 #pragma unroll
         for (int t = 0; t < T::KT; t++) sh.part[wave][b * T::KT + t][lane] = acc[b][t];
       __syncthreads();
-      for (int p = wave; p < g.nelt * T::KT; p += W) {
+      for (int p = wave; p < g.nelt * T::KT; p += kDescWaves) {
         f32x4v v = sh.part[0][p][lane];
 #pragma unroll
-        for (int w = 1; w < W; w++) v += sh.part[w][p][lane];
+        for (int w = 1; w < kDescWaves; w++) v += sh.part[w][p][lane];
         store_g<K>(v, p / T::KT, p % T::KT, g.tsym, Grow, geo.g_bf16);
       }
       return;
@@ -267,19 +268,19 @@ hipError_t force_wide(const ModelGeo &g, const Geom &geo, const double4 *pos, in
 // slots accumulated by the descriptor kernel
 constexpr int desc_slots(int nelt) { return nelt <= 1 ? 1 : (nelt <= 2 ? 2 : (nelt <= 4 ? 4 : 8)); }
 
-template <int K, int NS, int W>
+template <int K, int NS>
 hipError_t desc_wide(const ModelGeo &g, const Geom &geo, const double4 *pos, const uint32_t *nbr, const int *nn, int cap,
                      const int *row2atom, int rbase, int nrows, const float4 *tab, float *G, uint32_t *kl, hipStream_t s)
 {
   if constexpr (NS * Tiling<K>::KT <= 8) {
     size_t offs[3];
-    const size_t lds = std::max(desc_lds<K>(cap, offs), sizeof(DescWide<K, NS, W>));
+    const size_t lds = std::max(desc_lds<K>(cap, offs), sizeof(DescWide<K, NS>));
     if (lds > 160 * 1024) return hipErrorInvalidConfiguration;
-    if (hipError_t ae = hipFuncSetAttribute((const void *) k_descriptor_wide<K, NS, W>,
+    if (hipError_t ae = hipFuncSetAttribute((const void *) k_descriptor_wide<K, NS>,
                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds);
         ae != hipSuccess)
       return ae;
-    k_descriptor_wide<K, NS, W><<<nrows - rbase, 64 * W, lds, s>>>(g, geo, pos, nbr, nn, cap, row2atom, rbase, nrows,
+    k_descriptor_wide<K, NS><<<nrows - rbase, 64 * kDescWaves, lds, s>>>(g, geo, pos, nbr, nn, cap, row2atom, rbase, nrows,
                                                                    tab, G, kl);
     return hipGetLastError();
   } else {
@@ -291,7 +292,8 @@ hipError_t desc_wide(const ModelGeo &g, const Geom &geo, const double4 *pos, con
 
 // Waves per atom (K <= 32).  Several shorten a wave's chain but add barriers
 // and, in the lane-per-neighbor parts, idle lanes, so they pay while a CU has
-// few atoms.  us, descriptor / force, 1, 2 and 4 waves per atom:
+// few atoms.  (The descriptor's two-wave form won 1 us in a narrow band and
+// is not built.)  us, descriptor / force, 1, 2 and 4 waves per atom:
 //   rows, elements, K      1              2              4
 //     256, 4, 24     10.8 / 15.3     9.2 / 12.9     8.5 / 12.0
 //     512, 4, 24     11.1 / 16.4     9.9 / 13.6     9.2 / 12.4
@@ -310,25 +312,21 @@ int force_waves(const ModelGeo &g, int rows)
   return rows <= (g.nelt <= 2 ? 2048 : kWide2Rows) ? 2 : 1;
 }
 
-// two waves take lists of up to 128 entries; the sums of the waves' P fit
-// beside four workgroups' others up to 8 filter tiles
-int desc_waves(const ModelGeo &g, int rows, int cap)
+// the sums of the waves' P fit beside four workgroups' others up to 8 filter
+// tiles
+bool desc_wide_ok(const ModelGeo &g, int rows)
 {
-  if (g.k > 32 || desc_slots(g.nelt) * ((g.k + 15) / 16) > 8) return 1;
-  if (rows <= kWide4Rows) return 4;
-  return rows <= kWide2Rows && cap <= 128 ? 2 : 1;
+  return g.k <= 32 && desc_slots(g.nelt) * ((g.k + 15) / 16) <= 8 && rows <= kWide4Rows;
 }
 
 hipError_t launch_descriptor_wide(const ModelGeo &g, const Geom &geo, const double4 *pos, const uint32_t *nbr,
                                   const int *nn, int cap, const int *row2atom, int nrows, const float4 *tab, float *G,
                                   uint32_t *kl, hipStream_t s, int row_begin)
 {
-  const int w = desc_waves(g, nrows - row_begin, cap);
-  if (w <= 1 || g.nelt < 1 || g.nelt > kMaxElts) return hipErrorInvalidValue;
-#define TMD_NS(K, NS)                                                                                               \
-  case NS:                                                                                                          \
-    return w == 4 ? desc_wide<K, NS, 4>(g, geo, pos, nbr, nn, cap, row2atom, row_begin, nrows, tab, G, kl, s)       \
-                  : desc_wide<K, NS, 2>(g, geo, pos, nbr, nn, cap, row2atom, row_begin, nrows, tab, G, kl, s);
+  if (!desc_wide_ok(g, nrows - row_begin) || g.nelt < 1 || g.nelt > kMaxElts) return hipErrorInvalidValue;
+#define TMD_NS(K, NS) \
+  case NS:            \
+    return desc_wide<K, NS>(g, geo, pos, nbr, nn, cap, row2atom, row_begin, nrows, tab, G, kl, s);
 #define TMD_K_CASE(K)              \
   case K:                          \
     switch (desc_slots(g.nelt)) {  \

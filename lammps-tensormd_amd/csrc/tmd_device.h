@@ -203,7 +203,7 @@ hipError_t launch_force_hm(const ModelGeo &g, const Geom &geo, const double4 *po
 // the launches, which launch_descriptor/launch_force call.  Not for batches
 // (Geom::dyn): their sums' order, and so a structure's last bits, must not
 // depend on the batch's capacity.
-int desc_waves(const ModelGeo &g, int rows, int cap);
+bool desc_wide_ok(const ModelGeo &g, int rows);
 int force_waves(const ModelGeo &g, int rows);
 hipError_t launch_descriptor_wide(const ModelGeo &g, const Geom &geo, const double4 *pos, const uint32_t *nbr,
                                   const int *nn, int cap, const int *row2atom, int nrows, const float4 *tab, float *G,
@@ -231,6 +231,15 @@ hipError_t launch_mlp(int mode, const RowLayout &rl, const MlpParams &mp, const 
                       float *dEdG, hipStream_t stream, int rtile = 0,
                       const BatchDims *dyn = nullptr, int row_begin = 0, int row_end = -1,
                       bool g_bf16 = false);
+// its precisions, at R rows per tile and with the LDS layout of mlp_lds_bytes
+hipError_t launch_mlp_fp32(int R, const RowLayout &rl, const MlpParams &mp, const float *G, double *E, float *dEdG,
+                           size_t lds, hipStream_t s, const BatchDims *dyn, int row_begin, int row_end, bool g_bf16);
+hipError_t launch_mlp_bf16(int R, const RowLayout &rl, const MlpParams &mp, const float *G, double *E, float *dEdG,
+                           size_t lds, hipStream_t s, const BatchDims *dyn, int row_begin, int row_end, bool g_bf16);
+hipError_t launch_mlp_fp8(int R, const RowLayout &rl, const MlpParams &mp, const float *G, double *E, float *dEdG,
+                          size_t lds, hipStream_t s, const BatchDims *dyn, int row_begin, int row_end, bool g_bf16);
+hipError_t launch_mlp_bf16x3(int R, const RowLayout &rl, const MlpParams &mp, const float *G, double *E, float *dEdG,
+                             size_t lds, hipStream_t s, const BatchDims *dyn, int row_begin, int row_end, bool g_bf16);
 // the MLP launch takes BF16 descriptor rows: BF16 mode, tanh, a compile-time
 // layer shape
 bool mlp_bf16_rows(const MlpParams &mp, int mode);
