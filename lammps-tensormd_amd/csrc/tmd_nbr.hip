@@ -389,7 +389,7 @@ __global__ __launch_bounds__(256) void k_nb_list(NbrBuild nb, const double4 *pos
         cnt = nb.bin_count[b];
         code = (uint32_t) ((s0 + 3) * 49 + (s1 + 3) * 7 + (s2 + 3)) << kNbrJBits;
       }
-      // this round's candidates in order, as many at a time as fit
+      // these bins' candidates in order, as many at a time as fit
       const int incl = wave_scan(cnt);
       const int excl = incl - cnt, total = __builtin_amdgcn_readlane(incl, 63);
       if (ncand + total > kCand) flush();
