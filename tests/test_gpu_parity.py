@@ -1251,3 +1251,29 @@ def test_waves_per_atom(tmp_path, k, nelt):
         assert abs(got["vatom"].reshape(copies, -1, 6) - ref["vatom"]).max() <= 6.0 * bar
         assert abs(got["energy"] / copies - ref["energy"]) <= 1e-6 * len(nl)
         assert abs(G - g0).max() <= 4e-6 * max(1.0, abs(g0).max())
+
+
+@pytest.mark.parametrize("cells", [(4, 4, 4), (16, 16, 8), (16, 16, 9), (24, 24, 24)])
+def test_state_transfers(synth_models, cells):
+    """Positions and velocities set and read back on both sides of the line
+    (4,096 atoms) between kernels that read host memory and a copy before
+    them, twice with new values: the same bits, wrapped into the cell, and the
+    forces of a new system at the same positions."""
+    x, t, cell = W.crystal("bcc", 3.2, cells, nelt=4, sigma=0.05, seed=95)
+    rng = np.random.default_rng(96)
+    m = TensorMD(synth_models["c2"], ["Mo", "Nb", "Ta", "W"], "fp32", 0.001)
+    s = m.system(x, t, cell, skin=1.0)
+    L = np.array(cells) * 3.2
+    for _ in range(2):
+        x2 = x + rng.normal(scale=0.3, size=x.shape)
+        v = rng.normal(size=x.shape)
+        s.set_positions(x2)
+        s.set_velocities(v)
+        r = s.compute()
+        ref = m.system(x2, t, cell, skin=1.0).compute()
+        say("case:", len(x), "atoms, max |dF|", abs(r["f"] - ref["f"]).max())
+        # one rounding of the wrapped coordinate
+        assert abs(r["x"] - (x2 - np.floor(x2 / L) * L)).max() <= np.spacing(L.max())
+        assert np.array_equal(r["x"], ref["x"]) and np.array_equal(r["v"], v)
+        # the same kernels on the same values: FP64 sums in any order
+        assert abs(r["f"] - ref["f"]).max() <= 1e-10 and np.array_equal(r["eatom"], ref["eatom"])
