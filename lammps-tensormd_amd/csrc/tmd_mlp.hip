@@ -174,7 +174,8 @@ hipError_t launch_mlp(int mode, const RowLayout &rl, const MlpParams &mp, const 
     int R = Rs[q];
     MlpParams m;
     size_t lds = mlp_lds_bytes(mp, mode, R, &m);
-    if (lds > limit) continue;
+    // tiles of fewer than 16 rows read the descriptor rows from LDS only
+    if (lds > limit || (R < 16 && !m.stage_g)) continue;
     auto launch = mode == 0 ? launch_mlp_fp32 : (mode == 1 ? launch_mlp_bf16 : (mode == 2 ? launch_mlp_fp8 : launch_mlp_bf16x3));
     return launch(R, rl, m, G, E, dEdG, lds, s, dyn, row_begin, row_end, g_bf16);
   }

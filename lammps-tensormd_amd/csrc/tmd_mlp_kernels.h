@@ -868,6 +868,7 @@ __device__ inline void gemm_t(const void *W, int t0, const T *X, int ldx, const 
                               int grow0, int K, const float *rinv, f32x4 (&acc)[4][R / kRB<R>])
 {
   constexpr int KS = kFastKS<MODE>, RB = kRB<R>, RT = R / RB;
+  static_assert(!XG || RB == 16, "ld_graw reads 16 rows");
   constexpr int DW = (RB == 4 ? 16 : 8) / NTW;
   constexpr int D = XG ? 2 : (DW >= 2 ? DW : 2);  // layer 0 also rings its raw rows
   using F = typename Frag<MODE>::A;
@@ -1042,12 +1043,16 @@ __global__ __launch_bounds__(64 * NW, (kMlpWaves<MODE, R, SH>)) void k_mlp_fast(
 #pragma unroll
       for (int r = 0; r < RT; r++) mx[r] = 0.0f;
       if (ntw > 0) {
-        if constexpr (MODE == 2)
+        // tiles of fewer than 16 rows always have theirs staged (launch_mlp)
+        constexpr bool kUnstaged = MODE != 2 && !SH && RB == 16;
+        if constexpr (MODE == 2) {
           gemm_n<MODE, R, false, uint8_t>(W, t0, ntw, Q, mp.ldq, nullptr, gw, row0, K, rs + R, acc);
-        else if (!SH && l == 0 && !mp.stage_g)
-          gemm_n<MODE, R, true, T>(W, t0, ntw, nullptr, 0, Gd, gw, row0, K, rs + R, acc);
-        else
+        } else if (kUnstaged && l == 0 && !mp.stage_g) {
+          if constexpr (kUnstaged)
+            gemm_n<MODE, R, true, T>(W, t0, ntw, nullptr, 0, Gd, gw, row0, K, rs + R, acc);
+        } else {
           gemm_n<MODE, R, false, T>(W, t0, ntw, Hin, ldi, nullptr, gw, row0, K, rs + R, acc);
+        }
       }
       if (over) {
         __syncthreads();
@@ -1289,7 +1294,7 @@ template <int MODE, int R>
 hipError_t launch_r(const RowLayout &rl, const MlpParams &mp, const float *G, double *E, float *dEdG,
                     size_t lds, hipStream_t s, const BatchDims *dyn, int rb, int re, bool gb = false)
 {
-  if (rb % R || re % R) return hipErrorInvalidValue;
+  if (rb % R || re % R || (R < 16 && !mp.stage_g)) return hipErrorInvalidValue;
   dim3 grid((re - rb) / R);
   const bool fast = mlp_fast_ok(mp, MODE);
   if constexpr (MODE == 2 || MODE == 3 || R < 16) {  // these exist on the fast path only

@@ -1277,3 +1277,30 @@ def test_state_transfers(synth_models, cells):
         assert np.array_equal(r["x"], ref["x"]) and np.array_equal(r["v"], v)
         # the same kernels on the same values: FP64 sums in any order
         assert abs(r["f"] - ref["f"]).max() <= 1e-10 and np.array_equal(r["eatom"], ref["eatom"])
+
+
+@pytest.mark.parametrize("layers,act,cells", [
+    ([1024, 1024, 64, 1], "tanh", [(8, 8, 8), (8, 8, 9), (8, 16, 8)]),
+    ([576, 576, 64, 1], "squareplus", [(8, 8, 8), (8, 8, 9), (8, 16, 8)]),
+])
+def test_network_rows_not_staged(tmp_path, layers, act, cells):
+    """Networks of 512 inputs whose first layer is wider than one pass of the
+    waves (512) and whose 8-row tiles are too large to hold their descriptor
+    rows in LDS beside the activations: such tiles are not taken, and the
+    16-row ones read the rows from memory.  4-row tiles (1,024 rows and fewer)
+    have room for them.  Bars as in test_network_tiles."""
+    path = W.write_model(str(tmp_path / "m.npz"), symbols=["W"], masses=[183.84], rmax=5.0, num_filters=128,
+                         layer_sizes=layers, actfn=act, seed=131, radial_scale=0.2)
+    z = dict(np.load(path))
+    m = TensorMD(path, ["W"], "fp32", 0.001)
+    for c in cells:
+        x, t, cell = W.crystal("bcc", 3.2, c, nelt=1, sigma=0.08, seed=132)
+        say("case: network, rows not staged", layers, act, len(x), "atoms")
+        s = m.system(x, t, cell, skin=0.6)
+        r = s.compute()
+        G, dG = s.descriptors(m.info()["width"])
+        s.close()
+        E, sE, g, sg = _network_spread(z, G, len(layers), act, False, 0.0)
+        e0, e1 = abs(r["eatom"] - E) / sE, abs(dG - g) / sg
+        say("largest error / spread: E", e0.max(), "dE/dG", e1.max())
+        assert e0.max() <= 8.0 and e1.max() <= 8.0, (len(x), e0.max(), e1.max())
