@@ -125,14 +125,22 @@ bool mlp_bf16_rows(const MlpParams &mp, int mode)
 }
 
 namespace {
+constexpr long kMlpLds = 160 * 1024;  // of a CU
+
 // Rows per tile.  16 while 32-row tiles would not give every CU one (a tile
-// is a serial chain of layers, and its length goes with its rows); 64 in the
-// BF16 mode once they give every CU two (half the weight reads, and their
-// accumulators still fit four waves per SIMD); else 32.  FP32 tiles of 4 and
-// 8 rows while those give no CU a second one: a lone 16-row tile is bound by
-// its CU's matrix cores, 0.11 us per 1,000 weights, so they pay where that is
-// most of its time (16 K weights: 15.9 us at 16 rows, 16.4 and 17.3 at 4 and
-// 8; 82 K: 32.7, 29.5 and 32.4).  us, network alone, 384-256-128-64-1
+// is a serial chain of layers, and its length goes with its rows), or where
+// only a tile of 16 has room for its descriptor rows in LDS (BF16
+// 256-640-256-1, 16,000 rows: 74 us against 93 at 32); else 32.  64 in the
+// BF16 mode once they give every CU two (half the weight reads), where two of
+// them fit a CU: the compile-time shapes run four waves per SIMD at 64 rows
+// (spilling 6 registers and 1; the other widths take 202), with at most 80 KB
+// of LDS each.  384-256-256-128-1 has 83 KB: 128,000 rows take 218 us at 32
+// rows and 257 at 64; 256-128-128-128-128-1 with skips 224 and 271.
+// FP32 tiles of 4 and 8 rows while those give no CU a second one: a lone
+// 16-row tile is bound by its CU's matrix cores, 0.11 us per 1,000 weights,
+// so they pay where that is most of its time (16 K weights: 15.9 us at 16
+// rows, 16.4 and 17.3 at 4 and 8; 82 K: 32.7, 29.5 and 32.4).  us, network
+// alone, 384-256-128-64-1
 // (139 K weights):     4 rows   8 rows  16 rows  32 rows  64 rows
 //   FP32       128      18.3     23.5     32.5     52.0
 //            1,024      22.1     24.3     32.6     52.4
@@ -154,7 +162,14 @@ int tile_rows(const MlpParams &mp, int mode, int nrows, bool batch)
     if (w >= 64 * 1024) return nrows <= 4 * kCUs ? 4 : 8;
   }
   if (nrows <= 32 * kCUs) return 16;
-  return mode == 1 && nrows >= 64 * 2 * kCUs ? 64 : 32;
+  MlpParams m16, m32;
+  mlp_lds_bytes(mp, mode, 16, &m16);
+  mlp_lds_bytes(mp, mode, 32, &m32);
+  if (m16.stage_g && !m32.stage_g) return 16;
+  if (mode == 1 && nrows >= 64 * 2 * kCUs && mp.act == 2 && mlp_shape(mp) != 0 &&
+      2 * (long) mlp_lds_bytes(mp, mode, 64, nullptr) <= kMlpLds)
+    return 64;
+  return 32;
 }
 }  // namespace
 
@@ -166,20 +181,20 @@ hipError_t launch_mlp(int mode, const RowLayout &rl, const MlpParams &mp, const 
   if (row_end < 0 || row_end > rl.nrows) row_end = rl.nrows;
   if (row_begin < 0 || row_begin > row_end) return hipErrorInvalidValue;
   if (row_end == row_begin) return hipSuccess;
-  const size_t limit = 160 * 1024;
-  // rtile (16/32/64) overrides the rule
-  int Rs[3] = {mlp_fast_ok(mp, mode) ? tile_rows(mp, mode, row_end - row_begin, dyn != nullptr) : 32, 16, 16};
-  if (rtile == 16 || rtile == 32 || rtile == 64) Rs[0] = rtile;
-  for (int q = 0; q < 3; q++) {
-    int R = Rs[q];
+  // rtile (16/32/64) overrides the rule; where its tile does not fit, the next
+  // smaller of 32 and 16 rows
+  int R = mlp_fast_ok(mp, mode) ? tile_rows(mp, mode, row_end - row_begin, dyn != nullptr) : 32;
+  if (rtile == 16 || rtile == 32 || rtile == 64) R = rtile;
+  for (;; R = R > 32 ? 32 : 16) {
     MlpParams m;
-    size_t lds = mlp_lds_bytes(mp, mode, R, &m);
+    const long lds = (long) mlp_lds_bytes(mp, mode, R, &m);
     // tiles of fewer than 16 rows read the descriptor rows from LDS only
-    if (lds > limit || (R < 16 && !m.stage_g)) continue;
-    auto launch = mode == 0 ? launch_mlp_fp32 : (mode == 1 ? launch_mlp_bf16 : (mode == 2 ? launch_mlp_fp8 : launch_mlp_bf16x3));
-    return launch(R, rl, m, G, E, dEdG, lds, s, dyn, row_begin, row_end, g_bf16);
+    if (lds <= kMlpLds && (R >= 16 || m.stage_g)) {
+      auto launch = mode == 0 ? launch_mlp_fp32 : (mode == 1 ? launch_mlp_bf16 : (mode == 2 ? launch_mlp_fp8 : launch_mlp_bf16x3));
+      return launch(R, rl, m, G, E, dEdG, lds, s, dyn, row_begin, row_end, g_bf16);
+    }
+    if (R == 16) return hipErrorInvalidConfiguration;
   }
-  return hipErrorInvalidConfiguration;
 }
 
 }  // namespace tmd

@@ -1304,3 +1304,45 @@ def test_network_rows_not_staged(tmp_path, layers, act, cells):
         e0, e1 = abs(r["eatom"] - E) / sE, abs(dG - g) / sg
         say("largest error / spread: E", e0.max(), "dE/dG", e1.max())
         assert e0.max() <= 8.0 and e1.max() <= 8.0, (len(x), e0.max(), e1.max())
+
+
+@pytest.mark.parametrize("prec,k,nelt,layers,act,resnet,copies", [
+    ("fp32", 24, 4, [256, 128, 64, 1], "tanh", False, [20, 80]),
+    ("bf16", 24, 4, [256, 128, 64, 1], "tanh", False, [20, 80, 260]),
+    ("bf16", 24, 4, [256, 256, 128, 1], "tanh", False, [20, 80, 260]),
+    ("bf16", 32, 1, [128, 64, 1], "tanh", False, [20, 80, 260]),
+    ("bf16", 32, 2, [128] * 5 + [1], "squareplus", True, [20, 80, 260]),
+])
+def test_tile_rows_agree(tmp_path, prec, k, nelt, layers, act, resnet, copies):
+    """Tiles of 16, 32 and 64 rows give the same bits: clusters of 128 centers,
+    repeated until the number of rows takes the next tile (or, where a larger
+    tile never pays, the same one).  Energies equal those of the first copy of
+    the fewest rows; forces, whose FP64 sums are in any order, to 1e-12."""
+    el, ma = ["Mo", "Nb", "Ta", "W"][:nelt], [95.95, 92.906, 180.95, 183.84][:nelt]
+    path = W.write_model(str(tmp_path / "m.npz"), symbols=el, masses=ma, rmax=6.0, num_filters=k,
+                         layer_sizes=layers, actfn=act, use_resnet_dt=resnet, seed=140 + k, radial_scale=0.1)
+    m = TensorMD(path, el, prec, 0.001)
+    rng = np.random.default_rng(141)
+    base, nb = 128, 9
+    xs, ts = [], []
+    for _ in range(base):
+        x, t = _cluster(rng, m.cutoff, list(np.bincount(rng.integers(0, nelt, nb), minlength=nelt)))
+        t[0] = rng.integers(1, nelt + 1)
+        xs.append(x)
+        ts.append(t)
+    x1, t1, size = np.concatenate(xs), np.concatenate(ts), base * (nb + 1)
+    first = None
+    for c in copies:
+        say("case:", prec, k, nelt, layers, c * base, "rows")
+        il = (np.arange(c * base) * (nb + 1)).tolist()
+        num = np.zeros(c * size, dtype=np.int32)
+        num[il] = nb
+        flat = np.delete(np.arange(c * size), il)
+        got = m.compute_list(c * size, np.tile(x1, (c, 1)), np.tile(t1, c), il, num, flat)
+        e = got["eatom"][il].reshape(c, base)
+        f = got["f"].reshape(c, size, 3)
+        if first is None:
+            first = e[0].copy(), f[0].copy()
+            assert np.isfinite(first[0]).all() and np.ptp(first[0]) > 0 and abs(first[1]).max() > 0
+        assert np.array_equal(e, np.broadcast_to(first[0], e.shape))
+        assert abs(f - first[1]).max() <= 1e-12 * max(1.0, abs(first[1]).max())
