@@ -93,7 +93,7 @@ size_t mlp_lds_bytes(const MlpParams &mp, int mode, int R, MlpParams *out)
   m.ldx = m.ld[0];
   if (mode != 2 && mlp_fast_ok(mp, mode)) {
     const size_t xn = (size_t) R * m.ldx;
-    if (mp.sizes[1] / 16 <= 4 * NW && xn * esz <= 128 * 1024) {
+    if (mp.sizes[1] / 16 <= 4 * mlp_waves(mp, mode, R) && xn * esz <= 128 * 1024) {
       m.stage_g = m.g_over = 1;
       off = std::max(off, xn);
     } else if ((off + xn) * esz <= 80 * 1024) {
@@ -136,6 +136,11 @@ constexpr long kMlpLds = 160 * 1024;  // of a CU
 // (spilling 6 registers and 1; the other widths take 202), with at most 80 KB
 // of LDS each.  384-256-256-128-1 has 83 KB: 128,000 rows take 218 us at 32
 // rows and 257 at 64; 256-128-128-128-128-1 with skips 224 and 271.
+// In the FP8 and split-BF16 modes, widths unknown at compile time: 16 or 32,
+// whichever takes the chip fewer rounds of resident workgroups, 16 in a tie
+// (FP8 1024-128-128-1, two and three workgroups per CU: 11,664 rows 42.9 at 16
+// and 48.1 at 32 rows, 16,000 rows 66.0 and 55.4, 24,334 rows 84.5 and 97.2;
+// split BF16 64-128-64-1: 16,384 rows 27.2 and 21.0).
 // FP32 tiles of 4 and 8 rows while those give no CU a second one: a lone
 // 16-row tile is bound by its CU's matrix cores, 0.11 us per 1,000 weights,
 // so they pay where that is most of its time (16 K weights: 15.9 us at 16
@@ -155,18 +160,26 @@ constexpr long kMlpLds = 160 * 1024;  // of a CU
 //          128,000                         245      191      150
 int tile_rows(const MlpParams &mp, int mode, int nrows, bool batch)
 {
-  constexpr int kCUs = 256;
   if (mode == 0 && nrows <= 8 * kCUs && !batch) {
     long w = 0;
     for (int l = 0; l < mp.nl - 1; l++) w += (long) mp.sizes[l] * mp.sizes[l + 1];
     if (w >= 64 * 1024) return nrows <= 4 * kCUs ? 4 : 8;
+  }
+  if (mode >= 2 && !mlp_shape_kernel(mp, mode, 16)) {
+    // rounds that the chip takes for all tiles, by its resident workgroups
+    auto rounds = [&](int R) {
+      const long lds = (long) mlp_lds_bytes(mp, mode, R, nullptr), fit = kMlpLds / lds;
+      const long tiles = (nrows + R - 1) / R, held = kCUs * std::min(fit, mlp_waves(mp, mode, R) == 4 ? 3l : 1l);
+      return held > 0 ? (tiles + held - 1) / held : tiles + 1;
+    };
+    return rounds(32) < rounds(16) ? 32 : 16;
   }
   if (nrows <= 32 * kCUs) return 16;
   MlpParams m16, m32;
   mlp_lds_bytes(mp, mode, 16, &m16);
   mlp_lds_bytes(mp, mode, 32, &m32);
   if (m16.stage_g && !m32.stage_g) return 16;
-  if (mode == 1 && nrows >= 64 * 2 * kCUs && mp.act == 2 && mlp_shape(mp) != 0 &&
+  if (mode == 1 && nrows >= 64 * 2 * kCUs && mlp_shape_kernel(mp, mode, 64) &&
       2 * (long) mlp_lds_bytes(mp, mode, 64, nullptr) <= kMlpLds)
     return 64;
   return 32;

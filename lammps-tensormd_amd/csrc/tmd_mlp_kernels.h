@@ -28,9 +28,11 @@
 //
 // The kernels are compiled one precision to a file (tmd_mlp_fp32.hip, ..): a
 // process loads a file's code at its first launch, and all of them together
-// are 4.5 MB.
+// are 5 MB.
 #pragma once
 #include "tmd_desc_common.h"
+
+#include <climits>
 
 namespace tmd {
 
@@ -530,13 +532,6 @@ __device__ inline typename Frag<MODE>::A ld_x(const T *X, int ld, int r0, int k,
   }
 }
 
-// Waves of a workgroup.  Eight share a tile's rows: each reads half the
-// weights that four would, a small system's few tiles have twice the loads in
-// flight, and the FP32 modes, whose LDS admits two workgroups per CU, run
-// four waves per SIMD instead of two (FP32 network of 2,000 atoms 65 -> 40 us,
-// of 128,000 atoms 785 -> 694 us against four waves; 16 waves are slower).
-constexpr int NW = 8;
-
 // 8 consecutive values of row r at column c: the FP32 descriptor rows in
 // HBM (XG) or a BF16 LDS tile
 template <bool XG>
@@ -807,7 +802,7 @@ __device__ inline void st4(uint16_t *p, const float v[4])
 // -> X [R][ld] in the activations' type (the BF16 mode rounds FP32 rows here,
 // once for all waves; GB rows are BF16 already).  Reading them step by step
 // as MFMA operands put one trip to HBM into every step of the inner loop.
-template <int MODE, int R, bool GB, int GW, typename T>
+template <int MODE, int R, int NW, bool GB, int GW, typename T>
 __device__ inline void stage_g(const float *G, int gw_, int grow0, T *X, int ld)
 {
   static_assert(MODE != 2, "FP8 rows are quantized instead");
@@ -863,7 +858,7 @@ __device__ inline void stage_g(const float *G, int gw_, int grow0, T *X, int ld)
 // same number of loads (past the last step they repeat it), which lets the
 // compiler wait for exactly the step being consumed.  Activations in LDS
 // are read at the step that uses them.
-template <int MODE, int R, bool XG, int NTW, typename T>
+template <int MODE, int R, int NW, bool XG, int NTW, typename T>
 __device__ inline void gemm_t(const void *W, int t0, const T *X, int ldx, const float *G, int gw,
                               int grow0, int K, const float *rinv, f32x4 (&acc)[4][R / kRB<R>])
 {
@@ -918,28 +913,29 @@ __device__ inline void gemm_t(const void *W, int t0, const T *X, int ldx, const 
 }
 
 // gemm_t for a runtime tile count ntw in 1..4 (wave-uniform)
-template <int MODE, int R, bool XG, typename T>
+template <int MODE, int R, int NW, bool XG, typename T>
 __device__ inline void gemm_n(const void *W, int t0, int ntw, const T *X, int ldx, const float *G,
                               int gw, int grow0, int K, const float *rinv, f32x4 (&acc)[4][R / kRB<R>])
 {
   if (ntw >= 4)
-    gemm_t<MODE, R, XG, 4, T>(W, t0, X, ldx, G, gw, grow0, K, rinv, acc);
+    gemm_t<MODE, R, NW, XG, 4, T>(W, t0, X, ldx, G, gw, grow0, K, rinv, acc);
   else if (ntw == 3)
-    gemm_t<MODE, R, XG, 3, T>(W, t0, X, ldx, G, gw, grow0, K, rinv, acc);
+    gemm_t<MODE, R, NW, XG, 3, T>(W, t0, X, ldx, G, gw, grow0, K, rinv, acc);
   else if (ntw == 2)
-    gemm_t<MODE, R, XG, 2, T>(W, t0, X, ldx, G, gw, grow0, K, rinv, acc);
+    gemm_t<MODE, R, NW, XG, 2, T>(W, t0, X, ldx, G, gw, grow0, K, rinv, acc);
   else
-    gemm_t<MODE, R, XG, 1, T>(W, t0, X, ldx, G, gw, grow0, K, rinv, acc);
+    gemm_t<MODE, R, NW, XG, 1, T>(W, t0, X, ldx, G, gw, grow0, K, rinv, acc);
 }
 
 }  // namespace
 
-// Waves per SIMD asked of the fast kernel; a workgroup has two.  Four where
-// the registers allow it (the compile-time shapes, and the FP32 and BF16
-// modes up to 32 rows), else two; two in tiles of fewer than 16 rows, which
-// are taken where a CU has one tile.
-template <int MODE, int R, int SH>
-constexpr int kMlpWaves = R < 16 ? 2 : SH ? 4 : ((R <= 32 && MODE <= 1) ? 4 : 2);
+// Waves per SIMD asked of the fast kernel; a workgroup of eight waves has two,
+// of four one.  Four where the registers allow it (the compile-time shapes,
+// and the FP32 and BF16 modes up to 32 rows), three in the workgroups of four
+// waves up to 32 rows, else two; two in tiles of fewer than 16 rows, which are
+// taken where a CU has one tile.
+template <int MODE, int R, int SH, int NW>
+constexpr int kMlpWaves = R < 16 ? 2 : (SH || (R <= 32 && MODE <= 1)) ? 4 : (NW == 4 && R <= 32 ? 3 : 2);
 
 // bytes per weight of the fast kernel's A operands
 template <int MODE>
@@ -964,8 +960,8 @@ struct MlpShape<2> {  // 384-256-256-128-1
 };
 
 // GB: Gd holds BF16 descriptor rows (MODE 1 only)
-template <int MODE, int ACT, int R, int SH = 0, bool GB = false>
-__global__ __launch_bounds__(64 * NW, (kMlpWaves<MODE, R, SH>)) void k_mlp_fast(RowLayout rl_cap, MlpParams mp, const float *Gd,
+template <int MODE, int ACT, int R, int SH = 0, int NW = 8, bool GB = false>
+__global__ __launch_bounds__(64 * NW, (kMlpWaves<MODE, R, SH, NW>)) void k_mlp_fast(RowLayout rl_cap, MlpParams mp, const float *Gd,
                                                   double *E, float *dEdG, const BatchDims *dyn, int rbase, int rend)
 {
   const RowLayout rl = dyn ? dyn->rl : rl_cap;
@@ -1001,7 +997,7 @@ __global__ __launch_bounds__(64 * NW, (kMlpWaves<MODE, R, SH>)) void k_mlp_fast(
   T *X0 = sm + mp.offX;
   if constexpr (MODE != 2) {
     if (SH || mp.stage_g) {
-      stage_g<MODE, R, GB, SH ? MlpShape<SH>::w(0) : 0>(Gd, gw, row0, X0, mp.ldx);
+      stage_g<MODE, R, NW, GB, SH ? MlpShape<SH>::w(0) : 0>(Gd, gw, row0, X0, mp.ldx);
       __syncthreads();
     }
   }
@@ -1046,12 +1042,12 @@ __global__ __launch_bounds__(64 * NW, (kMlpWaves<MODE, R, SH>)) void k_mlp_fast(
         // tiles of fewer than 16 rows always have theirs staged (launch_mlp)
         constexpr bool kUnstaged = MODE != 2 && !SH && RB == 16;
         if constexpr (MODE == 2) {
-          gemm_n<MODE, R, false, uint8_t>(W, t0, ntw, Q, mp.ldq, nullptr, gw, row0, K, rs + R, acc);
+          gemm_n<MODE, R, NW, false, uint8_t>(W, t0, ntw, Q, mp.ldq, nullptr, gw, row0, K, rs + R, acc);
         } else if (kUnstaged && l == 0 && !mp.stage_g) {
           if constexpr (kUnstaged)
-            gemm_n<MODE, R, true, T>(W, t0, ntw, nullptr, 0, Gd, gw, row0, K, rs + R, acc);
+            gemm_n<MODE, R, NW, true, T>(W, t0, ntw, nullptr, 0, Gd, gw, row0, K, rs + R, acc);
         } else {
-          gemm_n<MODE, R, false, T>(W, t0, ntw, Hin, ldi, nullptr, gw, row0, K, rs + R, acc);
+          gemm_n<MODE, R, NW, false, T>(W, t0, ntw, Hin, ldi, nullptr, gw, row0, K, rs + R, acc);
         }
       }
       if (over) {
@@ -1179,9 +1175,9 @@ __global__ __launch_bounds__(64 * NW, (kMlpWaves<MODE, R, SH>)) void k_mlp_fast(
 #pragma unroll
       for (int r = 0; r < RT; r++) mx[r] = 0.0f;
       if constexpr (MODE == 2)
-        gemm_n<MODE, R, false, uint8_t>(W, t0, ntw, Q, mp.ldq, nullptr, gw, row0, N, rs + R, acc);
+        gemm_n<MODE, R, NW, false, uint8_t>(W, t0, ntw, Q, mp.ldq, nullptr, gw, row0, N, rs + R, acc);
       else
-        gemm_n<MODE, R, false, T>(W, t0, ntw, Gl, ldg, nullptr, gw, row0, N, rs + R, acc);
+        gemm_n<MODE, R, NW, false, T>(W, t0, ntw, Gl, ldg, nullptr, gw, row0, N, rs + R, acc);
 #pragma unroll
       for (int j = 0; j < 4; j++) {
         if (j >= ntw) continue;
@@ -1256,10 +1252,46 @@ int mlp_shape(const MlpParams &mp)
   return 0;
 }
 
+constexpr long kCUs = 256;
+
 // Tiles at which a mode's compile-time shapes are built: those that
 // tile_rows() takes.
+constexpr bool shape_tile(int mode, int R) { return R <= 32 || mode == 1; }
 template <int MODE, int R>
-constexpr bool kShapeTile = R <= 32 || MODE == 1;
+constexpr bool kShapeTile = shape_tile(MODE, R);
+// a compile-time shape's kernel runs
+bool mlp_shape_kernel(const MlpParams &mp, int mode, int R)
+{
+  return mp.act == 2 && shape_tile(mode, R) && mlp_shape(mp) != 0;
+}
+
+// Waves of a workgroup of the fast kernel.  Eight share a tile's rows: each
+// reads half the weights that four would, a small system's few tiles have
+// twice the loads in flight, and the FP32 modes, whose LDS admits two
+// workgroups per CU, run four waves per SIMD instead of two (FP32 network of
+// 2,000 atoms 65 -> 40 us, of 128,000 atoms 785 -> 694 us against four waves;
+// 16 waves are slower).  Four in the FP8 and split-BF16 kernels of widths not
+// known at compile time: their 138 to 176 registers leave two or three waves
+// per SIMD, which is one workgroup of eight per CU but three of four (us,
+// eight -> four waves, both at their best of 16 and 32 rows: FP8
+// 256-128-128-128-128-1 with skips, 35,152 rows, 166 -> 108; split BF16
+// 64-128-64-1, 37,044 rows, 68 -> 38).  Eight there too
+//  - in split BF16 where the first layer has more than 256 outputs, which four
+//    waves do not cover in one pass, so that the descriptor rows would not be
+//    staged (384-512-256-128-1, 93,312 rows: 690 against 852 us);
+//  - while 16-row tiles give a CU one workgroup at most, if a layer has 64 K
+//    weights or more, whose loads then bound the tile (FP8, 3,456 rows:
+//    1024-128-128-1 29.6 against 33.0 us, the network above 35.8 against 41.3;
+//    256-128-128-128-128-1, of 32 K: 36.4 against 30.6).
+int mlp_waves(const MlpParams &mp, int mode, int R, long rows = LONG_MAX)
+{
+  if (mode <= 1 || mlp_shape_kernel(mp, mode, R)) return 8;
+  if (mode == 3 && mp.sizes[1] > 256) return 8;
+  if (R > 16 || rows > 16 * kCUs) return 4;
+  for (int l = 0; l < mp.nl - 1; l++)
+    if ((long) mp.sizes[l] * mp.sizes[l + 1] >= 64 * 1024) return 8;
+  return 4;
+}
 
 // k_mlp_fast with the model's compile-time shape where one exists (tanh
 // models), else the generic widths.  The constant tile counts, inner steps
@@ -1269,25 +1301,32 @@ template <int MODE, int A, int R>
 hipError_t launch_fast(dim3 grid, size_t lds, hipStream_t s, const RowLayout &rl, const MlpParams &mp,
                        const float *G, double *E, float *dEdG, const BatchDims *dyn, int rb, bool gb)
 {
+  const int waves = mlp_waves(mp, MODE, R, (long) grid.x * R);
   auto go = [&](auto kern) -> hipError_t {
     if (hipError_t ae = hipFuncSetAttribute((const void *) kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds);
         ae != hipSuccess)
       return ae;
-    kern<<<grid, 64 * NW, lds, s>>>(rl, mp, G, E, dEdG, dyn, rb, rb + (int) grid.x * R);
+    kern<<<grid, 64 * waves, lds, s>>>(rl, mp, G, E, dEdG, dyn, rb, rb + (int) grid.x * R);
     return hipGetLastError();
   };
   if constexpr (A == 2 && kShapeTile<MODE, R>) {
     const int sh = mlp_shape(mp);
     if constexpr (MODE == 1) {
-      if (gb && sh == 1) return go(k_mlp_fast<MODE, A, R, 1, true>);
-      if (gb && sh == 2) return go(k_mlp_fast<MODE, A, R, 2, true>);
+      if (gb && sh == 1) return go(k_mlp_fast<MODE, A, R, 1, 8, true>);
+      if (gb && sh == 2) return go(k_mlp_fast<MODE, A, R, 2, 8, true>);
     }
     if (gb) return hipErrorInvalidValue;
     if (sh == 1) return go(k_mlp_fast<MODE, A, R, 1>);
     if (sh == 2) return go(k_mlp_fast<MODE, A, R, 2>);
   }
   if (gb) return hipErrorInvalidValue;
-  return go(k_mlp_fast<MODE, A, R, 0>);
+  if constexpr (MODE >= 2) {
+    if (waves == 4) return go(k_mlp_fast<MODE, A, R, 0, 4>);
+  }
+  if constexpr (MODE != 2 || R == 16)
+    return go(k_mlp_fast<MODE, A, R, 0>);
+  else
+    return hipErrorInvalidValue;
 }
 
 template <int MODE, int R>

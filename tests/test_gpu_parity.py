@@ -1312,6 +1312,13 @@ def test_network_rows_not_staged(tmp_path, layers, act, cells):
     ("bf16", 24, 4, [256, 256, 128, 1], "tanh", False, [20, 80, 260]),
     ("bf16", 32, 1, [128, 64, 1], "tanh", False, [20, 80, 260]),
     ("bf16", 32, 2, [128] * 5 + [1], "squareplus", True, [20, 80, 260]),
+    ("bf16x3", 24, 4, [256, 128, 64, 1], "tanh", False, [20, 80]),
+    ("bf16x3", 32, 1, [128, 64, 1], "tanh", False, [20, 96, 97]),
+    ("bf16x3", 64, 1, [512, 128, 1], "tanh", False, [20, 40]),
+    ("bf16x3", 64, 1, [128] * 4 + [1], "squareplus", True, [20, 130]),
+    ("fp8", 24, 4, [256, 256, 128, 1], "tanh", False, [20, 80]),
+    ("fp8", 128, 1, [128, 128, 1], "tanh", False, [20, 96, 97]),
+    ("fp8", 64, 1, [128] * 4 + [1], "squareplus", True, [20, 130]),
 ])
 def test_tile_rows_agree(tmp_path, prec, k, nelt, layers, act, resnet, copies):
     """Tiles of 16, 32 and 64 rows give the same bits: clusters of 128 centers,
