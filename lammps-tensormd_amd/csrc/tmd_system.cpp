@@ -255,9 +255,10 @@ hipError_t staging_free(hipEvent_t &ev)
   return hipEventSynchronize(ev);
 }
 
-// Atoms staged at a time on the way in or out (page-locked memory stays
-// below 64 MB).
-constexpr int kIoAtoms = 800000;
+// Atoms staged at a time on the way in or out.  They bound the page-locked
+// memory that a system keeps: 24 bytes per atom for positions, 24 for
+// velocities and 80 on the way out, each buffer a quarter larger, 64 MB.
+constexpr int kIoAtoms = 400000;
 // Up to this many atoms the kernel reads the staged positions itself; more
 // are copied to the device first, at the full rate of the copy engine.
 constexpr int kDirectIn = 4096;

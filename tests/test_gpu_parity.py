@@ -1353,3 +1353,34 @@ def test_tile_rows_agree(tmp_path, prec, k, nelt, layers, act, resnet, copies):
             assert np.isfinite(first[0]).all() and np.ptp(first[0]) > 0 and abs(first[1]).max() > 0
         assert np.array_equal(e, np.broadcast_to(first[0], e.shape))
         assert abs(f - first[1]).max() <= 1e-12 * max(1.0, abs(first[1]).max())
+
+
+def test_state_transfers_in_pieces(synth_models):
+    """Positions, velocities and results of a system larger than one piece of
+    a transfer (400,000 atoms): eight periodic copies of a 54,000-atom crystal,
+    set twice with new values.  Positions and velocities come back to the bit;
+    forces and energies of every copy equal those of the crystal alone (FP32
+    evaluations of the same environments)."""
+    x0, t, cell = W.crystal("bcc", 3.2, (30, 30, 30), nelt=4, sigma=0.05, seed=151)
+    rng = np.random.default_rng(152)
+    L = 30 * 3.2
+    shifts = np.array([[a, b, c] for a in (0, 1) for b in (0, 1) for c in (0, 1)]) * L
+    m = TensorMD(synth_models["c2"], ["Mo", "Nb", "Ta", "W"], "fp32", 0.001)
+    base = m.system(x0, t, cell, skin=0.5)
+    s = m.system((x0 + shifts[:, None]).reshape(-1, 3), np.tile(t, 8), 2 * cell, skin=0.5)
+    for _ in range(2):
+        x1 = W.wrap(x0 + rng.normal(scale=0.1, size=x0.shape), cell)
+        x = (x1 + shifts[:, None]).reshape(-1, 3)
+        v = rng.normal(size=x.shape)
+        s.set_positions(x)
+        s.set_velocities(v)
+        r = s.get()
+        assert np.array_equal(r["x"], x) and np.array_equal(r["v"], v)
+        r = s.compute()
+        base.set_positions(x1)
+        ref = base.compute()
+        df = abs(r["f"].reshape(8, -1, 3) - ref["f"]).max()
+        de = abs(r["eatom"].reshape(8, -1) - ref["eatom"]).max()
+        say("case:", len(x), "atoms, max |dF|", df, "max |dE|", de)
+        assert df <= 2 * F_TOL * max(1.0, abs(ref["f"]).max()) and de <= 2e-6 * max(1.0, abs(ref["eatom"]).max())
+        assert np.array_equal(r["v"], v) and abs(r["x"] - x).max() <= np.spacing(2 * L)
