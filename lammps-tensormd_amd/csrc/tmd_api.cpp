@@ -85,6 +85,7 @@ hipError_t PinnedBuffer::ensure(size_t nbytes)
   hipError_t e = hipHostMalloc(&p, want, hipHostMallocDefault);
   if (e != hipSuccess) {
     p = nullptr;
+    (void) hipGetLastError();  // a caller that goes on without must not find it at its next launch
     return e;
   }
   bytes = want;

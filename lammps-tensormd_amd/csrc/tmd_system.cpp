@@ -248,11 +248,14 @@ hipError_t snapshot(tmd_system *s, bool save)
                          s->step_counter(), s->ctx->stream);
 }
 
-// Waits until the last transfer from a staging buffer has left it.
-hipError_t staging_free(hipEvent_t &ev)
+// Waits until the last transfer from a staging buffer has left it, and
+// makes room for the next: *locked is false where no more memory can be
+// page-locked, and the transfer then goes from the caller's own.
+hipError_t take_staging(PinnedBuffer &b, hipEvent_t &ev, size_t bytes, bool *locked)
 {
-  if (!ev) return hipEventCreateWithFlags(&ev, hipEventDisableTiming);  // never used so far
-  return hipEventSynchronize(ev);
+  hipError_t e = ev ? hipEventSynchronize(ev) : hipEventCreateWithFlags(&ev, hipEventDisableTiming);
+  if (e == hipSuccess) *locked = b.ensure(bytes) == hipSuccess;
+  return e;
 }
 
 // Atoms staged at a time on the way in or out.  They bound the page-locked
@@ -433,17 +436,21 @@ int tmd_system_set_positions(tmd_system *s, const double *x)
   for (int first = 0; first < s->n && e == hipSuccess; first += kIoAtoms) {
     const int n = std::min(kIoAtoms, s->n - first);
     const size_t bytes = 3 * sizeof(double) * (size_t) n;
-    if ((e = staging_free(s->ev_x)) != hipSuccess || (e = s->in_x.ensure(bytes)) != hipSuccess) break;
-    const HostCopy cp{s->in_x.p, x + 3 * (size_t) first, bytes};
-    copy_threads(&cp, 1);
-    const double *src = (const double *) s->in_x.p;
-    if (n > kDirectIn) {
+    bool locked = false;
+    if ((e = take_staging(s->in_x, s->ev_x, bytes, &locked)) != hipSuccess) break;
+    const double *src = x + 3 * (size_t) first;
+    if (locked) {
+      const HostCopy cp{s->in_x.p, src, bytes};
+      copy_threads(&cp, 1);
+      src = (const double *) s->in_x.p;
+    }
+    if (n > kDirectIn || !locked) {
       if ((e = s->xin.ensure(bytes)) != hipSuccess) break;
-      if ((e = hipMemcpyAsync(s->xin.p, s->in_x.p, bytes, hipMemcpyHostToDevice, st)) != hipSuccess) break;
+      if ((e = hipMemcpyAsync(s->xin.p, src, bytes, hipMemcpyHostToDevice, st)) != hipSuccess) break;
       src = (const double *) s->xin.p;
     }
     e = launch_set_positions(first, n, src, (double4 *) s->w.pos.p, (unsigned long long *) s->ctl.p, st);
-    if (e == hipSuccess) e = hipEventRecord(s->ev_x, st);
+    if (e == hipSuccess) e = locked ? hipEventRecord(s->ev_x, st) : hipStreamSynchronize(st);
   }
   if (e != hipSuccess) return hip_fail(s->ctx, e, "set positions");
   s->have_forces = false;
@@ -460,12 +467,17 @@ int tmd_system_set_velocities(tmd_system *s, const double *v)
   for (int first = 0; first < s->n && e == hipSuccess; first += kIoAtoms) {
     const int n = std::min(kIoAtoms, s->n - first);
     const size_t bytes = 3 * sizeof(double) * (size_t) n;
-    if ((e = staging_free(s->ev_v)) != hipSuccess || (e = s->in_v.ensure(bytes)) != hipSuccess) break;
-    const HostCopy cp{s->in_v.p, v + 3 * (size_t) first, bytes};
-    copy_threads(&cp, 1);
-    e = hipMemcpyAsync((double *) s->vel.p + 3 * (size_t) first, s->in_v.p, bytes, hipMemcpyHostToDevice,
-                       s->ctx->stream);
-    if (e == hipSuccess) e = hipEventRecord(s->ev_v, s->ctx->stream);
+    bool locked = false;
+    if ((e = take_staging(s->in_v, s->ev_v, bytes, &locked)) != hipSuccess) break;
+    const double *src = v + 3 * (size_t) first;
+    if (locked) {
+      const HostCopy cp{s->in_v.p, src, bytes};
+      copy_threads(&cp, 1);
+      src = (const double *) s->in_v.p;
+    }
+    e = hipMemcpyAsync((double *) s->vel.p + 3 * (size_t) first, src, bytes, hipMemcpyHostToDevice, s->ctx->stream);
+    if (e == hipSuccess)
+      e = locked ? hipEventRecord(s->ev_v, s->ctx->stream) : hipStreamSynchronize(s->ctx->stream);
   }
   if (e != hipSuccess) return hip_fail(s->ctx, e, "set velocities");
   return TMD_OK;
@@ -503,37 +515,60 @@ int tmd_system_get(tmd_system *s, double *x, double *v, double *f, double *eatom
   const int per = (x ? 3 : 0) + (v ? 3 : 0) + (f ? 3 : 0) + (eatom ? 1 : 0);
   double red[8];
   const int chunk = std::min(s->n, kIoAtoms);
-  // the sums ride in front of the first chunk
-  if ((e = s->out.ensure(sizeof(double) * (8 + (size_t) per * chunk))) != hipSuccess)
-    return hip_fail(s->ctx, e, "tmd_system_get");
-  double *sums = (double *) s->out.p, *data = sums + 8;
   StateOut o{};
   if (x) o.pos = (const double4 *) s->w.pos.p;
-  if (v) o.v = (const double *) s->vel.p;
-  if (f) o.f = (const double *) s->w.f.p;
-  if (eatom) o.eatom = (const double *) s->w.ew.p;
-  o.out = data;
-  if (energy || virial) e = launch_copy_small((const double *) s->w.red.p, sums, 7, st);
-  for (int first = 0; first == 0 || first < s->n; first += chunk) {
-    const int n = std::min(chunk, s->n - first);
-    if (e == hipSuccess) e = launch_pack_state(first, n, o, st);
-    if (e == hipSuccess) e = hipStreamSynchronize(st);
+  if (s->out.ensure(sizeof(double) * (8 + (size_t) per * chunk)) != hipSuccess) {
+    // no more memory can be page-locked: copies into the caller's arrays
+    for (int first = 0; first < s->n && e == hipSuccess; first += chunk) {
+      const size_t n = (size_t) std::min(chunk, s->n - first), at = (size_t) first;
+      auto down = [&](double *dst, const void *src, size_t w) {
+        if (dst && e == hipSuccess)
+          e = hipMemcpyAsync(dst + w * at, src, sizeof(double) * w * n, hipMemcpyDeviceToHost, st);
+      };
+      if (x && (e = s->xin.ensure(3 * sizeof(double) * n)) == hipSuccess) {
+        o.out = (double *) s->xin.p;
+        e = launch_pack_state(first, (int) n, o, st);
+        down(x, o.out, 3);
+      }
+      down(v, (const double *) s->vel.p + 3 * at, 3);
+      down(f, (const double *) s->w.f.p + 3 * at, 3);
+      down(eatom, (const double *) s->w.ew.p + at, 1);
+      if (e == hipSuccess) e = hipStreamSynchronize(st);
+    }
+    if (e == hipSuccess && (energy || virial)) {
+      e = hipMemcpyAsync(red, s->w.red.p, 7 * sizeof(double), hipMemcpyDeviceToHost, st);
+      if (e == hipSuccess) e = hipStreamSynchronize(st);
+    }
     if (e != hipSuccess) return hip_fail(s->ctx, e, "tmd_system_get");
-    const double *src = data;
-    HostCopy cp[4];
-    int nc = 0;
-    auto take = [&](double *dst, int w) {
-      if (!dst) return;
-      cp[nc++] = {dst + (size_t) w * first, src, sizeof(double) * (size_t) w * n};
-      src += (size_t) w * n;
-    };
-    take(x, 3);
-    take(v, 3);
-    take(f, 3);
-    take(eatom, 1);
-    copy_threads(cp, nc);
+  } else {
+    // the sums ride in front of the first chunk
+    double *sums = (double *) s->out.p, *data = sums + 8;
+    if (v) o.v = (const double *) s->vel.p;
+    if (f) o.f = (const double *) s->w.f.p;
+    if (eatom) o.eatom = (const double *) s->w.ew.p;
+    o.out = data;
+    if (energy || virial) e = launch_copy_small((const double *) s->w.red.p, sums, 7, st);
+    for (int first = 0; first == 0 || first < s->n; first += chunk) {
+      const int n = std::min(chunk, s->n - first);
+      if (e == hipSuccess) e = launch_pack_state(first, n, o, st);
+      if (e == hipSuccess) e = hipStreamSynchronize(st);
+      if (e != hipSuccess) return hip_fail(s->ctx, e, "tmd_system_get");
+      const double *src = data;
+      HostCopy cp[4];
+      int nc = 0;
+      auto take = [&](double *dst, int w) {
+        if (!dst) return;
+        cp[nc++] = {dst + (size_t) w * first, src, sizeof(double) * (size_t) w * n};
+        src += (size_t) w * n;
+      };
+      take(x, 3);
+      take(v, 3);
+      take(f, 3);
+      take(eatom, 1);
+      copy_threads(cp, nc);
+    }
+    std::memcpy(red, sums, sizeof(red));
   }
-  std::memcpy(red, sums, sizeof(red));
   if (energy) *energy = red[0];
   if (virial)
     for (int q = 0; q < 6; q++) virial[q] = red[1 + q];

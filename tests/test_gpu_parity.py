@@ -4,13 +4,16 @@ Tolerances (FP32 path vs FP64 oracle): max-abs force error <= 1e-5 eV/A,
 energy error <= 1e-7 eV/atom.  BF16 MLP path: max-abs force error
 <= 5e-3 eV/A.  Integer work (the neighbor set) is compared bit-exactly.
 """
+import os
+import shutil
+import subprocess
 import sys
 
 import numpy as np
 import pytest
 
 import oracle
-from conftest import model_path
+from conftest import ROOT, model_path
 from tensormd_amd import TensorMD, workloads as W
 
 pytestmark = pytest.mark.gpu
@@ -1384,3 +1387,81 @@ def test_state_transfers_in_pieces(synth_models):
         say("case:", len(x), "atoms, max |dF|", df, "max |dE|", de)
         assert df <= 2 * F_TOL * max(1.0, abs(ref["f"]).max()) and de <= 2e-6 * max(1.0, abs(ref["eatom"]).max())
         assert np.array_equal(r["v"], v) and abs(r["x"] - x).max() <= np.spacing(2 * L)
+
+
+_REFUSE = """
+#include <dlfcn.h>
+#include <cstddef>
+// refuses to page-lock more than 64 KB: asks the runtime for a petabyte, so
+// that its own last error is set as well
+static int refused = 0;
+extern "C" int refusals() { return refused; }
+extern "C" int hipHostMalloc(void **p, size_t n, unsigned flags)
+{
+  using F = int (*)(void **, size_t, unsigned);
+  static F real = (F) dlsym(RTLD_NEXT, "hipHostMalloc");
+  if (n > 65536) {
+    refused++;
+    return real(p, (size_t) 1 << 50, flags);
+  }
+  return real(p, n, flags);
+}
+"""
+
+_REFUSED_RUN = """
+import ctypes, sys
+refuse = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+sys.path.insert(0, sys.argv[2])
+import numpy as np
+from tensormd_amd import TensorMD
+z = np.load(sys.argv[3])
+s = TensorMD(sys.argv[4], ["Mo", "Nb", "Ta", "W"], "fp32", 0.001).system(z["x0"], z["t"], z["cell"], skin=1.0)
+s.set_positions(z["x"])
+s.set_velocities(z["v"])
+a = s.get()
+r = s.compute()
+ep, ek = s.md_run(2, 0.001)
+e = s.get()
+np.savez(sys.argv[5], n=refuse.refusals(), xa=a["x"], va=a["v"], ep=ep, ek=ek, xe=e["x"], ve=e["v"], fe=e["f"],
+         **{k: r[k] for k in ("x", "v", "f", "eatom", "energy", "virial")})
+print("done", flush=True)
+"""
+
+
+@pytest.mark.parametrize("cells", [(12, 12, 12), (24, 24, 24)])
+def test_transfers_without_page_locked_memory(synth_models, tmp_path, cells):
+    """Where the runtime page-locks no more memory, positions, velocities and
+    results cross through the caller's own arrays: in a process whose large
+    page-locked allocations are refused, on both sides of the direct-read line
+    (4,096 atoms), the same values as here."""
+    if shutil.which("g++") is None:
+        pytest.skip("no g++")
+    src, so = tmp_path / "refuse.cpp", tmp_path / "refuse.so"
+    src.write_text(_REFUSE)
+    subprocess.run(["g++", "-O1", "-shared", "-fPIC", str(src), "-o", str(so), "-L/opt/rocm/lib",
+                    "-Wl,--no-as-needed", "-lamdhip64", "-ldl"], check=True)
+    x0, t, cell = W.crystal("bcc", 3.2, cells, nelt=4, sigma=0.05, seed=161)
+    rng = np.random.default_rng(162)
+    x = W.wrap(x0 + rng.normal(scale=0.1, size=x0.shape), cell)
+    v = W.maxwell_boltzmann(np.array([95.95, 92.906, 180.95, 183.84])[t - 1], 300.0, seed=163)
+    np.savez(tmp_path / "in.npz", x0=x0, t=t, cell=cell, x=x, v=v)
+    (tmp_path / "run.py").write_text(_REFUSED_RUN)
+    say("case:", len(x), "atoms, page-locked memory refused")
+    subprocess.run([sys.executable, str(tmp_path / "run.py"), str(so), os.path.join(ROOT, "lammps-tensormd_amd"),
+                    str(tmp_path / "in.npz"), synth_models["c2"], str(tmp_path / "out.npz")], check=True, timeout=100)
+    got = np.load(tmp_path / "out.npz")
+    assert got["n"] >= 2  # velocities, results (and positions)
+    assert np.array_equal(got["xa"], x) and np.array_equal(got["va"], v)
+    s = TensorMD(synth_models["c2"], ["Mo", "Nb", "Ta", "W"], "fp32", 0.001).system(x0, t, cell, skin=1.0)
+    s.set_positions(x)
+    s.set_velocities(v)
+    r = s.compute()
+    ep, ek = s.md_run(2, 0.001)
+    e = s.get()
+    # the same kernels on the same values: FP64 sums of forces in any order
+    for k in ("x", "v", "eatom", "energy"):
+        assert np.array_equal(got[k], r[k]), k
+    assert abs(got["f"] - r["f"]).max() <= 1e-10 and abs(got["virial"] - r["virial"]).max() <= 1e-8
+    for k, w in (("xe", e["x"]), ("ve", e["v"]), ("fe", e["f"])):
+        assert abs(got[k] - w).max() <= 1e-5, k
+    assert abs(got["ep"] - ep).max() <= 1e-6 * abs(ep).max() and abs(got["ek"] - ek).max() <= 1e-9 * ek.max()
