@@ -19,6 +19,7 @@
 #include <functional>
 #include <mutex>
 #include <string>
+#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -153,8 +154,14 @@ class HostPool {
  private:
   HostPool()
   {
-    nworkers = (int) std::min<unsigned>(15u, std::max(1u, std::thread::hardware_concurrency()) - 1);
-    for (int i = 0; i < nworkers; i++) workers.emplace_back([this] { loop(); });
+    const int want = (int) std::min<unsigned>(15u, std::max(1u, std::thread::hardware_concurrency()) - 1);
+    workers.reserve(want);
+    try {
+      for (int i = 0; i < want; i++) workers.emplace_back([this] { loop(); });
+    } catch (const std::system_error &) {
+      // the process may start no more threads: those there are do the work
+    }
+    nworkers = (int) workers.size();
   }
   // takes jobs of the current run until none is left
   void work()
