@@ -293,17 +293,34 @@ hipError_t desc_wide(const ModelGeo &g, const Geom &geo, const double4 *pos, con
 // Waves per atom (K <= 32).  Several shorten a wave's chain but add barriers
 // and, in the lane-per-neighbor parts, idle lanes, so they pay while a CU has
 // few atoms.  (The descriptor's two-wave form won 1 us in a narrow band and
-// is not built.)  us, descriptor / force, 1, 2 and 4 waves per atom:
-//   rows, elements, K      1              2              4
-//     256, 4, 24     10.8 / 15.3     9.2 / 12.9     8.5 / 12.0
-//     512, 4, 24     11.1 / 16.4     9.9 / 13.6     9.2 / 12.4
-//   1,024, 4, 24     11.4 / 16.7    10.3 / 14.5    12.9 / 17.6
-//   2,048, 4, 24     13.7 / 22.2    16.7 / 23.1    18.9 / 25.5
-//     256, 1, 16     10.1 / 14.1       - / 12.6     7.6 / 12.2
-//   2,048, 1, 16     12.6 / 20.6       - / 18.2    12.6 / 21.8
-//   4,000, 1, 16     15.9 / 26.6       - / 27.7    18.9 / 32.5
-//   2,048, 2, 32     12.7 / 23.0    13.9 / 22.0    15.0 / 23.9
-constexpr int kWide4Rows = 640, kWide2Rows = 1280;
+// is not built.)  us, descriptor with 1 and 4 waves, force with 1, 2 and 4:
+//   elements, K   rows   descriptor        force
+//     1, 16        512   10.2   7.9   14.7  13.5  12.8
+//                1,408   11.7  11.0   17.1  16.3  18.6
+//                2,048   12.1  12.4   20.0  18.1  21.7
+//                2,944   13.6  15.3   23.9  25.5  27.1
+//     1, 24      1,024    9.7   9.0   15.4  13.6  13.5
+//                2,048   11.1  12.9   20.4  20.7  20.9
+//     1, 32        704    9.7   8.5   15.8  13.4  12.6
+//                2,048   11.4  13.4   22.5  20.7  23.8
+//                3,456   14.5  19.3   28.4  28.5  33.3
+//     2, 32        512   10.0   8.4   15.9  13.7  11.9
+//                1,408   11.4  12.4   19.8  16.7  18.5
+//                2,944   14.1  18.8   26.3  25.3  29.2
+//     3, 16        576    9.6   8.4   14.4  13.0  12.2
+//                1,536   10.9  12.6   19.3  18.1  18.8
+//                2,688   12.4  17.7   21.8  23.8  24.5
+//     4, 24        512   10.7   9.2   15.9  13.7  12.4
+//                  768   10.8   9.8   16.1  13.9  12.9
+//                1,024   11.1  13.0   16.4  14.6  17.8
+//                1,536   12.2  14.9   21.6  18.4  20.9
+//                2,048   12.7  18.8   21.5  23.3  25.9
+//     5, 24        640                 16.6  14.2  12.8
+//                1,600                 22.8  20.1  21.9
+//                2,240                 23.4  25.8  28.4
+//     8, 32        512                 20.9  15.3  13.2
+//                2,048                 30.8  28.4  28.7
+constexpr int kWide4Rows = 640, kWide2Rows = 1600;
 
 int force_waves(const ModelGeo &g, int rows)
 {
