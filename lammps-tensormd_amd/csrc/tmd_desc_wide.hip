@@ -40,7 +40,7 @@ __global__ __launch_bounds__(64 * kDescWaves) void k_descriptor_wide(ModelGeo g,
   using T = Tiling<K>;
   extern __shared__ __align__(16) unsigned char smem[];
   const int row = geo.order ? geo.order[rbase + (int) blockIdx.x] : rbase + (int) blockIdx.x;
-  if (row >= nrows || (geo.dyn && row >= geo.dyn->rl.nrows)) return;
+  if (row >= nrows) return;
   float *Grow;
   const int i = descriptor_begin(g, geo, K, row, row2atom, G, Grow);
   if (i < 0) return;
@@ -140,7 +140,7 @@ __global__ __launch_bounds__(64 * W, (K <= 16 ? 4 : 3)) void k_force_wide(ModelG
   __shared__ __align__(16) f32x4v part[SHARE > 1 ? W : 1][T::KT][64];
   __shared__ double facc[2][9];
   const int row = geo.order ? geo.order[rbase + (int) blockIdx.x] : rbase + (int) blockIdx.x;
-  if (row >= nrows || (geo.dyn && row >= geo.dyn->rl.nrows)) return;
+  if (row >= nrows) return;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int i = row2atom[row];
   if (i < 0) return;  // padding row
@@ -340,7 +340,7 @@ hipError_t launch_descriptor_wide(const ModelGeo &g, const Geom &geo, const doub
                                   const int *nn, int cap, const int *row2atom, int nrows, const float4 *tab, float *G,
                                   uint32_t *kl, hipStream_t s, int row_begin)
 {
-  if (!desc_wide_ok(g, nrows - row_begin) || g.nelt < 1 || g.nelt > kMaxElts) return hipErrorInvalidValue;
+  if (geo.dyn || !desc_wide_ok(g, nrows - row_begin) || g.nelt < 1 || g.nelt > kMaxElts) return hipErrorInvalidValue;
 #define TMD_NS(K, NS) \
   case NS:            \
     return desc_wide<K, NS>(g, geo, pos, nbr, nn, cap, row2atom, row_begin, nrows, tab, G, kl, s);
@@ -369,7 +369,7 @@ hipError_t launch_force_wide(const ModelGeo &g, const Geom &geo, const double4 *
                              int row_begin)
 {
   const int w = force_waves(g, nrows - row_begin);
-  if (w <= 1) return hipErrorInvalidValue;
+  if (geo.dyn || w <= 1) return hipErrorInvalidValue;
 #define TMD_K_CASE(K)                                                                                               \
   case K:                                                                                                           \
     return w == 4 ? force_wide<K, 4>(g, geo, pos, cap, row2atom, row_begin, nrows, tab, kl, dEdG, E, scale, f,      \

@@ -289,7 +289,6 @@ int enqueue_batch(Server *S, Slot &sl, const Bucket &b, int rtile)
   c.f = (double *) sl.w.f.p;
   c.fbytes = 24 * (size_t) b.caps.atoms;
   c.f_cleared = true;  // by the unpack kernel
-  c.nb = &nb;
   c.natoms = S->full.atoms;  // eatom/watom layout of the slot
   c.no_sums = true;  // with the results' copy
   c.rtile = rtile;
