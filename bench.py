@@ -466,11 +466,13 @@ def main():
             row = dict(kernel=f"k_mlp_fast {prec} (fused per-element MLP fwd+bwd on "
                               f"{unit.get(prec, 'FP32')} MFMA)", bound="mfma")
         else:
-            # fused FP32 gather/scatter kernels without MFMA: arithmetic
-            # intensity 50-80 FLOP/B, so the binding roof is FP32 vector
-            # issue (VALU), not HBM
+            # fused FP32 gather/scatter kernels, contractions on FP32 MFMA:
+            # arithmetic intensity 50-80 FLOP/B, so the binding roof is the
+            # issue of vector and matrix instructions, which do not overlap on
+            # a SIMD, not HBM; both units have the same FP32 peak
             peak = PEAK["fp32_tflops"]
-            row = dict(kernel=f"k_{kname} (fused FP32 {kname} kernel, VALU)", bound="valu",
+            row = dict(kernel=f"k_{kname} (fused FP32 {kname} kernel, contractions on MFMA, the rest on "
+                              f"the VALU)", bound="mfma+valu",
                        valu_peak_without_packed_fp32=PEAK["fp32_tflops"] / 2)
         row.update(precision=prec, achieved=flops, peak=peak, unit="TFLOP/s", frac=flops / peak,
                    hbm_achieved_gbs=gbs, hbm_peak_gbs=PEAK["hbm_gbs"], hbm_frac=gbs / PEAK["hbm_gbs"],

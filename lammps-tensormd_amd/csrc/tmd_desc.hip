@@ -33,10 +33,12 @@
 //
 // What bounds the kernels (128,000 atoms, 4 elements, 24 filters, 63
 // neighbors): vector and matrix instructions, which do not overlap on a SIMD
-// here, fill about 95 % of the force kernel's time (0.38 + 0.19 of 0.61 ms;
-// 0.42 ms with neither matrix instructions nor atomics) and 90 % of the
-// descriptor's 0.30 ms.  With the monomials on the vector ALU they took 0.95
-// and 0.42 ms.
+// here, fill about 95 % of the force kernel's time (0.38 + 0.19 of 0.61 ms,
+// single evaluations of the lattice; 0.42 ms with neither matrix instructions
+// nor atomics) and 90 % of the descriptor's 0.30 ms.  With the monomials on
+// the vector ALU they took 0.95 and 0.42 ms.  Along MD runs, which heat up, the
+// force kernel's mean is 0.59 ms over 300 steps and 0.63 over 1,000 (69
+// neighbors).
 //
 // Nothing per neighbor is stored in HBM: the reference materialises R, M,
 // H, dH/dr, P, dE/dS, V, F1, F2 per padded slot (kernel.cu:1545-1582).
@@ -60,7 +62,11 @@ __global__ __launch_bounds__(64) void k_descriptor(ModelGeo g, Geom geo, const d
   if (i >= 0) descriptor_row<K, NS, MP>(g, geo, row, i, pos, nbr, nn, cap, tab, Grow, kl, smem);
 }
 
-// Waves per SIMD asked of the force kernel: what its LDS leaves room for
+// Waves per SIMD asked of the force kernel: what its LDS leaves room for.
+// K = 32 spills 11 registers for it, and is still faster than at three waves
+// or with one tile per slot in registers instead of two (Tiling::RT), neither
+// of which spills (us, 1-2 elements, 62,500 atoms 250, 259 and 297; 65,536
+// atoms 292, 304 and 288; eight elements, 65,536 atoms 532, 502 and 450).
 template <int K>
 constexpr int kForceWaves = K <= 32 ? 4 : (K == 64 ? 3 : 2);
 

@@ -37,7 +37,9 @@ struct Tiling {
   static constexpr int SBUF = K * SS;
   static constexpr int BUF = kSRegs ? (DBUF > SBUF ? DBUF : SBUF) : DBUF + SBUF;
   // staged neighbors of the force kernel: what leaves 16 waves per CU
-  // (10 KB each) up to K = 32
+  // (10 KB each) up to K = 32; above, one per lane (a CU holds 11 and 8 waves
+  // of K = 64 and 128).  A longer list goes slot by slot, at no step in time:
+  // K = 64, 35,152 atoms, 291 us with 56 neighbors and 296 with 75.
   static constexpr int WIN = K == 16 ? 96 : (K == 24 ? 84 : (K == 32 ? 72 : 64));
   // tiles of a slot whose H and dH stay in registers between P and the
   // chain rule (2 NFB registers each)
